@@ -257,10 +257,7 @@ int mpid_energy_gradients(mpid_context* ctx, const double* positions, const doub
 int mpid_get_stats(const mpid_context* ctx, mpid_stats* stats);
 /* Profiling (no counterpart in the reference): mpid_set_profiling times every
  * family (enable != 0) or none; mpid_set_profile_mask times the families
- * whose bit (1 << MPID_PROF_x) is set.  When a family issued inside a solver
- * iteration is timed (spread, FFT, gather, induced pairs, covalent pairs,
- * solver), the iterations run as individual launches; otherwise they are
- * replayed from a captured graph, as without profiling. */
+ * whose bit (1 << MPID_PROF_x) is set. */
 int mpid_set_profiling(mpid_context* ctx, int enable);
 int mpid_set_profile_mask(mpid_context* ctx, unsigned mask);
 /* times_ms[MPID_PROF_COUNT], counts[MPID_PROF_COUNT] (launches); resets them when reset != 0 */

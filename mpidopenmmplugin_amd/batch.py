@@ -9,7 +9,7 @@ small system fills a few dozen of the 256 CUs and its solver is bound by
 kernel-launch latency, so one system after another leaves the chip idle.
 
 ``BatchEvaluator`` keeps one ``HipCalcMPIDForceKernel`` (its own three
-streams, lists, grids and solver graph) per system and drives them from a
+streams, lists and grids) per system and drives them from a
 pool of host threads: the C ABI releases the GIL for the whole evaluation,
 so the launches of several systems are in flight at once and their kernels
 share the chip.  Each context issues its work on a single HIP stream: the

@@ -107,7 +107,7 @@ template <class R> struct PairParams {
     R scale14;
     int mutual;        // 1 when the induced-induced terms enter the forces
     int fix_torque;    // 1: energy-conserving induced-induced torques (MPID_FLAG_CONSERVATIVE_TORQUES)
-    const double* skip;  // the solver's stop flag in the induced-field kernels of a solver iteration, else null
+    const double* skip;  // the solver's stop flag in the field kernels of a solver iteration, else null
 };
 
 // Precision-specific per-atom inputs of the pair kernels (sorted order).
@@ -151,7 +151,7 @@ void launch_torque_to_force(hipStream_t s, int n, Box<double> box, const double4
                             const acc_t* torque, acc_t* force, int exact_threefold);
 void launch_output_forces(hipStream_t s, int n, const int* perm, const acc_t* force, double* out, int accumulate);
 void launch_unpermute3(hipStream_t s, int n, const int* perm, const double* in, double* out);
-void launch_zero_acc(hipStream_t s, acc_t* p, size_t count, const double* skip = nullptr);
+void launch_zero_acc(hipStream_t s, acc_t* p, size_t count);
 size_t sort_temp_bytes(int n);
 int launch_sort_pairs(hipStream_t s, void* temp, size_t bytes, unsigned* kin, unsigned* kout, int* vin, int* vout, int n);
 // out = acc + erecip + selfc * mu (field of the induced dipoles, double)
@@ -163,15 +163,7 @@ template <class R> void launch_fill(hipStream_t s, R* p, size_t count, R v);
 template <class R>
 void launch_fixed_field_finish(hipStream_t s, int n, const R* phi, const double* lab, const acc_t* acc,
                                FracT<double> A, double selfc, double* E0);
-// mu0 = alpha_lab E0 ; y0 = S E0 ; b = S E0
-void launch_solver_init(hipStream_t s, int n, const double* sqrtpol, const double* E0, double* b, double* y);
-// mu = S y (double and precision copies)
-template <class R> void launch_apply_S(hipStream_t s, int n, const double* sqrtpol, const double* y, R* mu, double* mud);
-// Ap = p - S (acc + Erecip + selfc mu)
-template <class R>
-void launch_matvec_finish(hipStream_t s, int n, const double* sqrtpol, const acc_t* acc, const R* erecip,
-                          const R* mu, double selfc, const double* p, double* Ap);
-// deterministic FP64 reductions
+// deterministic FP64 reduction
 void launch_dot(hipStream_t s, int m, const double* a, const double* b, double* partial, double* result);
 // Getters after an evaluation (sorted-order state).  Potential at npts points
 // of the charges, dipoles plus induced dipoles and quadrupoles (FP64).
@@ -214,28 +206,9 @@ void launch_extrap_combine(hipStream_t s, int n, const ExtrapCoefficients& cp, c
 // the dipole-response forces and torques into the fixed-point accumulators
 void launch_extrap_response(hipStream_t s, int n, const ExtrapCoefficients& cp, const double* mus, const double* Es,
                             const double* Gs, const int* aniso, acc_t* force, acc_t* torque);
-// The solver's device-side state in scal: [0] rr, [1] pAp, [2] rr_new,
-// [3] |S r|^2, [7] beta, [kCgCount] iterations done, [kCgStop] 1 once the
-// stopping test has passed.  Kernels of an iteration given the stop flag
-// return at once when it is set, so that the host may issue an iteration
-// before it has read the previous one's check.
-constexpr int kCgCount = 9;
-constexpr int kCgStop = 10;
-constexpr int kScalars = 16;
-// Check 0 of a solve: the stopping test on the initial |S r|^2 (scal[3]),
-// published to scal and to hcheck (pinned, mapped host memory, two slots of
-// (|S r|^2, stop); check c goes to slot c & 1).
-void launch_cg_begin(hipStream_t s, int n, double* scal, double* hcheck, double stop_eps);
-// One CG iteration once the operator's field for mu = S p is complete (acc,
-// erec): Ap, a = rr / pAp, x += a p, r -= a Ap, the norms rr and |S r|^2,
-// beta, the iteration's check, p = r + beta p and the next operator input
-// mu = S p.
+// mu0 = alpha_lab E0 at every atom, in both precisions (Extrapolated)
 template <class R>
-void launch_cg_iteration(hipStream_t s, int n, const double* sqrtpol, const acc_t* acc, const R* erec, R* mu,
-                         double selfc, double* p, double* Ap, double* x, double* r, double* partial, double* scal,
-                         double* hcheck, double stop_eps);
-void launch_residual_norm(hipStream_t s, int n, const double* sqrtpol, const double* r, double* partial,
-                          double* result);
+void launch_extrap_init(hipStream_t s, int n, const double* labpol, const double* E0, double* mu, R* mu_r);
 void launch_axpy(hipStream_t s, int m, double a, const double* x, double* y);
 void launch_sub(hipStream_t s, int m, const double* a, const double* b, double* out);
 // reciprocal-space energy, forces and torques, self terms (per atom)
@@ -284,7 +257,8 @@ void launch_spread_induced_owner(hipStream_t s, const R4<R>* pos, const R* mu, P
 template <class R>
 void launch_spread_fixed(hipStream_t s, int n, const R4<R>* pos, const R* lab, PmeGeom<R> g, R* grid);
 template <class R>
-void launch_spread_induced(hipStream_t s, int n, const R4<R>* pos, const R* mu, PmeGeom<R> g, R* grid);
+void launch_spread_induced(hipStream_t s, int natoms, const int* atoms, const R4<R>* pos, const R* mu, PmeGeom<R> g,
+                           R* grid);
 template <class R>
 void launch_gather_phi(hipStream_t s, int n, const R4<R>* pos, PmeGeom<R> g, const R* grid, R* phi);
 template <class R>
@@ -335,10 +309,11 @@ template <class R> void launch_influence_table(hipStream_t s, InflParams ip, con
 // of its lower neighbours (launch_fold handles any tiling)
 bool fold_by_tiles(const TileGeom& tg);
 template <class R> void launch_fold_tiles(hipStream_t s, PmeGeom<R> g, TileGeom tg, const R* scratch, R* grid);
-// Q (real grid) -> S (half spectrum) -> convolution -> Q (potential grid)
-// (every pass returns at once when cp.skip is set)
+// Q (charge grid) -> S (half spectrum) -> convolution -> V (potential grid).
+// V == Q works in place; with a V of its own, Q is left zero for the next
+// spreading.  (Every pass returns at once when cp.skip is set.)
 template <class R>
-void launch_recip_convolution(hipStream_t s, const FftPlan<R>& p, R* Q, R2<R>* S, ConvParams<R> cp);
+void launch_recip_convolution(hipStream_t s, const FftPlan<R>& p, R* Q, R2<R>* S, R* V, ConvParams<R> cp);
 
 // ---- real space (kernels_pairs.hip) -------------------------------------------
 template <class R>
@@ -400,6 +375,58 @@ void launch_cov_induced_field(hipStream_t s, int n, PairAtoms<R> a, const R* mu,
 template <class R>
 void launch_cov_electrostatics(hipStream_t s, int n, PairAtoms<R> a, const R* mu, PairParams<R> p, acc_t* force,
                                acc_t* torque, acc_t* energy, acc_t* pot = nullptr);
+
+// ---- mutual-polarization solver (kernels_solver.hip) -----------------------------
+// Its vectors hold the polarisable sites only (entry t: atom idx[t]); S by atom.
+struct SolverSites {
+    int npol;
+    const int* idx;
+    const double* S;  // alpha^(1/2), 6 per atom
+};
+// The solver's device-side state in scal: |r|^2 after c iterations in
+// [c & 1], [kCgCount] iterations done, [kCgStop] 1 once the stopping test has
+// passed, [kCgCur] the iteration in flight.  Kernels of an iteration given
+// the stop flag return at once when it is set, so that the host may issue an
+// iteration before it has read the previous one's check.
+constexpr int kCgCount = 9;
+constexpr int kCgStop = 10;
+constexpr int kCgCur = 11;
+constexpr int kScalars = 16;
+constexpr int kMaxPartials = 1024;  // workgroups of a reducing kernel, at most
+constexpr int kOneSites = 2048;     // sites whose update fits one workgroup
+// real-space field of mu at the polarisable sites (lists and covalent partners)
+template <class R>
+void launch_list_field(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p, const R* mu,
+                       R* field);
+// Av = v - S (E_rec + E_real + selfc mu), mu = S v in place; pot: the potential
+// grid (null: none).  field: launch_list_field's, or null to add the
+// real-space field in the same kernel.  Returns the number of partial sums of
+// v.Av left in partial (if given).
+template <class R>
+int launch_operator(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const R* field, NbrList l,
+                    PairAtoms<R> a, PairParams<R> p, const R* mu, double selfc, const double* v, double* Av,
+                    double* partial);
+// Check 0 of a solve: r = rhs - Ax (Ax null: x = 0), p = r, mu = S p; the
+// stopping test on |S r|^2, published to scal and to hcheck (pinned, mapped
+// host memory, two slots of (|S r|^2, stop); check c goes to slot c & 1).
+template <class R>
+void launch_cg_start(hipStream_t s, SolverSites st, const double* rhs, const double* Ax, double* x, double* r,
+                     double* p, R* mu, double* partial, double* scal, double* hcheck, int n, double stop_eps);
+// The rest of an iteration after launch_operator left A p and npap partials
+// of p.Ap: x += a p, r -= a Ap, the check, p = r + beta p and mu = S p.
+template <class R>
+void launch_cg_iteration(hipStream_t s, SolverSites st, const double* Ap, double* x, double* r, double* p, R* mu,
+                         int npap, double* partial, double* scal, double* hcheck, int n, double stop_eps);
+// b = x = S E0 and mu = S x (zero at the other atoms of mu, mu2, mud)
+template <class R>
+void launch_solver_init(hipStream_t s, SolverSites st, int n, const double4* pos, const double* E0, double* b,
+                        double* x, R* mu, double* mu2, double* mud);
+// S v: by atom in mu and mud, by site in at (each may be null)
+template <class R>
+void launch_apply_S(hipStream_t s, SolverSites st, const double* v, R* mu, double* mud, double* at);
+// rt = b - Ax (Ax null: rt as it is); out[0] = |S rt|^2, out[1] = x.rt (mapped host memory)
+void launch_residual(hipStream_t s, SolverSites st, const double* b, const double* Ax, const double* x, double* rt,
+                     double* partial, double* out);
 
 // ---- energy gradients ------------------------------------------------------------
 // The final pass of the gradients: launch_electrostatics_pairs plus the

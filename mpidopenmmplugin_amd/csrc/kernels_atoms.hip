@@ -263,47 +263,6 @@ __global__ void k_fixed_field_finish(int n, const R* __restrict__ phi, const dou
     E0[3 * (size_t)s + 2] = -c1.z + selfc * m[3] + acc_get(acc[3 * (size_t)s + 2]);
 }
 
-__global__ void k_solver_init(int n, const double* __restrict__ S, const double* __restrict__ E0, double* b,
-                              double* y) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    D3 v = sym_mul(S + 6 * (size_t)s, mk(E0[3 * (size_t)s], E0[3 * (size_t)s + 1], E0[3 * (size_t)s + 2]));
-    b[3 * (size_t)s] = y[3 * (size_t)s] = v.x;
-    b[3 * (size_t)s + 1] = y[3 * (size_t)s + 1] = v.y;
-    b[3 * (size_t)s + 2] = y[3 * (size_t)s + 2] = v.z;
-}
-
-template <class R>
-__global__ void k_apply_S(int n, const double* __restrict__ S, const double* __restrict__ y, R* mu, double* mud) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    D3 v = sym_mul(S + 6 * (size_t)s, mk(y[3 * (size_t)s], y[3 * (size_t)s + 1], y[3 * (size_t)s + 2]));
-    mu[3 * (size_t)s] = (R)v.x;
-    mu[3 * (size_t)s + 1] = (R)v.y;
-    mu[3 * (size_t)s + 2] = (R)v.z;
-    if (mud) {
-        mud[3 * (size_t)s] = v.x;
-        mud[3 * (size_t)s + 1] = v.y;
-        mud[3 * (size_t)s + 2] = v.z;
-    }
-}
-
-template <class R>
-__global__ void k_matvec_finish(int n, const double* __restrict__ S, const acc_t* __restrict__ acc,
-                                const R* __restrict__ erec, const R* __restrict__ mu, double selfc,
-                                const double* __restrict__ p, double* Ap) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    D3 E;
-    E.x = acc_get(acc[3 * (size_t)s]) + (double)erec[3 * (size_t)s] + selfc * (double)mu[3 * (size_t)s];
-    E.y = acc_get(acc[3 * (size_t)s + 1]) + (double)erec[3 * (size_t)s + 1] + selfc * (double)mu[3 * (size_t)s + 1];
-    E.z = acc_get(acc[3 * (size_t)s + 2]) + (double)erec[3 * (size_t)s + 2] + selfc * (double)mu[3 * (size_t)s + 2];
-    D3 v = sym_mul(S + 6 * (size_t)s, E);
-    Ap[3 * (size_t)s] = p[3 * (size_t)s] - v.x;
-    Ap[3 * (size_t)s + 1] = p[3 * (size_t)s + 1] - v.y;
-    Ap[3 * (size_t)s + 2] = p[3 * (size_t)s + 2] - v.z;
-}
-
 // Deterministic block reductions: 256 threads, fixed tree order.
 constexpr int kRedThreads = 256;
 constexpr int kRedBlocks = 512;
@@ -331,8 +290,7 @@ __global__ __launch_bounds__(kRedThreads) void k_dot_partial(int m, const double
 
 // Sums kRedBlocks partials per output slot; nout outputs stored back to back.
 __global__ __launch_bounds__(kRedThreads) void k_reduce_partials(const double* __restrict__ partial, int nout,
-                                                                 double* result, const double* skip) {
-    if (skipped(skip)) return;
+                                                                 double* result) {
     __shared__ double sh[kRedThreads];
     for (int o = 0; o < nout; o++) {
         double v = 0;
@@ -340,159 +298,6 @@ __global__ __launch_bounds__(kRedThreads) void k_reduce_partials(const double* _
         v = block_sum(v, sh);
         if (threadIdx.x == 0) result[o] = v;
     }
-}
-
-// x += a p, r -= a Ap with a = rr / pAp; partial sums of r.r and |S r|^2
-__global__ __launch_bounds__(kRedThreads) void k_cg_step(int n, const double* __restrict__ S,
-                                                         const double* __restrict__ scal,
-                                                         const double* __restrict__ p, const double* __restrict__ Ap,
-                                                         double* x, double* r, double* partial) {
-    if (scal[kCgStop] != 0.0) return;
-    __shared__ double sh[kRedThreads];
-    const double pAp = scal[1];
-    const double a = pAp != 0.0 ? scal[0] / pAp : 0.0;
-    double rr = 0, ss = 0;
-    for (int s = blockIdx.x * kRedThreads + threadIdx.x; s < n; s += kRedBlocks * kRedThreads) {
-        D3 rv;
-        for (int k = 0; k < 3; k++) {
-            const size_t id = 3 * (size_t)s + k;
-            x[id] += a * p[id];
-            const double nr = r[id] - a * Ap[id];
-            r[id] = nr;
-            rr += nr * nr;
-        }
-        rv = mk(r[3 * (size_t)s], r[3 * (size_t)s + 1], r[3 * (size_t)s + 2]);
-        D3 sr = sym_mul(S + 6 * (size_t)s, rv);
-        ss += dot(sr, sr);
-    }
-    rr = block_sum(rr, sh);
-    ss = block_sum(ss, sh);
-    if (threadIdx.x == 0) {
-        partial[blockIdx.x] = rr;
-        partial[kRedBlocks + blockIdx.x] = ss;
-    }
-}
-
-__global__ __launch_bounds__(kRedThreads) void k_residual_norm(int n, const double* __restrict__ S,
-                                                               const double* __restrict__ r, double* partial) {
-    __shared__ double sh[kRedThreads];
-    double rr = 0, ss = 0;
-    for (int s = blockIdx.x * kRedThreads + threadIdx.x; s < n; s += kRedBlocks * kRedThreads) {
-        D3 rv = mk(r[3 * (size_t)s], r[3 * (size_t)s + 1], r[3 * (size_t)s + 2]);
-        rr += dot(rv, rv);
-        D3 sr = sym_mul(S + 6 * (size_t)s, rv);
-        ss += dot(sr, sr);
-    }
-    rr = block_sum(rr, sh);
-    ss = block_sum(ss, sh);
-    if (threadIdx.x == 0) {
-        partial[blockIdx.x] = rr;
-        partial[kRedBlocks + blockIdx.x] = ss;
-    }
-}
-
-// The solver's operator output fused with the CG inner product: Ap as in
-// k_matvec_finish and the partial sums of p.Ap per block (kRedBlocks blocks).
-template <class R>
-__global__ __launch_bounds__(kRedThreads) void k_matvec_finish_dot(int n, const double* __restrict__ S,
-                                                                   const acc_t* __restrict__ acc,
-                                                                   const R* __restrict__ erec,
-                                                                   const R* __restrict__ mu, double selfc,
-                                                                   const double* __restrict__ p, double* Ap,
-                                                                   double* partial, const double* __restrict__ scal) {
-    if (scal[kCgStop] != 0.0) return;
-    __shared__ double sh[kRedThreads];
-    double v = 0;
-    for (int s = blockIdx.x * kRedThreads + threadIdx.x; s < n; s += kRedBlocks * kRedThreads) {
-        D3 E;
-        E.x = acc_get(acc[3 * (size_t)s]) + (double)erec[3 * (size_t)s] + selfc * (double)mu[3 * (size_t)s];
-        E.y = acc_get(acc[3 * (size_t)s + 1]) + (double)erec[3 * (size_t)s + 1] +
-              selfc * (double)mu[3 * (size_t)s + 1];
-        E.z = acc_get(acc[3 * (size_t)s + 2]) + (double)erec[3 * (size_t)s + 2] +
-              selfc * (double)mu[3 * (size_t)s + 2];
-        const D3 w = sym_mul(S + 6 * (size_t)s, E);
-        const D3 pv = mk(p[3 * (size_t)s], p[3 * (size_t)s + 1], p[3 * (size_t)s + 2]);
-        const D3 a = mk(pv.x - w.x, pv.y - w.y, pv.z - w.z);
-        Ap[3 * (size_t)s] = a.x;
-        Ap[3 * (size_t)s + 1] = a.y;
-        Ap[3 * (size_t)s + 2] = a.z;
-        v += dot(pv, a);
-    }
-    v = block_sum(v, sh);
-    if (threadIdx.x == 0) partial[blockIdx.x] = v;
-}
-
-// The solver's stopping test, the same expression as the host's report:
-// converged when the RMS of S r, in Debye, is below stop_eps.
-__device__ __forceinline__ double cg_stopped(double ss, int n, double stop_eps) {
-    return kDebye * sqrt(ss / (double)n) >= stop_eps ? 0.0 : 1.0;
-}
-
-// Publishes check c of a solve (the state after c iterations): scal[kCgCount]
-// = c, scal[kCgStop] = the stopping test, and in host slot c & 1 the pair
-// (|S r|^2, stop).  Slots alternate so that the host can read check c while
-// the iteration after it is already running.
-__device__ __forceinline__ void cg_publish(double* scal, double* hcheck, double c, double ss, double stop) {
-    scal[kCgCount] = c;
-    scal[kCgStop] = stop;
-    double* slot = hcheck + 2 * ((int)c & 1);
-    slot[0] = ss;
-    slot[1] = stop;
-}
-
-// Check 0 of a solve, from the initial residual's |S r|^2 in scal[3].
-__global__ void k_cg_begin(double* scal, double* hcheck, int n, double stop_eps) {
-    if (threadIdx.x != 0) return;
-    const double ss = scal[3];
-    cg_publish(scal, hcheck, 0.0, ss, cg_stopped(ss, n, stop_eps));
-}
-
-// One block: the partial sums of k_cg_step give rr_new (scal[2], scal[0]) and
-// ss (scal[3]); beta = rr_new / rr_old goes to scal[7], then the iteration's
-// check is published.  Thread 0 reads the old scal[0] before it writes the new
-// one.
-__global__ __launch_bounds__(kRedThreads) void k_cg_reduce_beta(const double* __restrict__ partial, double* scal,
-                                                                double* hcheck, int n, double stop_eps) {
-    if (scal[kCgStop] != 0.0) return;
-    __shared__ double sh[kRedThreads];
-    double rr = 0, ss = 0;
-    for (int i = threadIdx.x; i < kRedBlocks; i += kRedThreads) {
-        rr += partial[i];
-        ss += partial[kRedBlocks + i];
-    }
-    rr = block_sum(rr, sh);
-    ss = block_sum(ss, sh);
-    if (threadIdx.x == 0) {
-        const double old = scal[0];
-        scal[7] = old != 0.0 ? rr / old : 0.0;
-        scal[0] = rr;
-        scal[2] = rr;
-        scal[3] = ss;
-        cg_publish(scal, hcheck, scal[kCgCount] + 1.0, ss, cg_stopped(ss, n, stop_eps));
-    }
-}
-
-// p = r + beta p (beta = scal[7]), fused with the next operator input mu = S p.
-// Skipped once the solve has stopped, also after the iteration that stops it:
-// the solver does not read p or mu after its last check.
-template <class R>
-__global__ void k_cg_direction_apply(int n, const double* __restrict__ S, const double* __restrict__ scal,
-                                     const double* __restrict__ r, double* p, R* mu) {
-    if (scal[kCgStop] != 0.0) return;
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const double beta = scal[7];
-    D3 pv;
-    pv.x = r[3 * (size_t)s] + beta * p[3 * (size_t)s];
-    pv.y = r[3 * (size_t)s + 1] + beta * p[3 * (size_t)s + 1];
-    pv.z = r[3 * (size_t)s + 2] + beta * p[3 * (size_t)s + 2];
-    p[3 * (size_t)s] = pv.x;
-    p[3 * (size_t)s + 1] = pv.y;
-    p[3 * (size_t)s + 2] = pv.z;
-    const D3 v = sym_mul(S + 6 * (size_t)s, pv);
-    mu[3 * (size_t)s] = (R)v.x;
-    mu[3 * (size_t)s + 1] = (R)v.y;
-    mu[3 * (size_t)s + 2] = (R)v.z;
 }
 
 template <class R>
@@ -505,6 +310,20 @@ __device__ void cart_potential(const R* ph, const FracT<double>& A, double* c1, 
 // (gacc) - A phi_2 A^T (A the grid-coordinate transform; :4094-4127), kept
 // for the response forces; then mu_(m+1) = alpha_lab E, in FP64 and in the
 // precision of the next order's kernels.
+template <class R>
+__global__ void k_extrap_init(int n, const double* __restrict__ labpol, const double* __restrict__ E0, double* mu,
+                              R* mu_r) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= n) return;
+    const size_t i3 = 3 * (size_t)s;
+    const D3 m = sym_mul(labpol + 6 * (size_t)s, mk(E0[i3], E0[i3 + 1], E0[i3 + 2]));
+    mu[i3] = m.x;
+    mu[i3 + 1] = m.y;
+    mu[i3 + 2] = m.z;
+    mu_r[i3] = (R)m.x;
+    mu_r[i3 + 1] = (R)m.y;
+    mu_r[i3 + 2] = (R)m.z;
+}
 template <class R>
 __global__ void k_extrap_order(int n, const acc_t* __restrict__ field, const acc_t* __restrict__ gacc,
                                const R* __restrict__ phidp, FracT<double> A, double selfc,
@@ -710,8 +529,7 @@ __global__ void k_sub(int m, const double* __restrict__ a, const double* __restr
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x) out[i] = a[i] - b[i];
 }
 
-__global__ void k_zero_acc(acc_t* p, size_t count, const double* skip) {
-    if (skipped(skip)) return;
+__global__ void k_zero_acc(acc_t* p, size_t count) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x)
         p[i] = 0;
 }
@@ -1385,10 +1203,10 @@ void launch_output_forces(hipStream_t s, int n, const int* perm, const acc_t* fo
 void launch_unpermute3(hipStream_t s, int n, const int* perm, const double* in, double* out) {
     hipLaunchKernelGGL(k_unpermute3, blocks_for(n, 256), dim3(256), 0, s, n, perm, in, out);
 }
-void launch_zero_acc(hipStream_t s, acc_t* p, size_t count, const double* skip) {
+void launch_zero_acc(hipStream_t s, acc_t* p, size_t count) {
     int b = (int)std::min<size_t>((count + 255) / 256, 4096);
     if (b < 1) b = 1;
-    hipLaunchKernelGGL(k_zero_acc, dim3(b), dim3(256), 0, s, p, count, skip);
+    hipLaunchKernelGGL(k_zero_acc, dim3(b), dim3(256), 0, s, p, count);
 }
 template <class R> void launch_fill(hipStream_t s, R* p, size_t count, R v) {
     int b = (int)std::min<size_t>((count + 255) / 256, 8192);
@@ -1400,41 +1218,13 @@ void launch_fixed_field_finish(hipStream_t s, int n, const R* phi, const double*
                                FracT<double> A, double selfc, double* E0) {
     hipLaunchKernelGGL(k_fixed_field_finish<R>, blocks_for(n, 256), dim3(256), 0, s, n, phi, lab, acc, A, selfc, E0);
 }
-void launch_solver_init(hipStream_t s, int n, const double* S, const double* E0, double* b, double* y) {
-    hipLaunchKernelGGL(k_solver_init, blocks_for(n, 256), dim3(256), 0, s, n, S, E0, b, y);
-}
-template <class R> void launch_apply_S(hipStream_t s, int n, const double* S, const double* y, R* mu, double* mud) {
-    hipLaunchKernelGGL(k_apply_S<R>, blocks_for(n, 256), dim3(256), 0, s, n, S, y, mu, mud);
-}
-template <class R>
-void launch_matvec_finish(hipStream_t s, int n, const double* S, const acc_t* acc, const R* erecip, const R* mu,
-                          double selfc, const double* p, double* Ap) {
-    hipLaunchKernelGGL(k_matvec_finish<R>, blocks_for(n, 256), dim3(256), 0, s, n, S, acc, erecip, mu, selfc, p, Ap);
-}
 void launch_dot(hipStream_t s, int m, const double* a, const double* b, double* partial, double* result) {
     hipLaunchKernelGGL(k_dot_partial, dim3(kRedBlocks), dim3(kRedThreads), 0, s, m, a, b, partial);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kRedThreads), 0, s, partial, 1, result, nullptr);
+    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kRedThreads), 0, s, partial, 1, result);
 }
-void launch_residual_norm(hipStream_t s, int n, const double* S, const double* r, double* partial, double* result) {
-    hipLaunchKernelGGL(k_residual_norm, dim3(kRedBlocks), dim3(kRedThreads), 0, s, n, S, r, partial);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kRedThreads), 0, s, partial, 2, result, nullptr);
-}
-// One CG iteration after the operator's field is complete (scal slots:
-// [0] rr, [1] pAp, [2] rr_new, [3] ss, [7] beta): Ap and pAp, x += a p,
-// r -= a Ap with their norms, the iteration's check, then the next direction
-// p and its mu = S p.  Deterministic reductions: per-block partials, then
-// one block in block order.  Every kernel returns at once when the solve
-// has stopped before the iteration.
 template <class R>
-void launch_cg_iteration(hipStream_t s, int n, const double* S, const acc_t* acc, const R* erec, R* mu, double selfc,
-                         double* p, double* Ap, double* x, double* r, double* partial, double* scal, double* hcheck,
-                         double stop_eps) {
-    hipLaunchKernelGGL(k_matvec_finish_dot<R>, dim3(kRedBlocks), dim3(kRedThreads), 0, s, n, S, acc, erec, mu, selfc,
-                       p, Ap, partial, scal);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kRedThreads), 0, s, partial, 1, scal + 1, scal + kCgStop);
-    hipLaunchKernelGGL(k_cg_step, dim3(kRedBlocks), dim3(kRedThreads), 0, s, n, S, scal, p, Ap, x, r, partial);
-    hipLaunchKernelGGL(k_cg_reduce_beta, dim3(1), dim3(kRedThreads), 0, s, partial, scal, hcheck, n, stop_eps);
-    hipLaunchKernelGGL(k_cg_direction_apply<R>, blocks_for(n, 256), dim3(256), 0, s, n, S, scal, r, p, mu);
+void launch_extrap_init(hipStream_t s, int n, const double* labpol, const double* E0, double* mu, R* mu_r) {
+    hipLaunchKernelGGL(k_extrap_init<R>, blocks_for(n, 256), dim3(256), 0, s, n, labpol, E0, mu, mu_r);
 }
 template <class R>
 void launch_extrap_order(hipStream_t s, int n, const acc_t* field, const acc_t* gacc, const R* phidp,
@@ -1492,9 +1282,6 @@ void launch_multipole_moments(hipStream_t s, int n, const int* perm, const doubl
                               const double* lab, const double* mu, double* out) {
     hipLaunchKernelGGL(k_multipole_moments, dim3(1), dim3(kMomThreads), 0, s, n, perm, pos, masses, lab, mu, out);
 }
-void launch_cg_begin(hipStream_t s, int n, double* scal, double* hcheck, double stop_eps) {
-    hipLaunchKernelGGL(k_cg_begin, dim3(1), dim3(64), 0, s, scal, hcheck, n, stop_eps);
-}
 void launch_axpy(hipStream_t s, int m, double a, const double* x, double* y) {
     int b = std::min((m + 255) / 256, 4096);
     if (b < 1) b = 1;
@@ -1519,14 +1306,10 @@ void launch_recip_atoms(hipStream_t s, int n, int mutual, const double* phi, con
     template void launch_fill<R>(hipStream_t, R*, size_t, R);                                                        \
     template void launch_fixed_field_finish<R>(hipStream_t, int, const R*, const double*, const acc_t*, FracT<double>, \
                                                double, double*);                                                    \
-    template void launch_apply_S<R>(hipStream_t, int, const double*, const double*, R*, double*);                   \
-    template void launch_matvec_finish<R>(hipStream_t, int, const double*, const acc_t*, const R*, const R*, double, \
-                                          const double*, double*);                                                  \
+    template void launch_extrap_init<R>(hipStream_t, int, const double*, const double*, double*, R*);                  \
     template void launch_extrap_order<R>(hipStream_t, int, const acc_t*, const acc_t*, const R*, FracT<double>, double,   \
                                          const double*, const double*, double*, double*, double*, R*);              \
     template void launch_extrap_combine<R>(hipStream_t, int, const ExtrapCoefficients&, const double*, double*, R*); \
-    template void launch_cg_iteration<R>(hipStream_t, int, const double*, const acc_t*, const R*, R*, double,       \
-                                         double*, double*, double*, double*, double*, double*, double*, double);    \
     template void launch_recip_atoms<R>(hipStream_t, int, int, const double*, const R*, const double*, const double*,\
                                         const int*, FracT<double>, double, acc_t*, acc_t*, acc_t*);                      \
     template void launch_field_sum<R>(hipStream_t, int, const acc_t*, const R*, const R*, double, double*);                    \

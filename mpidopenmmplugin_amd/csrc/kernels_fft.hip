@@ -151,13 +151,15 @@ template <class R> constexpr int max_per_thread() {
 // contiguous run; pass 2 (lines along y) reads and writes whole contiguous
 // blocks of T lines; pass 3 (lines along x) reads runs of T consecutive y.
 
-// Pass 1 (dir = -1): lines l along z, real Q[l][z] -> S[kz][l].
+// Pass 1 (dir = -1): lines l along z, real Q[l][z] -> S[kz][l]; with `clear`
+// Q is left zero, ready for the next spreading's atomic adds (a fill kernel
+// of its own cost a dependent dispatch per cycle).
 // Pass 5 (dir = +1): S[kz][l] -> real Q[l][z] (Hermitian completion).
 // A batch is T consecutive lines l0 .. l0 + T - 1.
 template <class R>
 __global__ __launch_bounds__(fft_threads<R>()) void k_fft_z(R* __restrict__ Q, R2<R>* __restrict__ S, FftAxis ax, int T,
                                                        int Tshift, const R2<R>* __restrict__ tw, int nlines, int dir,
-                                                       const double* skip) {
+                                                       int clear, const double* skip) {
     if (skipped(skip)) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int n = ax.n;
@@ -171,13 +173,20 @@ __global__ __launch_bounds__(fft_threads<R>()) void k_fft_z(R* __restrict__ Q, R
     constexpr int MP = max_per_thread<R>();
     const int total = T * n;
     if (dir < 0) {
-        const R* src = Q + (size_t)l0 * n;
+        R* src = Q + (size_t)l0 * n;
         const int lim = count * n;
         R v[MP];
 #pragma unroll
         for (int u = 0; u < MP; u++) {
             const int idx = threadIdx.x + u * fft_threads<R>();
             v[u] = idx < lim ? src[idx] : R(0);
+        }
+        if (clear) {
+#pragma unroll
+            for (int u = 0; u < MP; u++) {
+                const int idx = threadIdx.x + u * fft_threads<R>();
+                if (idx < lim) src[idx] = R(0);
+            }
         }
 #pragma unroll
         for (int u = 0; u < MP; u++) {
@@ -590,9 +599,9 @@ __device__ __forceinline__ int at(int t, int z) { return t * kPitch + (z >> 3) *
 }  // namespace zline
 
 template <class R>
-__global__ __launch_bounds__(zline::threads<R>()) void k_fft_z128_r2c(const R* __restrict__ Q, R2<R>* __restrict__ S,
+__global__ __launch_bounds__(zline::threads<R>()) void k_fft_z128_r2c(R* __restrict__ Q, R2<R>* __restrict__ S,
                                                                      const R2<R>* __restrict__ tw, int nlines,
-                                                                     const double* skip) {
+                                                                     int clear, const double* skip) {
     if (skipped(skip)) return;
     using namespace zline;
     typedef Cx<R> C;
@@ -606,10 +615,14 @@ __global__ __launch_bounds__(zline::threads<R>()) void k_fft_z128_r2c(const R* _
     {
         // T lines of N reals in 16-byte loads
         constexpr int kLoads = T * N / kV / kThreads;
-        const vec* src = reinterpret_cast<const vec*>(Q + (size_t)l0 * N);
+        vec* src = reinterpret_cast<vec*>(Q + (size_t)l0 * N);
         vec v[kLoads];
 #pragma unroll
         for (int u = 0; u < kLoads; u++) v[u] = src[threadIdx.x + u * kThreads];
+        if (clear) {
+#pragma unroll
+            for (int u = 0; u < kLoads; u++) src[threadIdx.x + u * kThreads] = vec(R(0));
+        }
 #pragma unroll
         for (int u = 0; u < kLoads; u++) {
             const int f = threadIdx.x + u * kThreads, t = f / (N / kV), z = (f % (N / kV)) * kV;
@@ -757,13 +770,13 @@ template <class R> static size_t fft_lds(int T, int n) { return (2 * (size_t)T *
 // the z passes with the register-step kernels where they apply (n2 = 128,
 // whole batches of 64 lines in FP32, 32 in FP64)
 template <class R>
-static bool zline_pass(hipStream_t s, const FftPlan<R>& p, R* Q, R2<R>* S, int dir, const double* skip) {
+static bool zline_pass(hipStream_t s, const FftPlan<R>& p, R* Q, R2<R>* S, int dir, int clear, const double* skip) {
     constexpr int T = zline::lines<R>();
     const int nlines = p.ax[0].n * p.ax[1].n;
     if (p.ax[2].n != zline::N || nlines % T != 0) return false;
     if (dir < 0)
         hipLaunchKernelGGL(k_fft_z128_r2c<R>, dim3(nlines / T), dim3(zline::threads<R>()), 0, s, Q, S, p.tw[2], nlines,
-                           skip);
+                           clear, skip);
     else
         hipLaunchKernelGGL(k_fft_z128_c2r<R>, dim3(nlines / T), dim3(zline::threads<R>()), 0, s, Q, S, p.tw[2], nlines,
                            skip);
@@ -825,17 +838,18 @@ template void launch_influence_table<float>(hipStream_t, InflParams, const doubl
 template void launch_influence_table<double>(hipStream_t, InflParams, const double*, double*);
 
 template <class R>
-void launch_recip_convolution(hipStream_t s, const FftPlan<R>& p, R* Q, R2<R>* S, ConvParams<R> cp) {
+void launch_recip_convolution(hipStream_t s, const FftPlan<R>& p, R* Q, R2<R>* S, R* V, ConvParams<R> cp) {
     const int n0 = p.ax[0].n, n1 = p.ax[1].n, n2 = p.ax[2].n;
     const int n2h = n2 / 2 + 1;
     const int nlines = n0 * n1;
     const int Tz = lines_per_group<R>(n2);
     const int Ty = lines_per_group<R>(n1), nxb = (n0 + Ty - 1) / Ty;
     const int Tx = lines_per_group<R>(n0), nyb = (n1 + Tx - 1) / Tx;
+    const int clear = V != Q ? 1 : 0;
     // 1. z forward
-    if (!zline_pass<R>(s, p, Q, S, -1, cp.skip))
+    if (!zline_pass<R>(s, p, Q, S, -1, clear, cp.skip))
         hipLaunchKernelGGL(k_fft_z<R>, dim3((nlines + Tz - 1) / Tz), dim3(fft_threads<R>()), fft_lds<R>(Tz, n2), s, Q,
-                           S, p.ax[2], Tz, log2i(Tz), p.tw[2], nlines, -1, cp.skip);
+                           S, p.ax[2], Tz, log2i(Tz), p.tw[2], nlines, -1, clear, cp.skip);
     if (!plane_pass<R>(s, p, S, n2h, n2, cp) && !plane_small_pass<R>(s, p, S, n2h, n2, cp)) {
         // 2. y forward
         hipLaunchKernelGGL(k_fft_y<R>, dim3(n2h * nxb), dim3(fft_threads<R>()), fft_lds<R>(Ty, n1), s, S, p.ax[1], Ty,
@@ -848,14 +862,14 @@ void launch_recip_convolution(hipStream_t s, const FftPlan<R>& p, R* Q, R2<R>* S
                            p.tw[1], n0, nxb, 1, cp.skip);
     }
     // 5. z backward
-    if (!zline_pass<R>(s, p, Q, S, 1, cp.skip))
-        hipLaunchKernelGGL(k_fft_z<R>, dim3((nlines + Tz - 1) / Tz), dim3(fft_threads<R>()), fft_lds<R>(Tz, n2), s, Q,
-                           S, p.ax[2], Tz, log2i(Tz), p.tw[2], nlines, 1, cp.skip);
+    if (!zline_pass<R>(s, p, V, S, 1, 0, cp.skip))
+        hipLaunchKernelGGL(k_fft_z<R>, dim3((nlines + Tz - 1) / Tz), dim3(fft_threads<R>()), fft_lds<R>(Tz, n2), s, V,
+                           S, p.ax[2], Tz, log2i(Tz), p.tw[2], nlines, 1, 0, cp.skip);
 }
 
-template void launch_recip_convolution<float>(hipStream_t, const FftPlan<float>&, float*, R2<float>*,
+template void launch_recip_convolution<float>(hipStream_t, const FftPlan<float>&, float*, R2<float>*, float*,
                                               ConvParams<float>);
-template void launch_recip_convolution<double>(hipStream_t, const FftPlan<double>&, double*, R2<double>*,
+template void launch_recip_convolution<double>(hipStream_t, const FftPlan<double>&, double*, R2<double>*, double*,
                                                ConvParams<double>);
 
 }  // namespace mpid

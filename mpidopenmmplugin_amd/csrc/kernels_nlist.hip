@@ -443,7 +443,6 @@ template <class R, bool GRAD>
 __global__ __launch_bounds__(256) void k_nl_induced_field(NbrList L, const int* __restrict__ atoms, int natoms,
                                                           PairAtoms<R> A, const R* __restrict__ mu, PairParams<R> P,
                                                           acc_t* __restrict__ field, acc_t* __restrict__ grad) {
-    if (skipped(P.skip)) return;
     const unsigned g = (unsigned)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     const int t = (int)(g / kNlSplit), sub = (int)(g % kNlSplit);
     const int n = P.n;

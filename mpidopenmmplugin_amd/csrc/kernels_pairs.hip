@@ -484,7 +484,6 @@ template <class R, bool GRAD>
 __global__ __launch_bounds__(256) void k_cov_induced_field(PairAtoms<R> A, const R* __restrict__ mu, PairParams<R> P,
                                                            int pol_only, acc_t* __restrict__ field,
                                                            acc_t* __restrict__ grad) {
-    if (skipped(P.skip)) return;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= P.n) return;
     const int np = A.npart[i];

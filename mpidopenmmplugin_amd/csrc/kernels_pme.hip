@@ -10,72 +10,11 @@
 // :3532-3573, computeFixedPotentialFromGrid :3368-3530.  The grid has x
 // slowest and z fastest, as the reference's; it holds only the real part,
 // which is all the reference ever fills.
-#include "engine.h"
+#include "pme_math.h"
 
 #include <algorithm>
 
 namespace mpid {
-
-// Order-6 B-spline weights of the 6 grid points and their first ND derivatives:
-// Cox-de Boor recursion, derivatives as backward differences of lower orders.
-template <class R, int ND>
-__device__ __forceinline__ void bspline6(R w, R th[kOrder][ND + 1]) {
-    R c[kOrder + 1][kOrder + 1];
-    c[1][0] = R(1);
-#pragma unroll
-    for (int p = 2; p <= kOrder; p++) {
-#pragma unroll
-        for (int m = 0; m < p; m++) {
-            R left = (m >= 1) ? c[p - 1][m - 1] : R(0);
-            R right = (m <= p - 2) ? c[p - 1][m] : R(0);
-            c[p][m] = ((w + R(p - 1 - m)) * left + (R(m + 1) - w) * right) * R(1.0 / (p - 1));
-        }
-    }
-#pragma unroll
-    for (int r = 0; r <= ND; r++) {
-        R cur[kOrder + 1];
-        const int p = kOrder - r;
-#pragma unroll
-        for (int m = 0; m < kOrder + 1; m++) cur[m] = (m < p) ? c[p][m] : R(0);
-        int len = p;
-#pragma unroll
-        for (int s = 0; s < r; s++) {
-            R nxt[kOrder + 1];
-#pragma unroll
-            for (int m = 0; m < kOrder + 1; m++)
-                nxt[m] = ((m >= 1 && m - 1 < len) ? cur[m - 1] : R(0)) - ((m < len) ? cur[m] : R(0));
-            len++;
-#pragma unroll
-            for (int m = 0; m < kOrder + 1; m++) cur[m] = nxt[m];
-        }
-#pragma unroll
-        for (int m = 0; m < kOrder; m++) th[m][r] = cur[m];
-    }
-}
-
-__device__ __forceinline__ unsigned spread_bits_pme(unsigned v) {
-    v &= 0x3ffu;
-    v = (v | (v << 16)) & 0x030000ffu;
-    v = (v | (v << 8)) & 0x0300f00fu;
-    v = (v | (v << 4)) & 0x030c30c3u;
-    v = (v | (v << 2)) & 0x09249249u;
-    return v;
-}
-
-// Grid origin and spline offset of one atom along an axis of n points from
-// its fractional coordinate f along that box vector, as the reference
-// computes them (f wrapped to [-1/2, 1/2), then shifted by one half box,
-// MPIDReferenceForce.cpp:3049-3075).
-template <class R>
-__device__ __forceinline__ void grid_coord(R f, int n, int& ig, R& w) {
-    f -= floor(f + R(0.5));
-    const R fr = R(n) * (f + R(0.5));
-    const int ifr = (int)floor(fr);
-    w = fr - R(ifr);
-    ig = ifr - kOrder + 1;
-    ig %= n;
-    if (ig < 0) ig += n;
-}
 
 // ---------------------------------------------------------------------------
 // spreading
@@ -87,18 +26,6 @@ __device__ __forceinline__ void grid_coord(R f, int n, int& ig, R& w) {
 // of its own, so that a small system still spreads over many CUs.  Every
 // lane evaluates the atom's splines and selects its (ix, iy, iz) entries with
 // unrolled compares (no dynamically indexed register arrays).
-template <class R, int ND>
-__device__ __forceinline__ void spline_at(const R (&t)[kOrder][ND + 1], int k, R (&out)[ND + 1]) {
-#pragma unroll
-    for (int d = 0; d <= ND; d++) out[d] = t[0][d];
-#pragma unroll
-    for (int m = 1; m < kOrder; m++)
-        if (k == m) {
-#pragma unroll
-            for (int d = 0; d <= ND; d++) out[d] = t[m][d];
-        }
-}
-
 constexpr int kSpreadWaves = 4;  // atoms (wavefronts) per 256-thread block
 
 template <class R>
@@ -152,11 +79,14 @@ __global__ __launch_bounds__(256) void k_spread_fixed(int n, const R4<R>* __rest
 }
 
 template <class R>
-__global__ __launch_bounds__(256) void k_spread_induced(int n, const R4<R>* __restrict__ pos, const R* __restrict__ mu,
+__global__ __launch_bounds__(256) void k_spread_induced(int natoms, const int* __restrict__ atoms,
+                                                         const R4<R>* __restrict__ pos, const R* __restrict__ mu,
                                                          PmeGeom<R> g, R* __restrict__ grid) {
-    const int i = blockIdx.x * kSpreadWaves + (threadIdx.x >> 6);
+    if (skipped(g.skip)) return;
+    const int t = blockIdx.x * kSpreadWaves + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (i >= n) return;
+    if (t >= natoms) return;
+    const int i = atoms ? atoms[t] : t;
     const V3<R> uf = frac_vector(mk(mu[3 * (size_t)i], mu[3 * (size_t)i + 1], mu[3 * (size_t)i + 2]), g.A);
     const R ux = uf.x, uy = uf.y, uz = uf.z;
     // a site without a dipole adds nothing (the whole wave leaves together)
@@ -236,6 +166,7 @@ __global__ __launch_bounds__(256) void k_spread_tiled(const R4<R>* __restrict__ 
     constexpr int ND = MODE == 0 ? 3 : 1;   // spline derivatives needed
     constexpr int NC = MODE == 0 ? 20 : 3;  // fractional components
     constexpr int CH = 32;                  // atoms staged per pass
+    if (skipped(g.skip)) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int W0 = tg.W[0], W1 = tg.W[1], W2 = tg.W[2];
     const int WV = W0 * W1 * W2;
@@ -536,6 +467,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 template <class R>
 __global__ __launch_bounds__(256) void k_fold(PmeGeom<R> g, TileGeom tg, const R* __restrict__ scratch,
                                                R* __restrict__ grid) {
+    if (skipped(g.skip)) return;
     const size_t total = (size_t)g.n[0] * g.n[1] * g.n[2];
     const int WV = tg.W[0] * tg.W[1] * tg.W[2];
     const int nt = tg.tiles_per_axis;
@@ -583,6 +515,7 @@ __global__ __launch_bounds__(256) void k_fold(PmeGeom<R> g, TileGeom tg, const R
 template <class R>
 __global__ __launch_bounds__(256) void k_fold_tiles(PmeGeom<R> g, TileGeom tg, FastDiv t2, FastDiv t12,
                                                      const R* __restrict__ scratch, R* __restrict__ grid) {
+    if (skipped(g.skip)) return;
     const int t = blockIdx.x;
     const int nt = tg.tiles_per_axis;
     const int c[3] = {(int)compact_bits((unsigned)t >> 2), (int)compact_bits((unsigned)t >> 1),
@@ -735,7 +668,6 @@ template <class R>
 __global__ __launch_bounds__(256) void k_gather_field(int natoms, const int* __restrict__ atoms,
                                                        const R4<R>* __restrict__ pos, PmeGeom<R> g,
                                                        const R* __restrict__ grid, R* __restrict__ field) {
-    if (skipped(g.skip)) return;
     const int gt = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     const int t = gt >> 3, iz = gt & 7;
     const bool tv = t < natoms;
@@ -812,10 +744,11 @@ void launch_spread_fixed(hipStream_t s, int n, const R4<R>* pos, const R* lab, P
                        n, pos, lab, g, grid);
 }
 template <class R>
-void launch_spread_induced(hipStream_t s, int n, const R4<R>* pos, const R* mu, PmeGeom<R> g, R* grid) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_spread_induced<R>, dim3((n + kSpreadWaves - 1) / kSpreadWaves), dim3(64 * kSpreadWaves), 0,
-                       s, n, pos, mu, g, grid);
+void launch_spread_induced(hipStream_t s, int natoms, const int* atoms, const R4<R>* pos, const R* mu, PmeGeom<R> g,
+                           R* grid) {
+    if (natoms <= 0) return;
+    hipLaunchKernelGGL(k_spread_induced<R>, dim3((natoms + kSpreadWaves - 1) / kSpreadWaves), dim3(64 * kSpreadWaves),
+                       0, s, natoms, atoms, pos, mu, g, grid);
 }
 void launch_tile_ranges(hipStream_t s, int n, const unsigned* keys_sorted, const int* idx, const int* count,
                         int shift, int* tstart, int* tend) {
@@ -902,7 +835,8 @@ void launch_gather_field(hipStream_t s, int natoms, const int* atoms, const R4<R
 
 #define MPID_INSTANTIATE(R)                                                                                   \
     template void launch_spread_fixed<R>(hipStream_t, int, const R4<R>*, const R*, PmeGeom<R>, R*);           \
-    template void launch_spread_induced<R>(hipStream_t, int, const R4<R>*, const R*, PmeGeom<R>, R*);         \
+    template void launch_spread_induced<R>(hipStream_t, int, const int*, const R4<R>*, const R*, PmeGeom<R>,  \
+                                           R*);                                                              \
     template void launch_gather_phi<R>(hipStream_t, int, const R4<R>*, PmeGeom<R>, const R*, R*);            \
     template void launch_gather_field<R>(hipStream_t, int, const int*, const R4<R>*, PmeGeom<R>, const R*,   \
                                          R*);                                                                \

@@ -1,0 +1,677 @@
+// The mutual-polarization solver's kernels: the operator A = I - S T S on the
+// polarisable sites, the conjugate-gradient update and the residual norms.
+//
+// The solver's vectors (b, x, r, p, A p) hold the polarisable sites only, in
+// the order of their sorted index (t-th entry: atom idx[t]); a site without
+// polarisability has S = 0 and a zero entry in every one of them.  The
+// operator's input mu = S p is stored by atom, with zeros elsewhere, for the
+// spreading and the neighbour lists.
+//
+// A solver iteration is a chain of short dependent kernels, so its time on
+// small systems is their number times the 4-6 us a dependent dispatch takes.
+// The chain is therefore kept short: the operator's kernel gathers the
+// reciprocal field, adds the real-space field, applies S and leaves the
+// partial sums of p.Ap; the update kernels fold the reductions in (every
+// workgroup sums the previous kernel's partials in the same order, so the
+// result is the same in each and from run to run).
+#include "pair_math.h"
+#include "pme_math.h"
+
+#include <algorithm>
+
+namespace mpid {
+
+typedef V3<double> D3;
+
+__device__ __forceinline__ D3 sym_mul6(const double* S, D3 v) {
+    return mk(S[0] * v.x + S[1] * v.y + S[2] * v.z, S[1] * v.x + S[3] * v.y + S[4] * v.z,
+              S[2] * v.x + S[4] * v.y + S[5] * v.z);
+}
+__device__ __forceinline__ D3 load3(const double* a, size_t t) { return mk(a[3 * t], a[3 * t + 1], a[3 * t + 2]); }
+__device__ __forceinline__ void store3(double* a, size_t t, D3 v) {
+    a[3 * t] = v.x;
+    a[3 * t + 1] = v.y;
+    a[3 * t + 2] = v.z;
+}
+template <class R> __device__ __forceinline__ void store_mu(R* mu, size_t i, D3 v) {
+    mu[3 * i] = (R)v.x;
+    mu[3 * i + 1] = (R)v.y;
+    mu[3 * i + 2] = (R)v.z;
+}
+
+// Sums over a workgroup of THREADS threads in a fixed order, the result in
+// every thread; sh: THREADS / 64 * K words.
+template <int THREADS, int K> __device__ __forceinline__ void group_sum(double (&v)[K], double* sh) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < K; k++) v[k] += __shfl_xor(v[k], off);
+    constexpr int kWaves = THREADS / 64;
+    if constexpr (kWaves > 1) {
+        __syncthreads();  // sh may still be read from a previous sum
+        if ((threadIdx.x & 63) == 0)
+#pragma unroll
+            for (int k = 0; k < K; k++) sh[(threadIdx.x >> 6) * K + k] = v[k];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            double s = 0.0;
+#pragma unroll
+            for (int w = 0; w < kWaves; w++) s += sh[w * K + k];
+            v[k] = s;
+        }
+    }
+}
+// The same over `count` partials of each of K sums, stored one sum after the
+// other at a stride of kMaxPartials.
+template <int THREADS, int K>
+__device__ __forceinline__ void sum_partials(const double* __restrict__ partial, int count, double (&v)[K], double* sh) {
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        v[k] = 0.0;
+        for (int i = threadIdx.x; i < count; i += THREADS) v[k] += partial[k * kMaxPartials + i];
+    }
+    group_sum<THREADS, K>(v, sh);
+}
+
+// ---------------------------------------------------------------------------
+// operator
+// ---------------------------------------------------------------------------
+// Av_t = v_t - S (E_rec + E_real + selfc mu) at polarisable site t, and with
+// `partial` one partial sum of v.Av per workgroup.
+template <class R>
+__device__ __forceinline__ double operator_row(const SolverSites& st, int t, int i, D3 e, const R* __restrict__ mu,
+                                               double selfc, const double* __restrict__ v, double* Av) {
+    e.x += selfc * (double)mu[3 * (size_t)i];
+    e.y += selfc * (double)mu[3 * (size_t)i + 1];
+    e.z += selfc * (double)mu[3 * (size_t)i + 2];
+    const D3 w = sym_mul6(st.S + 6 * (size_t)i, e);
+    const D3 pv = load3(v, t);
+    const D3 a = pv - w;
+    store3(Av, t, a);
+    return dot(pv, a);
+}
+
+// Everything after the inverse transform in one kernel, 32 lanes per site:
+// the site's splines (lanes 0-2, one axis each, through LDS), the stencil's
+// points over the lanes, the neighbours over the lanes, the covalent partners.
+// For systems whose kernels do not fill the chip (kFusedSites): there the
+// list of a site is walked in 3 steps instead of the 18-24 of four lanes, and
+// five dispatches become one.
+constexpr int kOpLanes = 32;
+constexpr int kOpSites = 256 / kOpLanes;  // sites per workgroup
+template <class R>
+__global__ __launch_bounds__(256) void k_operator_fused(SolverSites st, PmeGeom<R> g, const R* __restrict__ pot,
+                                                        NbrList L, PairAtoms<R> A, PairParams<R> P,
+                                                        const R* __restrict__ mu, double selfc,
+                                                        const double* __restrict__ v, double* __restrict__ Av,
+                                                        double* __restrict__ partial) {
+    if (skipped(P.skip)) return;
+    __shared__ R sth[kOpSites][3][kOrder][2];
+    __shared__ int sig[kOpSites][3];
+    __shared__ double sdot[kOpSites];
+    const int grp = threadIdx.x / kOpLanes, lane = threadIdx.x % kOpLanes;
+    double acc = 0.0;
+    for (int t0 = blockIdx.x * kOpSites; t0 < st.npol; t0 += gridDim.x * kOpSites) {
+        const int t = min(t0 + grp, st.npol - 1);
+        const bool tv = t0 + grp < st.npol;
+        const int i = st.idx[t];
+        const R4<R> pi = A.pos[i];
+        R ex = 0, ey = 0, ez = 0;
+        if (pot) {  // no reciprocal space without a grid
+            if (lane < 3) {
+                const V3<R> f = to_frac(mk(pi.x, pi.y, pi.z), g.box);
+                int ig;
+                R w;
+                grid_coord(lane == 0 ? f.x : (lane == 1 ? f.y : f.z), g.n[lane], ig, w);
+                R th[kOrder][2];
+                bspline6<R, 1>(w, th);
+#pragma unroll
+                for (int m = 0; m < kOrder; m++) {
+                    sth[grp][lane][m][0] = th[m][0];
+                    sth[grp][lane][m][1] = th[m][1];
+                }
+                sig[grp][lane] = ig;
+            }
+            __syncthreads();
+            const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
+            const int gx = sig[grp][0], gy = sig[grp][1], gz = sig[grp][2];
+            constexpr int kPoints = kOrder * kOrder * kOrder;
+            constexpr int kSteps = (kPoints + kOpLanes - 1) / kOpLanes;
+            R q[kSteps];
+#pragma unroll
+            for (int u = 0; u < kSteps; u++) {
+                const int s = min(lane + u * kOpLanes, kPoints - 1);
+                const int ix = s / (kOrder * kOrder), rem = s - ix * kOrder * kOrder;
+                const int iy = rem / kOrder, iz = rem - iy * kOrder;
+                int x = gx + ix, y = gy + iy, z = gz + iz;
+                if (x >= nx) x -= nx;
+                if (y >= ny) y -= ny;
+                if (z >= nz) z -= nz;
+                q[u] = pot[((size_t)x * ny + y) * nz + z];
+            }
+            R s100 = 0, s010 = 0, s001 = 0;
+#pragma unroll
+            for (int u = 0; u < kSteps; u++) {
+                const int s0 = lane + u * kOpLanes, s = min(s0, kPoints - 1);
+                const int ix = s / (kOrder * kOrder), rem = s - ix * kOrder * kOrder;
+                const int iy = rem / kOrder, iz = rem - iy * kOrder;
+                const R a0 = sth[grp][0][ix][0], a1 = sth[grp][0][ix][1];
+                const R b0 = sth[grp][1][iy][0], b1 = sth[grp][1][iy][1];
+                const R c0 = sth[grp][2][iz][0], c1 = sth[grp][2][iz][1];
+                const R qv = s0 < kPoints ? q[u] : R(0);
+                s100 += qv * a1 * b0 * c0;
+                s010 += qv * a0 * b1 * c0;
+                s001 += qv * a0 * b0 * c1;
+            }
+            const V3<R> e = cart_vector(mk(s100, s010, s001), g.A);
+            ex = -e.x;
+            ey = -e.y;
+            ez = -e.z;
+            __syncthreads();  // the tables are read before the next sites' replace them
+        }
+        R rx = 0, ry = 0, rz = 0;
+        const int cnt = tv ? L.count[i] : 0;
+        for (int k = lane; k < cnt; k += kOpLanes) {
+            const int j = L.nbr[((size_t)(k / kNlSplit) * st.npol + t) * kNlSplit + k % kNlSplit];
+            const R4<R> pj = A.pos[j];
+            const V3<R> dr = min_image(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), P.box);
+            const V3<R> uj = mk(mu[3 * (size_t)j], mu[3 * (size_t)j + 1], mu[3 * (size_t)j + 2]);
+            const V3<R> fi =
+                induced_field_from<R>(uj, dr, induced_field_radial<R>(dot(dr, dr), pi.w, pj.w, P.default_thole, P));
+            rx += fi.x;
+            ry += fi.y;
+            rz += fi.z;
+        }
+        const V3<R> c = partner_field<R>(i, lane, kOpLanes, A, mu, P);
+        rx += c.x;
+        ry += c.y;
+        rz += c.z;
+#pragma unroll
+        for (int off = 1; off < kOpLanes; off <<= 1) {
+            ex += __shfl_xor(ex, off);
+            ey += __shfl_xor(ey, off);
+            ez += __shfl_xor(ez, off);
+            rx += __shfl_xor(rx, off);
+            ry += __shfl_xor(ry, off);
+            rz += __shfl_xor(rz, off);
+        }
+        if (tv && lane == 0)
+            acc += operator_row<R>(st, t, i, mk((double)ex + (double)rx, (double)ey + (double)ry, (double)ez + (double)rz),
+                                   mu, selfc, v, Av);
+    }
+    if (partial) {
+        if (lane == 0) sdot[grp] = acc;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double s = 0.0;
+#pragma unroll
+            for (int k = 0; k < kOpSites; k++) s += sdot[k];
+            partial[blockIdx.x] = s;
+        }
+    }
+}
+
+// The same in two kernels for systems that fill the chip: the real-space field
+// (k_list_field, beside the reciprocal chain on another stream), and the
+// gather with the rest, 8 lanes per site (lane iz < 6: the 36 points of a z
+// plane, all loads in flight).
+template <class R>
+__global__ __launch_bounds__(256) void k_list_field(SolverSites st, NbrList L, PairAtoms<R> A, PairParams<R> P,
+                                                    const R* __restrict__ mu, R* __restrict__ field) {
+    if (skipped(P.skip)) return;
+    const unsigned gth = (unsigned)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int t = (int)(gth / kNlSplit), sub = (int)(gth % kNlSplit);
+    const bool tv = t < st.npol;
+    const int tc = tv ? t : st.npol - 1;
+    const int i = st.idx[tc];
+    const R4<R> pi = A.pos[i];
+    const int cnt = tv ? L.count[i] : 0;
+    const int* lp = L.nbr + (size_t)tc * kNlSplit + sub;
+    const size_t stride = (size_t)st.npol * kNlSplit;
+    int jn = sub < cnt ? lp[0] : 0;
+    R ex = 0, ey = 0, ez = 0;
+    for (int k = sub; k < cnt; k += kNlSplit) {
+        const int j = jn;
+        lp += stride;
+        if (k + kNlSplit < cnt) jn = *lp;  // next index in flight during this pair
+        const R4<R> pj = A.pos[j];
+        const V3<R> dr = min_image(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), P.box);
+        const V3<R> uj = mk(mu[3 * (size_t)j], mu[3 * (size_t)j + 1], mu[3 * (size_t)j + 2]);
+        const V3<R> fi =
+            induced_field_from<R>(uj, dr, induced_field_radial<R>(dot(dr, dr), pi.w, pj.w, P.default_thole, P));
+        ex += fi.x;
+        ey += fi.y;
+        ez += fi.z;
+    }
+    const V3<R> c = partner_field<R>(i, sub, kNlSplit, A, mu, P);
+    ex += c.x;
+    ey += c.y;
+    ez += c.z;
+#pragma unroll
+    for (int off = 1; off < kNlSplit; off <<= 1) {
+        ex += __shfl_xor(ex, off);
+        ey += __shfl_xor(ey, off);
+        ez += __shfl_xor(ez, off);
+    }
+    if (tv && sub == 0) {
+        field[3 * (size_t)t] = ex;
+        field[3 * (size_t)t + 1] = ey;
+        field[3 * (size_t)t + 2] = ez;
+    }
+}
+
+constexpr int kGatherSites = 32;  // sites per workgroup
+template <class R>
+__global__ __launch_bounds__(256) void k_operator_gather(SolverSites st, PmeGeom<R> g, const R* __restrict__ pot,
+                                                         const R* __restrict__ field, const R4<R>* __restrict__ pos,
+                                                         const R* __restrict__ mu, double selfc,
+                                                         const double* __restrict__ v, double* __restrict__ Av,
+                                                         double* __restrict__ partial) {
+    if (skipped(g.skip)) return;
+    __shared__ double sdot[kGatherSites];
+    const int grp = threadIdx.x >> 3, iz = threadIdx.x & 7;
+    double acc = 0.0;
+    for (int t0 = xcd_block(blockIdx.x, gridDim.x) * kGatherSites; t0 < st.npol; t0 += gridDim.x * kGatherSites) {
+        const int t = min(t0 + grp, st.npol - 1);
+        const bool tv = t0 + grp < st.npol;
+        const int i = st.idx[t];
+        R s100 = 0, s010 = 0, s001 = 0;
+        if (pot) {
+            const R4<R> p = pos[i];
+            int ig[3];
+            R w[3];
+            {
+                const V3<R> f = to_frac(mk(p.x, p.y, p.z), g.box);
+                grid_coord(f.x, g.n[0], ig[0], w[0]);
+                grid_coord(f.y, g.n[1], ig[1], w[1]);
+                grid_coord(f.z, g.n[2], ig[2], w[2]);
+            }
+            R tx[kOrder][2], ty[kOrder][2], tz[kOrder][2];
+            bspline6<R, 1>(w[0], tx);
+            bspline6<R, 1>(w[1], ty);
+            bspline6<R, 1>(w[2], tz);
+            const int ny = g.n[1], nz = g.n[2];
+            if (iz < kOrder) {
+                int z = ig[2] + iz;
+                if (z >= nz) z -= nz;
+                R q[kOrder][kOrder];
+#pragma unroll
+                for (int iy = 0; iy < kOrder; iy++) {
+                    int y = ig[1] + iy;
+                    if (y >= ny) y -= ny;
+#pragma unroll
+                    for (int ix = 0; ix < kOrder; ix++) {
+                        int x = ig[0] + ix;
+                        if (x >= g.n[0]) x -= g.n[0];
+                        q[iy][ix] = pot[((size_t)x * ny + y) * nz + z];
+                    }
+                }
+                R b00 = 0, b10 = 0, b01 = 0;
+#pragma unroll
+                for (int iy = 0; iy < kOrder; iy++) {
+                    R a0 = 0, a1 = 0;
+#pragma unroll
+                    for (int ix = 0; ix < kOrder; ix++) {
+                        a0 += q[iy][ix] * tx[ix][0];
+                        a1 += q[iy][ix] * tx[ix][1];
+                    }
+                    b00 += a0 * ty[iy][0];
+                    b10 += a1 * ty[iy][0];
+                    b01 += a0 * ty[iy][1];
+                }
+                // this lane's z weights (a select: a runtime index would put the table in scratch memory)
+                R c[2];
+                spline_at<R, 1>(tz, iz, c);
+                s100 = b10 * c[0];
+                s010 = b01 * c[0];
+                s001 = b00 * c[1];
+            }
+#pragma unroll
+            for (int off = 1; off < 8; off <<= 1) {
+                s100 += __shfl_xor(s100, off);
+                s010 += __shfl_xor(s010, off);
+                s001 += __shfl_xor(s001, off);
+            }
+        }
+        if (tv && iz == 0) {
+            const V3<R> e = cart_vector(mk(s100, s010, s001), g.A);
+            const R* f = field + 3 * (size_t)t;
+            acc += operator_row<R>(st, t, i, mk((double)f[0] - (double)e.x, (double)f[1] - (double)e.y,
+                                                (double)f[2] - (double)e.z),
+                                   mu, selfc, v, Av);
+        }
+    }
+    if (partial) {
+        if (iz == 0) sdot[grp] = acc;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double s = 0.0;
+#pragma unroll
+            for (int k = 0; k < kGatherSites; k++) s += sdot[k];
+            partial[blockIdx.x] = s;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// conjugate gradients
+// ---------------------------------------------------------------------------
+// The solver's stopping test, the same expression as the host's report:
+// converged when the RMS of S r, in Debye, is below stop_eps.
+__device__ __forceinline__ double cg_stopped(double ss, int n, double stop_eps) {
+    return kDebye * sqrt(ss / (double)n) >= stop_eps ? 0.0 : 1.0;
+}
+// Publishes check c of a solve (the state after c iterations): |r|^2 in
+// scal[c & 1], scal[kCgCount] = c, scal[kCgStop] = the stopping test, and in
+// host slot c & 1 the pair (|S r|^2, stop).  Slots alternate so that the host
+// can read check c while the iteration after it is already running.
+__device__ __forceinline__ void cg_publish(double* scal, double* hcheck, int c, double rr, double ss, double stop) {
+    scal[c & 1] = rr;
+    scal[kCgCount] = (double)c;
+    scal[kCgStop] = stop;
+    double* slot = hcheck + 2 * (c & 1);
+    slot[0] = ss;
+    slot[1] = stop;
+}
+
+// At most kOneSites sites: a whole update in one workgroup of 1024 threads
+// (two sites a thread, everything loaded at once).  START: check 0 of a solve,
+// r = rhs - Ax (Ax null: x = 0, r = rhs), p = r, mu = S p.  Else one iteration
+// from Ap and the partials of p.Ap: a = rr / p.Ap, x += a p, r -= a Ap, the
+// check, p = r + beta p and mu = S p.  More sites: the same in two kernels
+// (k_cg_step, k_cg_direction) over many workgroups.
+constexpr int kOneThreads = 1024, kOnePer = kOneSites / kOneThreads;
+template <class R, bool START>
+__global__ __launch_bounds__(kOneThreads) void k_cg_one(SolverSites st, const double* __restrict__ rhs,
+                                                        const double* __restrict__ Ap, double* x, double* r, double* p,
+                                                        R* __restrict__ mu, const double* __restrict__ partial,
+                                                        int npartial, double* scal, double* hcheck, int n,
+                                                        double stop_eps) {
+    if (!START && scal[kCgStop] != 0.0) return;
+    __shared__ double sh[2 * kOneThreads / 64];
+    const int c0 = START ? 0 : (int)scal[kCgCount];
+    const double rr0 = START ? 0.0 : scal[c0 & 1];
+    D3 rv[kOnePer], pv[kOnePer], av[kOnePer], xv[kOnePer];
+    double S[kOnePer][6];
+    int idx[kOnePer];
+#pragma unroll
+    for (int u = 0; u < kOnePer; u++) {
+        const int t = threadIdx.x + u * kOneThreads;
+        if (t >= st.npol) continue;
+        idx[u] = st.idx[t];
+        av[u] = Ap ? load3(Ap, t) : mk(0.0, 0.0, 0.0);
+        rv[u] = load3(START ? rhs : r, t);
+        if (!START) {
+            pv[u] = load3(p, t);
+            xv[u] = load3(x, t);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kOnePer; u++)
+        if ((int)threadIdx.x + u * kOneThreads < st.npol)
+#pragma unroll
+            for (int k = 0; k < 6; k++) S[u][k] = st.S[6 * (size_t)idx[u] + k];
+    double a = 1.0;
+    if (!START) {
+        double pAp[1];
+        sum_partials<kOneThreads, 1>(partial, npartial, pAp, sh);
+        a = pAp[0] != 0.0 ? rr0 / pAp[0] : 0.0;
+    }
+    double s2[2] = {0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < kOnePer; u++) {
+        if ((int)threadIdx.x + u * kOneThreads >= st.npol) continue;
+        if (!START) xv[u] = xv[u] + pv[u] * a;
+        rv[u] = rv[u] - av[u] * a;
+        const D3 sr = sym_mul6(S[u], rv[u]);
+        s2[0] += dot(rv[u], rv[u]);
+        s2[1] += dot(sr, sr);
+    }
+    group_sum<kOneThreads, 2>(s2, sh);  // every thread has read scal by its barriers
+    const double beta = START || rr0 == 0.0 ? 0.0 : s2[0] / rr0;
+    if (threadIdx.x == 0)
+        cg_publish(scal, hcheck, START ? 0 : c0 + 1, s2[0], s2[1], cg_stopped(s2[1], n, stop_eps));
+#pragma unroll
+    for (int u = 0; u < kOnePer; u++) {
+        const int t = threadIdx.x + u * kOneThreads;
+        if (t >= st.npol) continue;
+        const D3 d = START ? rv[u] : rv[u] + pv[u] * beta;
+        if (!START) store3(x, t, xv[u]);
+        else if (!Ap) store3(x, t, mk(0.0, 0.0, 0.0));
+        store3(r, t, rv[u]);
+        store3(p, t, d);
+        store_mu<R>(mu, idx[u], sym_mul6(S[u], d));
+    }
+}
+
+// x += a p, r -= a Ap (START: r = rhs - Ax) with partial sums of r.r and |S r|^2
+template <bool START>
+__global__ __launch_bounds__(256) void k_cg_step(SolverSites st, const double* __restrict__ rhs,
+                                                 const double* __restrict__ Ap, double* x, double* r,
+                                                 const double* __restrict__ p, const double* __restrict__ pap,
+                                                 int npap, double* __restrict__ partial, double* scal) {
+    if (!START && scal[kCgStop] != 0.0) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) scal[kCgCur] = -1.0;
+        return;
+    }
+    __shared__ double sh[2 * 4];
+    double a = 1.0;
+    if (!START) {
+        const int c = (int)scal[kCgCount];
+        double pAp[1];
+        sum_partials<256, 1>(pap, npap, pAp, sh);
+        a = pAp[0] != 0.0 ? scal[c & 1] / pAp[0] : 0.0;
+        // k_cg_direction takes the count from here: it rewrites the other
+        if (blockIdx.x == 0 && threadIdx.x == 0) scal[kCgCur] = (double)c;
+    }
+    double s2[2] = {0.0, 0.0};
+    for (int t = blockIdx.x * 256 + threadIdx.x; t < st.npol; t += gridDim.x * 256) {
+        D3 rv = load3(START ? rhs : r, t);
+        if (Ap) rv = rv - load3(Ap, t) * a;
+        if (!START) store3(x, t, load3(x, t) + load3(p, t) * a);
+        else if (!Ap) store3(x, t, mk(0.0, 0.0, 0.0));
+        store3(r, t, rv);
+        const D3 sr = sym_mul6(st.S + 6 * (size_t)st.idx[t], rv);
+        s2[0] += dot(rv, rv);
+        s2[1] += dot(sr, sr);
+    }
+    group_sum<256, 2>(s2, sh);
+    if (threadIdx.x == 0) {
+        partial[blockIdx.x] = s2[0];
+        partial[kMaxPartials + blockIdx.x] = s2[1];
+    }
+}
+// beta and the iteration's check (workgroup 0 publishes it), p = r + beta p
+// and the next operator input mu = S p.  The iteration's number comes from
+// k_cg_step in scal[kCgCur] (-1: the solve had stopped), which no workgroup
+// of this kernel writes.
+template <class R, bool START>
+__global__ __launch_bounds__(256) void k_cg_direction(SolverSites st, const double* __restrict__ r, double* p,
+                                                      R* __restrict__ mu, const double* __restrict__ partial,
+                                                      int npartial, double* scal, double* hcheck, int n,
+                                                      double stop_eps) {
+    __shared__ double sh[2 * 4];
+    const int c = START ? 0 : (int)scal[kCgCur];
+    if (c < 0) return;
+    const double rr0 = START ? 0.0 : scal[c & 1];
+    double s2[2];
+    sum_partials<256, 2>(partial, npartial, s2, sh);
+    const double beta = rr0 != 0.0 ? s2[0] / rr0 : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        cg_publish(scal, hcheck, START ? 0 : c + 1, s2[0], s2[1], cg_stopped(s2[1], n, stop_eps));
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= st.npol) return;
+    D3 d = load3(r, t);
+    if (!START) d = d + load3(p, t) * beta;
+    store3(p, t, d);
+    const int i = st.idx[t];
+    store_mu<R>(mu, i, sym_mul6(st.S + 6 * (size_t)i, d));
+}
+
+// ---------------------------------------------------------------------------
+// vectors
+// ---------------------------------------------------------------------------
+// b = S E0, x = b and the first operator input mu = S x (in both precisions
+// where mu2 is given); zeros at every other atom of mu, mu2 and mud.
+template <class R>
+__global__ __launch_bounds__(256) void k_solver_init(SolverSites st, int n, const double4* __restrict__ pos,
+                                                     const double* __restrict__ E0, double* b, double* x,
+                                                     R* __restrict__ mu, double* __restrict__ mu2,
+                                                     double* __restrict__ mud) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t < n && pos[t].w == 0.0) {
+        const D3 z = mk(0.0, 0.0, 0.0);
+        store_mu<R>(mu, t, z);
+        store3(mud, t, z);
+        if (mu2) store3(mu2, t, z);
+    }
+    if (t >= st.npol) return;
+    const int i = st.idx[t];
+    const double* S = st.S + 6 * (size_t)i;
+    const D3 v = sym_mul6(S, load3(E0, i));
+    store3(b, t, v);
+    store3(x, t, v);
+    const D3 m = sym_mul6(S, v);
+    store_mu<R>(mu, i, m);
+    store3(mud, i, m);
+}
+
+// mu = S v by atom (and mud, its FP64 copy); at: by site (DIIS's errors)
+template <class R>
+__global__ __launch_bounds__(256) void k_apply_S(SolverSites st, const double* __restrict__ v, R* mu, double* mud,
+                                                 double* at) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= st.npol) return;
+    const int i = st.idx[t];
+    const D3 m = sym_mul6(st.S + 6 * (size_t)i, load3(v, t));
+    if (mu) store_mu<R>(mu, i, m);
+    if (mud) store3(mud, i, m);
+    if (at) store3(at, t, m);
+}
+
+// rt = b - A x (given Ax; null: rt is read), |S rt|^2 and x.rt: partial sums
+// per workgroup, then one workgroup writes out[0], out[1] (mapped host memory)
+__global__ __launch_bounds__(256) void k_residual(SolverSites st, const double* __restrict__ b,
+                                                  const double* __restrict__ Ax, const double* __restrict__ x,
+                                                  double* rt, double* __restrict__ partial) {
+    __shared__ double sh[2 * 4];
+    double s2[2] = {0.0, 0.0};
+    for (int t = blockIdx.x * 256 + threadIdx.x; t < st.npol; t += gridDim.x * 256) {
+        D3 v;
+        if (Ax) {
+            v = load3(b, t) - load3(Ax, t);
+            store3(rt, t, v);
+        } else {
+            v = load3(rt, t);
+        }
+        const D3 sr = sym_mul6(st.S + 6 * (size_t)st.idx[t], v);
+        s2[0] += dot(sr, sr);
+        s2[1] += dot(load3(x, t), v);
+    }
+    group_sum<256, 2>(s2, sh);
+    if (threadIdx.x == 0) {
+        partial[blockIdx.x] = s2[0];
+        partial[kMaxPartials + blockIdx.x] = s2[1];
+    }
+}
+__global__ __launch_bounds__(256) void k_residual_sum(const double* __restrict__ partial, int npartial, double* out) {
+    __shared__ double sh[2 * 4];
+    double s2[2];
+    sum_partials<256, 2>(partial, npartial, s2, sh);
+    if (threadIdx.x == 0) {
+        out[0] = s2[0];
+        out[1] = s2[1];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// launchers
+// ---------------------------------------------------------------------------
+static int site_blocks(int npol) { return std::max(1, std::min((npol + 255) / 256, kMaxPartials)); }
+
+template <class R>
+void launch_list_field(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p, const R* mu,
+                       R* field) {
+    if (st.npol <= 0) return;
+    const unsigned blocks = ((unsigned)st.npol * kNlSplit + 255) / 256;
+    hipLaunchKernelGGL(k_list_field<R>, dim3(blocks), dim3(256), 0, s, st, l, a, p, mu, field);
+}
+template <class R>
+int launch_operator(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const R* field, NbrList l,
+                    PairAtoms<R> a, PairParams<R> p, const R* mu, double selfc, const double* v, double* Av,
+                    double* partial) {
+    if (st.npol <= 0) return 0;
+    const int per = field ? kGatherSites : kOpSites;
+    const int blocks = std::min((st.npol + per - 1) / per, kMaxPartials);
+    if (field)
+        hipLaunchKernelGGL(k_operator_gather<R>, dim3(blocks), dim3(256), 0, s, st, g, pot, field, a.pos, mu, selfc, v,
+                           Av, partial);
+    else
+        hipLaunchKernelGGL(k_operator_fused<R>, dim3(blocks), dim3(256), 0, s, st, g, pot, l, a, p, mu, selfc, v, Av,
+                           partial);
+    return blocks;
+}
+template <class R>
+void launch_cg_start(hipStream_t s, SolverSites st, const double* rhs, const double* Ax, double* x, double* r,
+                     double* p, R* mu, double* partial, double* scal, double* hcheck, int n, double stop_eps) {
+    if (st.npol <= kOneSites) {
+        hipLaunchKernelGGL((k_cg_one<R, true>), dim3(1), dim3(kOneThreads), 0, s, st, rhs, Ax, x, r, p, mu, nullptr, 0,
+                           scal, hcheck, n, stop_eps);
+        return;
+    }
+    const int blocks = site_blocks(st.npol);
+    hipLaunchKernelGGL(k_cg_step<true>, dim3(blocks), dim3(256), 0, s, st, rhs, Ax, x, r, p, nullptr, 0, partial, scal);
+    hipLaunchKernelGGL((k_cg_direction<R, true>), dim3((st.npol + 255) / 256), dim3(256), 0, s, st, r, p, mu, partial,
+                       blocks, scal, hcheck, n, stop_eps);
+}
+template <class R>
+void launch_cg_iteration(hipStream_t s, SolverSites st, const double* Ap, double* x, double* r, double* p, R* mu,
+                         int npap, double* partial, double* scal, double* hcheck, int n, double stop_eps) {
+    if (st.npol <= kOneSites) {
+        hipLaunchKernelGGL((k_cg_one<R, false>), dim3(1), dim3(kOneThreads), 0, s, st, nullptr, Ap, x, r, p, mu,
+                           partial, npap, scal, hcheck, n, stop_eps);
+        return;
+    }
+    const int blocks = site_blocks(st.npol);
+    double* norms = partial + kMaxPartials;
+    hipLaunchKernelGGL(k_cg_step<false>, dim3(blocks), dim3(256), 0, s, st, nullptr, Ap, x, r, p, partial, npap, norms,
+                       scal);
+    hipLaunchKernelGGL((k_cg_direction<R, false>), dim3((st.npol + 255) / 256), dim3(256), 0, s, st, r, p, mu, norms,
+                       blocks, scal, hcheck, n, stop_eps);
+}
+template <class R>
+void launch_solver_init(hipStream_t s, SolverSites st, int n, const double4* pos, const double* E0, double* b,
+                        double* x, R* mu, double* mu2, double* mud) {
+    hipLaunchKernelGGL(k_solver_init<R>, dim3((n + 255) / 256), dim3(256), 0, s, st, n, pos, E0, b, x, mu, mu2, mud);
+}
+template <class R>
+void launch_apply_S(hipStream_t s, SolverSites st, const double* v, R* mu, double* mud, double* at) {
+    if (st.npol <= 0) return;
+    hipLaunchKernelGGL(k_apply_S<R>, dim3((st.npol + 255) / 256), dim3(256), 0, s, st, v, mu, mud, at);
+}
+void launch_residual(hipStream_t s, SolverSites st, const double* b, const double* Ax, const double* x, double* rt,
+                     double* partial, double* out) {
+    const int blocks = site_blocks(st.npol);
+    hipLaunchKernelGGL(k_residual, dim3(blocks), dim3(256), 0, s, st, b, Ax, x, rt, partial);
+    hipLaunchKernelGGL(k_residual_sum, dim3(1), dim3(256), 0, s, partial, blocks, out);
+}
+
+#define MPID_INSTANTIATE(R)                                                                                         \
+    template void launch_list_field<R>(hipStream_t, SolverSites, NbrList, PairAtoms<R>, PairParams<R>, const R*,    \
+                                       R*);                                                                        \
+    template int launch_operator<R>(hipStream_t, SolverSites, PmeGeom<R>, const R*, const R*, NbrList,              \
+                                    PairAtoms<R>, PairParams<R>, const R*, double, const double*, double*,          \
+                                    double*);                                                                      \
+    template void launch_cg_start<R>(hipStream_t, SolverSites, const double*, const double*, double*, double*,      \
+                                     double*, R*, double*, double*, double*, int, double);                          \
+    template void launch_cg_iteration<R>(hipStream_t, SolverSites, const double*, double*, double*, double*, R*,    \
+                                         int, double*, double*, double*, int, double);                              \
+    template void launch_solver_init<R>(hipStream_t, SolverSites, int, const double4*, const double*, double*,      \
+                                        double*, R*, double*, double*);                                            \
+    template void launch_apply_S<R>(hipStream_t, SolverSites, const double*, R*, double*, double*);
+MPID_INSTANTIATE(float)
+MPID_INSTANTIATE(double)
+#undef MPID_INSTANTIATE
+
+}  // namespace mpid

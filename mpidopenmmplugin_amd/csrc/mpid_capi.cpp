@@ -159,9 +159,12 @@ template <class R> struct Prec {
     DBuf<R> lab;
     DBuf<R2<R>> td;
     DBuf<R> mu;       // induced dipoles in this precision (matvec input)
-    DBuf<R> erec;     // reciprocal induced field
+    DBuf<R> erec;     // reciprocal induced field (inspection entry point)
+    DBuf<R> elist;    // real-space induced field at the polarisable sites
     DBuf<R> phi, phidp;
-    DBuf<R> grid;       // real charge / potential grid [n0][n1][n2]
+    DBuf<R> grid;       // real charge grid [n0][n1][n2]; left zero between cycles unless owned cores write it whole
+    DBuf<R> pot;        // potential grid (the charge grid itself when owned cores write that whole)
+    bool grid_dirty = false;  // spread into, but its transform is not issued (an evaluation that failed in between)
     DBuf<R2<R>> spec;   // half spectrum [n0][n1][n2/2+1]
     DBuf<double> moduli;  // |b(k)|^2 in FP64, [n0 | n1 | n2]
     DBuf<R> infl;         // the influence function on the half spectrum (launch_influence_table)
@@ -233,12 +236,8 @@ struct mpid_context {
     hipEvent_t ev_v = nullptr, ev_vdone = nullptr;
     bool final_issued = false;  // the final pass of the current solution is on its way
     bool defer_final = false;   // the solve leaves the final pass to its caller (energy gradients)
-    // CG iterations are replayed from a graph captured once per solve (its
-    // kernel arguments are those of that solve); hscal is the pinned host
-    // copy of the residual norm that each replay leaves behind.
-    hipGraphExec_t cg_exec = nullptr;
     double* hscal_dev = nullptr;  // device address of hscal (pinned, mapped)
-    double* hscal = nullptr;  // [1] read_scalar, [2] energy-correction dot, [3] (as int) the block-row count,
+    double* hscal = nullptr;  // [1] |S r|^2 of the last residual, [2] its product with x, [3] (as int) the block-row count,
                               // [kCheck ..] the solver's two check slots (|S r|^2, stop)
     static constexpr int kCheck = 8;
     hipEvent_t ev_check[2] = {nullptr, nullptr};  // recorded after the work that publishes check c (c & 1)
@@ -318,11 +317,7 @@ struct mpid_context {
 
     // profiling: bit c of prof_mask times the work booked to category c
     unsigned prof_mask = 0;
-    bool capturing = false;  // recording the solver's iteration graph: no timing events
-    // the categories of the work inside one solver iteration; timing any of
-    // them makes the iterations run eagerly instead of from the graph
-    static constexpr unsigned kIterationCats = (1u << P_SPREAD) | (1u << P_FFT) | (1u << P_GATHER) |
-                                               (1u << P_INDUCED) | (1u << P_COV) | (1u << P_SOLVER);
+    bool in_iteration = false;  // issuing a solver iteration: its kernels take the stop flag
     struct Ev { int cat; hipEvent_t a, b; };
     std::vector<Ev> events;
     std::vector<hipEvent_t> pool;
@@ -338,7 +333,6 @@ struct mpid_context {
         for (hipStream_t s : {stream, rstream, vstream})
             if (s) (void)hipStreamSynchronize(s);
         for (auto e : pool) (void)hipEventDestroy(e);
-        if (cg_exec) (void)hipGraphExecDestroy(cg_exec);
         if (hscal) (void)hipHostFree(hscal);
         if (hnl) (void)hipHostFree(hnl);
         if (ev_fork) (void)hipEventDestroy(ev_fork);
@@ -365,7 +359,7 @@ struct mpid_context {
     // device time of the work that f issues to stream s, booked to cat
     template <class F> void timed_on(hipStream_t s, int cat, F&& f) {
         if (prof_override >= 0) cat = prof_override;
-        if (capturing || !((prof_mask >> cat) & 1u)) {
+        if (!((prof_mask >> cat) & 1u)) {
             f();
             return;
         }
@@ -606,13 +600,12 @@ struct mpid_context {
         P.td.resize(n);
         P.mu.resize(3 * (size_t)n);
         P.erec.resize(3 * (size_t)n);
-        // the solver gathers the field at polarisable sites only; the other
-        // entries stay zero (they are multiplied by S = 0, which needs them finite)
-        HIP_CHECK(hipMemsetAsync(P.erec.p, 0, P.erec.n * sizeof(R), stream));
+        P.elist.resize(3 * (size_t)n);
         P.phi.resize(35 * (size_t)n);
         P.phidp.resize(35 * (size_t)n);
         if (!pme()) {
             // no reciprocal space: the potentials and fields it would give stay zero
+            HIP_CHECK(hipMemsetAsync(P.erec.p, 0, P.erec.n * sizeof(R), stream));
             HIP_CHECK(hipMemsetAsync(P.phi.p, 0, P.phi.n * sizeof(R), stream));
             HIP_CHECK(hipMemsetAsync(P.phidp.p, 0, P.phidp.n * sizeof(R), stream));
             HIP_CHECK(hipStreamSynchronize(stream));
@@ -620,6 +613,10 @@ struct mpid_context {
             return;
         }
         P.grid.resize(G);
+        if (!owner_spread) {
+            P.pot.resize(G);
+            HIP_CHECK(hipMemsetAsync(P.grid.p, 0, G * sizeof(R), stream));
+        }
         P.spec.resize((size_t)opt.grid[0] * opt.grid[1] * (opt.grid[2] / 2 + 1));
         std::vector<double> mods;
         for (int k = 0; k < 3; k++) {
@@ -695,7 +692,7 @@ struct mpid_context {
         mud.resize(n3);
         tmp3n.resize(n3);
         fout.resize(n3);
-        partial.resize(2 * 512);
+        partial.resize(3 * kMaxPartials);
         scal.resize(kScalars);
         choose_tiles();
         if (opt.precision == MPID_PRECISION_MIXED) init_prec(pf);
@@ -822,9 +819,9 @@ struct mpid_context {
         g.skip = iteration_skip();
         return g;
     }
-    // Kernels recorded into the solver's iteration graph take the stop flag:
-    // an iteration issued after the solve has stopped does no work.
-    const double* iteration_skip() const { return capturing ? scal.p + kCgStop : nullptr; }
+    // Kernels of a solver iteration take the stop flag: an iteration issued
+    // after the solve has stopped does no work.
+    const double* iteration_skip() const { return in_iteration ? scal.p + kCgStop : nullptr; }
     template <class R> PairParams<R> pair_params() const {
         PairParams<R> P;
         P.box = rbox<R>();
@@ -1059,28 +1056,45 @@ struct mpid_context {
         P.infl_valid = true;
     }
 
-    // Reciprocal cycles: issued to rstream after a fork(); the caller joins
-    // before it reads their output (phi, phidp, erec).
-    // Issued in two parts: the spreading first, the transforms and the gather
-    // once the neighbour-list kernels are issued (the host's launches would
-    // otherwise hold those back while the spreading runs).
+    // Reciprocal cycles: spreading, transforms, and a gather.  An untiled or
+    // windowed spreading adds into a grid that the previous cycle's first
+    // transform left zero; owned cores write the grid whole and are
+    // transformed in place.
+    template <class R> R* potential(Prec<R>& P) const { return P.pot.p ? P.pot.p : P.grid.p; }
+    template <class R> void clean_grid(Prec<R>& P, hipStream_t s) {
+        if (P.grid_dirty && P.pot.p) launch_fill<R>(s, P.grid.p, P.grid.n, R(0));
+        P.grid_dirty = true;
+    }
+    template <class R> void fold(Prec<R>& P, const PmeGeom<R>& g, hipStream_t s) {
+        if (fold_by_tiles(tgeom)) launch_fold_tiles<R>(s, g, tgeom, P.scratch.p, P.grid.p);
+        else launch_fold<R>(s, g, tgeom, P.scratch.p, P.grid.p);
+    }
+    template <class R> void convolve(Prec<R>& P, hipStream_t s) {
+        timed_on(s, P_FFT, [&] {
+            launch_recip_convolution<R>(s, P.plan, P.grid.p, P.spec.p, potential(P), conv_params(P));
+        });
+        P.grid_dirty = false;
+    }
+    // The permanent multipoles' cycle, on rstream after a fork(); the caller
+    // joins before it reads phi.  Issued in two parts: the spreading first,
+    // the transforms and the gather once the neighbour-list kernels are
+    // issued (the host's launches would otherwise hold those back while the
+    // spreading runs).
     bool fixed_recip_rest = false;
     template <class R> void recip_cycle_fixed(Prec<R>& P) {
         if (!pme()) return;  // phi stays zero
         PmeGeom<R> g = geom<R>();
         fork();
-        const size_t G = P.grid.n;
         timed_on(rstream, P_SPREAD, [&] {
             if (owner_spread) {
                 launch_spread_fixed_owner<R>(rstream, P.pos.p, P.lab.p, g, tgeom, tstart.p, tend.p, P.grid.p);
                 return;
             }
-            launch_fill<R>(rstream, P.grid.p, G, R(0));
+            clean_grid(P, rstream);
             if (tiled_spread) {
                 launch_spread_fixed_tiled<R>(rstream, P.pos.p, P.lab.p, g, tgeom, tstart.p, tend.p, P.scratch.p,
                                              P.grid.p);
-                if (fold_by_tiles(tgeom)) launch_fold_tiles<R>(rstream, g, tgeom, P.scratch.p, P.grid.p);
-                else launch_fold<R>(rstream, g, tgeom, P.scratch.p, P.grid.p);
+                fold(P, g, rstream);
             } else {
                 launch_spread_fixed<R>(rstream, n, P.pos.p, P.lab.p, g, P.grid.p);
             }
@@ -1092,51 +1106,47 @@ struct mpid_context {
         if (!fixed_recip_rest) return;
         fixed_recip_rest = false;
         PmeGeom<R> g = geom<R>();
-        timed_on(rstream, P_FFT, [&] { launch_recip_convolution<R>(rstream, P.plan, P.grid.p, P.spec.p, conv_params(P)); });
-        timed_on(rstream, P_GATHER, [&] { launch_gather_phi<R>(rstream, n, P.pos.p, g, P.grid.p, P.phi.p); });
+        convolve(P, rstream);
+        timed_on(rstream, P_GATHER,
+                 [&] { launch_gather_phi<R>(rstream, n, P.pos.p, g, potential(P), P.phi.p); });
         check_launch();
     }
 
-    // Reciprocal part of the field of the induced dipoles in P.mu.  Unless
-    // all_atoms, mu is known to vanish on unpolarisable sites: only the
-    // polarisable ones are spread, and (full == false) only their field is
-    // gathered.  full: the 35 potential derivatives at every atom (forces).
-    // forked: the caller has already made rstream wait for its work
-    template <class R> void recip_cycle_induced(Prec<R>& P, bool full, bool all_atoms = false, bool forked = false) {
-        if (!pme()) return;  // erec and phidp stay zero
+    // The potential grid of the induced dipoles in P.mu.  Unless all_atoms,
+    // mu is known to vanish on unpolarisable sites: only the polarisable ones
+    // are spread.
+    template <class R> void recip_potential(Prec<R>& P, hipStream_t s, bool all_atoms = false) {
+        if (!pme()) return;
         PmeGeom<R> g = geom<R>();
-        if (!forked) fork();
-        const size_t G = P.grid.n;
-        timed_on(rstream, P_SPREAD, [&] {
+        const int* atoms = all_atoms ? nullptr : pol_idx.p;
+        const int* first = all_atoms ? tstart.p : tpstart.p;
+        const int* last = all_atoms ? tend.p : tpend.p;
+        timed_on(s, P_SPREAD, [&] {
             if (owner_spread) {
-                if (all_atoms)
-                    launch_spread_induced_owner<R>(rstream, P.pos.p, P.mu.p, g, tgeom, nullptr, tstart.p, tend.p,
-                                                   P.grid.p);
-                else
-                    launch_spread_induced_owner<R>(rstream, P.pos.p, P.mu.p, g, tgeom, pol_idx.p, tpstart.p,
-                                                   tpend.p, P.grid.p);
+                launch_spread_induced_owner<R>(s, P.pos.p, P.mu.p, g, tgeom, atoms, first, last, P.grid.p);
                 return;
             }
-            launch_fill<R>(rstream, P.grid.p, G, R(0));
+            clean_grid(P, s);
             if (tiled_spread) {
-                if (all_atoms)
-                    launch_spread_induced_tiled<R>(rstream, P.pos.p, P.mu.p, g, tgeom, nullptr, tstart.p, tend.p,
-                                                   P.scratch.p, P.grid.p);
-                else
-                    launch_spread_induced_tiled<R>(rstream, P.pos.p, P.mu.p, g, tgeom, pol_idx.p, tpstart.p, tpend.p,
-                                                   P.scratch.p, P.grid.p);
-                if (fold_by_tiles(tgeom)) launch_fold_tiles<R>(rstream, g, tgeom, P.scratch.p, P.grid.p);
-                else launch_fold<R>(rstream, g, tgeom, P.scratch.p, P.grid.p);
+                launch_spread_induced_tiled<R>(s, P.pos.p, P.mu.p, g, tgeom, atoms, first, last, P.scratch.p,
+                                               P.grid.p);
+                fold(P, g, s);
             } else {
-                launch_spread_induced<R>(rstream, n, P.pos.p, P.mu.p, g, P.grid.p);
+                launch_spread_induced<R>(s, all_atoms ? n : npol, atoms, P.pos.p, P.mu.p, g, P.grid.p);
             }
         });
-        timed_on(rstream, P_FFT, [&] { launch_recip_convolution<R>(rstream, P.plan, P.grid.p, P.spec.p, conv_params(P)); });
-        timed_on(rstream, P_GATHER, [&] {
-            if (full) launch_gather_phi<R>(rstream, n, P.pos.p, g, P.grid.p, P.phidp.p);
-            else if (all_atoms) launch_gather_field<R>(rstream, n, nullptr, P.pos.p, g, P.grid.p, P.erec.p);
-            else launch_gather_field<R>(rstream, npol, pol_idx.p, P.pos.p, g, P.grid.p, P.erec.p);
-        });
+        convolve(P, s);
+        check_launch();
+    }
+    // The 35 potential derivatives of the induced dipoles at every atom
+    // (phidp), on rstream after a fork(); the caller joins before it reads them.
+    template <class R> void recip_cycle_induced(Prec<R>& P) {
+        if (!pme()) return;  // phidp stays zero
+        fork();
+        recip_potential(P, rstream);
+        PmeGeom<R> g = geom<R>();
+        timed_on(rstream, P_GATHER,
+                 [&] { launch_gather_phi<R>(rstream, n, P.pos.p, g, potential(P), P.phidp.p); });
         check_launch();
     }
 
@@ -1170,78 +1180,55 @@ struct mpid_context {
         check_launch();
     }
 
-    // Field T*mu of the induced dipoles in P.mu: accumulator + P.erec.  In the
-    // solver (all_atoms false) mu vanishes on unpolarisable sites and the field
-    // is only used on polarisable ones, so only pairs of polarisable sites are
-    // visited; all_atoms gives the field of an arbitrary mu everywhere.
-    // The reciprocal part goes to rstream first and runs beside the pair
-    // kernels; the caller joins before it reads erec.
-    template <class R> void induced_field(Prec<R>& P, bool all_atoms = false) {
-        check_lists(all_atoms);
-        recip_cycle_induced(P, false, all_atoms);
-        timed(P_INDUCED, [&] {
-            launch_zero_acc(stream, field_acc.p, field_acc.n, iteration_skip());
-            if (all_atoms)
-                launch_nl_induced_field<R>(stream, n, nullptr, nlist(), pair_atoms(P), P.mu.p, pair_params<R>(),
-                                           field_acc.p);
-            else
-                launch_nl_induced_field<R>(stream, npol, pol_idx.p, nlist_pol(), pair_atoms(P), P.mu.p,
-                                           pair_params<R>(), field_acc.p);
-        });
-        timed(P_COV, [&] {
-            launch_cov_induced_field<R>(stream, n, pair_atoms(P), P.mu.p, pair_params<R>(), all_atoms ? 0 : 1,
-                                        field_acc.p);
-        });
+    // Field T*mu of an arbitrary mu in P.mu at every atom (the inspection
+    // entry point): accumulator + P.erec.
+    template <class R> void induced_field_all(Prec<R>& P) {
+        check_lists(true);
+        recip_potential(P, stream, true);
+        if (pme())
+            launch_gather_field<R>(stream, n, nullptr, P.pos.p, geom<R>(), potential(P), P.erec.p);
+        launch_zero_acc(stream, field_acc.p, field_acc.n);
+        launch_nl_induced_field<R>(stream, n, nullptr, nlist(), pair_atoms(P), P.mu.p, pair_params<R>(), field_acc.p);
+        launch_cov_induced_field<R>(stream, n, pair_atoms(P), P.mu.p, pair_params<R>(), 0, field_acc.p);
+        check_launch();
     }
 
-    // Av = v - S T S v
-    template <class R> void matvec(Prec<R>& P, const double* v, double* Av) {
-        timed(P_SOLVER, [&] { launch_apply_S<R>(stream, n, sqrtpol.p, v, P.mu.p, nullptr); });
-        induced_field(P);
-        join();
-        timed(P_SOLVER, [&] {
-            launch_matvec_finish<R>(stream, n, sqrtpol.p, field_acc.p, P.erec.p, P.mu.p, selfc(), v, Av);
+    SolverSites sites() const { return SolverSites{npol, pol_idx.p, sqrtpol.p}; }
+    // Up to kFusedSites polarisable sites the operator's kernel adds the
+    // real-space field itself; beyond, the list kernel runs on rstream beside
+    // the reciprocal chain.  At 4,096 sites an evaluation takes 0.91 ms this
+    // way against 1.03 ms with the two kernels and their cross-stream waits
+    // (FP64: 1.04 against 1.14 ms); at 32,768 sites the list walk (20 us in
+    // FP32) would sit on the critical path, where it now overlaps the chain.
+    static constexpr int kFusedSites = 8192;
+
+    // Av = v - S T S v with P.mu = S v in place; returns the number of partial
+    // sums of v.Av left in `part` (if given).
+    template <class R> int apply_operator(Prec<R>& P, const double* v, double* Av, double* part) {
+        check_lists(false);
+        const bool fused = npol <= kFusedSites;
+        const NbrList l = nlist_pol();
+        if (!fused) {
+            fork();
+            timed_on(rstream, P_INDUCED, [&] {
+                launch_list_field<R>(rstream, sites(), l, pair_atoms(P), pair_params<R>(), P.mu.p, P.elist.p);
+            });
+        }
+        recip_potential(P, stream);
+        if (!fused) join();
+        int parts = 0;
+        timed(fused ? P_INDUCED : P_GATHER, [&] {
+            parts = launch_operator<R>(stream, sites(), pme() ? geom<R>() : PmeGeom<R>{},
+                                       pme() ? potential(P) : nullptr, fused ? nullptr : P.elist.p, l, pair_atoms(P),
+                                       pair_params<R>(), P.mu.p, selfc(), v, Av, part);
         });
         check_launch();
         stats.matvecs++;
+        return parts;
     }
-
-    // Records f (one CG iteration on stream and rstream, which leaves the
-    // residual norm in hscal[0]) into cg_exec: the executable graph is
-    // updated in place when its topology is unchanged, else instantiated.
-    template <class F> void capture_cg(F&& f) {
-        hipGraph_t g = nullptr;
-        HIP_CHECK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        capturing = true;
-        try {
-            f();
-        } catch (...) {
-            capturing = false;
-            hipGraph_t dead = nullptr;
-            (void)hipStreamEndCapture(stream, &dead);
-            if (dead) (void)hipGraphDestroy(dead);
-            throw;
-        }
-        capturing = false;
-        HIP_CHECK(hipStreamEndCapture(stream, &g));
-        bool updated = false;
-        if (cg_exec) {
-            hipGraphNode_t err = nullptr;
-            hipGraphExecUpdateResult res = hipGraphExecUpdateError;
-            updated = hipGraphExecUpdate(cg_exec, g, &err, &res) == hipSuccess && res == hipGraphExecUpdateSuccess;
-            if (!updated) {
-                (void)hipGetLastError();
-                (void)hipGraphExecDestroy(cg_exec);
-                cg_exec = nullptr;
-            }
-        }
-        hipError_t e = hipSuccess;
-        if (!updated) e = hipGraphInstantiate(&cg_exec, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (e != hipSuccess) {
-            cg_exec = nullptr;
-            throw HipError(std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
-        }
+    template <class R> void matvec(Prec<R>& P, const double* v, double* Av) {
+        timed(P_SOLVER, [&] { launch_apply_S<R>(stream, sites(), v, P.mu.p, nullptr, nullptr); });
+        apply_operator<R>(P, v, Av, nullptr);
     }
 
     // Waits for the work issued to stream so far by polling an event: the
@@ -1258,73 +1245,54 @@ struct mpid_context {
             if (q != hipErrorNotReady) HIP_CHECK(q);
         }
     }
-    double read_scalar(const double* d) {
-        HIP_CHECK(hipMemcpyAsync(hscal + 1, d, sizeof(double), hipMemcpyDeviceToHost, stream));
-        wait_stream();
-        return hscal[1];
-    }
     double debye_eps(double ss) const { return kDebye * std::sqrt(ss / n); }
 
     // Conjugate gradients on (I - S T S) sol = rhs.  With zero_start the
     // iteration starts from sol = 0 (r = rhs), else from the current sol.
     // Stops when the RMS-Debye norm of S r falls below stop_eps; returns it.
     //
-    // The device makes the stopping test (check c after c iterations, see
-    // launch_cg_begin) and the host reads it from pinned memory.  Replayed
-    // from the graph, the next iteration is issued before the host reads the
-    // previous check, so the device never waits for the host; an iteration
-    // issued after the solve has stopped does no work.
+    // The device makes the stopping test (check c after c iterations) and the
+    // host reads it from pinned memory.  The next iteration is issued before
+    // the host reads the previous check, so the device never waits for the
+    // host; an iteration issued after the solve has stopped does no work.
+    // (The iterations are issued kernel by kernel: recording them into a
+    // graph cost 60-100 us of host time per solve, with the device idle on
+    // small systems, and saved nothing once an iteration was 6-9 kernels.)
+    // mu_ready: P.mu = S sol already.
     template <class R>
-    double cg(Prec<R>& P, double* sol, const double* rhs, bool zero_start, double stop_eps, int& iters, int max_iter) {
-        const int n3 = 3 * n;
-        auto body = [&] {
-            induced_field(P);
-            join();
-            timed(P_SOLVER, [&] {
-                launch_cg_iteration<R>(stream, n, sqrtpol.p, field_acc.p, P.erec.p, P.mu.p, selfc(), p.p, Ap.p, sol,
-                                       r.p, partial.p, scal.p, hscal_dev + kCheck, stop_eps);
-            });
-        };
-        // The iteration graph is recorded first: the host does it while the
-        // device still runs the work issued before.  (Timing events cannot sit
-        // in a graph: when the iteration's categories are timed, the loop runs
-        // eagerly and the host reads every check before the next iteration.)
-        const bool eager = (prof_mask & kIterationCats) != 0;
-        if (!eager && iters < max_iter) capture_cg(body);
-        timed(P_SOLVER, [&] {
-            if (zero_start) {
-                launch_fill<double>(stream, sol, n3, 0.0);
-                HIP_CHECK(hipMemcpyAsync(r.p, rhs, n3 * sizeof(double), hipMemcpyDeviceToDevice, stream));
-            }
-        });
+    double cg(Prec<R>& P, double* sol, const double* rhs, bool zero_start, double stop_eps, int& iters, int max_iter,
+              bool mu_ready = false) {
         if (!zero_start) {
-            matvec(P, sol, Ap.p);
-            timed(P_SOLVER, [&] { launch_sub(stream, n3, rhs, Ap.p, r.p); });
+            if (mu_ready) apply_operator<R>(P, sol, Ap.p, nullptr);
+            else matvec(P, sol, Ap.p);
         }
         timed(P_SOLVER, [&] {
-            HIP_CHECK(hipMemcpyAsync(p.p, r.p, n3 * sizeof(double), hipMemcpyDeviceToDevice, stream));
-            launch_residual_norm(stream, n, sqrtpol.p, r.p, partial.p, scal.p + 2);  // scal[2] = rr, scal[3] = ss
-            HIP_CHECK(hipMemcpyAsync(scal.p, scal.p + 2, sizeof(double), hipMemcpyDeviceToDevice, stream));
-            launch_cg_begin(stream, n, scal.p, hscal_dev + kCheck, stop_eps);
-            // the first direction's operator input (each iteration leaves the
-            // next one's behind); issued before the norm is known
-            launch_apply_S<R>(stream, n, sqrtpol.p, p.p, P.mu.p, nullptr);
+            launch_cg_start<R>(stream, sites(), rhs, zero_start ? nullptr : Ap.p, sol, r.p, p.p, P.mu.p, partial.p,
+                               scal.p, hscal_dev + kCheck, n, stop_eps);
         });
+        check_launch();
         HIP_CHECK(hipEventRecord(ev_check[0], stream));
-        const int iters0 = iters;
+        const int iters0 = iters, matvecs0 = stats.matvecs;
         int issued = 0, seen = 0;  // iterations issued; the check the host reads next
         auto issue = [&] {
             if (iters0 + issued >= max_iter) return;
-            if (eager) {
-                body();
+            in_iteration = true;
+            try {
+                const int parts = apply_operator<R>(P, p.p, Ap.p, partial.p);
+                timed(P_SOLVER, [&] {
+                    launch_cg_iteration<R>(stream, sites(), Ap.p, sol, r.p, p.p, P.mu.p, parts, partial.p, scal.p,
+                                           hscal_dev + kCheck, n, stop_eps);
+                });
                 check_launch();
-            } else {
-                HIP_CHECK(hipGraphLaunch(cg_exec, stream));
+            } catch (...) {
+                in_iteration = false;
+                throw;
             }
+            in_iteration = false;
             issued++;
             HIP_CHECK(hipEventRecord(ev_check[issued & 1], stream));
         };
-        if (!eager) issue();
+        issue();
         double eps;
         for (;;) {
             wait_event(ev_check[seen & 1]);
@@ -1332,13 +1300,12 @@ struct mpid_context {
             const double* c = hscal + kCheck + 2 * (seen & 1);
             eps = debye_eps(c[0]);
             if (c[1] != 0.0) break;  // converged: an iteration issued after this one does nothing
-            if (eager) issue();
             if (issued == seen) break;  // the iteration limit
             seen++;                     // iteration `seen` runs (issued, and the solve had not stopped)
-            if (!eager) issue();        // one iteration ahead of the host
+            issue();                    // one iteration ahead of the host
         }
         iters = iters0 + seen;
-        stats.matvecs += seen;
+        stats.matvecs = matvecs0 + seen;
         return eps;
     }
 
@@ -1357,9 +1324,9 @@ struct mpid_context {
         ptE.resize((size_t)std::max(1, N - 1) * n3);
         ptG.resize((size_t)std::max(1, N - 1) * n6);
         grad_acc.resize(n6);
-        timed(P_SOLVER, [&] { launch_apply_S<R>(stream, n, sqrtpol.p, b.p, P.mu.p, ptmu.p); });
+        timed(P_SOLVER, [&] { launch_extrap_init<R>(stream, n, labpol.p, E0.p, ptmu.p, P.mu.p); });
         for (int m = 0; m + 1 < N; m++) {
-            recip_cycle_induced(P, true);  // phidp of mu_(m) at every atom, on rstream
+            recip_cycle_induced(P);  // phidp of mu_(m) at every atom, on rstream
             timed(P_INDUCED, [&] {
                 launch_zero_acc(stream, field_acc.p, field_acc.n);
                 launch_zero_acc(stream, grad_acc.p, grad_acc.n);
@@ -1399,10 +1366,10 @@ struct mpid_context {
     static constexpr int kDiisHistory = 20;
     DBuf<double> diis_d, diis_e, diis_dots;
     template <class R> double diis(Prec<R>& P, int& iters) {
-        const int n3 = 3 * n;
+        const int n3 = 3 * npol;
         const int nslot = kDiisHistory + 1;  // a new entry is added before the oldest leaves
-        diis_d.resize((size_t)nslot * n3);
-        diis_e.resize((size_t)nslot * n3);
+        diis_d.resize((size_t)nslot * std::max(n3, 1));
+        diis_e.resize((size_t)nslot * std::max(n3, 1));
         diis_dots.resize(nslot);
         std::vector<int> hist;  // slots, oldest first
         std::vector<double> B((size_t)nslot * nslot, 0.0), dots(nslot);
@@ -1417,7 +1384,7 @@ struct mpid_context {
                 launch_sub(stream, n3, b.p, Ap.p, r.p);
                 HIP_CHECK(hipMemcpyAsync(d, x.p, n3 * sizeof(double), hipMemcpyDeviceToDevice, stream));
                 launch_axpy(stream, n3, 1.0, r.p, d);
-                launch_apply_S<double>(stream, n, sqrtpol.p, r.p, e, nullptr);
+                launch_apply_S<double>(stream, sites(), r.p, nullptr, nullptr, e);
                 for (int s2 : hist)
                     launch_dot(stream, n3, e, diis_e.p + (size_t)s2 * n3, partial.p, diis_dots.p + s2);
             });
@@ -1504,24 +1471,28 @@ struct mpid_context {
         return c;
     }
 
-    // residual with the FP64 operator: rt = b - A x; returns its RMS-Debye norm
+    // residual with the FP64 operator: rt = b - A x; returns its RMS-Debye
+    // norm and leaves x.rt in hscal[2]
     double true_residual() {
-        const int n3 = 3 * n;
         prof_override = P_REFINE;
         matvec(pd, x.p, Ap.p);
         prof_override = -1;
         timed(P_SOLVER, [&] {
-            launch_sub(stream, n3, b.p, Ap.p, rt.p);
-            launch_residual_norm(stream, n, sqrtpol.p, rt.p, partial.p, scal.p + 4);
+            launch_residual(stream, sites(), b.p, Ap.p, x.p, rt.p, partial.p, hscal_dev + 1);
         });
-        return debye_eps(read_scalar(scal.p + 5));
+        check_launch();
+        wait_stream();
+        return debye_eps(hscal[1]);
     }
 
     template <class R> void solve(Prec<R>& P) {
         stats.iterations = 0;
         stats.refinements = 0;
         stats.matvecs = 0;
-        timed(P_SOLVER, [&] { launch_solver_init(stream, n, sqrtpol.p, E0.p, b.p, x.p); });
+        timed(P_SOLVER, [&] {
+            launch_solver_init<R>(stream, sites(), n, pd.pos.p, E0.p, b.p, x.p, P.mu.p,
+                                  opt.precision == MPID_PRECISION_MIXED ? pd.mu.p : nullptr, mud.p);
+        });
         check_launch();
         energy_correction = 0.0;
         correction_pending = false;
@@ -1537,16 +1508,12 @@ struct mpid_context {
         }
         int iters = 0;
         double eps = (opt.flags & MPID_FLAG_DIIS) ? diis(P, iters)
-                                                 : cg(P, x.p, b.p, false, opt.target_epsilon, iters, opt.max_iterations);
+                                                 : cg(P, x.p, b.p, false, opt.target_epsilon, iters, opt.max_iterations, true);
         // Variational correction of the energy: the energy expression of the
         // reference is linear in the induced dipoles, U(mu) = E(mu) - eps/2 y.r
         // (r = b - A y) is stationary at the solution, so it carries no
         // first-order error from the solver tolerance.  It is read with the
         // energy at the end of the evaluation (forces_and_energy).
-        auto correction_dot = [&](const double* res) {
-            timed(P_SOLVER, [&] { launch_dot(stream, 3 * n, x.p, res, partial.p, scal.p + 6); });
-            HIP_CHECK(hipMemcpyAsync(hscal + 2, scal.p + 6, sizeof(double), hipMemcpyDeviceToHost, stream));
-        };
         if (opt.precision == MPID_PRECISION_MIXED) {
             // FP64 iterative refinement: the residual of the FP32 solution is
             // formed with the FP64 operator, the correction is solved with the
@@ -1566,16 +1533,17 @@ struct mpid_context {
                 const int before = iters;
                 cg(P, dx.p, rt.p, true, std::max(0.3 * opt.target_epsilon, 1e-4 * eps), iters, opt.max_iterations);
                 if (iters == before) iters++;
-                timed(P_SOLVER, [&] { launch_axpy(stream, 3 * n, 1.0, dx.p, x.p); });
+                timed(P_SOLVER, [&] { launch_axpy(stream, 3 * npol, 1.0, dx.p, x.p); });
                 mark_v();
                 if (!defer_final) issue_final_pass(P);
                 on_vstream([&] { eps = true_residual(); });
             }
             stats.refinements = refine;
-            on_vstream([&] { correction_dot(rt.p); });
             join_v();
-        } else {
-            correction_dot(r.p);
+        } else if (!defer_final) {
+            timed(P_SOLVER,
+                  [&] { launch_residual(stream, sites(), nullptr, nullptr, x.p, r.p, partial.p, hscal_dev + 1); });
+            check_launch();
         }
         correction_pending = true;
         stats.iterations = iters;
@@ -1598,7 +1566,7 @@ struct mpid_context {
         join();  // a previous final pass's reciprocal kernels have added into the accumulators
         // induced dipoles: mu = S x (double for the per-atom terms, R for the
         // kernels), unless they are in place already (Extrapolated)
-        if (!mu_set) timed(P_SOLVER, [&] { launch_apply_S<R>(stream, n, sqrtpol.p, x.p, P.mu.p, mud.p); });
+        if (!mu_set) timed(P_SOLVER, [&] { launch_apply_S<R>(stream, sites(), x.p, P.mu.p, mud.p, nullptr); });
         timed(P_OTHER, [&] {
             launch_zero_acc(stream, force_acc.p, force_acc.n);
             launch_zero_acc(stream, torque_acc.p, torque_acc.n);
@@ -1612,7 +1580,7 @@ struct mpid_context {
         // LDS blocks, which would wait for whole CUs behind the
         // electrostatics), then the electrostatics, then the per-atom
         // reciprocal terms and covalent pairs behind the chain on rstream.
-        recip_cycle_induced(P, true);  // phidp
+        recip_cycle_induced(P);  // phidp
         // this category's events bracket the one kernel (its live time in the benchmark)
         timed(P_ELEC, [&] {
             launch_electrostatics_pairs<R>(stream, tile_bound(), tile_act.p, brow_ustart.p + (n + kTile - 1) / kTile,
@@ -1755,17 +1723,17 @@ struct mpid_context {
             // right-hand side: the FP64 residual of the solution (mixed: formed
             // by the check of the solution; FP64: the solver's residual)
             if (opt.precision != MPID_PRECISION_MIXED)
-                HIP_CHECK(hipMemcpyAsync(rt.p, r.p, n3 * sizeof(double), hipMemcpyDeviceToDevice, stream));
+                HIP_CHECK(hipMemcpyAsync(rt.p, r.p, 3 * (size_t)npol * sizeof(double), hipMemcpyDeviceToDevice, stream));
             const double stop = 0.01 * stats.epsilon;
             if (stop > 0.0) {
                 int it = 0;
                 cg(P, dx.p, rt.p, true, stop, it, 20);
                 adjoint_iterations = it;
-                timed(P_SOLVER, [&] { launch_axpy(stream, n3, 1.0, dx.p, x.p); });
+                timed(P_SOLVER, [&] { launch_axpy(stream, 3 * npol, 1.0, dx.p, x.p); });
             }
         }
         // final pass at the refined dipoles, with the potential vectors
-        timed(P_SOLVER, [&] { launch_apply_S<R>(stream, n, sqrtpol.p, x.p, P.mu.p, mud.p); });
+        timed(P_SOLVER, [&] { launch_apply_S<R>(stream, sites(), x.p, P.mu.p, mud.p, nullptr); });
         timed(P_OTHER, [&] {
             launch_zero_acc(stream, force_acc.p, force_acc.n);
             launch_zero_acc(stream, torque_acc.p, torque_acc.n);
@@ -1776,7 +1744,7 @@ struct mpid_context {
             launch_zero_acc(stream, ht_acc.p, ht_acc.n);
             launch_zero_acc(stream, gdef_acc.p, gdef_acc.n);
         });
-        recip_cycle_induced(P, true);  // phidp at every atom
+        recip_cycle_induced(P);  // phidp at every atom
         timed(P_ELEC, [&] {
             launch_electrostatics_pot<R>(stream, tile_bound(), tile_act.p, brow_ustart.p + (n + kTile - 1) / kTile,
                                            brows.p, brow_owner.p,
@@ -2025,8 +1993,7 @@ struct mpid_context {
             for (int s = 0; s < n; s++)
                 for (int k = 0; k < 3; k++) ms[3 * (size_t)s + k] = (R)mu[3 * (size_t)pm[s] + k];
             HIP_CHECK(hipMemcpyAsync(P.mu.p, ms.data(), ms.size() * sizeof(R), hipMemcpyHostToDevice, stream));
-            induced_field(P, true);
-            join();
+            induced_field_all(P);
             launch_field_sum<R>(stream, n, field_acc.p, P.erec.p, P.mu.p, selfc(), tmp3n.p);
             check_launch();
             std::vector<double> f(3 * (size_t)n);

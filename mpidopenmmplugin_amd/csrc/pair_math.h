@@ -161,6 +161,31 @@ template <class R> MPID_HD V3<R> induced_field_from(V3<R> u, V3<R> dr, const Ind
     return dr * (dot(u, dr) * f.f2) + u * f.f1;
 }
 
+// Field at polarisable site i of the induced dipoles of its polarisable
+// covalent partners, which the lists leave out: every `lanes`-th partner from
+// `lane` on.
+template <class R>
+__device__ __forceinline__ V3<R> partner_field(int i, int lane, int lanes, const PairAtoms<R>& A, const R* mu,
+                                               const PairParams<R>& P) {
+    V3<R> e = mk(R(0), R(0), R(0));
+    const int np = A.npart[i];
+    for (int k = lane; k < np; k += lanes) {
+        const int en = A.partners[(size_t)i * A.pstride + k];
+        const int j = en >> 2;
+        const R2<R> tdj = A.td[j];
+        if (tdj.y == R(0)) continue;
+        const R4<R> pi = A.pos[i], pj = A.pos[j];
+        const V3<R> dr = min_image(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), P.box);
+        const R r2 = dot(dr, dr);
+        if (r2 > P.rc2) continue;
+        const R2<R> tdi = A.td[i];
+        const R a = partner_scale<R>(en, P.scale14) == R(0) ? tdi.x + tdj.x : P.default_thole;
+        const V3<R> uj = mk(mu[3 * (size_t)j], mu[3 * (size_t)j + 1], mu[3 * (size_t)j + 2]);
+        e = e + induced_field_from<R>(uj, dr, induced_field_radial<R>(r2, tdi.y, tdj.y, a, P));
+    }
+    return e;
+}
+
 // The field factors with the third one of the field gradient (Extrapolated
 // polarization): f3 = bn3 - 15 (1 - lambda7) / r^7 with the Thole factor
 // lambda7 of MPIDReferenceForce.cpp:4214 (the damped pair terms of

@@ -251,9 +251,7 @@ class HipCalcMPIDForceKernel:
         self._check(self._lib.mpid_set_profiling(self._ctx, int(enable)))
 
     def setProfileFamilies(self, names):
-        """Time only the named kernel families (see _capi.PROFILE_NAMES);
-        unless one of them runs inside a solver iteration, the iterations
-        keep their graph replays."""
+        """Time only the named kernel families (see _capi.PROFILE_NAMES)."""
         mask = 0
         for name in names:
             mask |= 1 << _capi.PROFILE_NAMES.index(name)

@@ -1,0 +1,102 @@
+"""The mutual-polarization solver at the sizes where its kernels change form.
+
+Small clusters without a cutoff, at site counts around the eight sites of an
+operator workgroup, against the FP64 oracle converged to 1e-10 Debye: the
+FP64 path at 1e-9 Debye within 1e-10 relative in energy (second order in the
+residual) and 1e-7 relative RMS in forces (first order: 1e-9 Debye is about
+1e-8 of the dipoles); the mixed path's forces within the workload bar of 1e-5
+(a small cluster's energy is a difference of large pair terms that a relative
+bar on the sum does not describe).
+
+Periodic boxes around 2,048 sites (one workgroup updates all sites, beyond it
+several do) and 8,192 sites (the operator's kernel adds the real-space field
+itself, beyond it the list kernel does): the dipoles must satisfy the
+equation they solve, mu = alpha (E0 + T mu), with E0 and T mu from the
+inspection entry points, whose kernels are others.  The FP64 solve stops
+below 1e-8 Debye RMS (over all atoms); E0 and T mu carry fixed-point sums of
+2^-32, 1e-11 Debye at this alpha, so the residual formed from them must stay
+below 1.01e-8 Debye.  The mixed path's dipoles agree with them to the
+workload bar of 1e-5 relative RMS.
+"""
+import numpy as np
+import pytest
+
+from mpidopenmmplugin_amd.kernel import HipCalcMPIDForceKernel
+from mpidopenmmplugin_amd.mpidforce import MPIDForce
+from mpidopenmmplugin_amd.waterbox import _o_parameters, _water_force, make_small_waterbox
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+
+DEBYE = 48.033324
+
+
+def rel_rms(a, b):
+    a = np.asarray(a, dtype=np.float64)
+    b = np.asarray(b, dtype=np.float64)
+    return np.sqrt(((a - b) ** 2).sum() / (b ** 2).sum())
+
+
+@pytest.mark.parametrize("waters", [1, 2, 7, 8, 9, 33])
+def test_small_clusters(waters):
+    force, pos, _ = make_small_waterbox(waters, 40 + waters)
+    force.setNonbondedMethod(MPIDForce.NoCutoff)
+    force.setMutualInducedTargetEpsilon(1e-10)
+    ref = oracle.evaluate(force.flatten(), pos, None)
+    force.setMutualInducedTargetEpsilon(1e-9)
+    for precision, e_tol, f_tol in (("double", 1e-10, 1e-7), ("mixed", None, 1e-5)):
+        if precision == "mixed":
+            force.setMutualInducedTargetEpsilon(1e-6)
+        k = HipCalcMPIDForceKernel(precision)
+        k.initialize(len(pos), force)
+        print(f"[gpu] cluster of {waters} waters, {precision}", flush=True)
+        e, F = k.execute(pos, None)
+        # one molecule alone has no real-space pairs: its energy is zero
+        if e_tol is not None:
+            assert abs(e - ref["energy_variational"]) <= e_tol * max(abs(ref["energy_variational"]), 1.0)
+        assert np.sqrt(((F - ref["forces"]) ** 2).sum()) <= f_tol * max(np.sqrt((ref["forces"] ** 2).sum()), 1.0)
+
+
+@pytest.mark.parametrize("waters", [2048, 2049, 8192, 8193])
+def test_dipoles_satisfy_their_equation(waters):
+    alpha = 0.001
+    rng = np.random.default_rng(waters)
+    params = _o_parameters(rng, True, False)  # isotropic
+    force, pos, box = make_small_waterbox(waters, waters, params)
+    force.setMutualInducedTargetEpsilon(1e-8)
+    k = HipCalcMPIDForceKernel("double")
+    k.initialize(len(pos), force, default_box=box)
+    print(f"[gpu] {waters} waters", flush=True)
+    mu = k.getInducedDipoles(pos, box)
+    st = k.stats()
+    assert st["converged"] and st["epsilon"] < 1e-8
+    assert not mu.reshape(-1, 3, 3)[:, 1:].any()  # hydrogens are not polarisable
+    field = k.computeFixedField(pos, box) + k.computeInducedField(pos, box, mu)
+    residual = (mu - alpha * field)[::3]
+    assert DEBYE * np.sqrt((residual ** 2).sum() / len(pos)) <= 1.01e-8
+    m = HipCalcMPIDForceKernel("mixed")
+    force.setMutualInducedTargetEpsilon(1e-6)
+    m.initialize(len(pos), force, default_box=box)
+    assert rel_rms(m.getInducedDipoles(pos, box), mu) <= 1e-5
+
+
+def test_no_polarisable_site():
+    """Charges and multipoles only: nothing to solve, no iteration."""
+    rng = np.random.default_rng(3)
+    dip, quad, octo, _ = _o_parameters(rng, True, True)
+    small, pos, box = make_small_waterbox(40, 3)
+    force = _water_force(40, (dip, quad, octo, [0.0] * 3))
+    force.setNonbondedMethod(MPIDForce.PME)
+    force.setCutoffDistance(small.getCutoffDistance())
+    force.setPMEParameters(*small.getPMEParameters())
+    force.setPolarizationType(MPIDForce.Mutual)
+    force.setMutualInducedTargetEpsilon(1e-6)
+    ref = oracle.evaluate(force.flatten(), pos, box)
+    for precision, e_tol, f_tol in (("double", 1e-9, 1e-9), ("mixed", 1e-6, 1e-5)):
+        k = HipCalcMPIDForceKernel(precision)
+        k.initialize(len(pos), force, default_box=box)
+        print(f"[gpu] no polarisable site, {precision}", flush=True)
+        e, F = k.execute(pos, box)
+        assert k.stats()["iterations"] == 0
+        assert abs(e - ref["energy"]) <= e_tol * abs(ref["energy"])
+        assert rel_rms(F, ref["forces"]) <= f_tol
