@@ -132,19 +132,61 @@ struct NbrList {
 };
 
 // ---- atoms / frames / solver vectors (kernels_atoms.hip) ---------------------
-void launch_morton_keys(hipStream_t s, int n, const double* pos, Box<double> box, unsigned* keys, int* vals);
-void launch_invert_perm(hipStream_t s, int n, const int* perm, int* inv);
-void launch_gather_sorted(hipStream_t s, int n, const int* perm, const int* inv, const double* pos, Box<double> box,
-                          const double* mol, const int4* axes, const double* thole, const double* pol,
-                          const int* partners, const int* npart, int pstride, double4* spos, double* smol,
-                          int4* saxes, double* sthole, double* spol, int* spartners, int* snpart);
-// chg[s] = 1: the site carries a charge only (no higher moment, no polarisability)
-void launch_rotate(hipStream_t s, int n, Box<double> box, const double4* pos, const int4* axes, const double* mol,
-                   const double* pol, double* lab, double* labpol, double* sqrtpol, double* damp, int* aniso,
-                   int* chg);
-template <class R>
-void launch_convert(hipStream_t s, int n, const double4* pos, const double* lab, const double* thole,
-                    const double* damp, R4<R>* rpos, R* rlab, R2<R>* rtd);
+// Sorts the atoms along the Morton curve (stable): perm, its inverse and the
+// sorted keys.  One kernel up to kRankSortMax atoms, a radix sort beyond.
+constexpr int kRankSortMax = 16384;  // 64 KB of keys in LDS
+int launch_sort_atoms(hipStream_t s, int n, const double* pos, Box<double> box, void* temp, size_t bytes,
+                      unsigned* keys, int* vals, int* perm, int* inv, unsigned* keys_sorted);
+// Per-atom parameters in the caller's order, and the permutation
+struct AtomParams {
+    const int* perm;
+    const int* inv;
+    const unsigned* keys_sorted;
+    const double* mol;
+    const int4* axes;
+    const double* thole;
+    const double* pol;
+    const int* partners;
+    const int* npart;
+    int pstride;
+};
+// What launch_sorted_atoms writes, in sorted order.  chg[s] = 1: the site
+// carries a charge only (no higher moment, no polarisability).  The pointers
+// named f*, tstart and E0 (with mud, dmu, fmu: cleared) may be null.
+struct AtomState {
+    double4* spos;
+    double* smol;
+    int4* saxes;
+    double* sthole;
+    double* spol;
+    int* spart;
+    int* snpart;
+    double* lab;
+    double* labpol;
+    double* sqrtpol;
+    double* damp;
+    int* aniso;
+    int* chg;
+    double4* dpos;
+    double2* dtd;
+    float4* fpos;
+    float* flab;
+    float2* ftd;
+    float4* bmin;  // per 64-atom block: bounding box, polarisable atoms and their number
+    float4* bmax;
+    unsigned long long* polmask;
+    int* polcnt;
+    int* nl_scalars;  // cleared
+    int* tstart;      // [ntiles + 1] first sorted atom of each spreading tile
+    int tile_shift;
+    int ntiles;
+    double* E0;
+    double* mud;
+    double* dmu;
+    float* fmu;
+};
+void launch_sorted_atoms(hipStream_t s, int n, Box<double> box, const double* pos, const AtomParams& in,
+                         const AtomState& out);
 // exact_threefold: ThreeFold frames by the exact chain rule (conservative
 // torques) instead of the reference's approximate projection
 void launch_torque_to_force(hipStream_t s, int n, Box<double> box, const double4* pos, const int4* axes,
@@ -153,7 +195,6 @@ void launch_output_forces(hipStream_t s, int n, const int* perm, const acc_t* fo
 void launch_unpermute3(hipStream_t s, int n, const int* perm, const double* in, double* out);
 void launch_zero_acc(hipStream_t s, acc_t* p, size_t count);
 size_t sort_temp_bytes(int n);
-int launch_sort_pairs(hipStream_t s, void* temp, size_t bytes, unsigned* kin, unsigned* kout, int* vin, int* vout, int n);
 // out = acc + erecip + selfc * mu (field of the induced dipoles, double)
 template <class R>
 void launch_field_sum(hipStream_t s, int n, const acc_t* acc, const R* erec, const R* mu, double selfc, double* out);
@@ -233,9 +274,6 @@ struct TileGeom {
     int T[3];
     int W[3];
 };
-// Morton-cell ranges of the sorted atoms, or (idx != nullptr) of the subsequence idx[0 .. *count)
-void launch_tile_ranges(hipStream_t s, int n, const unsigned* keys_sorted, const int* idx, const int* count,
-                        int shift, int* tstart, int* tend);
 size_t spread_tiled_lds_bytes(const TileGeom& tg, int double_precision);
 template <class R>
 void launch_spread_fixed_tiled(hipStream_t s, const R4<R>* pos, const R* lab, PmeGeom<R> g, TileGeom tg,
@@ -316,8 +354,6 @@ template <class R>
 void launch_recip_convolution(hipStream_t s, const FftPlan<R>& p, R* Q, R2<R>* S, R* V, ConvParams<R> cp);
 
 // ---- real space (kernels_pairs.hip) -------------------------------------------
-template <class R>
-void launch_block_bounds(hipStream_t s, int n, const R4<R>* pos, float4* bmin, float4* bmax);
 // One workgroup per tile act[0 .. *nact) (row entries r of block pairs
 // J >= I); the launch covers maxtiles >= *nact.
 // tmask: pairs with a multipole or a polarisable site; tmaskcc: pairs of two
@@ -332,17 +368,21 @@ void launch_electrostatics_pairs(hipStream_t s, int maxtiles, const int4* act, c
                                  PairParams<R> p, const double4* pos64, const double* lab64, PairParams<double> p64,
                                  acc_t* force, acc_t* torque, acc_t* energy);
 // ---- neighbour lists (kernels_nlist.hip) ---------------------------------------
-// Block pairs within the cutoff: counts and upper (those with J >= I) when
-// rows == nullptr, or the rows at start[I] (at most cap entries are stored;
-// the count may exceed it)
+// Block rows: for each block I the blocks J within the cutoff, ascending, at
+// rows[start[I] ..] with I in owner[] (at most cap entries are stored; the
+// count start[nb] may exceed it), ustart: the exclusive scan of each row's
+// entries with J >= I, polstart: that of polcnt.  *total (mapped host memory)
+// takes the count, *nact the length of the electrostatics kernels' work list
+// (the entries with J >= I; 0 when the rows overflow, so that a pass issued
+// before the host has seen that reads nothing).  work: 2 nb ints.
+constexpr int kOneRows = 256;  // blocks whose rows one workgroup builds
 void launch_block_rows(hipStream_t s, int nb, const float4* bmin, const float4* bmax, Box<float> box, float cutoff,
-                       const int* start, int* counts, int* upper, int* rows, int* owner, int cap);
-void launch_exclusive_scan(hipStream_t s, int m, const int* counts, int* start);
+                       const int* polcnt, int* work, int* start, int* ustart, int* polstart, int* rows, int* owner,
+                       int cap, int* total, int* nact);
 // pos.w of the FP64 positions is the damping factor: nonzero iff the site is polarisable
 // Masks, then lists: all = true gives the full list of every atom stored by
 // atom index; all = false the full and polarisable-neighbour lists of the
-// polarisable atoms, stored by position in their sorted index (polstart,
-// the exclusive scan of polcnt, is written on the way).  nmask: 64 words per
+// polarisable atoms, stored by position in their sorted index.  nmask: 64 words per
 // row entry (nrows entries); polmask: one word per block; scalars[0]:
 // largest stored list length, scalars[1]: nonzero if a block pair lacked its
 // mirror entry.  act[ustart[I] + k] = {r, I, J} for the k-th row entry r of
@@ -351,13 +391,15 @@ void launch_exclusive_scan(hipStream_t s, int m, const int* counts, int* start);
 // number of such entries).  nrows: row entries launched (the count, or the capacity
 // when the count is not known on the host: entries past rstart[nb] return);
 // rcap: the capacity of rows / nmask (entries beyond it are ignored).
+// pol_idx: the sorted indices of the polarisable atoms; tpstart (may be
+// null): the first entry of pol_idx in each spreading tile, from tstart.
 void launch_nl_build(hipStream_t s, int n, int nrows, int rcap, bool all, const int* rstart, const int* rows,
                      const int* owner, const float4* bmin, const float4* bmax, const double4* pos,
                      const int* partners, const int* npart, int pstride, Box<double> box, double rc2, int cap,
-                     unsigned long long* nmask, unsigned long long* polmask, int* polcnt, int* polstart, int* nbr,
+                     unsigned long long* nmask, const unsigned long long* polmask, const int* polstart, int* nbr,
                      int* count, int* scalars, unsigned long long* tmask, int* pnbr, int* pcount, const int* chg,
-                     unsigned long long* tmaskcc, int4* act, const int* ustart);
-void launch_pol_fill(hipStream_t s, int n, const double4* pos, const int* start, int* idx);
+                     unsigned long long* tmaskcc, int4* act, const int* ustart, int* pol_idx, int ntiles,
+                     const int* tstart, int* tpstart);
 // fields at the atoms atoms[0..natoms) (all atoms when atoms == nullptr, natoms = n)
 template <class R>
 void launch_nl_fixed_field(hipStream_t s, int natoms, const int* atoms, NbrList l, PairAtoms<R> a, PairParams<R> p,
@@ -417,10 +459,19 @@ void launch_cg_start(hipStream_t s, SolverSites st, const double* rhs, const dou
 template <class R>
 void launch_cg_iteration(hipStream_t s, SolverSites st, const double* Ap, double* x, double* r, double* p, R* mu,
                          int npap, double* partial, double* scal, double* hcheck, int n, double stop_eps);
-// b = x = S E0 and mu = S x (zero at the other atoms of mu, mu2, mud)
+// Permanent field of the lists (in R) and of the covalent partners (FP64) at
+// the polarisable sites, by site
 template <class R>
-void launch_solver_init(hipStream_t s, SolverSites st, int n, const double4* pos, const double* E0, double* b,
-                        double* x, R* mu, double* mu2, double* mud);
+void launch_fixed_list(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p,
+                       PairAtoms<double> a64, PairParams<double> p64, double* field);
+// The rest: E0 (by atom) = field + reciprocal (phi, 35 per atom) + self,
+// b = x = S E0, mu = mud = S x.  field null: launch_fixed_list's sums in the
+// same kernel.  nl_scalars go to hnl (mapped host memory).
+template <class R>
+void launch_solver_init(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p,
+                        PairAtoms<double> a64, PairParams<double> p64, const double* field, const double* phi,
+                        FracT<double> A, double selfc, double* E0, double* b, double* x, R* mu, double* mud,
+                        const int* nl_scalars, int* hnl);
 // S v: by atom in mu and mud, by site in at (each may be null)
 template <class R>
 void launch_apply_S(hipStream_t s, SolverSites st, const double* v, R* mu, double* mud, double* at);

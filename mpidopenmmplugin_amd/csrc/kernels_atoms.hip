@@ -41,11 +41,9 @@ __device__ __forceinline__ unsigned spread_bits(unsigned v) {
     return v;
 }
 
-__global__ void k_morton_keys(int n, const double* __restrict__ pos, Box<double> box, unsigned* keys, int* vals) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+__device__ __forceinline__ unsigned morton_key(const double* pos, const Box<double>& box) {
     unsigned c[3];
-    const D3 fr = to_frac(mk(pos[3 * (size_t)i], pos[3 * (size_t)i + 1], pos[3 * (size_t)i + 2]), box);
+    const D3 fr = to_frac(mk(pos[0], pos[1], pos[2]), box);
     const double fs[3] = {fr.x, fr.y, fr.z};
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -54,7 +52,13 @@ __global__ void k_morton_keys(int n, const double* __restrict__ pos, Box<double>
         int q = (int)(f * 1024.0);
         c[k] = (unsigned)min(max(q, 0), 1023);
     }
-    keys[i] = (spread_bits(c[0]) << 2) | (spread_bits(c[1]) << 1) | spread_bits(c[2]);
+    return (spread_bits(c[0]) << 2) | (spread_bits(c[1]) << 1) | spread_bits(c[2]);
+}
+
+__global__ void k_morton_keys(int n, const double* __restrict__ pos, Box<double> box, unsigned* keys, int* vals) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    keys[i] = morton_key(pos + 3 * (size_t)i, box);
     vals[i] = i;
 }
 
@@ -63,46 +67,63 @@ __global__ void k_invert_perm(int n, const int* __restrict__ perm, int* inv) {
     if (s < n) inv[perm[s]] = s;
 }
 
-__global__ void k_gather_sorted(int n, const int* __restrict__ perm, const int* __restrict__ inv,
-                                const double* __restrict__ pos, Box<double> box, const double* __restrict__ mol,
-                                const int4* __restrict__ axes, const double* __restrict__ thole,
-                                const double* __restrict__ pol, const int* __restrict__ partners,
-                                const int* __restrict__ npart, int pstride, double4* spos, double* smol,
-                                int4* saxes, double* sthole, double* spol, int* spartners, int* snpart) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int a = perm[s];
-    // wrapped into the cell (fractional coordinates in [0, 1)); without
-    // periodicity (zero box) the positions stay as they are
-    D3 w = mk(pos[3 * (size_t)a], pos[3 * (size_t)a + 1], pos[3 * (size_t)a + 2]);
-    if (box.L[0] > 0.0) {
-        D3 f = to_frac(w, box);
-        f.x -= floor(f.x);
-        f.y -= floor(f.y);
-        f.z -= floor(f.z);
-        w = from_frac(f, box);
+// Up to kRankSortMax atoms: keys, stable sort and both permutations in one
+// kernel, by ranks.  A workgroup computes every key into LDS and ranks 64
+// atoms (lane: atom), its 16 wavefronts counting over the 64-key blocks in
+// turn; the counts meet in LDS.  n^2 / 64 four-byte compares from broadcast
+// LDS reads: 11 us of VALU work at 12,288 atoms and under 1 us at 3,000,
+// where key, sort (five radix passes from 4,096 keys on) and inversion
+// kernels took 35-40 us and 20 us as dependent dispatches.
+constexpr int kRankThreads = 1024;
+__global__ __launch_bounds__(kRankThreads) void k_rank_sort(int n, const double* __restrict__ pos, Box<double> box,
+                                                            int* __restrict__ perm, int* __restrict__ inv,
+                                                            unsigned* __restrict__ keys_sorted) {
+    extern __shared__ __align__(16) unsigned skey[];  // nb * 64 keys, the last block filled up
+    __shared__ int scnt[kRankThreads / kTile][kTile];
+    const int nb = (n + kTile - 1) / kTile;
+    for (int i = threadIdx.x; i < nb * kTile; i += kRankThreads)
+        skey[i] = i < n ? morton_key(pos + 3 * (size_t)i, box) : 0xffffffffu;
+    __syncthreads();
+    const int I = blockIdx.x, lane = threadIdx.x & (kTile - 1), w = threadIdx.x / kTile;
+    const int i = I * kTile + lane;
+    const unsigned ki = skey[i];
+    int c = 0;
+    for (int J = w; J < nb; J += kRankThreads / kTile) {
+        const uint4* kj = reinterpret_cast<const uint4*>(skey + J * kTile);
+        if (J == I) {
+            for (int j = 0; j < kTile; j++) {
+                const unsigned k = skey[J * kTile + j];
+                c += (k < ki || (k == ki && j < lane)) ? 1 : 0;
+            }
+            continue;
+        }
+        const unsigned lim = J < I ? ki + 1u : ki;  // equal keys keep their order
+#pragma unroll 4
+        for (int j = 0; j < kTile / 4; j++) {
+            const uint4 k = kj[j];
+            c += (k.x < lim) + (k.y < lim) + (k.z < lim) + (k.w < lim);
+        }
     }
-    const double x[3] = {w.x, w.y, w.z};
-    spos[s] = make_double4(x[0], x[1], x[2], mol[(size_t)a * kMP]);
-    for (int k = 0; k < kMP; k++) smol[(size_t)s * kMP + k] = mol[(size_t)a * kMP + k];
-    int4 ax = axes[a];
-    saxes[s] = make_int4(ax.x >= 0 ? inv[ax.x] : -1, ax.y >= 0 ? inv[ax.y] : -1, ax.z >= 0 ? inv[ax.z] : -1, ax.w);
-    sthole[s] = thole[a];
-    for (int k = 0; k < 3; k++) spol[3 * (size_t)s + k] = pol[3 * (size_t)a + k];
-    const int np = npart[a];
-    snpart[s] = np;
-    for (int k = 0; k < np; k++) {
-        int e = partners[(size_t)a * pstride + k];
-        spartners[(size_t)s * pstride + k] = (inv[e >> 2] << 2) | (e & 3);
+    scnt[w][lane] = c;
+    __syncthreads();
+    if (w == 0 && i < n) {
+        int r = 0;
+#pragma unroll
+        for (int k = 0; k < kRankThreads / kTile; k++) r += scnt[k][lane];
+        perm[r] = i;
+        inv[i] = r;
+        keys_sorted[r] = ki;
     }
 }
 
 // ---------------------------------------------------------------------------
 // lab frame
 // ---------------------------------------------------------------------------
-// Molecular frame axes of atom s (rows x, y, z in lab components); identity
-// for NoAxisType.  ZOnly picks its x axis from the lab axes.
-__device__ void frame_axes(int s, const double4* __restrict__ pos, int4 ax, const Box<double>& box, D3 e[3]) {
+// Molecular frame axes of an atom at pi (rows x, y, z in lab components);
+// identity for NoAxisType.  ZOnly picks its x axis from the lab axes.  at(k):
+// position of frame atom k.
+template <class At>
+__device__ void frame_axes(D3 pi, At at, int4 ax, const Box<double>& box, D3 e[3]) {
     const int t = ax.w;
     if (t == 5 || ax.x < 0) {
         e[0] = mk(1.0, 0.0, 0.0);
@@ -110,27 +131,26 @@ __device__ void frame_axes(int s, const double4* __restrict__ pos, int4 ax, cons
         e[2] = mk(0.0, 0.0, 1.0);
         return;
     }
-    const D3 pi = d3(pos[s]);
-    D3 vz = min_image(d3(pos[ax.x]) - pi, box);
+    D3 vz = min_image(at(ax.x) - pi, box);
     dnorm(vz);
     D3 vx;
     if (t == 4) {
         vx = fabs(vz.x) < 0.866 ? mk(1.0, 0.0, 0.0) : mk(0.0, 1.0, 0.0);
     } else {
-        vx = min_image(d3(pos[ax.y]) - pi, box);
+        vx = min_image(at(ax.y) - pi, box);
         if (t == 1) {
             dnorm(vx);
             vz = vz + vx;
             dnorm(vz);
         } else if (t == 2) {
             dnorm(vx);
-            D3 vy = min_image(d3(pos[ax.z]) - pi, box);
+            D3 vy = min_image(at(ax.z) - pi, box);
             dnorm(vy);
             vx = vx + vy;
             dnorm(vx);
         } else if (t == 3) {
             dnorm(vx);
-            D3 vy = min_image(d3(pos[ax.z]) - pi, box);
+            D3 vy = min_image(at(ax.z) - pi, box);
             dnorm(vy);
             vz = vz + vx + vy;
             dnorm(vz);
@@ -155,25 +175,95 @@ __device__ __forceinline__ int i3(int a, int b, int c) {
     return t[lo][mid][hi];
 }
 
-// axes: x = z-axis atom, y = x-axis atom, z = y-axis atom, w = axis type (all sorted indices)
-__global__ __launch_bounds__(128) void k_rotate(int n, Box<double> box, const double4* __restrict__ pos,
-                                                 const int4* __restrict__ axes, const double* __restrict__ mol,
-                                                 const double* __restrict__ pol, double* lab, double* labpol,
-                                                 double* sqrtpol, double* damp, int* aniso, int* chg) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int4 ax = axes[s];
+// Everything an evaluation needs per atom in sorted order, one wavefront per
+// 64-atom block: the gathered parameters and wrapped position, the lab-frame
+// moments and polarisability (frames from the unsorted positions, so that no
+// other block's output is waited for), the precision copies, the block's
+// bounding box and polarisable atoms, the first atoms of the spreading tiles,
+// and zeros where the solver writes polarisable sites only.
+// axes: x = z-axis atom, y = x-axis atom, z = y-axis atom, w = axis type
+// (original indices; stored as sorted ones).
+__global__ __launch_bounds__(kTile) void k_sorted_atoms(int n, Box<double> box, const double* __restrict__ pos,
+                                                        AtomParams in, AtomState o) {
+    const int s = blockIdx.x * kTile + threadIdx.x;
+    const bool v = s < n;
+    const int a = in.perm[v ? s : n - 1];
+    // wrapped into the cell (fractional coordinates in [0, 1)); without
+    // periodicity (zero box) the positions stay as they are
+    const D3 raw = mk(pos[3 * (size_t)a], pos[3 * (size_t)a + 1], pos[3 * (size_t)a + 2]);
+    D3 w = raw;
+    if (box.L[0] > 0.0) {
+        D3 f = to_frac(w, box);
+        f.x -= floor(f.x);
+        f.y -= floor(f.y);
+        f.z -= floor(f.z);
+        w = from_frac(f, box);
+    }
+    // the block's bounding box (lanes past the last atom repeat it)
+    {
+        float lo[3] = {(float)w.x, (float)w.y, (float)w.z}, hi[3] = {lo[0], lo[1], lo[2]};
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                lo[k] = fminf(lo[k], __shfl_xor(lo[k], off));
+                hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], off));
+            }
+        }
+        if (threadIdx.x == 0) {
+            o.bmin[blockIdx.x] = make_float4(lo[0], lo[1], lo[2], 0.f);
+            o.bmax[blockIdx.x] = make_float4(hi[0], hi[1], hi[2], 0.f);
+        }
+    }
+    const double p0 = in.pol[3 * (size_t)a], p1 = in.pol[3 * (size_t)a + 1], p2 = in.pol[3 * (size_t)a + 2];
+    // MPIDForce.h:531 / MPIDReferenceKernels.cpp:134
+    const double damp = pow((p0 + p1 + p2) / 3.0, 1.0 / 6.0);
+    {
+        const unsigned long long pm = __ballot(v && damp != 0.0);
+        if (threadIdx.x == 0) {
+            o.polmask[blockIdx.x] = pm;
+            o.polcnt[blockIdx.x] = __popcll(pm);
+            if (blockIdx.x == 0) o.nl_scalars[0] = o.nl_scalars[1] = 0;
+        }
+    }
+    if (!v) return;
+    if (o.tstart) {
+        // tile t starts at the first atom whose key is in t or beyond: atom s
+        // opens the tiles after its predecessor's up to its own, the last
+        // atom closes the rest
+        const int t1 = (int)(in.keys_sorted[s] >> o.tile_shift);
+        const int t0 = s == 0 ? -1 : (int)(in.keys_sorted[s - 1] >> o.tile_shift);
+        for (int t = t0 + 1; t <= t1; t++) o.tstart[t] = s;
+        if (s == n - 1)
+            for (int t = t1 + 1; t <= o.ntiles; t++) o.tstart[t] = n;
+    }
+    const int4 ax = in.axes[a];
     double m[kMP];
     bool bare = true;  // charge only: no higher moment, no polarisability
     for (int k = 0; k < kMP; k++) {
-        m[k] = mol[(size_t)s * kMP + k];
+        m[k] = in.mol[(size_t)a * kMP + k];
+        o.smol[(size_t)s * kMP + k] = m[k];
         if (k > 0 && m[k] != 0.0) bare = false;
     }
+    o.spos[s] = make_double4(w.x, w.y, w.z, m[0]);
+    o.saxes[s] = make_int4(ax.x >= 0 ? in.inv[ax.x] : -1, ax.y >= 0 ? in.inv[ax.y] : -1,
+                           ax.z >= 0 ? in.inv[ax.z] : -1, ax.w);
+    const double th = in.thole[a];
+    o.sthole[s] = th;
+    o.spol[3 * (size_t)s] = p0;
+    o.spol[3 * (size_t)s + 1] = p1;
+    o.spol[3 * (size_t)s + 2] = p2;
+    const int np = in.npart[a];
+    o.snpart[s] = np;
+    for (int k = 0; k < np; k++) {
+        const int e = in.partners[(size_t)a * in.pstride + k];
+        o.spart[(size_t)s * in.pstride + k] = (in.inv[e >> 2] << 2) | (e & 3);
+    }
     // chirality (ZThenX with a y atom): flip y-odd dipole/quadrupole components
+    auto at = [&](int k) { return mk(pos[3 * (size_t)k], pos[3 * (size_t)k + 1], pos[3 * (size_t)k + 2]); };
     if (ax.w == 0 && ax.z >= 0) {
-        const D3 py = d3(pos[ax.z]);
-        D3 ad = min_image(d3(pos[s]) - py, box), bd = min_image(d3(pos[ax.x]) - py, box),
-           cd = min_image(d3(pos[ax.y]) - py, box);
+        const D3 py = at(ax.z);
+        D3 ad = min_image(raw - py, box), bd = min_image(at(ax.x) - py, box), cd = min_image(at(ax.y) - py, box);
         if (dot(cross(bd, cd), ad) < 0.0) {
             m[2] = -m[2];
             m[5] = -m[5];
@@ -181,65 +271,67 @@ __global__ __launch_bounds__(128) void k_rotate(int n, Box<double> box, const do
         }
     }
     D3 e[3];
-    frame_axes(s, pos, ax, box, e);
+    frame_axes(raw, at, ax, box, e);
     double E[3][3];  // E[k][a] = component a of molecular axis k
     for (int k = 0; k < 3; k++) {
         E[k][0] = e[k].x;
         E[k][1] = e[k].y;
         E[k][2] = e[k].z;
     }
-    double* o = lab + (size_t)s * kMP;
-    o[0] = m[0];
-    for (int a = 0; a < 3; a++) {
-        double v = 0;
-        for (int k = 0; k < 3; k++) v += E[k][a] * m[1 + k];
-        o[1 + a] = v;
+    double r[kMP];
+    r[0] = m[0];
+    for (int c = 0; c < 3; c++) {
+        double x = 0;
+        for (int k = 0; k < 3; k++) x += E[k][c] * m[1 + k];
+        r[1 + c] = x;
     }
-    for (int a = 0; a < 3; a++)
-        for (int b = a; b < 3; b++) {
-            double v = 0;
+    for (int c = 0; c < 3; c++)
+        for (int b = c; b < 3; b++) {
+            double x = 0;
             for (int k = 0; k < 3; k++)
-                for (int l = 0; l < 3; l++) v += E[k][a] * E[l][b] * m[4 + i2(k, l)];
-            o[4 + i2(a, b)] = v;
+                for (int l = 0; l < 3; l++) x += E[k][c] * E[l][b] * m[4 + i2(k, l)];
+            r[4 + i2(c, b)] = x;
         }
-    for (int a = 0; a < 3; a++)
-        for (int b = a; b < 3; b++)
-            for (int c = b; c < 3; c++) {
-                double v = 0;
+    for (int c = 0; c < 3; c++)
+        for (int b = c; b < 3; b++)
+            for (int d = b; d < 3; d++) {
+                double x = 0;
                 for (int k = 0; k < 3; k++)
                     for (int l = 0; l < 3; l++)
-                        for (int q = 0; q < 3; q++) v += E[k][a] * E[l][b] * E[q][c] * m[10 + i3(k, l, q)];
-                o[10 + i3(a, b, c)] = v;
+                        for (int q = 0; q < 3; q++) x += E[k][c] * E[l][b] * E[q][d] * m[10 + i3(k, l, q)];
+                r[10 + i3(c, b, d)] = x;
             }
-    const double p0 = pol[3 * (size_t)s], p1 = pol[3 * (size_t)s + 1], p2 = pol[3 * (size_t)s + 2];
     const double pk[3] = {p0, p1, p2};
     const double sk[3] = {sqrt(fmax(p0, 0.0)), sqrt(fmax(p1, 0.0)), sqrt(fmax(p2, 0.0))};
-    for (int a = 0; a < 3; a++)
-        for (int b = a; b < 3; b++) {
-            double v = 0, w = 0;
+    for (int c = 0; c < 3; c++)
+        for (int b = c; b < 3; b++) {
+            double x = 0, y = 0;
             for (int k = 0; k < 3; k++) {
-                v += E[k][a] * E[k][b] * pk[k];
-                w += E[k][a] * E[k][b] * sk[k];
+                x += E[k][c] * E[k][b] * pk[k];
+                y += E[k][c] * E[k][b] * sk[k];
             }
-            labpol[6 * (size_t)s + i2(a, b)] = v;
-            sqrtpol[6 * (size_t)s + i2(a, b)] = w;
+            o.labpol[6 * (size_t)s + i2(c, b)] = x;
+            o.sqrtpol[6 * (size_t)s + i2(c, b)] = y;
         }
-    // MPIDForce.h:531 / MPIDReferenceKernels.cpp:134
-    damp[s] = pow((p0 + p1 + p2) / 3.0, 1.0 / 6.0);
-    aniso[s] = (p0 != p1 || p0 != p2) ? 1 : 0;
-    chg[s] = (bare && p0 == 0.0 && p1 == 0.0 && p2 == 0.0) ? 1 : 0;
-}
-
-template <class R>
-__global__ void k_convert(int n, const double4* __restrict__ pos, const double* __restrict__ lab,
-                          const double* __restrict__ thole, const double* __restrict__ damp, R4<R>* rpos, R* rlab,
-                          R2<R>* rtd) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    double4 p = pos[s];
-    rpos[s] = R4<R>{(R)p.x, (R)p.y, (R)p.z, (R)damp[s]};  // w: damping factor
-    for (int k = 0; k < kMP; k++) rlab[(size_t)s * kMP + k] = (R)lab[(size_t)s * kMP + k];
-    rtd[s] = R2<R>{(R)thole[s], (R)damp[s]};
+    o.damp[s] = damp;
+    o.aniso[s] = (p0 != p1 || p0 != p2) ? 1 : 0;
+    o.chg[s] = (bare && p0 == 0.0 && p1 == 0.0 && p2 == 0.0) ? 1 : 0;
+    for (int k = 0; k < kMP; k++) o.lab[(size_t)s * kMP + k] = r[k];
+    o.dpos[s] = make_double4(w.x, w.y, w.z, damp);  // w: damping factor
+    o.dtd[s] = make_double2(th, damp);
+    if (o.fpos) {
+        o.fpos[s] = make_float4((float)w.x, (float)w.y, (float)w.z, (float)damp);
+        o.ftd[s] = make_float2((float)th, (float)damp);
+        for (int k = 0; k < kMP; k++) o.flab[(size_t)s * kMP + k] = (float)r[k];
+    }
+    if (o.E0) {
+        for (int k = 0; k < 3; k++) {
+            o.E0[3 * (size_t)s + k] = 0.0;
+            o.mud[3 * (size_t)s + k] = 0.0;
+            o.dmu[3 * (size_t)s + k] = 0.0;
+            if (o.fmu) o.fmu[3 * (size_t)s + k] = 0.f;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -902,7 +994,7 @@ __global__ __launch_bounds__(128) void k_param_gradients(int n, int all_sites, c
         double v[kMP];
         for (int k = 0; k < kMP; k++) v[k] = (bare && k > 0) ? 0.0 : acc_get(pot[kMP * (size_t)s + k]);
         D3 e[3];
-        frame_axes(s, pos, ax, box, e);
+        frame_axes(d3(pos[s]), [&](int k) { return d3(pos[k]); }, ax, box, e);
         double E[3][3];
         for (int k = 0; k < 3; k++) {
             E[k][0] = e[k].x;
@@ -1137,7 +1229,7 @@ size_t sort_temp_bytes(int n) {
                               (size_t)n, 0, 30);
     return bytes;
 }
-int launch_sort_pairs(hipStream_t s, void* temp, size_t bytes, unsigned* kin, unsigned* kout, int* vin, int* vout,
+static int launch_sort_pairs(hipStream_t s, void* temp, size_t bytes, unsigned* kin, unsigned* kout, int* vin, int* vout,
                       int n) {
     return (int)rocprim::radix_sort_pairs(temp, bytes, kin, kout, vin, vout, (size_t)n, 0, 30, s);
 }
@@ -1148,29 +1240,25 @@ void launch_field_sum(hipStream_t s, int n, const acc_t* acc, const R* erec, con
 
 static inline dim3 blocks_for(size_t n, int t) { return dim3((unsigned)((n + t - 1) / t)); }
 
-void launch_morton_keys(hipStream_t s, int n, const double* pos, Box<double> box, unsigned* keys, int* vals) {
+static void launch_morton_keys(hipStream_t s, int n, const double* pos, Box<double> box, unsigned* keys, int* vals) {
     hipLaunchKernelGGL(k_morton_keys, blocks_for(n, 256), dim3(256), 0, s, n, pos, box, keys, vals);
 }
-void launch_invert_perm(hipStream_t s, int n, const int* perm, int* inv) {
+int launch_sort_atoms(hipStream_t s, int n, const double* pos, Box<double> box, void* temp, size_t bytes,
+                      unsigned* keys, int* vals, int* perm, int* inv, unsigned* keys_sorted) {
+    if (n <= kRankSortMax) {
+        const int nb = (n + kTile - 1) / kTile;
+        hipLaunchKernelGGL(k_rank_sort, dim3(nb), dim3(kRankThreads), (size_t)nb * kTile * sizeof(unsigned), s, n, pos,
+                           box, perm, inv, keys_sorted);
+        return 0;
+    }
+    launch_morton_keys(s, n, pos, box, keys, vals);
+    const int rc = launch_sort_pairs(s, temp, bytes, keys, keys_sorted, vals, perm, n);
     hipLaunchKernelGGL(k_invert_perm, blocks_for(n, 256), dim3(256), 0, s, n, perm, inv);
+    return rc;
 }
-void launch_gather_sorted(hipStream_t s, int n, const int* perm, const int* inv, const double* pos, Box<double> box,
-                          const double* mol, const int4* axes, const double* thole, const double* pol,
-                          const int* partners, const int* npart, int pstride, double4* spos, double* smol,
-                          int4* saxes, double* sthole, double* spol, int* spartners, int* snpart) {
-    hipLaunchKernelGGL(k_gather_sorted, blocks_for(n, 128), dim3(128), 0, s, n, perm, inv, pos, box, mol, axes, thole,
-                       pol, partners, npart, pstride, spos, smol, saxes, sthole, spol, spartners, snpart);
-}
-void launch_rotate(hipStream_t s, int n, Box<double> box, const double4* pos, const int4* axes, const double* mol,
-                   const double* pol, double* lab, double* labpol, double* sqrtpol, double* damp, int* aniso,
-                   int* chg) {
-    hipLaunchKernelGGL(k_rotate, blocks_for(n, 128), dim3(128), 0, s, n, box, pos, axes, mol, pol, lab, labpol,
-                       sqrtpol, damp, aniso, chg);
-}
-template <class R>
-void launch_convert(hipStream_t s, int n, const double4* pos, const double* lab, const double* thole,
-                    const double* damp, R4<R>* rpos, R* rlab, R2<R>* rtd) {
-    hipLaunchKernelGGL(k_convert<R>, blocks_for(n, 256), dim3(256), 0, s, n, pos, lab, thole, damp, rpos, rlab, rtd);
+void launch_sorted_atoms(hipStream_t s, int n, Box<double> box, const double* pos, const AtomParams& in,
+                         const AtomState& out) {
+    hipLaunchKernelGGL(k_sorted_atoms, dim3((n + kTile - 1) / kTile), dim3(kTile), 0, s, n, box, pos, in, out);
 }
 template <class R>
 void launch_recip_potential(hipStream_t s, int n, int pme, const double* phi, const R* phidp, const double* lab,
@@ -1301,8 +1389,6 @@ void launch_recip_atoms(hipStream_t s, int n, int mutual, const double* phi, con
 }
 
 #define MPID_INSTANTIATE(R)                                                                                         \
-    template void launch_convert<R>(hipStream_t, int, const double4*, const double*, const double*, const double*,  \
-                                    R4<R>*, R*, R2<R>*);                                                            \
     template void launch_fill<R>(hipStream_t, R*, size_t, R);                                                        \
     template void launch_fixed_field_finish<R>(hipStream_t, int, const R*, const double*, const acc_t*, FracT<double>, \
                                                double, double*);                                                    \
@@ -1319,6 +1405,7 @@ void launch_recip_atoms(hipStream_t s, int n, int mutual, const double* phi, con
                                         const double*, double, double*);
 MPID_INSTANTIATE(float)
 MPID_INSTANTIATE(double)
+template void launch_fill<int>(hipStream_t, int*, size_t, int);
 #undef MPID_INSTANTIATE
 
 }  // namespace mpid

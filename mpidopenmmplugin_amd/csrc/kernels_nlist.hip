@@ -97,12 +97,14 @@ __device__ __forceinline__ bool blocks_within(float4 a0, float4 a1, float4 b0, f
 // One wavefront per block I.  Count mode (rows == nullptr) writes counts[I]
 // and upper[I], the number of those blocks J with J >= I; fill mode writes
 // the row at rows[start[I] ...] in ascending J, and I into owner[] at the
-// same positions.
+// same positions; *nact takes the number of entries with J >= I (ustart[nb]),
+// or 0 when the rows overflow their capacity.
 __global__ __launch_bounds__(64) void k_block_rows(int nb, const float4* __restrict__ bmin,
                                                    const float4* __restrict__ bmax, Box<float> box, float cutoff,
                                                    const int* __restrict__ start, int* __restrict__ counts,
                                                    int* __restrict__ upper, int* __restrict__ rows,
-                                                   int* __restrict__ owner, int cap) {
+                                                   int* __restrict__ owner, int cap, const int* __restrict__ ustart,
+                                                   int* __restrict__ nact) {
     const int I = blockIdx.x, lane = threadIdx.x;
     const float4 a0 = bmin[I], a1 = bmax[I];
     const int base = rows ? start[I] : 0;
@@ -125,14 +127,22 @@ __global__ __launch_bounds__(64) void k_block_rows(int nb, const float4* __restr
         counts[I] = c;
         upper[I] = cu;
     }
+    if (rows && I == 0 && lane == 0) *nact = start[nb] <= cap ? ustart[nb] : 0;
 }
 
-// start[k] = counts[0] + ... + counts[k-1] for k = 0..m (one workgroup).
-__global__ __launch_bounds__(1024) void k_exclusive_scan(int m, const int* __restrict__ counts, int* __restrict__ start) {
+// Exclusive scans, one workgroup each: start[k] = counts[0] + ... +
+// counts[k-1] for k = 0..m.  The first one's total also goes to *total.
+struct Scans {
+    const int* counts[3];
+    int* start[3];
+};
+__global__ __launch_bounds__(1024) void k_exclusive_scans(int m, Scans sc, int* total) {
     __shared__ int part[1024];
+    const int* __restrict__ counts = sc.counts[blockIdx.x];
+    int* __restrict__ start = sc.start[blockIdx.x];
     const int t = threadIdx.x;
     const int per = (m + 1023) / 1024;
-    const int b = t * per, e = min(b + per, m);
+    const int b = min(t * per, m), e = min(b + per, m);
     int s = 0;
     for (int k = b; k < e; k++) s += counts[k];
     part[t] = s;
@@ -148,7 +158,84 @@ __global__ __launch_bounds__(1024) void k_exclusive_scan(int m, const int* __res
         start[k] = run;
         run += counts[k];
     }
-    if (t == 1023) start[m] = part[1023];
+    if (t == 1023) {
+        start[m] = part[1023];
+        if (blockIdx.x == 0) *total = part[1023];
+    }
+}
+
+// At most kOneRows blocks: counting, the three scans and the rows in one
+// workgroup (the boxes and the hit masks stay in LDS, so each block pair is
+// tested once): at 192 blocks about 9 us against 25-30 us for the two passes
+// and three scans as dependent dispatches.
+__global__ __launch_bounds__(1024) void k_block_rows_one(int nb, const float4* __restrict__ bmin,
+                                                         const float4* __restrict__ bmax, Box<float> box, float cutoff,
+                                                         const int* __restrict__ polcnt, int* __restrict__ start,
+                                                         int* __restrict__ ustart, int* __restrict__ polstart,
+                                                         int* __restrict__ rows, int* __restrict__ owner, int cap,
+                                                         int* total, int* __restrict__ nact) {
+    constexpr int kWords = kOneRows / kTile;
+    __shared__ float4 s0[kOneRows], s1[kOneRows];
+    __shared__ unsigned long long hit[kOneRows][kWords];
+    __shared__ int cnt[3][kOneRows];  // entries, entries with J >= I, polarisable atoms: then inclusive sums
+    const int lane = threadIdx.x & (kTile - 1), w = threadIdx.x / kTile;
+    for (int k = threadIdx.x; k < nb; k += 1024) {
+        s0[k] = bmin[k];
+        s1[k] = bmax[k];
+    }
+    if (threadIdx.x < kOneRows) cnt[2][threadIdx.x] = (int)threadIdx.x < nb ? polcnt[threadIdx.x] : 0;
+    __syncthreads();
+    for (int I = w; I < kOneRows; I += 1024 / kTile) {
+        int c = 0, cu = 0;
+        if (I < nb) {
+            const float4 a0 = s0[I], a1 = s1[I];
+            for (int J0 = 0; J0 < nb; J0 += kTile) {
+                const int J = J0 + lane;
+                const bool h = J < nb && blocks_within(a0, a1, s0[min(J, nb - 1)], s1[min(J, nb - 1)], box, cutoff);
+                const unsigned long long m = __ballot(h);
+                c += __popcll(m);
+                cu += __popcll(__ballot(h && J >= I));
+                if (lane == 0) hit[I][J0 / kTile] = m;
+            }
+        }
+        if (lane == 0) {
+            cnt[0][I] = c;
+            cnt[1][I] = cu;
+        }
+    }
+    __syncthreads();
+    for (int off = 1; off < kOneRows; off <<= 1) {
+        int v[3] = {0, 0, 0};
+        const int t = threadIdx.x;
+        if (t < kOneRows && t >= off)
+            for (int q = 0; q < 3; q++) v[q] = cnt[q][t - off];
+        __syncthreads();
+        if (t < kOneRows)
+            for (int q = 0; q < 3; q++) cnt[q][t] += v[q];
+        __syncthreads();
+    }
+    if ((int)threadIdx.x <= nb) {
+        const int t = threadIdx.x;
+        start[t] = t ? cnt[0][t - 1] : 0;
+        ustart[t] = t ? cnt[1][t - 1] : 0;
+        polstart[t] = t ? cnt[2][t - 1] : 0;
+        if (t == nb) {
+            *total = cnt[0][nb - 1];
+            *nact = cnt[0][nb - 1] <= cap ? cnt[1][nb - 1] : 0;
+        }
+    }
+    for (int I = w; I < nb; I += 1024 / kTile) {
+        int at = I ? cnt[0][I - 1] : 0;
+        for (int J0 = 0; J0 < nb; J0 += kTile) {
+            const unsigned long long m = hit[I][J0 / kTile];
+            const int k = at + __popcll(m & ((1ull << lane) - 1ull));
+            if (((m >> lane) & 1ull) && k < cap) {  // entries beyond the capacity: the host grows it and builds again
+                rows[k] = J0 + lane;
+                owner[k] = I;
+            }
+            at += __popcll(m);
+        }
+    }
 }
 
 // Phase 1 of the atom lists, one wavefront per row entry r = (I, J), J >= I
@@ -162,8 +249,7 @@ __global__ __launch_bounds__(1024) void k_exclusive_scan(int m, const int* __res
 // that entry exists (if not, flag[0] is set and the host raises an error).
 // Tile masks: bit jj for each listed j = J * 64 + jj with j > i, in
 // tmaskcc[r * 64 + lane] when i and j are both bare charges (chg), in
-// tmask[r * 64 + lane] otherwise.  The diagonal entry (I, I) writes
-// polmask[I], the polarisable atoms of block I, and their number polcnt[I].
+// tmask[r * 64 + lane] otherwise.
 __global__ __launch_bounds__(64) void k_nl_masks(int n, const int* __restrict__ rstart, const int* __restrict__ rows,
                                                  const int* __restrict__ owner, const float4* __restrict__ bmin,
                                                  const float4* __restrict__ bmax, const double4* __restrict__ pos,
@@ -278,7 +364,8 @@ __global__ __launch_bounds__(kFillWaves * kTile) void k_nl_fill(
     int n, int all, const int* __restrict__ rstart, const int* __restrict__ rows,
     const unsigned long long* __restrict__ polmask, const int* __restrict__ polstart,
     const unsigned long long* __restrict__ nmask, int cap, int* __restrict__ nbr, int* __restrict__ count,
-    int* __restrict__ maxcount, int* __restrict__ pnbr, int* __restrict__ pcount, int rcap) {
+    int* __restrict__ maxcount, int* __restrict__ pnbr, int* __restrict__ pcount, int rcap, int* __restrict__ pol_idx,
+    int ntiles, const int* __restrict__ tstart, int* __restrict__ tpstart) {
     __shared__ int scnt[kFillWaves][kTile], spcnt[kFillWaves][kTile];
     const int I = blockIdx.x, lane = threadIdx.x & (kTile - 1), w = threadIdx.x / kTile;
     const int nb = (n + kTile - 1) / kTile;
@@ -289,6 +376,15 @@ __global__ __launch_bounds__(kFillWaves * kTile) void k_nl_fill(
     const bool store = iv && (all || ipol);
     const int li = all ? i : polstart[I] + __popcll(pmI & ((1ull << lane) - 1ull));
     const int nrows = all ? n : polstart[nb];
+    // the sorted index of the polarisable atoms, and its spreading tiles: a
+    // tile's first polarisable atom is the first one at or after its first atom
+    if (w == 0 && ipol) pol_idx[polstart[I] + __popcll(pmI & ((1ull << lane) - 1ull))] = i;
+    if (tpstart)
+        for (int t = I * kFillWaves * kTile + threadIdx.x; t <= ntiles; t += nb * kFillWaves * kTile) {
+            const int f = tstart[t], B = f / kTile;
+            tpstart[t] = B >= nb ? polstart[nb]
+                                 : polstart[B] + __popcll(polmask[B] & ((1ull << (f & (kTile - 1))) - 1ull));
+        }
     // (rows beyond the capacity rcap were not stored; the host grows it and builds again)
     const int r0 = min(rstart[I], rcap), r1 = min(rstart[I + 1], rcap);
     const int per = (r1 - r0 + kFillWaves - 1) / kFillWaves;
@@ -355,30 +451,6 @@ __global__ __launch_bounds__(kFillWaves * kTile) void k_nl_fill(
         for (int off = 32; off >= 1; off >>= 1) lmax = max(lmax, __shfl_xor(lmax, off));
         if (lane == 0 && lmax > 0) atomicMax(maxcount, lmax);
     }
-}
-
-// The polarisable atoms of each block (damping factor nonzero): a mask and
-// its count, one wavefront per block.
-__global__ __launch_bounds__(64) void k_pol_mask(int n, const double4* __restrict__ pos,
-                                                 unsigned long long* __restrict__ polmask, int* __restrict__ polcnt) {
-    const int I = blockIdx.x, lane = threadIdx.x;
-    const int i = I * kTile + lane;
-    const unsigned long long pm = __ballot(i < n && pos[i < n ? i : n - 1].w != 0.0);
-    if (lane == 0) {
-        polmask[I] = pm;
-        polcnt[I] = __popcll(pm);
-    }
-}
-
-// Sorted indices of the polarisable atoms, in order: block I writes its
-// polarisable lanes from start[I].
-__global__ __launch_bounds__(64) void k_pol_fill(int n, const double4* __restrict__ pos, const int* __restrict__ start,
-                                                 int* __restrict__ idx) {
-    const int I = blockIdx.x, lane = threadIdx.x;
-    const int i = I * kTile + lane;
-    const bool p = i < n && pos[i].w != 0.0;
-    const unsigned long long m = __ballot(p);
-    if (p) idx[start[I] + __popcll(m & ((1ull << lane) - 1ull))] = i;
 }
 
 // ---------------------------------------------------------------------------
@@ -546,32 +618,35 @@ __global__ __launch_bounds__(256) void k_nl_thole(NbrList L, const int* __restri
 // launchers
 // ---------------------------------------------------------------------------
 void launch_block_rows(hipStream_t s, int nb, const float4* bmin, const float4* bmax, Box<float> box, float cutoff,
-                       const int* start, int* counts, int* upper, int* rows, int* owner, int cap) {
-    hipLaunchKernelGGL(k_block_rows, dim3(nb), dim3(kTile), 0, s, nb, bmin, bmax, box, cutoff, start, counts, upper,
-                       rows, owner, cap);
-}
-void launch_exclusive_scan(hipStream_t s, int m, const int* counts, int* start) {
-    hipLaunchKernelGGL(k_exclusive_scan, dim3(1), dim3(1024), 0, s, m, counts, start);
+                       const int* polcnt, int* work, int* start, int* ustart, int* polstart, int* rows, int* owner,
+                       int cap, int* total, int* nact) {
+    if (nb <= kOneRows) {
+        hipLaunchKernelGGL(k_block_rows_one, dim3(1), dim3(1024), 0, s, nb, bmin, bmax, box, cutoff, polcnt, start,
+                           ustart, polstart, rows, owner, cap, total, nact);
+        return;
+    }
+    hipLaunchKernelGGL(k_block_rows, dim3(nb), dim3(kTile), 0, s, nb, bmin, bmax, box, cutoff, nullptr, work, work + nb,
+                       nullptr, nullptr, 0, nullptr, nullptr);
+    const Scans sc{{work, work + nb, polcnt}, {start, ustart, polstart}};
+    hipLaunchKernelGGL(k_exclusive_scans, dim3(3), dim3(1024), 0, s, nb, sc, total);
+    if (cap > 0)
+        hipLaunchKernelGGL(k_block_rows, dim3(nb), dim3(kTile), 0, s, nb, bmin, bmax, box, cutoff, start, nullptr,
+                           nullptr, rows, owner, cap, ustart, nact);
 }
 void launch_nl_build(hipStream_t s, int n, int nrows, int rcap, bool all, const int* rstart, const int* rows,
                      const int* owner, const float4* bmin, const float4* bmax, const double4* pos,
                      const int* partners, const int* npart, int pstride, Box<double> box, double rc2, int cap,
-                     unsigned long long* nmask, unsigned long long* polmask, int* polcnt, int* polstart, int* nbr,
+                     unsigned long long* nmask, const unsigned long long* polmask, const int* polstart, int* nbr,
                      int* count, int* scalars, unsigned long long* tmask, int* pnbr, int* pcount, const int* chg,
-                     unsigned long long* tmaskcc, int4* act, const int* ustart) {
+                     unsigned long long* tmaskcc, int4* act, const int* ustart, int* pol_idx, int ntiles,
+                     const int* tstart, int* tpstart) {
     const int nb = (n + kTile - 1) / kTile;
-    hipLaunchKernelGGL(k_pol_mask, dim3(nb), dim3(kTile), 0, s, n, pos, polmask, polcnt);
     if (nrows > 0)
         hipLaunchKernelGGL(k_nl_masks, dim3(nrows), dim3(kTile), 0, s, n, rstart, rows, owner, bmin, bmax, pos,
                            partners, npart, pstride, box, rc2, chg, nmask, tmask, tmaskcc, scalars + 1, rcap, act,
                            ustart);
-    launch_exclusive_scan(s, nb, polcnt, polstart);
     hipLaunchKernelGGL(k_nl_fill, dim3(nb), dim3(kFillWaves * kTile), 0, s, n, all ? 1 : 0, rstart, rows, polmask,
-                       polstart, nmask, cap, nbr, count, scalars, pnbr, pcount, rcap);
-}
-void launch_pol_fill(hipStream_t s, int n, const double4* pos, const int* start, int* idx) {
-    const int nb = (n + kTile - 1) / kTile;
-    hipLaunchKernelGGL(k_pol_fill, dim3(nb), dim3(kTile), 0, s, n, pos, start, idx);
+                       polstart, nmask, cap, nbr, count, scalars, pnbr, pcount, rcap, pol_idx, ntiles, tstart, tpstart);
 }
 template <class R>
 void launch_nl_fixed_field(hipStream_t s, int natoms, const int* atoms, NbrList l, PairAtoms<R> a, PairParams<R> p,

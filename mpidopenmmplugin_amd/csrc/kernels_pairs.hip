@@ -20,40 +20,6 @@
 
 namespace mpid {
 
-// ---------------------------------------------------------------------------
-// blocks and tiles
-// ---------------------------------------------------------------------------
-template <class R>
-__global__ __launch_bounds__(64) void k_block_bounds(int n, const R4<R>* __restrict__ pos, float4* bmin,
-                                                      float4* bmax) {
-    int b = blockIdx.x, lane = threadIdx.x;
-    int i = b * kTile + lane;
-    float lo[3], hi[3];
-    if (i < n) {
-        R4<R> p = pos[i];
-        lo[0] = hi[0] = (float)p.x;
-        lo[1] = hi[1] = (float)p.y;
-        lo[2] = hi[2] = (float)p.z;
-    } else {
-        R4<R> p = pos[b * kTile];
-        lo[0] = hi[0] = (float)p.x;
-        lo[1] = hi[1] = (float)p.y;
-        lo[2] = hi[2] = (float)p.z;
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            lo[k] = fminf(lo[k], __shfl_xor(lo[k], off));
-            hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], off));
-        }
-    }
-    if (lane == 0) {
-        bmin[b] = make_float4(lo[0], lo[1], lo[2], 0.f);
-        bmax[b] = make_float4(hi[0], hi[1], hi[2], 0.f);
-    }
-}
-
 constexpr int kElecThreads = 256;  // four wavefronts share one tile
 
 // kPot (the energy gradients): also the potential vectors dE/dm of every
@@ -610,13 +576,6 @@ __global__ __launch_bounds__(128) void k_cov_electrostatics(PairAtoms<R> A, cons
 // launchers
 // ---------------------------------------------------------------------------
 template <class R>
-void launch_block_bounds(hipStream_t s, int n, const R4<R>* pos, float4* bmin, float4* bmax) {
-    int nb = (n + kTile - 1) / kTile;
-    hipLaunchKernelGGL(k_block_bounds<R>, dim3(nb), dim3(kTile), 0, s, n, pos, bmin, bmax);
-}
-
-
-template <class R>
 void launch_electrostatics_pairs(hipStream_t s, int maxtiles, const int4* act, const int* nact, const int* rows,
                                  const int* owner, const unsigned long long* tmask,
                                  const unsigned long long* tmaskcc, const int* chg, PairAtoms<R> a, const R* mu,
@@ -719,7 +678,6 @@ void launch_electrostatics_pot(hipStream_t s, int maxtiles, const int4* act, con
 }
 
 #define MPID_INSTANTIATE(R)                                                                                        \
-    template void launch_block_bounds<R>(hipStream_t, int, const R4<R>*, float4*, float4*);                         \
     template void launch_electrostatics_pairs<R>(hipStream_t, int, const int4*, const int*, const int*, const int*,\
                                                  const unsigned long long*, const unsigned long long*, const int*,   \
                                                  PairAtoms<R>, const R*, PairParams<R>, const double4*,             \

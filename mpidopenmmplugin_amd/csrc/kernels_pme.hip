@@ -144,19 +144,6 @@ __device__ __forceinline__ unsigned compact_bits(unsigned v) {
     return v;
 }
 
-// Range [tstart[t], tend[t]) of the atoms of Morton cell t.  With idx, over
-// the subsequence idx[0 .. *count) of the sorted atoms (still in Morton order).
-__global__ void k_tile_ranges(int n, const unsigned* __restrict__ keys, const int* __restrict__ idx,
-                              const int* __restrict__ count, int shift, int* tstart, int* tend) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    const int m = count ? *count : n;
-    if (s >= m) return;
-    auto key = [&](int k) { return keys[idx ? idx[k] : k] >> shift; };
-    const unsigned t = key(s);
-    if (s == 0 || key(s - 1) != t) tstart[t] = s;
-    if (s == m - 1 || key(s + 1) != t) tend[t] = s + 1;
-}
-
 template <class R, int MODE>
 __global__ __launch_bounds__(256) void k_spread_tiled(const R4<R>* __restrict__ pos, const R* __restrict__ src,
                                                        PmeGeom<R> g, TileGeom tg, const int* __restrict__ atoms,
@@ -750,12 +737,6 @@ void launch_spread_induced(hipStream_t s, int natoms, const int* atoms, const R4
     hipLaunchKernelGGL(k_spread_induced<R>, dim3((natoms + kSpreadWaves - 1) / kSpreadWaves), dim3(64 * kSpreadWaves),
                        0, s, natoms, atoms, pos, mu, g, grid);
 }
-void launch_tile_ranges(hipStream_t s, int n, const unsigned* keys_sorted, const int* idx, const int* count,
-                        int shift, int* tstart, int* tend) {
-    hipLaunchKernelGGL(k_tile_ranges, dim3((n + 255) / 256), dim3(256), 0, s, n, keys_sorted, idx, count, shift, tstart,
-                       tend);
-}
-
 template <class R, int MODE> static size_t tiled_lds(const TileGeom& tg) {
     constexpr int ND = MODE == 0 ? 3 : 1;
     constexpr int NC = MODE == 0 ? 20 : 3;

@@ -512,29 +512,97 @@ __global__ __launch_bounds__(256) void k_cg_direction(SolverSites st, const doub
 // ---------------------------------------------------------------------------
 // vectors
 // ---------------------------------------------------------------------------
-// b = S E0, x = b and the first operator input mu = S x (in both precisions
-// where mu2 is given); zeros at every other atom of mu, mu2 and mud.
+// Permanent field at a polarisable site: every kFixedLanes-th listed
+// neighbour from `lane` on, in R, and of the covalent partners in FP64 (their
+// screened and unscreened parts nearly cancel).
+constexpr int kFixedLanes = 16;
 template <class R>
-__global__ __launch_bounds__(256) void k_solver_init(SolverSites st, int n, const double4* __restrict__ pos,
-                                                     const double* __restrict__ E0, double* b, double* x,
-                                                     R* __restrict__ mu, double* __restrict__ mu2,
-                                                     double* __restrict__ mud) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t < n && pos[t].w == 0.0) {
-        const D3 z = mk(0.0, 0.0, 0.0);
-        store_mu<R>(mu, t, z);
-        store3(mud, t, z);
-        if (mu2) store3(mu2, t, z);
+__device__ __forceinline__ D3 fixed_field_part(const SolverSites& st, int t, int i, int lane, const NbrList& L,
+                                               const PairAtoms<R>& A, const PairParams<R>& P,
+                                               const PairAtoms<double>& A64, const PairParams<double>& P64) {
+    const R4<R> pi = A.pos[i];
+    const R2<R> tdi = A.td[i];
+    const int cnt = L.count[i];
+    R ex = 0, ey = 0, ez = 0;
+    for (int k = lane; k < cnt; k += kFixedLanes) {
+        const int j = L.nbr[((size_t)(k / kNlSplit) * st.npol + t) * kNlSplit + k % kNlSplit];
+        const R4<R> pj = A.pos[j];
+        const V3<R> dr = min_image(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), P.box);
+        R mj[kMP];
+#pragma unroll
+        for (int c = 0; c < kMP; c++) mj[c] = A.lab[(size_t)j * kMP + c];
+        // listed pairs are not covalent partners: scale 1, default Thole width
+        const FixedRadial<R> gr = fixed_field_radial<R>(dot(dr, dr), tdi, R2<R>{R(0), pj.w}, R(1), P);
+        const V3<R> f = fixed_field_from<R>(mj, dr, gr);
+        ex += f.x;
+        ey += f.y;
+        ez += f.z;
     }
-    if (t >= st.npol) return;
+    D3 e = mk((double)ex, (double)ey, (double)ez);
+    const int np = A64.npart[i];
+    for (int k = lane; k < np; k += kFixedLanes) {
+        const int en = A64.partners[(size_t)i * A64.pstride + k];
+        const int j = en >> 2;
+        const double4 qi = A64.pos[i], qj = A64.pos[j];
+        const D3 dr = min_image(mk(qj.x - qi.x, qj.y - qi.y, qj.z - qi.z), P64.box);
+        const double r2 = dot(dr, dr);
+        if (r2 > P64.rc2) continue;
+        const FixedRadial<double> gr =
+            fixed_field_radial<double>(r2, A64.td[i], A64.td[j], partner_scale<double>(en, P64.scale14), P64);
+        e = e + fixed_field_from<double>(A64.lab + (size_t)j * kMP, dr, gr);
+    }
+#pragma unroll
+    for (int off = 1; off < kFixedLanes; off <<= 1) {
+        e.x += __shfl_xor(e.x, off);
+        e.y += __shfl_xor(e.y, off);
+        e.z += __shfl_xor(e.z, off);
+    }
+    return e;
+}
+template <class R>
+__global__ __launch_bounds__(256) void k_fixed_list(SolverSites st, NbrList L, PairAtoms<R> A, PairParams<R> P,
+                                                    PairAtoms<double> A64, PairParams<double> P64,
+                                                    double* __restrict__ field) {
+    const int g = (int)(blockIdx.x * 256 + threadIdx.x) / kFixedLanes, lane = threadIdx.x % kFixedLanes;
+    const int t = min(g, st.npol - 1);
+    const D3 e = fixed_field_part<R>(st, t, st.idx[t], lane, L, A, P, A64, P64);
+    if (g < st.npol && lane == 0) store3(field, t, e);
+}
+// E0 = real space + reciprocal (-A phi_1) + self, b = x = S E0 and the first
+// operator input mu = S x.  LIST: the real-space part here, kFixedLanes lanes
+// per site (two dispatches less; the list walk then waits for phi); else one
+// thread per site with the part of k_fixed_list.
+template <class R, bool LIST>
+__global__ __launch_bounds__(256) void k_solver_init(SolverSites st, NbrList L, PairAtoms<R> A, PairParams<R> P,
+                                                     PairAtoms<double> A64, PairParams<double> P64,
+                                                     const double* __restrict__ field, const double* __restrict__ phi,
+                                                     FracT<double> F, double selfc, double* __restrict__ E0, double* b,
+                                                     double* x, R* __restrict__ mu, double* __restrict__ mud,
+                                                     const int* __restrict__ nl_scalars, int* hnl) {
+    constexpr int kLanes = LIST ? kFixedLanes : 1;
+    const int g = (int)(blockIdx.x * 256 + threadIdx.x) / kLanes, lane = threadIdx.x % kLanes;
+    if (blockIdx.x == 0 && threadIdx.x < 2) hnl[threadIdx.x] = nl_scalars[threadIdx.x];
+    if (st.npol == 0) return;
+    const int t = min(g, st.npol - 1);
     const int i = st.idx[t];
+    D3 e;
+    if (LIST) e = fixed_field_part<R>(st, t, i, lane, L, A, P, A64, P64);
+    else e = load3(field, t);
+    if (g >= st.npol || lane != 0) return;
+    const double* ph = phi + 35 * (size_t)i;
+    const double* m = A64.lab + (size_t)i * kMP;
+    const D3 c1 = cart_vector(mk(ph[1], ph[2], ph[3]), F);
+    e.x += selfc * m[1] - c1.x;
+    e.y += selfc * m[2] - c1.y;
+    e.z += selfc * m[3] - c1.z;
+    store3(E0, i, e);
     const double* S = st.S + 6 * (size_t)i;
-    const D3 v = sym_mul6(S, load3(E0, i));
+    const D3 v = sym_mul6(S, e);
     store3(b, t, v);
     store3(x, t, v);
-    const D3 m = sym_mul6(S, v);
-    store_mu<R>(mu, i, m);
-    store3(mud, i, m);
+    const D3 u = sym_mul6(S, v);
+    store_mu<R>(mu, i, u);
+    store3(mud, i, u);
 }
 
 // mu = S v by atom (and mud, its FP64 copy); at: by site (DIIS's errors)
@@ -641,9 +709,25 @@ void launch_cg_iteration(hipStream_t s, SolverSites st, const double* Ap, double
                        blocks, scal, hcheck, n, stop_eps);
 }
 template <class R>
-void launch_solver_init(hipStream_t s, SolverSites st, int n, const double4* pos, const double* E0, double* b,
-                        double* x, R* mu, double* mu2, double* mud) {
-    hipLaunchKernelGGL(k_solver_init<R>, dim3((n + 255) / 256), dim3(256), 0, s, st, n, pos, E0, b, x, mu, mu2, mud);
+void launch_fixed_list(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p,
+                       PairAtoms<double> a64, PairParams<double> p64, double* field) {
+    if (st.npol <= 0) return;
+    const unsigned blocks = ((unsigned)st.npol * kFixedLanes + 255) / 256;
+    hipLaunchKernelGGL(k_fixed_list<R>, dim3(blocks), dim3(256), 0, s, st, l, a, p, a64, p64, field);
+}
+template <class R>
+void launch_solver_init(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p,
+                        PairAtoms<double> a64, PairParams<double> p64, const double* field, const double* phi,
+                        FracT<double> A, double selfc, double* E0, double* b, double* x, R* mu, double* mud,
+                        const int* nl_scalars, int* hnl) {
+    const unsigned threads = std::max(1u, (unsigned)st.npol * (field ? 1 : kFixedLanes));
+    const dim3 blocks((threads + 255) / 256);
+    if (field)
+        hipLaunchKernelGGL((k_solver_init<R, false>), blocks, dim3(256), 0, s, st, l, a, p, a64, p64, field, phi, A,
+                           selfc, E0, b, x, mu, mud, nl_scalars, hnl);
+    else
+        hipLaunchKernelGGL((k_solver_init<R, true>), blocks, dim3(256), 0, s, st, l, a, p, a64, p64, field, phi, A,
+                           selfc, E0, b, x, mu, mud, nl_scalars, hnl);
 }
 template <class R>
 void launch_apply_S(hipStream_t s, SolverSites st, const double* v, R* mu, double* mud, double* at) {
@@ -667,8 +751,12 @@ void launch_residual(hipStream_t s, SolverSites st, const double* b, const doubl
                                      double*, R*, double*, double*, double*, int, double);                          \
     template void launch_cg_iteration<R>(hipStream_t, SolverSites, const double*, double*, double*, double*, R*,    \
                                          int, double*, double*, double*, int, double);                              \
-    template void launch_solver_init<R>(hipStream_t, SolverSites, int, const double4*, const double*, double*,      \
-                                        double*, R*, double*, double*);                                            \
+    template void launch_fixed_list<R>(hipStream_t, SolverSites, NbrList, PairAtoms<R>, PairParams<R>,              \
+                                       PairAtoms<double>, PairParams<double>, double*);                            \
+    template void launch_solver_init<R>(hipStream_t, SolverSites, NbrList, PairAtoms<R>, PairParams<R>,             \
+                                        PairAtoms<double>, PairParams<double>, const double*, const double*,        \
+                                        FracT<double>, double, double*, double*, double*, R*, double*, const int*,  \
+                                        int*);                                                                     \
     template void launch_apply_S<R>(hipStream_t, SolverSites, const double*, R*, double*, double*);
 MPID_INSTANTIATE(float)
 MPID_INSTANTIATE(double)

@@ -1,4 +1,13 @@
-"""The mutual-polarization solver at the sizes where its kernels change form.
+"""The evaluation's build and the mutual-polarization solver at the sizes where
+their kernels change form.
+
+Sorting and lab frames around whole 64-atom blocks and around 16,384 atoms (one
+kernel ranks the keys and one workgroup builds the block rows up to there, a
+radix sort and several kernels beyond): the lab-frame dipoles, which come back
+through the permutation, equal the frames written out in numpy to 2e-13 of
+the largest component (FP64 rounding: the O-H vectors carry 1e-15 of box edges
+up to 5.5 nm, 6e-15 of the 0.0957 nm bond, through two normalisations and the
+orthogonalisation, with a factor 10 in hand).
 
 Small clusters without a cutoff, at site counts around the eight sites of an
 operator workgroup, against the FP64 oracle converged to 1e-10 Debye: the
@@ -37,6 +46,33 @@ def rel_rms(a, b):
     return np.sqrt(((a - b) ** 2).sum() / (b ** 2).sum())
 
 
+@pytest.mark.parametrize("waters", [1, 21, 22, 64, 65, 5461, 5462])
+def test_lab_frames_through_the_sort(waters):
+    force, pos, box = make_small_waterbox(max(waters, 32), waters)
+    flat = force.flatten()
+    k = HipCalcMPIDForceKernel("double")
+    if waters < 32:  # a cluster: the smallest boxes hold 32 waters
+        pos = pos[:3 * waters]
+        force = _water_force(waters, _o_parameters(np.random.default_rng(waters), True, True))
+        force.setNonbondedMethod(MPIDForce.NoCutoff)
+        flat, box = force.flatten(), None
+    k.initialize(len(pos), force, default_box=box)
+    print(f"[gpu] frames of {waters} waters", flush=True)
+    found = k.getLabFramePermanentDipoles(pos, box)
+    o, h1, h2 = pos[0::3], pos[1::3], pos[2::3]
+
+    def unit(v):
+        return v / np.linalg.norm(v, axis=1, keepdims=True)
+
+    u1, u2 = unit(h1 - o), unit(h2 - o)
+    z = unit(u1 + u2)
+    x = unit(u2 - z * (z * u2).sum(1, keepdims=True))
+    d = flat["dipoles"].reshape(-1, 3)[0::3]
+    expected = d[:, :1] * x + d[:, 1:2] * np.cross(z, x) + d[:, 2:] * z
+    assert not found.reshape(-1, 3, 3)[:, 1:].any()
+    assert np.abs(found[::3] - expected).max() <= 1e-14 * 20 * np.abs(expected).max()
+
+
 @pytest.mark.parametrize("waters", [1, 2, 7, 8, 9, 33])
 def test_small_clusters(waters):
     force, pos, _ = make_small_waterbox(waters, 40 + waters)
@@ -57,7 +93,7 @@ def test_small_clusters(waters):
         assert np.sqrt(((F - ref["forces"]) ** 2).sum()) <= f_tol * max(np.sqrt((ref["forces"] ** 2).sum()), 1.0)
 
 
-@pytest.mark.parametrize("waters", [2048, 2049, 8192, 8193])
+@pytest.mark.parametrize("waters", [2048, 2049, 5461, 5462, 8192, 8193])
 def test_dipoles_satisfy_their_equation(waters):
     alpha = 0.001
     rng = np.random.default_rng(waters)
