@@ -191,7 +191,8 @@ void launch_sorted_atoms(hipStream_t s, int n, Box<double> box, const double* po
 // torques) instead of the reference's approximate projection
 void launch_torque_to_force(hipStream_t s, int n, Box<double> box, const double4* pos, const int4* axes,
                             const acc_t* torque, acc_t* force, int exact_threefold);
-void launch_output_forces(hipStream_t s, int n, const int* perm, const acc_t* force, double* out, int accumulate);
+void launch_output_forces(hipStream_t s, int n, const int* perm, const acc_t* force, double* out, int accumulate,
+                          const acc_t* energy, acc_t* esum);
 void launch_unpermute3(hipStream_t s, int n, const int* perm, const double* in, double* out);
 void launch_zero_acc(hipStream_t s, acc_t* p, size_t count);
 size_t sort_temp_bytes(int n);
@@ -252,11 +253,12 @@ template <class R>
 void launch_extrap_init(hipStream_t s, int n, const double* labpol, const double* E0, double* mu, R* mu_r);
 void launch_axpy(hipStream_t s, int m, double a, const double* x, double* y);
 void launch_sub(hipStream_t s, int m, const double* a, const double* b, double* out);
-// reciprocal-space energy, forces and torques, self terms (per atom)
+// reciprocal-space energy, forces and torques, self terms (per atom), and
+// (cov) the covalent pairs' electrostatics; energy: 2 kEnergySlots words
 template <class R>
-void launch_recip_atoms(hipStream_t s, int n, int mutual, const double* phi, const R* phidp, const double* lab,
-                        const double* mu, const int* aniso, FracT<double> A, double alpha, acc_t* force,
-                        acc_t* torque, acc_t* energy);
+void launch_final_atoms(hipStream_t s, int n, int mutual, const double* phi, const R* phidp, const double* mu,
+                        FracT<double> A, double alpha, PairAtoms<double> c, PairParams<double> p, bool cov,
+                        acc_t* force, acc_t* torque, acc_t* energy);
 
 // ---- PME (kernels_pme.hip) ----------------------------------------------------
 template <class R> struct PmeGeom {
@@ -413,10 +415,10 @@ template <class R> void launch_cov_fixed_field(hipStream_t s, int n, PairAtoms<R
 template <class R>
 void launch_cov_induced_field(hipStream_t s, int n, PairAtoms<R> a, const R* mu, PairParams<R> p, int pol_only,
                               acc_t* field, acc_t* grad = nullptr);
-// pot != nullptr: also each pair's potential vectors dE/dm (20 per atom)
+// the covalent pairs' electrostatics with their potential vectors dE/dm (20 per atom)
 template <class R>
-void launch_cov_electrostatics(hipStream_t s, int n, PairAtoms<R> a, const R* mu, PairParams<R> p, acc_t* force,
-                               acc_t* torque, acc_t* energy, acc_t* pot = nullptr);
+void launch_cov_electrostatics_pot(hipStream_t s, int n, PairAtoms<R> a, const R* mu, PairParams<R> p, acc_t* force,
+                                   acc_t* torque, acc_t* energy, acc_t* pot);
 
 // ---- mutual-polarization solver (kernels_solver.hip) -----------------------------
 // Its vectors hold the polarisable sites only (entry t: atom idx[t]); S by atom.
@@ -472,6 +474,10 @@ void launch_solver_init(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a
                         PairAtoms<double> a64, PairParams<double> p64, const double* field, const double* phi,
                         FracT<double> A, double selfc, double* E0, double* b, double* x, R* mu, double* mud,
                         const int* nl_scalars, int* hnl);
+// The final pass's start: mu = mud = S v (v null: they are in place) and the
+// accumulators cleared
+template <class R>
+void launch_final_start(hipStream_t s, SolverSites st, const double* v, R* mu, double* mud, acc_t* acc, size_t count);
 // S v: by atom in mu and mud, by site in at (each may be null)
 template <class R>
 void launch_apply_S(hipStream_t s, SolverSites st, const double* v, R* mu, double* mud, double* at);

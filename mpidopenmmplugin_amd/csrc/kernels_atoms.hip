@@ -11,7 +11,7 @@
 // computeReciprocalSpaceInducedDipoleForceAndEnergy :3871-4024,
 // calculatePmeSelfEnergy :4283-4318, calculatePmeSelfTorque :4320-4333,
 // mapTorqueToForceForParticle :1895-2110.
-#include "engine.h"
+#include "pair_math.h"
 
 #include <cstring>
 #include <map>
@@ -292,15 +292,35 @@ __global__ __launch_bounds__(kTile) void k_sorted_atoms(int n, Box<double> box, 
                 for (int l = 0; l < 3; l++) x += E[k][c] * E[l][b] * m[4 + i2(k, l)];
             r[4 + i2(c, b)] = x;
         }
-    for (int c = 0; c < 3; c++)
-        for (int b = c; b < 3; b++)
-            for (int d = b; d < 3; d++) {
-                double x = 0;
-                for (int k = 0; k < 3; k++)
-                    for (int l = 0; l < 3; l++)
-                        for (int q = 0; q < 3; q++) x += E[k][c] * E[l][b] * E[q][d] * m[10 + i3(k, l, q)];
-                r[10 + i3(c, b, d)] = x;
-            }
+    // octopole, one index at a time (O_klq E_qd, then E_lb, then E_kc: 140
+    // multiply-adds where the triple sum per component takes 810)
+    {
+        double o1[3][3][3], o2[3][3][3];  // [k][l][d] for l >= k, then [k][b][d] for d >= b
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+#pragma unroll
+            for (int l = k; l < 3; l++)
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    o1[k][l][d] = m[10 + i3(k, l, 0)] * E[0][d] + m[10 + i3(k, l, 1)] * E[1][d] +
+                                  m[10 + i3(k, l, 2)] * E[2][d];
+                    o1[l][k][d] = o1[k][l][d];
+                }
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+#pragma unroll
+            for (int b = 0; b < 3; b++)
+#pragma unroll
+                for (int d = b; d < 3; d++)
+                    o2[k][b][d] = o1[k][0][d] * E[0][b] + o1[k][1][d] * E[1][b] + o1[k][2][d] * E[2][b];
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+#pragma unroll
+            for (int b = c; b < 3; b++)
+#pragma unroll
+                for (int d = b; d < 3; d++)
+                    r[10 + i3(c, b, d)] = o2[0][b][d] * E[0][c] + o2[1][b][d] * E[1][c] + o2[2][b][d] * E[2][c];
+    }
     const double pk[3] = {p0, p1, p2};
     const double sk[3] = {sqrt(fmax(p0, 0.0)), sqrt(fmax(p1, 0.0)), sqrt(fmax(p2, 0.0))};
     for (int c = 0; c < 3; c++)
@@ -658,39 +678,29 @@ __device__ __forceinline__ double comp_mult(int k) {
     const double t[20] = {1, 1, 1, 1, 1, 2, 2, 1, 2, 1, 1, 3, 3, 3, 6, 3, 1, 3, 3, 1};
     return t[k];
 }
-__device__ __forceinline__ int levi(int a, int b, int c) {
-    if (a == b || b == c || a == c) return 0;
-    return ((a == 0 && b == 1) || (a == 1 && b == 2) || (a == 2 && b == 0)) ? 1 : -1;
-}
-
 // Torque -dE/dtheta of moments (d, Q, O) in a potential whose Cartesian
 // derivative tensors are c1, c2 (6), c3 (10); E = d.c1 + Q:c2 + O:c3 over all
-// index orderings.
-__device__ D3 multipole_torque(const double* d, const double* Q, const double* O, const double* c1, const double* c2,
-                               const double* c3) {
-    double t[3];
-    for (int k = 0; k < 3; k++) {
-        double s = 0;
-        for (int a = 0; a < 3; a++)
-            for (int i = 0; i < 3; i++) s += levi(a, k, i) * d[i] * c1[a];
-        for (int a = 0; a < 3; a++)
+// index orderings.  Turning the moments by theta changes E by theta.s with
+// s_k = eps_kia (d_i c1_a + 2 N2_ia + 3 N3_ia), N2_ia = Q_ib c2_ab and
+// N3_ia = O_ibc c3_abc.
+__device__ __forceinline__ D3 multipole_torque(const double* d, const double* Q, const double* O, const double* c1,
+                                               const double* c2, const double* c3) {
+    double n[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            if (i == a) continue;
+            double q = 0.0, o = 0.0;
+#pragma unroll
             for (int b = 0; b < 3; b++) {
-                double dq = 0;
-                for (int i = 0; i < 3; i++) dq += levi(a, k, i) * Q[i2(i, b)] + levi(b, k, i) * Q[i2(a, i)];
-                s += dq * c2[i2(a, b)];
+                q += Q[i2(i, b)] * c2[i2(a, b)];
+#pragma unroll
+                for (int c = b; c < 3; c++) o += (b == c ? 3.0 : 6.0) * O[i3(i, b, c)] * c3[i3(a, b, c)];
             }
-        for (int a = 0; a < 3; a++)
-            for (int b = 0; b < 3; b++)
-                for (int c = 0; c < 3; c++) {
-                    double dq = 0;
-                    for (int i = 0; i < 3; i++)
-                        dq += levi(a, k, i) * O[i3(i, b, c)] + levi(b, k, i) * O[i3(a, i, c)] +
-                              levi(c, k, i) * O[i3(a, b, i)];
-                    s += dq * c3[i3(a, b, c)];
-                }
-        t[k] = -s;
-    }
-    return mk(t[0], t[1], t[2]);
+            n[i][a] = d[i] * c1[a] + 2.0 * q + o;
+        }
+    return mk(n[2][1] - n[1][2], n[0][2] - n[2][0], n[1][0] - n[0][1]);
 }
 
 // Cartesian derivative tensors of the potential from grid-coordinate ones:
@@ -766,110 +776,119 @@ __device__ void cart_potential(const R* ph, const FracT<double>& A, double* c1, 
 }
 
 template <class R>
-__global__ __launch_bounds__(128) void k_recip_atoms(int n, int mutual, const double* __restrict__ phi,
-                                                      const R* __restrict__ phidp, const double* __restrict__ lab,
-                                                      const double* __restrict__ mu, const int* __restrict__ aniso,
-                                                      FracT<double> A, double alpha, acc_t* force, acc_t* torque,
-                                                      acc_t* energy) {
-    __shared__ double sh[128];
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    double en = 0;
-    if (s < n) {
-        const double* m = lab + (size_t)s * kMP;
-        const double* ph = phi + (size_t)s * 35;
-        const R* pd = phidp + (size_t)s * 35;
-        const double u[3] = {mu[3 * (size_t)s], mu[3 * (size_t)s + 1], mu[3 * (size_t)s + 2]};
-        const bool an = aniso[s] != 0;
-        // fractional multipoles
-        double mf[20];
-        frac_moments<double>(m, A, mf);
-        // fixed: energy 1/2 eps M.phi, force -eps grad, torque
-        double ef = 0, f[3] = {0, 0, 0}, fi[3] = {0, 0, 0};
-        for (int k = 0; k < 20; k++) {
-            int e[3];
-            comp_exp(k, e);
-            ef += mf[k] * (double)ph[phi_idx(e[0], e[1], e[2])];
-            for (int a = 0; a < 3; a++) {
-                int e2[3] = {e[0], e[1], e[2]};
-                e2[a]++;
-                const int id = phi_idx(e2[0], e2[1], e2[2]);
-                f[a] += mf[k] * (double)ph[id];
-                fi[a] += 2.0 * mf[k] * (double)pd[id];
-            }
+__device__ __forceinline__ double recip_atom(int s, int mutual, const double* __restrict__ phi,
+                                             const R* __restrict__ phidp, const double* __restrict__ lab,
+                                             const double* __restrict__ mu, const int* __restrict__ aniso,
+                                             const FracT<double>& A, double alpha, acc_t* force, acc_t* torque) {
+    const double* m = lab + (size_t)s * kMP;
+    const double* ph = phi + (size_t)s * 35;
+    const R* pd = phidp + (size_t)s * 35;
+    const double u[3] = {mu[3 * (size_t)s], mu[3 * (size_t)s + 1], mu[3 * (size_t)s + 2]};
+    const bool an = aniso[s] != 0;
+    // fractional multipoles
+    double mf[20];
+    frac_moments<double>(m, A, mf);
+    // fixed: energy 1/2 eps M.phi, force -eps grad, torque
+    double ef = 0, f[3] = {0, 0, 0}, fi[3] = {0, 0, 0};
+    for (int k = 0; k < 20; k++) {
+        int e[3];
+        comp_exp(k, e);
+        ef += mf[k] * (double)ph[phi_idx(e[0], e[1], e[2])];
+        for (int a = 0; a < 3; a++) {
+            int e2[3] = {e[0], e[1], e[2]};
+            e2[a]++;
+            const int id = phi_idx(e2[0], e2[1], e2[2]);
+            f[a] += mf[k] * (double)ph[id];
+            fi[a] += 2.0 * mf[k] * (double)pd[id];
         }
-        // induced: energy 1/4 eps 2 u'.grad phi, force
-        const D3 ufv = frac_vector(mk(u[0], u[1], u[2]), A);
-        const double uf[3] = {ufv.x, ufv.y, ufv.z};
-        double ei = 0;
-        for (int k = 0; k < 3; k++) {
-            int e[3] = {0, 0, 0};
-            e[k]++;
-            ei += 2.0 * uf[k] * (double)ph[phi_idx(e[0], e[1], e[2])];
-            for (int a = 0; a < 3; a++) {
-                int e2[3] = {0, 0, 0};
-                e2[k]++;
-                e2[a]++;
-                const int id = phi_idx(e2[0], e2[1], e2[2]);
-                fi[a] += 2.0 * uf[k] * (double)ph[id];
-                if (mutual) fi[a] += 2.0 * uf[k] * (double)pd[id];
-            }
-        }
-        const D3 Fc = cart_vector(mk(kElectric * f[0] + 0.5 * kElectric * fi[0], kElectric * f[1] + 0.5 * kElectric * fi[1],
-                                     kElectric * f[2] + 0.5 * kElectric * fi[2]),
-                                  A);
-        const double F[3] = {-Fc.x, -Fc.y, -Fc.z};
-        // torques
-        double c1[3], c2[6], c3[10];
-        double dd[3] = {m[1], m[2], m[3]};
-        if (an) {
-            dd[0] += u[0];
-            dd[1] += u[1];
-            dd[2] += u[2];
-        }
-        cart_potential<double>(ph, A, c1, c2, c3);
-        D3 T = multipole_torque(dd, m + 4, m + 10, c1, c2, c3) * kElectric;
-        double di[3] = {m[1], m[2], m[3]};
-        if (mutual && an) {
-            di[0] += u[0];
-            di[1] += u[1];
-            di[2] += u[2];
-        }
-        cart_potential<R>(pd, A, c1, c2, c3);
-        T = T + multipole_torque(di, m + 4, m + 10, c1, c2, c3) * kElectric;
-        // self energy and torque
-        const double sqp = 1.7320508075688772;
-        const double sq[5] = {3.0 * m[9], 2.0 * sqp * m[6], 2.0 * sqp * m[8], sqp * (m[4] - m[7]), 2.0 * sqp * m[5]};
-        const double r32 = 1.2247448713915890, r35 = 0.7745966692414834, r110 = 0.31622776601683794;
-        const double so[7] = {15.0 * m[19], 15.0 * r32 * m[15], 15.0 * r32 * m[18], 15.0 * r35 * (m[12] - m[17]),
-                              30.0 * r35 * m[14], 15.0 * r110 * (m[10] - 3.0 * m[13]),
-                              15.0 * r110 * (3.0 * m[11] - m[16])};
-        double qq = 0, oo = 0;
-        for (int k = 0; k < 5; k++) qq += sq[k] * sq[k];
-        for (int k = 0; k < 7; k++) oo += so[k] * so[k];
-        const double a2 = alpha * alpha;
-        const double dud = m[1] * (m[1] + u[0]) + m[2] * (m[2] + u[1]) + m[3] * (m[3] + u[2]);
-        const double eself = -alpha * kElectric / kSqrtPi *
-                             (m[0] * m[0] + (2.0 / 3.0) * a2 * dud + (4.0 / 15.0) * a2 * a2 * qq +
-                              (8.0 / 105.0) * a2 * a2 * a2 * oo);
-        if (!an) {
-            const double term = (2.0 / 3.0) * kElectric * alpha * a2 / kSqrtPi;
-            T = T + cross(mk(m[1], m[2], m[3]), mk(2.0 * u[0], 2.0 * u[1], 2.0 * u[2])) * term;
-        }
-        en = 0.5 * kElectric * ef + 0.25 * kElectric * ei + eself;
-        acc_add(&force[3 * (size_t)s + 0], F[0]);
-        acc_add(&force[3 * (size_t)s + 1], F[1]);
-        acc_add(&force[3 * (size_t)s + 2], F[2]);
-        acc_add(&torque[3 * (size_t)s + 0], T.x);
-        acc_add(&torque[3 * (size_t)s + 1], T.y);
-        acc_add(&torque[3 * (size_t)s + 2], T.z);
     }
-    sh[threadIdx.x] = en;
-    __syncthreads();
-    for (int off = 64; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-        __syncthreads();
+    // induced: energy 1/4 eps 2 u'.grad phi, force
+    const D3 ufv = frac_vector(mk(u[0], u[1], u[2]), A);
+    const double uf[3] = {ufv.x, ufv.y, ufv.z};
+    double ei = 0;
+    for (int k = 0; k < 3; k++) {
+        int e[3] = {0, 0, 0};
+        e[k]++;
+        ei += 2.0 * uf[k] * (double)ph[phi_idx(e[0], e[1], e[2])];
+        for (int a = 0; a < 3; a++) {
+            int e2[3] = {0, 0, 0};
+            e2[k]++;
+            e2[a]++;
+            const int id = phi_idx(e2[0], e2[1], e2[2]);
+            fi[a] += 2.0 * uf[k] * (double)ph[id];
+            if (mutual) fi[a] += 2.0 * uf[k] * (double)pd[id];
+        }
     }
-    if (threadIdx.x == 0) acc_add(energy + (blockIdx.x & (kEnergySlots - 1)), sh[0]);
+    const D3 Fc = cart_vector(mk(kElectric * f[0] + 0.5 * kElectric * fi[0], kElectric * f[1] + 0.5 * kElectric * fi[1],
+                                 kElectric * f[2] + 0.5 * kElectric * fi[2]),
+                              A);
+    const double F[3] = {-Fc.x, -Fc.y, -Fc.z};
+    // torques
+    double c1[3], c2[6], c3[10];
+    double dd[3] = {m[1], m[2], m[3]};
+    if (an) {
+        dd[0] += u[0];
+        dd[1] += u[1];
+        dd[2] += u[2];
+    }
+    cart_potential<double>(ph, A, c1, c2, c3);
+    D3 T = multipole_torque(dd, m + 4, m + 10, c1, c2, c3) * kElectric;
+    double di[3] = {m[1], m[2], m[3]};
+    if (mutual && an) {
+        di[0] += u[0];
+        di[1] += u[1];
+        di[2] += u[2];
+    }
+    cart_potential<R>(pd, A, c1, c2, c3);
+    T = T + multipole_torque(di, m + 4, m + 10, c1, c2, c3) * kElectric;
+    // self energy and torque
+    const double sqp = 1.7320508075688772;
+    const double sq[5] = {3.0 * m[9], 2.0 * sqp * m[6], 2.0 * sqp * m[8], sqp * (m[4] - m[7]), 2.0 * sqp * m[5]};
+    const double r32 = 1.2247448713915890, r35 = 0.7745966692414834, r110 = 0.31622776601683794;
+    const double so[7] = {15.0 * m[19], 15.0 * r32 * m[15], 15.0 * r32 * m[18], 15.0 * r35 * (m[12] - m[17]),
+                          30.0 * r35 * m[14], 15.0 * r110 * (m[10] - 3.0 * m[13]),
+                          15.0 * r110 * (3.0 * m[11] - m[16])};
+    double qq = 0, oo = 0;
+    for (int k = 0; k < 5; k++) qq += sq[k] * sq[k];
+    for (int k = 0; k < 7; k++) oo += so[k] * so[k];
+    const double a2 = alpha * alpha;
+    const double dud = m[1] * (m[1] + u[0]) + m[2] * (m[2] + u[1]) + m[3] * (m[3] + u[2]);
+    const double eself = -alpha * kElectric / kSqrtPi *
+                         (m[0] * m[0] + (2.0 / 3.0) * a2 * dud + (4.0 / 15.0) * a2 * a2 * qq +
+                          (8.0 / 105.0) * a2 * a2 * a2 * oo);
+    if (!an) {
+        const double term = (2.0 / 3.0) * kElectric * alpha * a2 / kSqrtPi;
+        T = T + cross(mk(m[1], m[2], m[3]), mk(2.0 * u[0], 2.0 * u[1], 2.0 * u[2])) * term;
+    }
+    acc_add(&force[3 * (size_t)s + 0], F[0]);
+    acc_add(&force[3 * (size_t)s + 1], F[1]);
+    acc_add(&force[3 * (size_t)s + 2], F[2]);
+    acc_add(&torque[3 * (size_t)s + 0], T.x);
+    acc_add(&torque[3 * (size_t)s + 1], T.y);
+    acc_add(&torque[3 * (size_t)s + 2], T.z);
+    return 0.5 * kElectric * ef + 0.25 * kElectric * ei + eself;
+}
+
+// The per-atom terms of the final pass, one dispatch: workgroups [0, nb) take
+// the reciprocal and self terms of 64 atoms each (their energy to the second
+// kEnergySlots words), workgroups [nb, 2 nb) the covalent pairs (to the first).
+template <class R, bool COV>
+__global__ __launch_bounds__(kTile) void k_final_atoms(int n, int nb, int mutual, const double* __restrict__ phi,
+                                                       const R* __restrict__ phidp, const double* __restrict__ mu,
+                                                       FracT<double> A, double alpha, PairAtoms<double> C,
+                                                       PairParams<double> P, acc_t* force, acc_t* torque,
+                                                       acc_t* energy) {
+    const bool cov = COV && (int)blockIdx.x >= nb;
+    const int block = cov ? blockIdx.x - nb : blockIdx.x;
+    const int s = block * kTile + threadIdx.x;
+    double en = 0.0;
+    if (s < n)
+        en = cov ? cov_electrostatics<double, false>(s, C, mu, P, force, torque, nullptr)
+                 : recip_atom<R>(s, mutual, phi, phidp, C.lab, mu, C.aniso, A, alpha, force, torque);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) en += __shfl_xor(en, off);
+    if (threadIdx.x == 0 && en != 0.0)
+        acc_add(energy + (cov ? 0 : kEnergySlots) + (block & (kEnergySlots - 1)), en);
 }
 
 // ---------------------------------------------------------------------------
@@ -964,7 +983,7 @@ __global__ void k_total_field(int n, int mutual, const double* __restrict__ E0, 
 // Per-atom gradients of the energy with respect to the force's parameters,
 // written in the caller's atom order (perm: sorted -> caller):
 //  gmol[20]  dE/dm of the molecular-frame record (internal order), the lab
-//            potential vector pot taken back through the rotation of k_rotate
+//            potential vector pot taken back through the rotation of k_sorted_atoms
 //            and the chirality flip (a transpose: lab = L m);
 //  gpol[3]   dE/dalpha_k of the molecular-frame polarisabilities: at fixed
 //            induced dipoles the energy holds 1/2 mu alpha_lab^-1 mu, whose
@@ -1001,7 +1020,7 @@ __global__ __launch_bounds__(128) void k_param_gradients(int n, int all_sites, c
             E[k][1] = e[k].y;
             E[k][2] = e[k].z;
         }
-        // transpose of the rotation in k_rotate
+        // transpose of the rotation in k_sorted_atoms
         double g[kMP];
         g[0] = v[0];
         for (int k = 0; k < 3; k++) {
@@ -1026,7 +1045,7 @@ __global__ __launch_bounds__(128) void k_param_gradients(int n, int all_sites, c
                             for (int r = q; r < 3; r++) t += E[k][p] * E[l][q] * E[w][r] * v[10 + i3(p, q, r)];
                     g[10 + i3(k, l, w)] += t;
                 }
-        // chirality (ZThenX with a y atom): k_rotate flips these components
+        // chirality (ZThenX with a y atom): k_sorted_atoms flips these components
         if (ax.w == 0 && ax.z >= 0) {
             const D3 py = d3(pos[ax.z]);
             D3 ad = min_image(d3(pos[s]) - py, box), bd = min_image(d3(pos[ax.x]) - py, box),
@@ -1190,10 +1209,30 @@ __global__ __launch_bounds__(128) void k_torque_to_force(int n, Box<double> box,
     acc_add(&force[3 * (size_t)s + 2], fI.z);
 }
 
-__global__ void k_output_forces(int n, const int* __restrict__ perm, const acc_t* __restrict__ force, double* out,
-                                int accumulate) {
+// Forces to the caller's order (out null: none), and the energies' slots
+// summed by the first wavefront into esum[0..1] (mapped host memory; integer
+// sums, so any order gives the same bits).
+__global__ __launch_bounds__(256) void k_output_forces(int n, const int* __restrict__ perm,
+                                                       const acc_t* __restrict__ force, double* out, int accumulate,
+                                                       const acc_t* __restrict__ energy, acc_t* esum) {
+    if (blockIdx.x == 0 && threadIdx.x < kTile) {
+        acc_t e0 = 0, e1 = 0;
+        for (int k = threadIdx.x; k < kEnergySlots; k += kTile) {
+            e0 += energy[k];
+            e1 += energy[kEnergySlots + k];
+        }
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) {
+            e0 += __shfl_xor(e0, off);
+            e1 += __shfl_xor(e1, off);
+        }
+        if (threadIdx.x == 0) {
+            esum[0] = e0;
+            esum[1] = e1;
+        }
+    }
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
+    if (s >= n || !out) return;
     const int a = perm[s];
     for (int k = 0; k < 3; k++) {
         const double v = acc_get(force[3 * (size_t)s + k]);
@@ -1285,8 +1324,10 @@ void launch_torque_to_force(hipStream_t s, int n, Box<double> box, const double4
     hipLaunchKernelGGL(k_torque_to_force, blocks_for(n, 128), dim3(128), 0, s, n, box, pos, axes, torque, force,
                        exact_threefold);
 }
-void launch_output_forces(hipStream_t s, int n, const int* perm, const acc_t* force, double* out, int accumulate) {
-    hipLaunchKernelGGL(k_output_forces, blocks_for(n, 256), dim3(256), 0, s, n, perm, force, out, accumulate);
+void launch_output_forces(hipStream_t s, int n, const int* perm, const acc_t* force, double* out, int accumulate,
+                          const acc_t* energy, acc_t* esum) {
+    hipLaunchKernelGGL(k_output_forces, out ? blocks_for(n, 256) : dim3(1), dim3(256), 0, s, n, perm, force, out,
+                       accumulate, energy, esum);
 }
 void launch_unpermute3(hipStream_t s, int n, const int* perm, const double* in, double* out) {
     hipLaunchKernelGGL(k_unpermute3, blocks_for(n, 256), dim3(256), 0, s, n, perm, in, out);
@@ -1381,11 +1422,16 @@ void launch_sub(hipStream_t s, int m, const double* a, const double* b_, double*
     hipLaunchKernelGGL(k_sub, dim3(b), dim3(256), 0, s, m, a, b_, out);
 }
 template <class R>
-void launch_recip_atoms(hipStream_t s, int n, int mutual, const double* phi, const R* phidp, const double* lab,
-                        const double* mu, const int* aniso, FracT<double> A, double alpha, acc_t* force,
-                        acc_t* torque, acc_t* energy) {
-    hipLaunchKernelGGL(k_recip_atoms<R>, blocks_for(n, 128), dim3(128), 0, s, n, mutual, phi, phidp, lab, mu, aniso,
-                       A, alpha, force, torque, energy);
+void launch_final_atoms(hipStream_t s, int n, int mutual, const double* phi, const R* phidp, const double* mu,
+                        FracT<double> A, double alpha, PairAtoms<double> c, PairParams<double> p, bool cov,
+                        acc_t* force, acc_t* torque, acc_t* energy) {
+    const int nb = (n + kTile - 1) / kTile;
+    if (cov)
+        hipLaunchKernelGGL((k_final_atoms<R, true>), dim3(2 * nb), dim3(kTile), 0, s, n, nb, mutual, phi, phidp, mu, A,
+                           alpha, c, p, force, torque, energy);
+    else
+        hipLaunchKernelGGL((k_final_atoms<R, false>), dim3(nb), dim3(kTile), 0, s, n, nb, mutual, phi, phidp, mu, A,
+                           alpha, c, p, force, torque, energy);
 }
 
 #define MPID_INSTANTIATE(R)                                                                                         \
@@ -1396,8 +1442,9 @@ void launch_recip_atoms(hipStream_t s, int n, int mutual, const double* phi, con
     template void launch_extrap_order<R>(hipStream_t, int, const acc_t*, const acc_t*, const R*, FracT<double>, double,   \
                                          const double*, const double*, double*, double*, double*, R*);              \
     template void launch_extrap_combine<R>(hipStream_t, int, const ExtrapCoefficients&, const double*, double*, R*); \
-    template void launch_recip_atoms<R>(hipStream_t, int, int, const double*, const R*, const double*, const double*,\
-                                        const int*, FracT<double>, double, acc_t*, acc_t*, acc_t*);                      \
+    template void launch_final_atoms<R>(hipStream_t, int, int, const double*, const R*, const double*,              \
+                                        FracT<double>, double, PairAtoms<double>, PairParams<double>, bool, acc_t*, \
+                                        acc_t*, acc_t*);                                                           \
     template void launch_field_sum<R>(hipStream_t, int, const acc_t*, const R*, const R*, double, double*);                    \
     template void launch_recip_potential<R>(hipStream_t, int, int, const double*, const R*, const double*,            \
                                             const double*, FracT<double>, double, acc_t*);                                 \

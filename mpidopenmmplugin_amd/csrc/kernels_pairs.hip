@@ -503,69 +503,15 @@ __global__ __launch_bounds__(256) void k_cov_induced_field(PairAtoms<R> A, const
     }
 }
 
-// kPot: also the pairs' potential vectors (dE/dm, 20 per atom) into pot.
-template <class R, bool kPot>
-__global__ __launch_bounds__(128) void k_cov_electrostatics(PairAtoms<R> A, const R* __restrict__ mu, PairParams<R> P,
-                                                            acc_t* __restrict__ force, acc_t* __restrict__ torque,
-                                                            acc_t* __restrict__ energy, acc_t* __restrict__ pot) {
+// Covalent electrostatics with the potential vectors (the energy gradients;
+// an evaluation's are in the per-atom kernel of its final pass).
+template <class R>
+__global__ __launch_bounds__(128) void k_cov_electrostatics_pot(PairAtoms<R> A, const R* __restrict__ mu,
+                                                                PairParams<R> P, acc_t* __restrict__ force,
+                                                                acc_t* __restrict__ torque,
+                                                                acc_t* __restrict__ energy, acc_t* __restrict__ pot) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double en = 0.0;
-    if (i < P.n && A.npart[i] > 0) {
-        const int np = A.npart[i];
-        const R4<R> pi = A.pos[i];
-        const R* mi = A.lab + (size_t)i * kMP;
-        const V3<R> ui = mk(mu[3 * (size_t)i], mu[3 * (size_t)i + 1], mu[3 * (size_t)i + 2]);
-        const R2<R> tdi = A.td[i];
-        const bool ani = A.aniso[i] != 0;
-        R fx = 0, fy = 0, fz = 0, tx = 0, ty = 0, tz = 0;
-        R pi_[kPot ? kMP : 1] = {};
-        bool any = false;
-        for (int k = 0; k < np; k++) {
-            const int e = A.partners[(size_t)i * A.pstride + k];
-            const int j = e >> 2;
-            if (j <= i) continue;
-            const R4<R> pj = A.pos[j];
-            const V3<R> dr = min_image(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), P.box);
-            const R r2 = dot(dr, dr);
-            if (r2 > P.rc2) continue;
-            const R sc = partner_scale<R>(e, P.scale14);
-            R pj_[kPot ? kMP : 1] = {};
-            const ElecOut<R> o =
-                elec_pair<R, kPot>(dr, r2, mi, A.lab + (size_t)j * kMP, ui,
-                                   mk(mu[3 * (size_t)j], mu[3 * (size_t)j + 1], mu[3 * (size_t)j + 2]), tdi, A.td[j],
-                                   ani, A.aniso[j] != 0, sc, sc, P, true, pi_, pj_);
-            if constexpr (kPot) {
-#pragma unroll
-                for (int c = 0; c < kMP; c++) acc_add(&pot[kMP * (size_t)j + c], pj_[c]);
-            }
-            any = true;
-            en += (double)o.energy;
-            fx -= o.f.x;
-            fy -= o.f.y;
-            fz -= o.f.z;
-            tx += o.ti.x;
-            ty += o.ti.y;
-            tz += o.ti.z;
-            acc_add(&force[3 * (size_t)j + 0], o.f.x);
-            acc_add(&force[3 * (size_t)j + 1], o.f.y);
-            acc_add(&force[3 * (size_t)j + 2], o.f.z);
-            acc_add(&torque[3 * (size_t)j + 0], o.tj.x);
-            acc_add(&torque[3 * (size_t)j + 1], o.tj.y);
-            acc_add(&torque[3 * (size_t)j + 2], o.tj.z);
-        }
-        if (any) {
-            acc_add(&force[3 * (size_t)i + 0], fx);
-            acc_add(&force[3 * (size_t)i + 1], fy);
-            acc_add(&force[3 * (size_t)i + 2], fz);
-            acc_add(&torque[3 * (size_t)i + 0], tx);
-            acc_add(&torque[3 * (size_t)i + 1], ty);
-            acc_add(&torque[3 * (size_t)i + 2], tz);
-            if constexpr (kPot) {
-#pragma unroll
-                for (int c = 0; c < kMP; c++) acc_add(&pot[kMP * (size_t)i + c], pi_[c]);
-            }
-        }
-    }
+    double en = i < P.n ? cov_electrostatics<R, true>(i, A, mu, P, force, torque, pot) : 0.0;
     // every lane reaches the reduction
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) en += __shfl_xor(en, off);
@@ -600,14 +546,10 @@ void launch_cov_induced_field(hipStream_t s, int n, PairAtoms<R> a, const R* mu,
                            pol_only, field, nullptr);
 }
 template <class R>
-void launch_cov_electrostatics(hipStream_t s, int n, PairAtoms<R> a, const R* mu, PairParams<R> p, acc_t* force,
-                               acc_t* torque, acc_t* energy, acc_t* pot) {
-    if (pot)
-        hipLaunchKernelGGL((k_cov_electrostatics<R, true>), dim3((n + 127) / 128), dim3(128), 0, s, a, mu, p, force,
-                           torque, energy, pot);
-    else
-        hipLaunchKernelGGL((k_cov_electrostatics<R, false>), dim3((n + 127) / 128), dim3(128), 0, s, a, mu, p, force,
-                           torque, energy, nullptr);
+void launch_cov_electrostatics_pot(hipStream_t s, int n, PairAtoms<R> a, const R* mu, PairParams<R> p, acc_t* force,
+                                   acc_t* torque, acc_t* energy, acc_t* pot) {
+    hipLaunchKernelGGL(k_cov_electrostatics_pot<R>, dim3((n + 127) / 128), dim3(128), 0, s, a, mu, p, force, torque,
+                       energy, pot);
 }
 
 // ---------------------------------------------------------------------------
@@ -685,8 +627,8 @@ void launch_electrostatics_pot(hipStream_t s, int maxtiles, const int4* act, con
     template void launch_cov_fixed_field<R>(hipStream_t, int, PairAtoms<R>, PairParams<R>, acc_t*);                \
     template void launch_cov_induced_field<R>(hipStream_t, int, PairAtoms<R>, const R*, PairParams<R>, int,        \
                                               acc_t*, acc_t*);                                                    \
-    template void launch_cov_electrostatics<R>(hipStream_t, int, PairAtoms<R>, const R*, PairParams<R>, acc_t*,    \
-                                               acc_t*, acc_t*, acc_t*);                                             \
+    template void launch_cov_electrostatics_pot<R>(hipStream_t, int, PairAtoms<R>, const R*, PairParams<R>,        \
+                                                   acc_t*, acc_t*, acc_t*, acc_t*);                                 \
     template void launch_cov_thole<R>(hipStream_t, int, PairAtoms<R>, const R*, PairParams<R>, acc_t*, acc_t*,      \
                                       acc_t*);                                                                      \
     template void launch_electrostatics_pot<R>(hipStream_t, int, const int4*, const int*, const int*, const int*,   \

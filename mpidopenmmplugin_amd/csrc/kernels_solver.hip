@@ -618,6 +618,18 @@ __global__ __launch_bounds__(256) void k_apply_S(SolverSites st, const double* _
     if (at) store3(at, t, m);
 }
 
+template <class R>
+__global__ __launch_bounds__(256) void k_final_start(SolverSites st, const double* __restrict__ v, R* mu, double* mud,
+                                                     acc_t* __restrict__ acc, size_t count) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    for (size_t k = t; k < count; k += (size_t)gridDim.x * 256) acc[k] = 0;
+    if (!v || t >= st.npol) return;
+    const int i = st.idx[t];
+    const D3 m = sym_mul6(st.S + 6 * (size_t)i, load3(v, t));
+    store_mu<R>(mu, i, m);
+    store3(mud, i, m);
+}
+
 // rt = b - A x (given Ax; null: rt is read), |S rt|^2 and x.rt: partial sums
 // per workgroup, then one workgroup writes out[0], out[1] (mapped host memory)
 __global__ __launch_bounds__(256) void k_residual(SolverSites st, const double* __restrict__ b,
@@ -734,6 +746,12 @@ void launch_apply_S(hipStream_t s, SolverSites st, const double* v, R* mu, doubl
     if (st.npol <= 0) return;
     hipLaunchKernelGGL(k_apply_S<R>, dim3((st.npol + 255) / 256), dim3(256), 0, s, st, v, mu, mud, at);
 }
+template <class R>
+void launch_final_start(hipStream_t s, SolverSites st, const double* v, R* mu, double* mud, acc_t* acc, size_t count) {
+    const size_t blocks = std::max<size_t>((st.npol + 255) / 256, std::min<size_t>((count + 255) / 256, 2048));
+    hipLaunchKernelGGL(k_final_start<R>, dim3((unsigned)std::max<size_t>(blocks, 1)), dim3(256), 0, s, st, v, mu, mud,
+                       acc, count);
+}
 void launch_residual(hipStream_t s, SolverSites st, const double* b, const double* Ax, const double* x, double* rt,
                      double* partial, double* out) {
     const int blocks = site_blocks(st.npol);
@@ -757,6 +775,7 @@ void launch_residual(hipStream_t s, SolverSites st, const double* b, const doubl
                                         PairAtoms<double>, PairParams<double>, const double*, const double*,        \
                                         FracT<double>, double, double*, double*, double*, R*, double*, const int*,  \
                                         int*);                                                                     \
+    template void launch_final_start<R>(hipStream_t, SolverSites, const double*, R*, double*, acc_t*, size_t);      \
     template void launch_apply_S<R>(hipStream_t, SolverSites, const double*, R*, double*, double*);
 MPID_INSTANTIATE(float)
 MPID_INSTANTIATE(double)

@@ -240,6 +240,9 @@ struct mpid_context {
     double* hscal = nullptr;  // [1] |S r|^2 of the last residual, [2] its product with x,
                               // [kCheck ..] the solver's two check slots (|S r|^2, stop)
     static constexpr int kCheck = 8;
+    // the energies' two sums (fixed point), in words 4 and 5
+    const acc_t* esum() const { return reinterpret_cast<const acc_t*>(hscal + 4); }
+    acc_t* esum_dev() const { return reinterpret_cast<acc_t*>(hscal_dev + 4); }
     hipEvent_t ev_check[2] = {nullptr, nullptr};  // recorded after the work that publishes check c (c & 1)
     hipEvent_t ev_sync = nullptr;
     std::string error;
@@ -295,7 +298,11 @@ struct mpid_context {
     int* hnl = nullptr;  // pinned, mapped: [0] largest list length, [1] mirror flag, [2] block-row count
     int* hnl_dev = nullptr;  // its device address
     // accumulators
-    DBuf<acc_t> field_acc, force_acc, torque_acc, energy_acc;
+    DBuf<acc_t> field_acc;
+    DBuf<acc_t> final_acc;  // the final pass's: force [3n], torque [3n], energy [2 kEnergySlots]
+    acc_t* force_acc() const { return final_acc.p; }
+    acc_t* torque_acc() const { return final_acc.p + 3 * (size_t)n; }
+    acc_t* energy_acc() const { return final_acc.p + 6 * (size_t)n; }
     // Extrapolated polarization: coefficient partial sums, the order dipoles
     // mu_(m) [N][3n], the fields E_(m) and gradients G_(m) of mu_(0..N-2)
     // ([N-1][3n], [N-1][6n]) and the real-space gradient accumulator
@@ -678,9 +685,7 @@ struct mpid_context {
         pol_idx.resize(n);
         nl_scalars.resize(4);
         field_acc.resize(n3);
-        force_acc.resize(n3);
-        torque_acc.resize(n3);
-        energy_acc.resize(2 * kEnergySlots);
+        final_acc.resize(2 * n3 + 2 * kEnergySlots);
         E0.resize(n3);
         b.resize(n3);
         x.resize(n3);
@@ -1569,15 +1574,12 @@ struct mpid_context {
         join();  // a previous final pass's reciprocal kernels have added into the accumulators
         // induced dipoles: mu = S x (double for the per-atom terms, R for the
         // kernels), unless they are in place already (Extrapolated)
-        if (!mu_set) timed(P_SOLVER, [&] { launch_apply_S<R>(stream, sites(), x.p, P.mu.p, mud.p, nullptr); });
-        timed(P_OTHER, [&] {
-            launch_zero_acc(stream, force_acc.p, force_acc.n);
-            launch_zero_acc(stream, torque_acc.p, torque_acc.n);
-            launch_zero_acc(stream, energy_acc.p, 2 * kEnergySlots);
+        timed(P_SOLVER, [&] {
+            launch_final_start<R>(stream, sites(), mu_set ? nullptr : x.p, P.mu.p, mud.p, final_acc.p, final_acc.n);
         });
         if (opt.polarization == MPID_POLARIZATION_EXTRAPOLATED)
             timed(P_SOLVER, [&] {
-                launch_extrap_response(stream, n, ext_cp, ptmu.p, ptE.p, ptG.p, aniso.p, force_acc.p, torque_acc.p);
+                launch_extrap_response(stream, n, ext_cp, ptmu.p, ptE.p, ptG.p, aniso.p, force_acc(), torque_acc());
             });
         // Order of issue: the reciprocal chain first (short kernels with large
         // LDS blocks, which would wait for whole CUs behind the
@@ -1590,16 +1592,12 @@ struct mpid_context {
                                            brows.p, brow_owner.p,
                                            tmask.p, tmaskcc.p, chg.p,
                                            pair_atoms(P), P.mu.p, pair_params<R>(), pd.pos.p, lab.p,
-                                           pair_params<double>(), force_acc.p, torque_acc.p, energy_acc.p);
+                                           pair_params<double>(), force_acc(), torque_acc(), energy_acc());
         });
         timed_on(rstream, P_RECIP, [&] {
-            launch_recip_atoms<R>(rstream, n, opt.polarization == MPID_POLARIZATION_MUTUAL ? 1 : 0, pd.phi.p,
-                                  P.phidp.p, lab.p, mud.p, aniso.p, frac_transform<double>(), opt.ewald_alpha, force_acc.p,
-                                  torque_acc.p, energy_acc.p + kEnergySlots);
-        });
-        timed_on(rstream, P_COV, [&] {
-            launch_cov_electrostatics<double>(rstream, n, pair_atoms(pd), mud.p, pair_params<double>(), force_acc.p,
-                                              torque_acc.p, energy_acc.p);
+            launch_final_atoms<R>(rstream, n, opt.polarization == MPID_POLARIZATION_MUTUAL ? 1 : 0, pd.phi.p,
+                                  P.phidp.p, mud.p, frac_transform<double>(), opt.ewald_alpha, pair_atoms(pd),
+                                  pair_params<double>(), true, force_acc(), torque_acc(), energy_acc());
         });
         check_launch();
         final_issued = true;
@@ -1611,19 +1609,13 @@ struct mpid_context {
         mu_valid = true;
         join();
         timed(P_OTHER, [&] {
-            launch_torque_to_force(stream, n, dbox, spos.p, saxes.p, torque_acc.p, force_acc.p,
+            launch_torque_to_force(stream, n, dbox, spos.p, saxes.p, torque_acc(), force_acc(),
                                    (opt.flags & MPID_FLAG_CONSERVATIVE_TORQUES) ? 1 : 0);
-            if (d_forces_out) launch_output_forces(stream, n, perm.p, force_acc.p, d_forces_out, 1);
+            launch_output_forces(stream, n, perm.p, force_acc(), d_forces_out, 1, energy_acc(), esum_dev());
         });
         check_launch();
-        acc_t e[2] = {0, 0};
-        acc_t slots[2 * kEnergySlots];
-        HIP_CHECK(hipMemcpyAsync(slots, energy_acc.p, sizeof(slots), hipMemcpyDeviceToHost, stream));
         HIP_CHECK(hipStreamSynchronize(stream));
-        for (int k = 0; k < kEnergySlots; k++) {  // integer sums: any order gives the same bits
-            e[0] += slots[k];
-            e[1] += slots[kEnergySlots + k];
-        }
+        const acc_t* e = esum();
         if (correction_pending) {
             energy_correction = -0.5 * kElectric * hscal[2];
             correction_pending = false;
@@ -1736,11 +1728,9 @@ struct mpid_context {
             }
         }
         // final pass at the refined dipoles, with the potential vectors
-        timed(P_SOLVER, [&] { launch_apply_S<R>(stream, sites(), x.p, P.mu.p, mud.p, nullptr); });
+        timed(P_SOLVER,
+              [&] { launch_final_start<R>(stream, sites(), x.p, P.mu.p, mud.p, final_acc.p, final_acc.n); });
         timed(P_OTHER, [&] {
-            launch_zero_acc(stream, force_acc.p, force_acc.n);
-            launch_zero_acc(stream, torque_acc.p, torque_acc.n);
-            launch_zero_acc(stream, energy_acc.p, 2 * kEnergySlots);
             launch_zero_acc(stream, pot_acc.p, pot_acc.n);
             launch_zero_acc(stream, hd_acc.p, hd_acc.n);
             launch_zero_acc(stream, hdef_acc.p, hdef_acc.n);
@@ -1753,18 +1743,19 @@ struct mpid_context {
                                            brows.p, brow_owner.p,
                                          tmask.p, tmaskcc.p, chg.p,
                                          pair_atoms(P), P.mu.p, pair_params<R>(), pd.pos.p, lab.p,
-                                         pair_params<double>(), force_acc.p, torque_acc.p, energy_acc.p, pot_acc.p,
+                                         pair_params<double>(), force_acc(), torque_acc(), energy_acc(), pot_acc.p,
                                          all_sites ? 1 : 0);
         });
         timed_on(rstream, P_RECIP, [&] {
-            launch_recip_atoms<R>(rstream, n, mutual ? 1 : 0, pd.phi.p, P.phidp.p, lab.p, mud.p, aniso.p, frac_transform<double>(),
-                                  opt.ewald_alpha, force_acc.p, torque_acc.p, energy_acc.p + kEnergySlots);
+            launch_final_atoms<R>(rstream, n, mutual ? 1 : 0, pd.phi.p, P.phidp.p, mud.p, frac_transform<double>(),
+                                  opt.ewald_alpha, pair_atoms(pd), pair_params<double>(), false, force_acc(),
+                                  torque_acc(), energy_acc());
             launch_recip_potential<R>(rstream, n, pme() ? 1 : 0, pd.phi.p, P.phidp.p, lab.p, mud.p, frac_transform<double>(),
                                       opt.ewald_alpha, pot_acc.p);
         });
         timed_on(rstream, P_COV, [&] {
-            launch_cov_electrostatics<double>(rstream, n, pair_atoms(pd), mud.p, pair_params<double>(), force_acc.p,
-                                              torque_acc.p, energy_acc.p, pot_acc.p);
+            launch_cov_electrostatics_pot<double>(rstream, n, pair_atoms(pd), mud.p, pair_params<double>(),
+                                                  force_acc(), torque_acc(), energy_acc(), pot_acc.p);
         });
         // Thole damping of the pairs of polarisable sites
         timed(P_INDUCED, [&] {
@@ -1801,9 +1792,9 @@ struct mpid_context {
         timed(P_OTHER, [&] {
             launch_total_field<R>(stream, n, mutual ? 1 : 0, E0.p, field_acc.p, P.phidp.p, frac_transform<double>(), mud.p, selfc(),
                                   Etot.p);
-            launch_torque_to_force(stream, n, dbox, spos.p, saxes.p, torque_acc.p, force_acc.p,
+            launch_torque_to_force(stream, n, dbox, spos.p, saxes.p, torque_acc(), force_acc(),
                                    (opt.flags & MPID_FLAG_CONSERVATIVE_TORQUES) ? 1 : 0);
-            launch_output_forces(stream, n, perm.p, force_acc.p, gforce.p, 0);
+            launch_output_forces(stream, n, perm.p, force_acc(), gforce.p, 0, energy_acc(), esum_dev());
             launch_param_gradients(stream, n, all_sites ? 1 : 0, perm.p, dbox, spos.p, saxes.p, smol.p, spol.p,
                                    damp.p, chg.p, pot_acc.p, Etot.p, hd_acc.p, hdef_acc.p, ht_acc.p,
                                    opt.default_thole, gmol.p, gpol.p, gthole.p, gdef_acc.p);
@@ -1813,9 +1804,7 @@ struct mpid_context {
         out.mol.resize((size_t)kMP * n);
         out.pol.resize(n3);
         out.thole.resize(n);
-        acc_t slots[2 * kEnergySlots];
         acc_t gdef = 0;
-        HIP_CHECK(hipMemcpyAsync(slots, energy_acc.p, sizeof(slots), hipMemcpyDeviceToHost, stream));
         HIP_CHECK(hipMemcpyAsync(&gdef, gdef_acc.p, sizeof(acc_t), hipMemcpyDeviceToHost, stream));
         HIP_CHECK(hipMemcpyAsync(out.force.data(), gforce.p, n3 * sizeof(double), hipMemcpyDeviceToHost, stream));
         HIP_CHECK(hipMemcpyAsync(out.mol.data(), gmol.p, out.mol.size() * sizeof(double), hipMemcpyDeviceToHost,
@@ -1823,11 +1812,7 @@ struct mpid_context {
         HIP_CHECK(hipMemcpyAsync(out.pol.data(), gpol.p, n3 * sizeof(double), hipMemcpyDeviceToHost, stream));
         HIP_CHECK(hipMemcpyAsync(out.thole.data(), gthole.p, n * sizeof(double), hipMemcpyDeviceToHost, stream));
         HIP_CHECK(hipStreamSynchronize(stream));
-        acc_t e[2] = {0, 0};
-        for (int k = 0; k < kEnergySlots; k++) {
-            e[0] += slots[k];
-            e[1] += slots[kEnergySlots + k];
-        }
+        const acc_t* e = esum();
         out.default_thole = acc_get(gdef);
         stats.energy_terms[0] = acc_get(e[0]);
         stats.energy_terms[1] = acc_get(e[1]);

@@ -904,4 +904,69 @@ MPID_HD ElecBareOut<R> elec_pair_bare_cart(V3<R> dr, R r2, const R* ma, R qb, V3
     return o;
 }
 
+// Energy of atom i's covalent pairs with partners j > i; forces, torques and
+// (kPot) potential vectors (dE/dm, 20 per atom) of both sides are added to
+// the accumulators.
+template <class R, bool kPot>
+__device__ __forceinline__ double cov_electrostatics(int i, const PairAtoms<R>& A, const R* __restrict__ mu,
+                                                     const PairParams<R>& P, acc_t* force, acc_t* torque, acc_t* pot) {
+    double en = 0.0;
+    const int np = A.npart[i];
+    if (np == 0) return en;
+    const R4<R> pi = A.pos[i];
+    const R* mi = A.lab + (size_t)i * kMP;
+    const V3<R> ui = mk(mu[3 * (size_t)i], mu[3 * (size_t)i + 1], mu[3 * (size_t)i + 2]);
+    const R2<R> tdi = A.td[i];
+    const bool ani = A.aniso[i] != 0;
+    R fx = 0, fy = 0, fz = 0, tx = 0, ty = 0, tz = 0;
+    R pi_[kPot ? kMP : 1] = {};
+    bool any = false;
+    for (int k = 0; k < np; k++) {
+        const int e = A.partners[(size_t)i * A.pstride + k];
+        const int j = e >> 2;
+        if (j <= i) continue;
+        const R4<R> pj = A.pos[j];
+        const V3<R> dr = min_image(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), P.box);
+        const R r2 = dot(dr, dr);
+        if (r2 > P.rc2) continue;
+        const R sc = partner_scale<R>(e, P.scale14);
+        R pj_[kPot ? kMP : 1] = {};
+        const ElecOut<R> o =
+            elec_pair<R, kPot>(dr, r2, mi, A.lab + (size_t)j * kMP, ui,
+                               mk(mu[3 * (size_t)j], mu[3 * (size_t)j + 1], mu[3 * (size_t)j + 2]), tdi, A.td[j],
+                               ani, A.aniso[j] != 0, sc, sc, P, true, pi_, pj_);
+        if constexpr (kPot) {
+#pragma unroll
+            for (int c = 0; c < kMP; c++) acc_add(&pot[kMP * (size_t)j + c], pj_[c]);
+        }
+        any = true;
+        en += (double)o.energy;
+        fx -= o.f.x;
+        fy -= o.f.y;
+        fz -= o.f.z;
+        tx += o.ti.x;
+        ty += o.ti.y;
+        tz += o.ti.z;
+        acc_add(&force[3 * (size_t)j + 0], o.f.x);
+        acc_add(&force[3 * (size_t)j + 1], o.f.y);
+        acc_add(&force[3 * (size_t)j + 2], o.f.z);
+        acc_add(&torque[3 * (size_t)j + 0], o.tj.x);
+        acc_add(&torque[3 * (size_t)j + 1], o.tj.y);
+        acc_add(&torque[3 * (size_t)j + 2], o.tj.z);
+    }
+    if (any) {
+        acc_add(&force[3 * (size_t)i + 0], fx);
+        acc_add(&force[3 * (size_t)i + 1], fy);
+        acc_add(&force[3 * (size_t)i + 2], fz);
+        acc_add(&torque[3 * (size_t)i + 0], tx);
+        acc_add(&torque[3 * (size_t)i + 1], ty);
+        acc_add(&torque[3 * (size_t)i + 2], tz);
+        if constexpr (kPot) {
+#pragma unroll
+            for (int c = 0; c < kMP; c++) acc_add(&pot[kMP * (size_t)i + c], pi_[c]);
+        }
+    }
+    return en;
+}
+
 }  // namespace mpid
