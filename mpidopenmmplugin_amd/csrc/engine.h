@@ -234,31 +234,26 @@ struct ExtrapCoefficients {
     int n;
     double c[kMaxExtrapolation];
 };
-// One order: E_(m), G_(m) (field with the self term, gradient without it, of
-// mu_(m) at every atom, from the real-space accumulators, the reciprocal
-// potential derivatives phidp and the self term) and mu_(m+1) = alpha_lab E.
-template <class R>
-void launch_extrap_order(hipStream_t s, int n, const acc_t* field, const acc_t* gacc, const R* phidp, FracT<double> A,
-                         double selfc, const double* labpol, const double* mu, double* E, double* G, double* mu_next,
-                         R* mu_next_r);
-// mu = sum_o c'_o mu_(o) (mus: [order][3n])
-template <class R>
-void launch_extrap_combine(hipStream_t s, int n, const ExtrapCoefficients& cp, const double* mus, double* mud,
-                           R* mu_r);
-// the dipole-response forces and torques into the fixed-point accumulators
-void launch_extrap_response(hipStream_t s, int n, const ExtrapCoefficients& cp, const double* mus, const double* Es,
-                            const double* Gs, const int* aniso, acc_t* force, acc_t* torque);
-// mu0 = alpha_lab E0 at every atom, in both precisions (Extrapolated)
-template <class R>
-void launch_extrap_init(hipStream_t s, int n, const double* labpol, const double* E0, double* mu, R* mu_r);
 void launch_axpy(hipStream_t s, int m, double a, const double* x, double* y);
 void launch_sub(hipStream_t s, int m, const double* a, const double* b, double* out);
+// The orders of Extrapolated polarization by polarisable site, for their
+// response forces: mu_(m) [n][3 npol], fields E_(m) [n - 1][3 npol] and
+// gradients G_(m) [n - 1][6 npol].  npol = 0: none.
+struct ExtrapResponse {
+    ExtrapCoefficients cp;
+    int npol;
+    const int* idx;
+    const double* mus;
+    const double* E;
+    const double* G;
+};
 // reciprocal-space energy, forces and torques, self terms (per atom), and
-// (cov) the covalent pairs' electrostatics; energy: 2 kEnergySlots words
+// (cov) the covalent pairs' electrostatics and the response forces; energy:
+// 2 kEnergySlots words
 template <class R>
 void launch_final_atoms(hipStream_t s, int n, int mutual, const double* phi, const R* phidp, const double* mu,
                         FracT<double> A, double alpha, PairAtoms<double> c, PairParams<double> p, bool cov,
-                        acc_t* force, acc_t* torque, acc_t* energy);
+                        const ExtrapResponse& x, acc_t* force, acc_t* torque, acc_t* energy);
 
 // ---- PME (kernels_pme.hip) ----------------------------------------------------
 template <class R> struct PmeGeom {
@@ -406,15 +401,14 @@ void launch_nl_build(hipStream_t s, int n, int nrows, int rcap, bool all, const 
 template <class R>
 void launch_nl_fixed_field(hipStream_t s, int natoms, const int* atoms, NbrList l, PairAtoms<R> a, PairParams<R> p,
                            acc_t* field);
-// grad != nullptr: also the field gradient (xx yy zz xy xz yz per atom)
 template <class R>
 void launch_nl_induced_field(hipStream_t s, int natoms, const int* atoms, NbrList l, PairAtoms<R> a, const R* mu,
-                             PairParams<R> p, acc_t* field, acc_t* grad = nullptr);
+                             PairParams<R> p, acc_t* field);
 // the scaled covalent pairs, which the list and tile kernels leave out
 template <class R> void launch_cov_fixed_field(hipStream_t s, int n, PairAtoms<R> a, PairParams<R> p, acc_t* field);
 template <class R>
 void launch_cov_induced_field(hipStream_t s, int n, PairAtoms<R> a, const R* mu, PairParams<R> p, int pol_only,
-                              acc_t* field, acc_t* grad = nullptr);
+                              acc_t* field);
 // the covalent pairs' electrostatics with their potential vectors dE/dm (20 per atom)
 template <class R>
 void launch_cov_electrostatics_pot(hipStream_t s, int n, PairAtoms<R> a, const R* mu, PairParams<R> p, acc_t* force,
@@ -474,10 +468,30 @@ void launch_solver_init(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a
                         PairAtoms<double> a64, PairParams<double> p64, const double* field, const double* phi,
                         FracT<double> A, double selfc, double* E0, double* b, double* x, R* mu, double* mud,
                         const int* nl_scalars, int* hnl);
-// The final pass's start: mu = mud = S v (v null: they are in place) and the
-// accumulators cleared
+// The final pass's start: the accumulators cleared, and mu = mud = S v; v
+// null: the extrapolated sum of mus (ex.n > 0), or they are in place
 template <class R>
-void launch_final_start(hipStream_t s, SolverSites st, const double* v, R* mu, double* mud, acc_t* acc, size_t count);
+void launch_final_start(hipStream_t s, SolverSites st, const double* v, const ExtrapCoefficients& ex,
+                        const double* mus, R* mu, double* mud, acc_t* acc, size_t count);
+// One order of Extrapolated polarization: its dipoles (by site; null: mud, by
+// atom, which mu0 then takes), field, gradient and the next order's dipoles.
+struct ExtrapOrder {
+    const double* mus_in;
+    double* mu0;
+    double* E;
+    double* G;
+    double* mus_out;
+};
+// real-space field and gradient of mu (9 per site)
+template <class R>
+void launch_extrap_list(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p, const R* mu,
+                        R* field);
+// field null: the real-space part in the same kernel.  mu_next (by atom) must
+// not be mu.
+template <class R>
+void launch_extrap_order(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const R* field, NbrList l,
+                         PairAtoms<R> a, PairParams<R> p, const R* mu, R* mu_next, FracT<double> A, double selfc,
+                         const double* labpol, const ExtrapOrder& o, const double* mud);
 // S v: by atom in mu and mud, by site in at (each may be null)
 template <class R>
 void launch_apply_S(hipStream_t s, SolverSites st, const double* v, R* mu, double* mud, double* at);

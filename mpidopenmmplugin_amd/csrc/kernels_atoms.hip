@@ -412,117 +412,6 @@ __global__ __launch_bounds__(kRedThreads) void k_reduce_partials(const double* _
     }
 }
 
-template <class R>
-__device__ void cart_potential(const R* ph, const FracT<double>& A, double* c1, double* c2, double* c3);
-
-// ---- Extrapolated (OPT) polarization --------------------------------------
-// convergeInduceDipolesByExtrapolation, MPIDReferenceForce.cpp:1125-1180.
-// One order: the field of mu_(m) at every atom, E = real space (acc) +
-// reciprocal (-A phi_1) + selfc mu_(m), and its gradient G = real space
-// (gacc) - A phi_2 A^T (A the grid-coordinate transform; :4094-4127), kept
-// for the response forces; then mu_(m+1) = alpha_lab E, in FP64 and in the
-// precision of the next order's kernels.
-template <class R>
-__global__ void k_extrap_init(int n, const double* __restrict__ labpol, const double* __restrict__ E0, double* mu,
-                              R* mu_r) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const size_t i3 = 3 * (size_t)s;
-    const D3 m = sym_mul(labpol + 6 * (size_t)s, mk(E0[i3], E0[i3 + 1], E0[i3 + 2]));
-    mu[i3] = m.x;
-    mu[i3 + 1] = m.y;
-    mu[i3 + 2] = m.z;
-    mu_r[i3] = (R)m.x;
-    mu_r[i3 + 1] = (R)m.y;
-    mu_r[i3 + 2] = (R)m.z;
-}
-template <class R>
-__global__ void k_extrap_order(int n, const acc_t* __restrict__ field, const acc_t* __restrict__ gacc,
-                               const R* __restrict__ phidp, FracT<double> A, double selfc,
-                               const double* __restrict__ labpol, const double* __restrict__ mu, double* E,
-                               double* G, double* mu_next, R* mu_next_r) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const R* ph = phidp + 35 * (size_t)s;
-    const size_t i3 = 3 * (size_t)s, i6 = 6 * (size_t)s;
-    double c1[3], c2[6], c3[10];
-    cart_potential<R>(ph, A, c1, c2, c3);
-    D3 e;
-    e.x = acc_get(field[i3]) - c1[0] + selfc * mu[i3];
-    e.y = acc_get(field[i3 + 1]) - c1[1] + selfc * mu[i3 + 1];
-    e.z = acc_get(field[i3 + 2]) - c1[2] + selfc * mu[i3 + 2];
-    E[i3] = e.x;
-    E[i3 + 1] = e.y;
-    E[i3 + 2] = e.z;
-    // gradient order xx yy zz xy xz yz; c2 is XX XY XZ YY YZ ZZ
-    G[i6 + 0] = acc_get(gacc[i6 + 0]) - c2[0];
-    G[i6 + 1] = acc_get(gacc[i6 + 1]) - c2[3];
-    G[i6 + 2] = acc_get(gacc[i6 + 2]) - c2[5];
-    G[i6 + 3] = acc_get(gacc[i6 + 3]) - c2[1];
-    G[i6 + 4] = acc_get(gacc[i6 + 4]) - c2[2];
-    G[i6 + 5] = acc_get(gacc[i6 + 5]) - c2[4];
-    const D3 m = sym_mul(labpol + i6, e);
-    mu_next[i3] = m.x;
-    mu_next[i3 + 1] = m.y;
-    mu_next[i3 + 2] = m.z;
-    mu_next_r[i3] = (R)m.x;
-    mu_next_r[i3 + 1] = (R)m.y;
-    mu_next_r[i3 + 2] = (R)m.z;
-}
-
-// mu = sum_o c'_o mu_(o), c'_o = sum_{j >= o} c_j (setExtrapolationCoefficients,
-// MPIDReferenceForce.cpp:173-183; the sum at :1170-1177).
-template <class R>
-__global__ void k_extrap_combine(int n, ExtrapCoefficients cp, const double* __restrict__ mus, double* mud, R* mu_r) {
-    const int id = blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t n3 = 3 * (size_t)n;
-    if (id >= (int)n3) return;
-    double v = 0.0;
-    for (int o = 0; o < cp.n; o++) v += cp.c[o] * mus[o * n3 + id];
-    mud[id] = v;
-    mu_r[id] = (R)v;
-}
-
-// The dipole-response forces and torques, MPIDReferenceForce.cpp:4955-4985:
-// for l + m <= N - 2, c'_(l+m+1) times mu_(l) contracted with the gradient
-// of the field of mu_(m) (force) or crossed with that field (torque on
-// anisotropic sites).  Terms with |c'| < 1e-6 are skipped as there.
-__global__ void k_extrap_response(int n, ExtrapCoefficients cp, const double* __restrict__ mus,
-                                  const double* __restrict__ Es, const double* __restrict__ Gs,
-                                  const int* __restrict__ aniso, acc_t* force, acc_t* torque) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const size_t n3 = 3 * (size_t)n, n6 = 6 * (size_t)n;
-    const bool an = aniso[s] != 0;
-    D3 f = mk(0.0, 0.0, 0.0), t = mk(0.0, 0.0, 0.0);
-    for (int l = 0; l < cp.n - 1; l++) {
-        const double* u = mus + l * n3 + 3 * (size_t)s;
-        for (int m = 0; m < cp.n - 1 - l; m++) {
-            const double p = cp.c[l + m + 1];
-            if (fabs(p) < 1e-6) continue;
-            const double pf = p * kElectric;
-            const double* g = Gs + m * n6 + 6 * (size_t)s;
-            f.x += pf * (u[0] * g[0] + u[1] * g[3] + u[2] * g[4]);
-            f.y += pf * (u[0] * g[3] + u[1] * g[1] + u[2] * g[5]);
-            f.z += pf * (u[0] * g[4] + u[1] * g[5] + u[2] * g[2]);
-            if (an) {
-                const double* e = Es + m * n3 + 3 * (size_t)s;
-                t.x += pf * (u[1] * e[2] - u[2] * e[1]);
-                t.y += pf * (u[2] * e[0] - u[0] * e[2]);
-                t.z += pf * (u[0] * e[1] - u[1] * e[0]);
-            }
-        }
-    }
-    acc_add(&force[3 * (size_t)s + 0], f.x);
-    acc_add(&force[3 * (size_t)s + 1], f.y);
-    acc_add(&force[3 * (size_t)s + 2], f.z);
-    if (an) {
-        acc_add(&torque[3 * (size_t)s + 0], t.x);
-        acc_add(&torque[3 * (size_t)s + 1], t.y);
-        acc_add(&torque[3 * (size_t)s + 2], t.z);
-    }
-}
-
 // ---- getters after an evaluation -----------------------------------------
 // getElectrostaticPotential, MPIDReferenceForce.cpp:2464-2531: at each point,
 // the Coulomb constant times the bare potential of every particle's charge,
@@ -869,15 +758,60 @@ __device__ __forceinline__ double recip_atom(int s, int mutual, const double* __
     return 0.5 * kElectric * ef + 0.25 * kElectric * ei + eself;
 }
 
+// The dipole-response forces and torques of Extrapolated polarization at
+// polarisable site t, MPIDReferenceForce.cpp:4955-4985: for l + m <= N - 2,
+// c'_(l+m+1) times mu_(l) contracted with the gradient of the field of mu_(m)
+// (force) or crossed with that field (torque on anisotropic sites).  Terms
+// with |c'| < 1e-6 are skipped as there.
+__device__ __forceinline__ void extrap_response(const ExtrapResponse& x, int t, const int* __restrict__ aniso,
+                                                acc_t* force, acc_t* torque) {
+    const int s = x.idx[t];
+    const size_t n3 = 3 * (size_t)x.npol, n6 = 6 * (size_t)x.npol;
+    const bool an = aniso[s] != 0;
+    D3 f = mk(0.0, 0.0, 0.0), q = mk(0.0, 0.0, 0.0);
+    for (int l = 0; l < x.cp.n - 1; l++) {
+        const double* u = x.mus + l * n3 + 3 * (size_t)t;
+        for (int m = 0; m < x.cp.n - 1 - l; m++) {
+            const double p = x.cp.c[l + m + 1];
+            if (fabs(p) < 1e-6) continue;
+            const double pf = p * kElectric;
+            const double* g = x.G + m * n6 + 6 * (size_t)t;
+            f.x += pf * (u[0] * g[0] + u[1] * g[3] + u[2] * g[4]);
+            f.y += pf * (u[0] * g[3] + u[1] * g[1] + u[2] * g[5]);
+            f.z += pf * (u[0] * g[4] + u[1] * g[5] + u[2] * g[2]);
+            if (an) {
+                const double* e = x.E + m * n3 + 3 * (size_t)t;
+                q.x += pf * (u[1] * e[2] - u[2] * e[1]);
+                q.y += pf * (u[2] * e[0] - u[0] * e[2]);
+                q.z += pf * (u[0] * e[1] - u[1] * e[0]);
+            }
+        }
+    }
+    acc_add(&force[3 * (size_t)s + 0], f.x);
+    acc_add(&force[3 * (size_t)s + 1], f.y);
+    acc_add(&force[3 * (size_t)s + 2], f.z);
+    if (an) {
+        acc_add(&torque[3 * (size_t)s + 0], q.x);
+        acc_add(&torque[3 * (size_t)s + 1], q.y);
+        acc_add(&torque[3 * (size_t)s + 2], q.z);
+    }
+}
+
 // The per-atom terms of the final pass, one dispatch: workgroups [0, nb) take
 // the reciprocal and self terms of 64 atoms each (their energy to the second
-// kEnergySlots words), workgroups [nb, 2 nb) the covalent pairs (to the first).
+// kEnergySlots words), workgroups [nb, 2 nb) the covalent pairs (to the first),
+// workgroups beyond the response terms of Extrapolated polarization.
 template <class R, bool COV>
 __global__ __launch_bounds__(kTile) void k_final_atoms(int n, int nb, int mutual, const double* __restrict__ phi,
                                                        const R* __restrict__ phidp, const double* __restrict__ mu,
                                                        FracT<double> A, double alpha, PairAtoms<double> C,
-                                                       PairParams<double> P, acc_t* force, acc_t* torque,
-                                                       acc_t* energy) {
+                                                       PairParams<double> P, ExtrapResponse X, acc_t* force,
+                                                       acc_t* torque, acc_t* energy) {
+    if (COV && (int)blockIdx.x >= 2 * nb) {
+        const int t = (blockIdx.x - 2 * nb) * kTile + threadIdx.x;
+        if (t < X.npol) extrap_response(X, t, C.aniso, force, torque);
+        return;
+    }
     const bool cov = COV && (int)blockIdx.x >= nb;
     const int block = cov ? blockIdx.x - nb : blockIdx.x;
     const int s = block * kTile + threadIdx.x;
@@ -1351,27 +1285,6 @@ void launch_dot(hipStream_t s, int m, const double* a, const double* b, double* 
     hipLaunchKernelGGL(k_dot_partial, dim3(kRedBlocks), dim3(kRedThreads), 0, s, m, a, b, partial);
     hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kRedThreads), 0, s, partial, 1, result);
 }
-template <class R>
-void launch_extrap_init(hipStream_t s, int n, const double* labpol, const double* E0, double* mu, R* mu_r) {
-    hipLaunchKernelGGL(k_extrap_init<R>, blocks_for(n, 256), dim3(256), 0, s, n, labpol, E0, mu, mu_r);
-}
-template <class R>
-void launch_extrap_order(hipStream_t s, int n, const acc_t* field, const acc_t* gacc, const R* phidp,
-                         FracT<double> A, double selfc, const double* labpol, const double* mu, double* E, double* G,
-                         double* mu_next, R* mu_next_r) {
-    hipLaunchKernelGGL(k_extrap_order<R>, blocks_for(n, 256), dim3(256), 0, s, n, field, gacc, phidp, A, selfc,
-                       labpol, mu, E, G, mu_next, mu_next_r);
-}
-template <class R>
-void launch_extrap_combine(hipStream_t s, int n, const ExtrapCoefficients& cp, const double* mus, double* mud,
-                           R* mu_r) {
-    hipLaunchKernelGGL(k_extrap_combine<R>, blocks_for(3 * n, 256), dim3(256), 0, s, n, cp, mus, mud, mu_r);
-}
-void launch_extrap_response(hipStream_t s, int n, const ExtrapCoefficients& cp, const double* mus, const double* Es,
-                            const double* Gs, const int* aniso, acc_t* force, acc_t* torque) {
-    hipLaunchKernelGGL(k_extrap_response, blocks_for(n, 256), dim3(256), 0, s, n, cp, mus, Es, Gs, aniso, force,
-                       torque);
-}
 void launch_potential_points(hipStream_t s, int n, int npts, const double4* pos, const double* lab, const double* mu,
                              Box<double> box, const double* points, double* out) {
     if (npts <= 0) return;
@@ -1424,27 +1337,23 @@ void launch_sub(hipStream_t s, int m, const double* a, const double* b_, double*
 template <class R>
 void launch_final_atoms(hipStream_t s, int n, int mutual, const double* phi, const R* phidp, const double* mu,
                         FracT<double> A, double alpha, PairAtoms<double> c, PairParams<double> p, bool cov,
-                        acc_t* force, acc_t* torque, acc_t* energy) {
+                        const ExtrapResponse& x, acc_t* force, acc_t* torque, acc_t* energy) {
     const int nb = (n + kTile - 1) / kTile;
     if (cov)
-        hipLaunchKernelGGL((k_final_atoms<R, true>), dim3(2 * nb), dim3(kTile), 0, s, n, nb, mutual, phi, phidp, mu, A,
-                           alpha, c, p, force, torque, energy);
+        hipLaunchKernelGGL((k_final_atoms<R, true>), dim3(2 * nb + (x.npol + kTile - 1) / kTile), dim3(kTile), 0, s, n,
+                           nb, mutual, phi, phidp, mu, A, alpha, c, p, x, force, torque, energy);
     else
         hipLaunchKernelGGL((k_final_atoms<R, false>), dim3(nb), dim3(kTile), 0, s, n, nb, mutual, phi, phidp, mu, A,
-                           alpha, c, p, force, torque, energy);
+                           alpha, c, p, x, force, torque, energy);
 }
 
 #define MPID_INSTANTIATE(R)                                                                                         \
     template void launch_fill<R>(hipStream_t, R*, size_t, R);                                                        \
     template void launch_fixed_field_finish<R>(hipStream_t, int, const R*, const double*, const acc_t*, FracT<double>, \
                                                double, double*);                                                    \
-    template void launch_extrap_init<R>(hipStream_t, int, const double*, const double*, double*, R*);                  \
-    template void launch_extrap_order<R>(hipStream_t, int, const acc_t*, const acc_t*, const R*, FracT<double>, double,   \
-                                         const double*, const double*, double*, double*, double*, R*);              \
-    template void launch_extrap_combine<R>(hipStream_t, int, const ExtrapCoefficients&, const double*, double*, R*); \
     template void launch_final_atoms<R>(hipStream_t, int, int, const double*, const R*, const double*,              \
-                                        FracT<double>, double, PairAtoms<double>, PairParams<double>, bool, acc_t*, \
-                                        acc_t*, acc_t*);                                                           \
+                                        FracT<double>, double, PairAtoms<double>, PairParams<double>, bool,         \
+                                        const ExtrapResponse&, acc_t*, acc_t*, acc_t*);                             \
     template void launch_field_sum<R>(hipStream_t, int, const acc_t*, const R*, const R*, double, double*);                    \
     template void launch_recip_potential<R>(hipStream_t, int, int, const double*, const R*, const double*,            \
                                             const double*, FracT<double>, double, acc_t*);                                 \

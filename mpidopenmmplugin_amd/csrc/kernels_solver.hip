@@ -355,6 +355,279 @@ __global__ __launch_bounds__(256) void k_operator_gather(SolverSites st, PmeGeom
 }
 
 // ---------------------------------------------------------------------------
+// Extrapolated (OPT) polarization
+// (convergeInduceDipolesByExtrapolation, MPIDReferenceForce.cpp:1125-1180)
+// ---------------------------------------------------------------------------
+// One order at a polarisable site: E = real space + reciprocal (-A phi_1) +
+// selfc mu_(m) and its gradient G = real space - A phi_2 A^T (A the
+// grid-coordinate transform; :4094-4127), kept for the response forces, and
+// mu_(m+1) = alpha_lab E by site in FP64 and by atom in the precision of the
+// next order's kernels.  Only polarisable sites are visited: at the others
+// mu is zero, and every use of E and G is multiplied by it.
+// s: field and gradient (xx yy zz xy xz yz) of the lists; q: the potential's
+// grid derivatives 100 010 001 200 020 002 110 101 011.
+template <class R>
+__device__ __forceinline__ void extrap_finish(const SolverSites& st, int t, int i, const R (&s)[9], const R (&q)[9],
+                                              const FracT<double>& F, double selfc, const double* __restrict__ labpol,
+                                              const ExtrapOrder& o, const double* __restrict__ mud, R* __restrict__ mu) {
+    const D3 c1 = cart_vector(mk((double)q[0], (double)q[1], (double)q[2]), F);
+    // A phi_2 A^T, A lower triangular
+    const double xx = q[3], yy = q[4], zz = q[5], xy = q[6], xz = q[7], yz = q[8];
+    double c2[6];  // xx yy zz xy xz yz
+    if (!F.tri) {
+        c2[0] = F.a00 * F.a00 * xx;
+        c2[1] = F.a11 * F.a11 * yy;
+        c2[2] = F.a22 * F.a22 * zz;
+        c2[3] = F.a00 * F.a11 * xy;
+        c2[4] = F.a00 * F.a22 * xz;
+        c2[5] = F.a11 * F.a22 * yz;
+    } else {
+        const double m[3][3] = {{xx, xy, xz}, {xy, yy, yz}, {xz, yz, zz}};
+        const double a[3][3] = {{F.a00, 0.0, 0.0}, {F.a10, F.a11, 0.0}, {F.a20, F.a21, F.a22}};
+        double am[3][3];
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) am[r][c] = a[r][0] * m[0][c] + a[r][1] * m[1][c] + a[r][2] * m[2][c];
+        auto el = [&](int r, int c) { return am[r][0] * a[c][0] + am[r][1] * a[c][1] + am[r][2] * a[c][2]; };
+        c2[0] = el(0, 0);
+        c2[1] = el(1, 1);
+        c2[2] = el(2, 2);
+        c2[3] = el(0, 1);
+        c2[4] = el(0, 2);
+        c2[5] = el(1, 2);
+    }
+    const D3 m = o.mus_in ? load3(o.mus_in, t) : load3(mud, i);
+    if (!o.mus_in) store3(o.mu0, t, m);  // mu_(0) = alpha E0, so far by atom
+    const D3 e = mk((double)s[0] - c1.x + selfc * m.x, (double)s[1] - c1.y + selfc * m.y,
+                    (double)s[2] - c1.z + selfc * m.z);
+    store3(o.E, t, e);
+#pragma unroll
+    for (int c = 0; c < 6; c++) o.G[6 * (size_t)t + c] = (double)s[3 + c] - c2[c];
+    const D3 nx = sym_mul6(labpol + 6 * (size_t)i, e);
+    store3(o.mus_out, t, nx);
+    store_mu<R>(mu, i, nx);
+}
+
+// As k_operator_fused: 32 lanes per site for everything after the inverse
+// transform.  mu is read of the neighbours and written in a second array.
+template <class R>
+__global__ __launch_bounds__(256) void k_extrap_fused(SolverSites st, PmeGeom<R> g, const R* __restrict__ pot,
+                                                      NbrList L, PairAtoms<R> A, PairParams<R> P,
+                                                      const R* __restrict__ mu, R* __restrict__ mu_next,
+                                                      FracT<double> F, double selfc, const double* __restrict__ labpol,
+                                                      ExtrapOrder o, const double* __restrict__ mud) {
+    __shared__ R sth[kOpSites][3][kOrder][3];
+    __shared__ int sig[kOpSites][3];
+    const int grp = threadIdx.x / kOpLanes, lane = threadIdx.x % kOpLanes;
+    const int t0 = blockIdx.x * kOpSites + grp;
+    const int t = min(t0, st.npol - 1);
+    const bool tv = t0 < st.npol;
+    const int i = st.idx[t];
+    const R4<R> pi = A.pos[i];
+    R q[9] = {};
+    if (pot) {
+        if (lane < 3) {
+            const V3<R> f = to_frac(mk(pi.x, pi.y, pi.z), g.box);
+            int ig;
+            R w;
+            grid_coord(lane == 0 ? f.x : (lane == 1 ? f.y : f.z), g.n[lane], ig, w);
+            R th[kOrder][3];
+            bspline6<R, 2>(w, th);
+#pragma unroll
+            for (int m = 0; m < kOrder; m++)
+#pragma unroll
+                for (int d = 0; d < 3; d++) sth[grp][lane][m][d] = th[m][d];
+            sig[grp][lane] = ig;
+        }
+        __syncthreads();
+        const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
+        const int gx = sig[grp][0], gy = sig[grp][1], gz = sig[grp][2];
+        constexpr int kPoints = kOrder * kOrder * kOrder;
+        constexpr int kSteps = (kPoints + kOpLanes - 1) / kOpLanes;
+        R v[kSteps];
+#pragma unroll
+        for (int u = 0; u < kSteps; u++) {
+            const int s = min(lane + u * kOpLanes, kPoints - 1);
+            const int ix = s / (kOrder * kOrder), rem = s - ix * kOrder * kOrder;
+            const int iy = rem / kOrder, iz = rem - iy * kOrder;
+            int x = gx + ix, y = gy + iy, z = gz + iz;
+            if (x >= nx) x -= nx;
+            if (y >= ny) y -= ny;
+            if (z >= nz) z -= nz;
+            v[u] = pot[((size_t)x * ny + y) * nz + z];
+        }
+#pragma unroll
+        for (int u = 0; u < kSteps; u++) {
+            const int s0 = lane + u * kOpLanes, s = min(s0, kPoints - 1);
+            const int ix = s / (kOrder * kOrder), rem = s - ix * kOrder * kOrder;
+            const int iy = rem / kOrder, iz = rem - iy * kOrder;
+            const R* a = sth[grp][0][ix];
+            const R* b = sth[grp][1][iy];
+            const R* c = sth[grp][2][iz];
+            const R p = s0 < kPoints ? v[u] : R(0);
+            q[0] += p * a[1] * b[0] * c[0];
+            q[1] += p * a[0] * b[1] * c[0];
+            q[2] += p * a[0] * b[0] * c[1];
+            q[3] += p * a[2] * b[0] * c[0];
+            q[4] += p * a[0] * b[2] * c[0];
+            q[5] += p * a[0] * b[0] * c[2];
+            q[6] += p * a[1] * b[1] * c[0];
+            q[7] += p * a[1] * b[0] * c[1];
+            q[8] += p * a[0] * b[1] * c[1];
+        }
+    }
+    R s[9] = {};
+    const int cnt = tv ? L.count[i] : 0;
+    for (int k = lane; k < cnt; k += kOpLanes) {
+        const int j = L.nbr[((size_t)(k / kNlSplit) * st.npol + t) * kNlSplit + k % kNlSplit];
+        const R4<R> pj = A.pos[j];
+        const V3<R> dr = min_image(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), P.box);
+        const V3<R> uj = mk(mu[3 * (size_t)j], mu[3 * (size_t)j + 1], mu[3 * (size_t)j + 2]);
+        const InducedRadialGrad<R> f = induced_grad_radial<R>(dot(dr, dr), pi.w, pj.w, P.default_thole, P);
+        const V3<R> e = induced_field_from<R>(uj, dr, InducedRadial<R>{f.f1, f.f2});
+        s[0] += e.x;
+        s[1] += e.y;
+        s[2] += e.z;
+        induced_grad_add<R>(uj, dr, f.f2, f.f3, s + 3);
+    }
+    const V3<R> c = partner_field_grad<R>(i, lane, kOpLanes, A, mu, P, s + 3);
+    s[0] += c.x;
+    s[1] += c.y;
+    s[2] += c.z;
+#pragma unroll
+    for (int off = 1; off < kOpLanes; off <<= 1)
+#pragma unroll
+        for (int k = 0; k < 9; k++) {
+            q[k] += __shfl_xor(q[k], off);
+            s[k] += __shfl_xor(s[k], off);
+        }
+    if (tv && lane == 0) extrap_finish<R>(st, t, i, s, q, F, selfc, labpol, o, mud, mu_next);
+}
+
+// The same in two kernels (see k_list_field and k_operator_gather)
+template <class R>
+__global__ __launch_bounds__(256) void k_extrap_list(SolverSites st, NbrList L, PairAtoms<R> A, PairParams<R> P,
+                                                     const R* __restrict__ mu, R* __restrict__ field) {
+    const unsigned gth = (unsigned)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int t0 = (int)(gth / kNlSplit), sub = (int)(gth % kNlSplit);
+    const bool tv = t0 < st.npol;
+    const int t = tv ? t0 : st.npol - 1;
+    const int i = st.idx[t];
+    const R4<R> pi = A.pos[i];
+    const int cnt = tv ? L.count[i] : 0;
+    const int* lp = L.nbr + (size_t)t * kNlSplit + sub;
+    const size_t stride = (size_t)st.npol * kNlSplit;
+    int jn = sub < cnt ? lp[0] : 0;
+    R s[9] = {};
+    for (int k = sub; k < cnt; k += kNlSplit) {
+        const int j = jn;
+        lp += stride;
+        if (k + kNlSplit < cnt) jn = *lp;  // next index in flight during this pair
+        const R4<R> pj = A.pos[j];
+        const V3<R> dr = min_image(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), P.box);
+        const V3<R> uj = mk(mu[3 * (size_t)j], mu[3 * (size_t)j + 1], mu[3 * (size_t)j + 2]);
+        const InducedRadialGrad<R> f = induced_grad_radial<R>(dot(dr, dr), pi.w, pj.w, P.default_thole, P);
+        const V3<R> e = induced_field_from<R>(uj, dr, InducedRadial<R>{f.f1, f.f2});
+        s[0] += e.x;
+        s[1] += e.y;
+        s[2] += e.z;
+        induced_grad_add<R>(uj, dr, f.f2, f.f3, s + 3);
+    }
+    const V3<R> c = partner_field_grad<R>(i, sub, kNlSplit, A, mu, P, s + 3);
+    s[0] += c.x;
+    s[1] += c.y;
+    s[2] += c.z;
+#pragma unroll
+    for (int off = 1; off < kNlSplit; off <<= 1)
+#pragma unroll
+        for (int k = 0; k < 9; k++) s[k] += __shfl_xor(s[k], off);
+    if (tv && sub == 0)
+#pragma unroll
+        for (int k = 0; k < 9; k++) field[9 * (size_t)t + k] = s[k];
+}
+template <class R>
+__global__ __launch_bounds__(256) void k_extrap_gather(SolverSites st, PmeGeom<R> g, const R* __restrict__ pot,
+                                                       const R* __restrict__ field, const R4<R>* __restrict__ pos,
+                                                       FracT<double> F, double selfc,
+                                                       const double* __restrict__ labpol, ExtrapOrder o,
+                                                       const double* __restrict__ mud, R* __restrict__ mu_next) {
+    const int gt = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+    const int t0 = gt >> 3, iz = gt & 7;
+    const bool tv = t0 < st.npol;
+    const int t = tv ? t0 : st.npol - 1;
+    const int i = st.idx[t];
+    R q[9] = {};
+    if (pot) {
+        const R4<R> p = pos[i];
+        int ig[3];
+        R w[3];
+        {
+            const V3<R> f = to_frac(mk(p.x, p.y, p.z), g.box);
+            grid_coord(f.x, g.n[0], ig[0], w[0]);
+            grid_coord(f.y, g.n[1], ig[1], w[1]);
+            grid_coord(f.z, g.n[2], ig[2], w[2]);
+        }
+        R tx[kOrder][3], ty[kOrder][3], tz[kOrder][3];
+        bspline6<R, 2>(w[0], tx);
+        bspline6<R, 2>(w[1], ty);
+        bspline6<R, 2>(w[2], tz);
+        const int ny = g.n[1], nz = g.n[2];
+        if (iz < kOrder) {
+            int z = ig[2] + iz;
+            if (z >= nz) z -= nz;
+            R b00 = 0, b10 = 0, b01 = 0, b20 = 0, b11 = 0, b02 = 0;
+#pragma unroll
+            for (int iy = 0; iy < kOrder; iy++) {
+                int y = ig[1] + iy;
+                if (y >= ny) y -= ny;
+                R row[kOrder];
+#pragma unroll
+                for (int ix = 0; ix < kOrder; ix++) {
+                    int x = ig[0] + ix;
+                    if (x >= g.n[0]) x -= g.n[0];
+                    row[ix] = pot[((size_t)x * ny + y) * nz + z];
+                }
+                R a0 = 0, a1 = 0, a2 = 0;
+#pragma unroll
+                for (int ix = 0; ix < kOrder; ix++) {
+                    a0 += row[ix] * tx[ix][0];
+                    a1 += row[ix] * tx[ix][1];
+                    a2 += row[ix] * tx[ix][2];
+                }
+                b00 += a0 * ty[iy][0];
+                b10 += a1 * ty[iy][0];
+                b01 += a0 * ty[iy][1];
+                b20 += a2 * ty[iy][0];
+                b11 += a1 * ty[iy][1];
+                b02 += a0 * ty[iy][2];
+            }
+            R c[3];
+            spline_at<R, 2>(tz, iz, c);
+            q[0] = b10 * c[0];
+            q[1] = b01 * c[0];
+            q[2] = b00 * c[1];
+            q[3] = b20 * c[0];
+            q[4] = b02 * c[0];
+            q[5] = b00 * c[2];
+            q[6] = b11 * c[0];
+            q[7] = b10 * c[1];
+            q[8] = b01 * c[1];
+        }
+#pragma unroll
+        for (int off = 1; off < 8; off <<= 1)
+#pragma unroll
+            for (int k = 0; k < 9; k++) q[k] += __shfl_xor(q[k], off);
+    }
+    if (tv && iz == 0) {
+        R s[9];
+#pragma unroll
+        for (int k = 0; k < 9; k++) s[k] = field[9 * (size_t)t + k];
+        extrap_finish<R>(st, t, i, s, q, F, selfc, labpol, o, mud, mu_next);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // conjugate gradients
 // ---------------------------------------------------------------------------
 // The solver's stopping test, the same expression as the host's report:
@@ -618,14 +891,28 @@ __global__ __launch_bounds__(256) void k_apply_S(SolverSites st, const double* _
     if (at) store3(at, t, m);
 }
 
+// v: the mutual solution (mu = S v); null: the dipoles are in place
+// (Direct), or with ex.n > 0 the sum of the extrapolated orders, mu = sum_o
+// c'_o mu_(o) with c'_o = sum_{j >= o} c_j (setExtrapolationCoefficients,
+// MPIDReferenceForce.cpp:173-183; the sum at :1170-1177).  A single order is
+// the dipoles in place, scaled.
 template <class R>
-__global__ __launch_bounds__(256) void k_final_start(SolverSites st, const double* __restrict__ v, R* mu, double* mud,
-                                                     acc_t* __restrict__ acc, size_t count) {
+__global__ __launch_bounds__(256) void k_final_start(SolverSites st, const double* __restrict__ v,
+                                                     ExtrapCoefficients ex, const double* __restrict__ mus, R* mu,
+                                                     double* mud, acc_t* __restrict__ acc, size_t count) {
     const int t = blockIdx.x * 256 + threadIdx.x;
     for (size_t k = t; k < count; k += (size_t)gridDim.x * 256) acc[k] = 0;
-    if (!v || t >= st.npol) return;
+    if (t >= st.npol || (!v && ex.n == 0)) return;
     const int i = st.idx[t];
-    const D3 m = sym_mul6(st.S + 6 * (size_t)i, load3(v, t));
+    D3 m;
+    if (v) {
+        m = sym_mul6(st.S + 6 * (size_t)i, load3(v, t));
+    } else if (ex.n == 1) {
+        m = load3(mud, i) * ex.c[0];
+    } else {
+        m = mk(0.0, 0.0, 0.0);
+        for (int o = 0; o < ex.n; o++) m = m + load3(mus + (size_t)o * 3 * st.npol, t) * ex.c[o];
+    }
     store_mu<R>(mu, i, m);
     store3(mud, i, m);
 }
@@ -747,10 +1034,30 @@ void launch_apply_S(hipStream_t s, SolverSites st, const double* v, R* mu, doubl
     hipLaunchKernelGGL(k_apply_S<R>, dim3((st.npol + 255) / 256), dim3(256), 0, s, st, v, mu, mud, at);
 }
 template <class R>
-void launch_final_start(hipStream_t s, SolverSites st, const double* v, R* mu, double* mud, acc_t* acc, size_t count) {
+void launch_final_start(hipStream_t s, SolverSites st, const double* v, const ExtrapCoefficients& ex,
+                        const double* mus, R* mu, double* mud, acc_t* acc, size_t count) {
     const size_t blocks = std::max<size_t>((st.npol + 255) / 256, std::min<size_t>((count + 255) / 256, 2048));
-    hipLaunchKernelGGL(k_final_start<R>, dim3((unsigned)std::max<size_t>(blocks, 1)), dim3(256), 0, s, st, v, mu, mud,
-                       acc, count);
+    hipLaunchKernelGGL(k_final_start<R>, dim3((unsigned)std::max<size_t>(blocks, 1)), dim3(256), 0, s, st, v, ex, mus,
+                       mu, mud, acc, count);
+}
+template <class R>
+void launch_extrap_list(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p, const R* mu,
+                        R* field) {
+    if (st.npol <= 0) return;
+    const unsigned blocks = ((unsigned)st.npol * kNlSplit + 255) / 256;
+    hipLaunchKernelGGL(k_extrap_list<R>, dim3(blocks), dim3(256), 0, s, st, l, a, p, mu, field);
+}
+template <class R>
+void launch_extrap_order(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const R* field, NbrList l,
+                         PairAtoms<R> a, PairParams<R> p, const R* mu, R* mu_next, FracT<double> A, double selfc,
+                         const double* labpol, const ExtrapOrder& o, const double* mud) {
+    if (st.npol <= 0) return;
+    if (field)
+        hipLaunchKernelGGL(k_extrap_gather<R>, dim3(((unsigned)st.npol * 8 + 255) / 256), dim3(256), 0, s, st, g, pot,
+                           field, a.pos, A, selfc, labpol, o, mud, mu_next);
+    else
+        hipLaunchKernelGGL(k_extrap_fused<R>, dim3((st.npol + kOpSites - 1) / kOpSites), dim3(256), 0, s, st, g, pot, l,
+                           a, p, mu, mu_next, A, selfc, labpol, o, mud);
 }
 void launch_residual(hipStream_t s, SolverSites st, const double* b, const double* Ax, const double* x, double* rt,
                      double* partial, double* out) {
@@ -775,7 +1082,13 @@ void launch_residual(hipStream_t s, SolverSites st, const double* b, const doubl
                                         PairAtoms<double>, PairParams<double>, const double*, const double*,        \
                                         FracT<double>, double, double*, double*, double*, R*, double*, const int*,  \
                                         int*);                                                                     \
-    template void launch_final_start<R>(hipStream_t, SolverSites, const double*, R*, double*, acc_t*, size_t);      \
+    template void launch_final_start<R>(hipStream_t, SolverSites, const double*, const ExtrapCoefficients&,         \
+                                        const double*, R*, double*, acc_t*, size_t);                               \
+    template void launch_extrap_list<R>(hipStream_t, SolverSites, NbrList, PairAtoms<R>, PairParams<R>, const R*,   \
+                                        R*);                                                                       \
+    template void launch_extrap_order<R>(hipStream_t, SolverSites, PmeGeom<R>, const R*, const R*, NbrList,         \
+                                         PairAtoms<R>, PairParams<R>, const R*, R*, FracT<double>, double,          \
+                                         const double*, const ExtrapOrder&, const double*);                        \
     template void launch_apply_S<R>(hipStream_t, SolverSites, const double*, R*, double*, double*);
 MPID_INSTANTIATE(float)
 MPID_INSTANTIATE(double)

@@ -159,6 +159,7 @@ template <class R> struct Prec {
     DBuf<R> lab;
     DBuf<R2<R>> td;
     DBuf<R> mu;       // induced dipoles in this precision (matvec input)
+    DBuf<R> mu_next;  // Extrapolated polarization: the next order's
     DBuf<R> erec;     // reciprocal induced field (inspection entry point)
     DBuf<R> elist;    // real-space induced field at the polarisable sites
     DBuf<R> phi, phidp;
@@ -304,12 +305,10 @@ struct mpid_context {
     acc_t* torque_acc() const { return final_acc.p + 3 * (size_t)n; }
     acc_t* energy_acc() const { return final_acc.p + 6 * (size_t)n; }
     // Extrapolated polarization: coefficient partial sums, the order dipoles
-    // mu_(m) [N][3n], the fields E_(m) and gradients G_(m) of mu_(0..N-2)
-    // ([N-1][3n], [N-1][6n]) and the real-space gradient accumulator
+    // mu_(m) [N][3 npol], the fields E_(m) and gradients G_(m) of mu_(0..N-2)
+    // ([N-1][3 npol], [N-1][6 npol]), by polarisable site
     ExtrapCoefficients ext_cp{};
     DBuf<double> ptmu, ptE, ptG;
-    DBuf<acc_t> grad_acc;
-    bool mu_set = false;  // the induced dipoles are in place (Extrapolated); the final pass does not form S x
     // solver
     DBuf<double> E0, b, x, r, p, Ap, dx, rt, mud, partial, scal, tmp3n, fout;
     // precisions
@@ -1328,36 +1327,42 @@ struct mpid_context {
     template <class R> void extrapolate(Prec<R>& P) {
         check_lists(false);
         const int N = ext_cp.n;
-        const size_t n3 = 3 * (size_t)n, n6 = 6 * (size_t)n;
-        ptmu.resize((size_t)N * n3);
-        ptE.resize((size_t)std::max(1, N - 1) * n3);
-        ptG.resize((size_t)std::max(1, N - 1) * n6);
-        grad_acc.resize(n6);
-        timed(P_SOLVER, [&] { launch_extrap_init<R>(stream, n, labpol.p, E0.p, ptmu.p, P.mu.p); });
+        const size_t n3 = 3 * (size_t)npol, n6 = 6 * (size_t)npol;
+        ptmu.resize(std::max<size_t>(N * n3, 1));
+        ptE.resize(std::max<size_t>((N - 1) * n3, 1));
+        ptG.resize(std::max<size_t>((N - 1) * n6, 1));
+        P.mu_next.resize(P.mu.n);
+        if (N > 1) P.elist.resize(9 * (size_t)n);
+        const bool fused = npol <= kFusedSites;
+        const NbrList l = nlist_pol();
         for (int m = 0; m + 1 < N; m++) {
-            recip_cycle_induced(P);  // phidp of mu_(m) at every atom, on rstream
-            timed(P_INDUCED, [&] {
-                launch_zero_acc(stream, field_acc.p, field_acc.n);
-                launch_zero_acc(stream, grad_acc.p, grad_acc.n);
-                launch_nl_induced_field<R>(stream, npol, pol_idx.p, nlist_pol(), pair_atoms(P), P.mu.p,
-                                           pair_params<R>(), field_acc.p, grad_acc.p);
-            });
-            timed(P_COV, [&] {
-                launch_cov_induced_field<R>(stream, n, pair_atoms(P), P.mu.p, pair_params<R>(), 1, field_acc.p,
-                                            grad_acc.p);
-            });
-            join();
-            timed(P_SOLVER, [&] {
-                launch_extrap_order<R>(stream, n, field_acc.p, grad_acc.p, P.phidp.p, frac_transform<double>(), selfc(), labpol.p,
-                                       ptmu.p + m * n3, ptE.p + m * n3, ptG.p + m * n6, ptmu.p + (m + 1) * n3,
-                                       P.mu.p);
+            if (!fused) {
+                fork();
+                timed_on(rstream, P_INDUCED, [&] {
+                    launch_extrap_list<R>(rstream, sites(), l, pair_atoms(P), pair_params<R>(), P.mu.p, P.elist.p);
+                });
+            }
+            recip_potential(P, stream);
+            if (!fused) join();
+            timed(fused ? P_INDUCED : P_GATHER, [&] {
+                const ExtrapOrder o{m == 0 ? nullptr : ptmu.p + m * n3, ptmu.p, ptE.p + m * n3, ptG.p + m * n6,
+                                    ptmu.p + (m + 1) * n3};
+                launch_extrap_order<R>(stream, sites(), pme() ? geom<R>() : PmeGeom<R>{},
+                                       pme() ? potential(P) : nullptr, fused ? nullptr : P.elist.p, l, pair_atoms(P),
+                                       pair_params<R>(), P.mu.p, P.mu_next.p, frac_transform<double>(), selfc(),
+                                       labpol.p, o, mud.p);
             });
             check_launch();
+            std::swap(P.mu.p, P.mu_next.p);
             stats.matvecs++;
         }
-        timed(P_SOLVER, [&] { launch_extrap_combine<R>(stream, n, ext_cp, ptmu.p, mud.p, P.mu.p); });
-        check_launch();
-        mu_set = true;
+        // The orders read and write polarisable sites only.  The final pass
+        // takes the array that is zero elsewhere (and overwrites the sites).
+        if ((N - 1) % 2 != 0) std::swap(P.mu.p, P.mu_next.p);
+    }
+    ExtrapResponse extrap_response() const {
+        if (opt.polarization != MPID_POLARIZATION_EXTRAPOLATED) return ExtrapResponse{};
+        return ExtrapResponse{ext_cp, npol, pol_idx.p, ptmu.p, ptE.p, ptG.p};
     }
 
     // DIIS, the reference's solver for mutual polarization
@@ -1574,13 +1579,12 @@ struct mpid_context {
         join();  // a previous final pass's reciprocal kernels have added into the accumulators
         // induced dipoles: mu = S x (double for the per-atom terms, R for the
         // kernels), unless they are in place already (Extrapolated)
+        const bool extrap = opt.polarization == MPID_POLARIZATION_EXTRAPOLATED;
         timed(P_SOLVER, [&] {
-            launch_final_start<R>(stream, sites(), mu_set ? nullptr : x.p, P.mu.p, mud.p, final_acc.p, final_acc.n);
+            launch_final_start<R>(stream, sites(), opt.polarization == MPID_POLARIZATION_MUTUAL ? x.p : nullptr,
+                                  extrap ? ext_cp : ExtrapCoefficients{}, ptmu.p, P.mu.p, mud.p, final_acc.p,
+                                  final_acc.n);
         });
-        if (opt.polarization == MPID_POLARIZATION_EXTRAPOLATED)
-            timed(P_SOLVER, [&] {
-                launch_extrap_response(stream, n, ext_cp, ptmu.p, ptE.p, ptG.p, aniso.p, force_acc(), torque_acc());
-            });
         // Order of issue: the reciprocal chain first (short kernels with large
         // LDS blocks, which would wait for whole CUs behind the
         // electrostatics), then the electrostatics, then the per-atom
@@ -1597,7 +1601,8 @@ struct mpid_context {
         timed_on(rstream, P_RECIP, [&] {
             launch_final_atoms<R>(rstream, n, opt.polarization == MPID_POLARIZATION_MUTUAL ? 1 : 0, pd.phi.p,
                                   P.phidp.p, mud.p, frac_transform<double>(), opt.ewald_alpha, pair_atoms(pd),
-                                  pair_params<double>(), true, force_acc(), torque_acc(), energy_acc());
+                                  pair_params<double>(), true, extrap_response(), force_acc(), torque_acc(),
+                                  energy_acc());
         });
         check_launch();
         final_issued = true;
@@ -1632,7 +1637,6 @@ struct mpid_context {
         for (int attempt = 0;; attempt++) {
             try {
                 final_issued = false;
-                mu_set = false;
                 prepare(d_pos);
                 fixed_field(P);
                 solve(P);
@@ -1729,7 +1733,7 @@ struct mpid_context {
         }
         // final pass at the refined dipoles, with the potential vectors
         timed(P_SOLVER,
-              [&] { launch_final_start<R>(stream, sites(), x.p, P.mu.p, mud.p, final_acc.p, final_acc.n); });
+              [&] { launch_final_start<R>(stream, sites(), x.p, ExtrapCoefficients{}, nullptr, P.mu.p, mud.p, final_acc.p, final_acc.n); });
         timed(P_OTHER, [&] {
             launch_zero_acc(stream, pot_acc.p, pot_acc.n);
             launch_zero_acc(stream, hd_acc.p, hd_acc.n);
@@ -1748,7 +1752,7 @@ struct mpid_context {
         });
         timed_on(rstream, P_RECIP, [&] {
             launch_final_atoms<R>(rstream, n, mutual ? 1 : 0, pd.phi.p, P.phidp.p, mud.p, frac_transform<double>(),
-                                  opt.ewald_alpha, pair_atoms(pd), pair_params<double>(), false, force_acc(),
+                                  opt.ewald_alpha, pair_atoms(pd), pair_params<double>(), false, ExtrapResponse{}, force_acc(),
                                   torque_acc(), energy_acc());
             launch_recip_potential<R>(rstream, n, pme() ? 1 : 0, pd.phi.p, P.phidp.p, lab.p, mud.p, frac_transform<double>(),
                                       opt.ewald_alpha, pot_acc.p);

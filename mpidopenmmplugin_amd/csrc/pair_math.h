@@ -904,6 +904,31 @@ MPID_HD ElecBareOut<R> elec_pair_bare_cart(V3<R> dr, R r2, const R* ma, R qb, V3
     return o;
 }
 
+// partner_field with the field gradient (xx yy zz xy xz yz) added to gr.
+template <class R>
+__device__ __forceinline__ V3<R> partner_field_grad(int i, int lane, int lanes, const PairAtoms<R>& A, const R* mu,
+                                                    const PairParams<R>& P, R* gr) {
+    V3<R> e = mk(R(0), R(0), R(0));
+    const int np = A.npart[i];
+    for (int k = lane; k < np; k += lanes) {
+        const int en = A.partners[(size_t)i * A.pstride + k];
+        const int j = en >> 2;
+        const R2<R> tdj = A.td[j];
+        if (tdj.y == R(0)) continue;
+        const R4<R> pi = A.pos[i], pj = A.pos[j];
+        const V3<R> dr = min_image(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), P.box);
+        const R r2 = dot(dr, dr);
+        if (r2 > P.rc2) continue;
+        const R2<R> tdi = A.td[i];
+        const R a = partner_scale<R>(en, P.scale14) == R(0) ? tdi.x + tdj.x : P.default_thole;
+        const V3<R> uj = mk(mu[3 * (size_t)j], mu[3 * (size_t)j + 1], mu[3 * (size_t)j + 2]);
+        const InducedRadialGrad<R> f = induced_grad_radial<R>(r2, tdi.y, tdj.y, a, P);
+        e = e + induced_field_from<R>(uj, dr, InducedRadial<R>{f.f1, f.f2});
+        induced_grad_add<R>(uj, dr, f.f2, f.f3, gr);
+    }
+    return e;
+}
+
 // Energy of atom i's covalent pairs with partners j > i; forces, torques and
 // (kPot) potential vectors (dE/dm, 20 per atom) of both sides are added to
 // the accumulators.

@@ -17,6 +17,13 @@ residual) and 1e-7 relative RMS in forces (first order: 1e-9 Debye is about
 (a small cluster's energy is a difference of large pair terms that a relative
 bar on the sum does not describe).
 
+Extrapolated polarization with one to three coefficients (no order, one and two
+orders) in a triclinic cell against the oracle: there is no iteration, so the
+FP64 path differs by rounding and the fixed-point sums (1e-9 relative RMS in
+forces and dipoles), the mixed path by the workload bar; and around 8,192 sites
+the dipoles against the recursion written out with the inspection entry
+points, to 1e-9 relative RMS (their fixed-point sums of 2^-32).
+
 Periodic boxes around 2,048 sites (one workgroup updates all sites, beyond it
 several do) and 8,192 sites (the operator's kernel adds the real-space field
 itself, beyond it the list kernel does): the dipoles must satisfy the
@@ -136,3 +143,43 @@ def test_no_polarisable_site():
         assert k.stats()["iterations"] == 0
         assert abs(e - ref["energy"]) <= e_tol * abs(ref["energy"])
         assert rel_rms(F, ref["forces"]) <= f_tol
+
+
+@pytest.mark.parametrize("coefficients", [[0.7], [0.3, 0.6], [-0.1, 0.4, 0.5]])
+def test_extrapolation_orders(coefficients):
+    force, pos, box = make_small_waterbox(60, 5, polarization=MPIDForce.Extrapolated)
+    force.setExtrapolationCoefficients(coefficients)
+    cutoff = 0.42
+    force.setCutoffDistance(cutoff)
+    force.setPMEParameters(2.628 / cutoff, 18, 20, 24)
+    L = box[0]
+    cell = np.array([[L, 0, 0], [0.2 * L, L, 0], [-0.15 * L, 0.1 * L, L]])
+    ref = oracle.evaluate(force.flatten(), pos, cell, details=True)
+    for precision, tol in (("double", 1e-9), ("mixed", 1e-5)):
+        k = HipCalcMPIDForceKernel(precision)
+        k.initialize(len(pos), force, default_box=cell)
+        print(f"[gpu] {len(coefficients)} extrapolation coefficients, {precision}", flush=True)
+        e, F = k.execute(pos, cell)
+        assert rel_rms(F, ref["forces"]) <= tol
+        assert rel_rms(k.getInducedDipoles(pos, cell), ref["induced"]) <= tol
+
+
+@pytest.mark.parametrize("waters", [8192, 8193])
+def test_extrapolation_recursion(waters):
+    alpha = 0.001
+    params = _o_parameters(np.random.default_rng(waters), True, False)  # isotropic
+    force, pos, box = make_small_waterbox(waters, waters, params, polarization=MPIDForce.Extrapolated)
+    coefficients = [0.2, 0.3, 0.5]
+    force.setExtrapolationCoefficients(coefficients)
+    k = HipCalcMPIDForceKernel("double")
+    k.initialize(len(pos), force, default_box=box)
+    print(f"[gpu] {waters} waters, extrapolated", flush=True)
+    found = k.getInducedDipoles(pos, box)
+    site = np.zeros((len(pos), 1))
+    site[::3] = alpha
+    order = site * k.computeFixedField(pos, box)
+    expected = sum(coefficients) * order
+    for m in (1, 2):
+        order = site * k.computeInducedField(pos, box, order)
+        expected = expected + sum(coefficients[m:]) * order
+    assert rel_rms(found, expected) <= 1e-9
