@@ -192,7 +192,7 @@ void launch_sorted_atoms(hipStream_t s, int n, Box<double> box, const double* po
 void launch_torque_to_force(hipStream_t s, int n, Box<double> box, const double4* pos, const int4* axes,
                             const acc_t* torque, acc_t* force, int exact_threefold);
 void launch_output_forces(hipStream_t s, int n, const int* perm, const acc_t* force, double* out, int accumulate,
-                          const acc_t* energy, acc_t* esum);
+                          const acc_t* energy, acc_t* esum, const double* gate);
 void launch_unpermute3(hipStream_t s, int n, const int* perm, const double* in, double* out);
 void launch_zero_acc(hipStream_t s, acc_t* p, size_t count);
 size_t sort_temp_bytes(int n);
@@ -372,7 +372,7 @@ void launch_electrostatics_pairs(hipStream_t s, int maxtiles, const int4* act, c
 // takes the count, *nact the length of the electrostatics kernels' work list
 // (the entries with J >= I; 0 when the rows overflow, so that a pass issued
 // before the host has seen that reads nothing).  work: 2 nb ints.
-constexpr int kOneRows = 256;  // blocks whose rows one workgroup builds
+constexpr int kOneRows = 64;  // blocks whose rows one workgroup builds
 void launch_block_rows(hipStream_t s, int nb, const float4* bmin, const float4* bmax, Box<float> box, float cutoff,
                        const int* polcnt, int* work, int* start, int* ustart, int* polstart, int* rows, int* owner,
                        int cap, int* total, int* nact);
@@ -429,6 +429,7 @@ struct SolverSites {
 constexpr int kCgCount = 9;
 constexpr int kCgStop = 10;
 constexpr int kCgCur = 11;
+constexpr int kCheckPassed = 12;  // the FP64 check of the mixed path's solution
 constexpr int kScalars = 16;
 constexpr int kMaxPartials = 1024;  // workgroups of a reducing kernel, at most
 constexpr int kOneSites = 2048;     // sites whose update fits one workgroup
@@ -495,9 +496,11 @@ void launch_extrap_order(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* p
 // S v: by atom in mu and mud, by site in at (each may be null)
 template <class R>
 void launch_apply_S(hipStream_t s, SolverSites st, const double* v, R* mu, double* mud, double* at);
-// rt = b - Ax (Ax null: rt as it is); out[0] = |S rt|^2, out[1] = x.rt (mapped host memory)
+// rt = b - Ax (Ax null: rt as it is); out[0] = |S rt|^2, out[1] = x.rt (mapped
+// host memory), *passed (may be null) = 1 if the RMS-Debye norm over n atoms
+// is below target, else 0
 void launch_residual(hipStream_t s, SolverSites st, const double* b, const double* Ax, const double* x, double* rt,
-                     double* partial, double* out);
+                     double* partial, double* out, double* passed, int n, double target);
 
 // ---- energy gradients ------------------------------------------------------------
 // The final pass of the gradients: launch_electrostatics_pairs plus the

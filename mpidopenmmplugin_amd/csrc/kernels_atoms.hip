@@ -1145,10 +1145,12 @@ __global__ __launch_bounds__(128) void k_torque_to_force(int n, Box<double> box,
 
 // Forces to the caller's order (out null: none), and the energies' slots
 // summed by the first wavefront into esum[0..1] (mapped host memory; integer
-// sums, so any order gives the same bits).
+// sums, so any order gives the same bits).  Nothing is written to out while
+// *gate is 0.
 __global__ __launch_bounds__(256) void k_output_forces(int n, const int* __restrict__ perm,
                                                        const acc_t* __restrict__ force, double* out, int accumulate,
-                                                       const acc_t* __restrict__ energy, acc_t* esum) {
+                                                       const acc_t* __restrict__ energy, acc_t* esum,
+                                                       const double* __restrict__ gate) {
     if (blockIdx.x == 0 && threadIdx.x < kTile) {
         acc_t e0 = 0, e1 = 0;
         for (int k = threadIdx.x; k < kEnergySlots; k += kTile) {
@@ -1166,7 +1168,7 @@ __global__ __launch_bounds__(256) void k_output_forces(int n, const int* __restr
         }
     }
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n || !out) return;
+    if (s >= n || !out || (gate && *gate == 0.0)) return;
     const int a = perm[s];
     for (int k = 0; k < 3; k++) {
         const double v = acc_get(force[3 * (size_t)s + k]);
@@ -1259,9 +1261,9 @@ void launch_torque_to_force(hipStream_t s, int n, Box<double> box, const double4
                        exact_threefold);
 }
 void launch_output_forces(hipStream_t s, int n, const int* perm, const acc_t* force, double* out, int accumulate,
-                          const acc_t* energy, acc_t* esum) {
+                          const acc_t* energy, acc_t* esum, const double* gate) {
     hipLaunchKernelGGL(k_output_forces, out ? blocks_for(n, 256) : dim3(1), dim3(256), 0, s, n, perm, force, out,
-                       accumulate, energy, esum);
+                       accumulate, energy, esum, gate);
 }
 void launch_unpermute3(hipStream_t s, int n, const int* perm, const double* in, double* out) {
     hipLaunchKernelGGL(k_unpermute3, blocks_for(n, 256), dim3(256), 0, s, n, perm, in, out);

@@ -166,8 +166,9 @@ __global__ __launch_bounds__(1024) void k_exclusive_scans(int m, Scans sc, int* 
 
 // At most kOneRows blocks: counting, the three scans and the rows in one
 // workgroup (the boxes and the hit masks stay in LDS, so each block pair is
-// tested once): at 192 blocks about 9 us against 25-30 us for the two passes
-// and three scans as dependent dispatches.
+// tested once): 6 us at 11 blocks against 20-25 us for the two passes and the
+// scans as three dependent dispatches.  At 192 blocks one CU needs 45 us for
+// the 36,864 tests, so that larger systems take the three.
 __global__ __launch_bounds__(1024) void k_block_rows_one(int nb, const float4* __restrict__ bmin,
                                                          const float4* __restrict__ bmax, Box<float> box, float cutoff,
                                                          const int* __restrict__ polcnt, int* __restrict__ start,

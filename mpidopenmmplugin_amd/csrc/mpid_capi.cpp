@@ -1301,16 +1301,22 @@ struct mpid_context {
             HIP_CHECK(hipEventRecord(ev_check[issued & 1], stream));
         };
         issue();
-        double eps;
+        double eps, before = 0.0;
         for (;;) {
             wait_event(ev_check[seen & 1]);
             if (seen == 0) check_lists_pending();
             const double* c = hscal + kCheck + 2 * (seen & 1);
             eps = debye_eps(c[0]);
             if (c[1] != 0.0) break;  // converged: an iteration issued after this one does nothing
+            if (issued == seen) issue();
             if (issued == seen) break;  // the iteration limit
-            seen++;                     // iteration `seen` runs (issued, and the solve had not stopped)
-            issue();                    // one iteration ahead of the host
+            // One iteration ahead of the host, unless the next check is likely
+            // to pass (it continues this one's decrease): the empty launches of
+            // an iteration that is not needed take longer than the wait.
+            const bool last = before > 0.0 && eps * (eps / before) < stop_eps;
+            before = eps;
+            seen++;  // iteration `seen` runs (issued, and the solve had not stopped)
+            if (!last) issue();
         }
         iters = iters0 + seen;
         stats.matvecs = matvecs0 + seen;
@@ -1485,16 +1491,21 @@ struct mpid_context {
         return c;
     }
 
-    // residual with the FP64 operator: rt = b - A x; returns its RMS-Debye
-    // norm and leaves x.rt in hscal[2]
-    double true_residual() {
+    // residual with the FP64 operator: rt = b - A x; its |S rt|^2 goes to
+    // hscal[1], x.rt to hscal[2], and scal[kCheckPassed] = 1 if its RMS-Debye
+    // norm is below the target
+    void issue_true_residual() {
         prof_override = P_REFINE;
         matvec(pd, x.p, Ap.p);
         prof_override = -1;
         timed(P_SOLVER, [&] {
-            launch_residual(stream, sites(), b.p, Ap.p, x.p, rt.p, partial.p, hscal_dev + 1);
+            launch_residual(stream, sites(), b.p, Ap.p, x.p, rt.p, partial.p, hscal_dev + 1, scal.p + kCheckPassed, n,
+                            opt.target_epsilon);
         });
         check_launch();
+    }
+    double true_residual() {
+        issue_true_residual();
         wait_stream();
         return debye_eps(hscal[1]);
     }
@@ -1533,32 +1544,53 @@ struct mpid_context {
             // FP32 operator and added in FP64, until the target is met.  The
             // final pass needs only the solution: it is issued first, and the
             // FP64 residual runs on vstream beside it.  Outputs are written
-            // only once the check has passed (forces_and_energy); a
-            // correction issues the final pass again.
+            // only if the check has passed: the first one is not waited for
+            // here, the device makes the test and the output kernel reads it
+            // (forces_and_energy); a correction issues the final pass again.
             mark_v();
             if (!defer_final) issue_final_pass(P);
-            on_vstream([&] { eps = true_residual(); });
-            int refine = 0;
-            while (eps >= opt.target_epsilon && refine < 8 && iters < opt.max_iterations) {
-                join();    // the final pass's reciprocal chain has read mu
-                join_v();  // rt
-                refine++;
-                const int before = iters;
-                cg(P, dx.p, rt.p, true, std::max(0.3 * opt.target_epsilon, 1e-4 * eps), iters, opt.max_iterations);
-                if (iters == before) iters++;
-                timed(P_SOLVER, [&] { launch_axpy(stream, 3 * npol, 1.0, dx.p, x.p); });
-                mark_v();
-                if (!defer_final) issue_final_pass(P);
-                on_vstream([&] { eps = true_residual(); });
+            on_vstream([&] { issue_true_residual(); });
+            if (!defer_final) {
+                check_pending = true;
+                solved_iterations = iters;
+                correction_pending = true;
+                return;
             }
-            stats.refinements = refine;
+            on_vstream([&] { wait_stream(); });
+            eps = refine(P, debye_eps(hscal[1]), iters);
             join_v();
         } else if (!defer_final) {
             timed(P_SOLVER,
-                  [&] { launch_residual(stream, sites(), nullptr, nullptr, x.p, r.p, partial.p, hscal_dev + 1); });
+                  [&] {
+                      launch_residual(stream, sites(), nullptr, nullptr, x.p, r.p, partial.p, hscal_dev + 1, nullptr,
+                                      n, 0.0);
+                  });
             check_launch();
         }
         correction_pending = true;
+        solved(iters, eps);
+    }
+    // The refinement loop after a check of eps; returns the last check's.
+    template <class R> double refine(Prec<R>& P, double eps, int& iters) {
+        int refine = 0;
+        while (eps >= opt.target_epsilon && refine < 8 && iters < opt.max_iterations) {
+            join();    // the final pass's reciprocal chain has read mu
+            join_v();  // rt
+            refine++;
+            const int before = iters;
+            cg(P, dx.p, rt.p, true, std::max(0.3 * opt.target_epsilon, 1e-4 * eps), iters, opt.max_iterations);
+            if (iters == before) iters++;
+            timed(P_SOLVER, [&] { launch_axpy(stream, 3 * npol, 1.0, dx.p, x.p); });
+            mark_v();
+            if (!defer_final) issue_final_pass(P);
+            on_vstream([&] { eps = true_residual(); });
+        }
+        stats.refinements = refine;
+        return eps;
+    }
+    bool check_pending = false;  // the FP64 check of the solution is on its way (its result gates the outputs)
+    int solved_iterations = 0;
+    void solved(int iters, double eps) {
         stats.iterations = iters;
         stats.epsilon = eps;
         stats.converged = eps < opt.target_epsilon ? 1 : 0;
@@ -1608,18 +1640,39 @@ struct mpid_context {
         final_issued = true;
     }
 
-    template <class R> double forces_and_energy(Prec<R>& P, double* d_forces_out) {
-        if (!final_issued) issue_final_pass(P);
-        final_issued = false;
-        mu_valid = true;
+    // The torques' forces, and the outputs if *gate (null: always) is 1
+    void issue_outputs(double* d_forces_out, const double* gate) {
         join();
         timed(P_OTHER, [&] {
             launch_torque_to_force(stream, n, dbox, spos.p, saxes.p, torque_acc(), force_acc(),
                                    (opt.flags & MPID_FLAG_CONSERVATIVE_TORQUES) ? 1 : 0);
-            launch_output_forces(stream, n, perm.p, force_acc(), d_forces_out, 1, energy_acc(), esum_dev());
+            launch_output_forces(stream, n, perm.p, force_acc(), d_forces_out, 1, energy_acc(), esum_dev(), gate);
         });
         check_launch();
+    }
+
+    template <class R> double forces_and_energy(Prec<R>& P, double* d_forces_out) {
+        if (!final_issued) issue_final_pass(P);
+        final_issued = false;
+        if (check_pending) join_v();
+        issue_outputs(d_forces_out, check_pending ? scal.p + kCheckPassed : nullptr);
         HIP_CHECK(hipStreamSynchronize(stream));
+        if (check_pending) {
+            check_pending = false;
+            const double eps = debye_eps(hscal[1]);
+            int iters = solved_iterations;
+            if (eps < opt.target_epsilon) {
+                solved(iters, eps);
+            } else {  // nothing was written: correct the dipoles and issue the outputs again
+                const double refined = refine(P, eps, iters);
+                join_v();
+                solved(iters, refined);
+                final_issued = false;
+                issue_outputs(d_forces_out, nullptr);
+                HIP_CHECK(hipStreamSynchronize(stream));
+            }
+        }
+        mu_valid = true;
         const acc_t* e = esum();
         if (correction_pending) {
             energy_correction = -0.5 * kElectric * hscal[2];
@@ -1637,6 +1690,7 @@ struct mpid_context {
         for (int attempt = 0;; attempt++) {
             try {
                 final_issued = false;
+                check_pending = false;
                 prepare(d_pos);
                 fixed_field(P);
                 solve(P);
@@ -1798,7 +1852,7 @@ struct mpid_context {
                                   Etot.p);
             launch_torque_to_force(stream, n, dbox, spos.p, saxes.p, torque_acc(), force_acc(),
                                    (opt.flags & MPID_FLAG_CONSERVATIVE_TORQUES) ? 1 : 0);
-            launch_output_forces(stream, n, perm.p, force_acc(), gforce.p, 0, energy_acc(), esum_dev());
+            launch_output_forces(stream, n, perm.p, force_acc(), gforce.p, 0, energy_acc(), esum_dev(), nullptr);
             launch_param_gradients(stream, n, all_sites ? 1 : 0, perm.p, dbox, spos.p, saxes.p, smol.p, spol.p,
                                    damp.p, chg.p, pot_acc.p, Etot.p, hd_acc.p, hdef_acc.p, ht_acc.p,
                                    opt.default_thole, gmol.p, gpol.p, gthole.p, gdef_acc.p);
