@@ -1128,8 +1128,8 @@ struct mpid_context {
     // The 35 potential derivatives of the induced dipoles at every atom
     // (phidp), on rstream after a fork(); the caller joins before it reads them.
     template <class R> void recip_cycle_induced(Prec<R>& P) {
+        fork();  // (without PME too: the per-atom and covalent-pair kernels follow on rstream)
         if (!pme()) return;  // phidp stays zero
-        fork();
         recip_potential(P, rstream);
         PmeGeom<R> g = geom<R>();
         timed_on(rstream, P_GATHER,

@@ -183,3 +183,17 @@ def test_extrapolation_recursion(waters):
         order = site * k.computeInducedField(pos, box, order)
         expected = expected + sum(coefficients[m:]) * order
     assert rel_rms(found, expected) <= 1e-9
+
+
+@pytest.mark.parametrize("polarization", [MPIDForce.Mutual, MPIDForce.Direct, MPIDForce.Extrapolated],
+                         ids=["mutual", "direct", "extrapolated"])
+def test_repeated_evaluations_without_cutoff(polarization):
+    force, pos, _ = make_small_waterbox(216, 5, polarization=polarization)
+    force.setNonbondedMethod(MPIDForce.NoCutoff)
+    force.setMutualInducedTargetEpsilon(1e-9)
+    k = HipCalcMPIDForceKernel("double")
+    k.initialize(len(pos), force)
+    print(f"[gpu] repeated evaluations, polarization {polarization}", flush=True)
+    first = k.execute(pos, None)[1]
+    for _ in range(6):
+        assert rel_rms(k.execute(pos, None)[1], first) <= 1e-12
