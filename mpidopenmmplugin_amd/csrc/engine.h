@@ -176,6 +176,7 @@ struct AtomState {
     float4* bmax;
     unsigned long long* polmask;
     int* polcnt;
+    unsigned long long* bmask;  // the block's bare charges
     int* nl_scalars;  // cleared
     int* tstart;      // [ntiles + 1] first sorted atom of each spreading tile
     int tile_shift;
@@ -351,19 +352,39 @@ template <class R>
 void launch_recip_convolution(hipStream_t s, const FftPlan<R>& p, R* Q, R2<R>* S, R* V, ConvParams<R> cp);
 
 // ---- real space (kernels_pairs.hip) -------------------------------------------
-// One workgroup per tile act[0 .. *nact) (row entries r of block pairs
-// J >= I); the launch covers maxtiles >= *nact.
-// tmask: pairs with a multipole or a polarisable site; tmaskcc: pairs of two
-// bare charges; chg[i] != 0: atom i is a bare charge (pairs of tmask with one
-// such site take the reduced formula).  The charge-charge channel of all
-// pairs is evaluated in FP64 from pos64 (x, y, z) and the FP64 lab-frame
-// charges lab64[20 i].
+// The tiles (block pairs I, J >= I): tile u < *nact is act[u] = {two-bare
+// pairs | general pairs << 16, I, J, one-bare pairs}, and its pairs are
+// list[u * kTilePairs ..]: the two-bare and then the general ones from the
+// front, the ones with one bare charge from the back.  An entry is
+// atom of I << 8 | atom of J, bit 15 of a one-bare entry says that I's site is
+// the bare one.
+constexpr int kTilePairs = kTile * kTile;
+//
+// Groups: the electrostatics kernel's workgroups take m > 1 consecutive tiles
+// of one block row each.  Row I's groups are the slots ustart[I] / m + I up to
+// ustart[I + 1] / m + I of groups[], {first tile, tiles}; that is one slot
+// more than the row needs at most, which holds no tiles, and needs no scan of
+// its own.
+struct TileList {
+    const int4* act;
+    const int* nact;
+    const unsigned short* list;
+    const int2* groups;
+};
+MPID_HD int tile_groups(int tiles, int n, int m) { return tiles / m + (n + kTile - 1) / kTile; }
+// m, from an upper bound of the tile count: two in FP32 (TileShape), unless
+// that leaves CUs without eight workgroups
+inline int tiles_per_group(int maxtiles, bool fp64) { return maxtiles < 4096 || fp64 ? 1 : 2; }
+// Real-space electrostatics of all tiles; the launch covers maxtiles >= *nact.
+// bmask: the bare charges of each block (a pair with one takes the reduced
+// formula).  The charge-charge channel of all pairs is evaluated in FP64 from
+// pos64 (x, y, z) and the FP64 lab-frame charges lab64[20 i].  ustart[I]: the
+// first tile of block row I.
 template <class R>
-void launch_electrostatics_pairs(hipStream_t s, int maxtiles, const int4* act, const int* nact, const int* rows,
-                                 const int* owner, const unsigned long long* tmask,
-                                 const unsigned long long* tmaskcc, const int* chg, PairAtoms<R> a, const R* mu,
-                                 PairParams<R> p, const double4* pos64, const double* lab64, PairParams<double> p64,
-                                 acc_t* force, acc_t* torque, acc_t* energy);
+void launch_electrostatics_pairs(hipStream_t s, int n, int maxtiles, int group, const TileList& t, const int* ustart,
+                                 const unsigned long long* bmask, PairAtoms<R> a, const R* mu, PairParams<R> p,
+                                 const double4* pos64, const double* lab64, PairParams<double> p64, acc_t* force,
+                                 acc_t* torque, acc_t* energy);
 // ---- neighbour lists (kernels_nlist.hip) ---------------------------------------
 // Block rows: for each block I the blocks J within the cutoff, ascending, at
 // rows[start[I] ..] with I in owner[] (at most cap entries are stored; the
@@ -379,23 +400,23 @@ void launch_block_rows(hipStream_t s, int nb, const float4* bmin, const float4* 
 // pos.w of the FP64 positions is the damping factor: nonzero iff the site is polarisable
 // Masks, then lists: all = true gives the full list of every atom stored by
 // atom index; all = false the full and polarisable-neighbour lists of the
-// polarisable atoms, stored by position in their sorted index.  nmask: 64 words per
-// row entry (nrows entries); polmask: one word per block; scalars[0]:
-// largest stored list length, scalars[1]: nonzero if a block pair lacked its
-// mirror entry.  act[ustart[I] + k] = {r, I, J} for the k-th row entry r of
-// row I with J >= I, r = -1 if the block pair holds no pair (ustart: the
-// exclusive scan of launch_block_rows' upper, whose last element is the
-// number of such entries).  nrows: row entries launched (the count, or the capacity
-// when the count is not known on the host: entries past rstart[nb] return);
-// rcap: the capacity of rows / nmask (entries beyond it are ignored).
+// polarisable atoms, stored by position in their sorted index.  nmask: 64
+// words per row entry (nrows entries); scalars[0]: largest stored list length,
+// scalars[1]: nonzero if a block pair lacked its mirror entry.  act and plist:
+// the tiles and their pairs (TileList; ustart: the exclusive scan of the rows'
+// entries with J >= I; bmask: the bare charges of each block).  nrows: row
+// entries launched (the count, or the capacity when the count is not known on
+// the host: entries past rstart[nb] return); rcap: the capacity of rows /
+// nmask (entries beyond it are ignored); tcap: that of act and plist in tiles.
+// groups: the groups of `group` > 1 tiles (not written for 1).
 // pol_idx: the sorted indices of the polarisable atoms; tpstart (may be
 // null): the first entry of pol_idx in each spreading tile, from tstart.
 void launch_nl_build(hipStream_t s, int n, int nrows, int rcap, bool all, const int* rstart, const int* rows,
                      const int* owner, const float4* bmin, const float4* bmax, const double4* pos,
                      const int* partners, const int* npart, int pstride, Box<double> box, double rc2, int cap,
                      unsigned long long* nmask, const unsigned long long* polmask, const int* polstart, int* nbr,
-                     int* count, int* scalars, unsigned long long* tmask, int* pnbr, int* pcount, const int* chg,
-                     unsigned long long* tmaskcc, int4* act, const int* ustart, int* pol_idx, int ntiles,
+                     int* count, int* scalars, int* pnbr, int* pcount, const unsigned long long* bmask, int4* act,
+                     unsigned short* plist, int tcap, int2* groups, int group, const int* ustart, int* pol_idx, int ntiles,
                      const int* tstart, int* tpstart);
 // fields at the atoms atoms[0..natoms) (all atoms when atoms == nullptr, natoms = n)
 template <class R>
@@ -509,9 +530,8 @@ void launch_residual(hipStream_t s, SolverSites st, const double* b, const doubl
 // formula, so that bare-charge sites get all 20 components (else the charge
 // component only).
 template <class R>
-void launch_electrostatics_pot(hipStream_t s, int maxtiles, const int4* act, const int* nact, const int* rows,
-                               const int* owner, const unsigned long long* tmask, const unsigned long long* tmaskcc,
-                               const int* chg, PairAtoms<R> a, const R* mu, PairParams<R> p, const double4* pos64,
+void launch_electrostatics_pot(hipStream_t s, int maxtiles, const TileList& t, const unsigned long long* bmask,
+                               PairAtoms<R> a, const R* mu, PairParams<R> p, const double4* pos64,
                                const double* lab64, PairParams<double> p64, acc_t* force, acc_t* torque,
                                acc_t* energy, acc_t* pot, int all_general);
 // Thole damping derivatives h = u dE/du (thole_u_derivative) of the pairs of

@@ -335,7 +335,12 @@ __global__ __launch_bounds__(kTile) void k_sorted_atoms(int n, Box<double> box, 
         }
     o.damp[s] = damp;
     o.aniso[s] = (p0 != p1 || p0 != p2) ? 1 : 0;
-    o.chg[s] = (bare && p0 == 0.0 && p1 == 0.0 && p2 == 0.0) ? 1 : 0;
+    const bool charge = bare && p0 == 0.0 && p1 == 0.0 && p2 == 0.0;
+    o.chg[s] = charge ? 1 : 0;
+    {
+        const unsigned long long bm = __ballot(charge);  // lanes past the last atom have left: 0
+        if (threadIdx.x == 0) o.bmask[blockIdx.x] = bm;
+    }
     for (int k = 0; k < kMP; k++) o.lab[(size_t)s * kMP + k] = r[k];
     o.dpos[s] = make_double4(w.x, w.y, w.z, damp);  // w: damping factor
     o.dtd[s] = make_double2(th, damp);

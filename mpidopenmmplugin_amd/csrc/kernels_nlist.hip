@@ -244,26 +244,37 @@ __global__ __launch_bounds__(1024) void k_block_rows_one(int nb, const float4* _
 // distances, the test of the reference: r2 > cutoff^2 is out), skipping
 // itself and its scaled covalent partners (those pairs go to the
 // covalent-pair kernels), and writes the 64-bit neighbour mask of i within J
-// to nmask[r * 64 + lane].  For J > I the 64 x 64 bit matrix is transposed
-// (one ballot per column) into the masks of J's atoms within I, written at
-// the mirrored entry (J, I) of J's row; the block-box test is symmetric, so
-// that entry exists (if not, flag[0] is set and the host raises an error).
-// Tile masks: bit jj for each listed j = J * 64 + jj with j > i, in
-// tmaskcc[r * 64 + lane] when i and j are both bare charges (chg), in
-// tmask[r * 64 + lane] otherwise.
-__global__ __launch_bounds__(64) void k_nl_masks(int n, const int* __restrict__ rstart, const int* __restrict__ rows,
+// to nmask[r * 64 + lane].  For J > I the masks of J's atoms within I (one
+// ballot per tested atom) go to the mirrored entry (J, I) of J's row; the
+// block-box test is symmetric, so that entry exists (if not, flag[0] is set
+// and the host raises an error).
+//
+// One workgroup of W wavefronts per entry; each tests every W-th atom of J
+// against the 64 of I.  A ballot per tested atom, kept in LDS, gives its
+// pairs (j > i); a scan of their counts places them in the tile's pair list by
+// class (TileList, kernels_pairs.hip).  (The electrostatics kernel used to rank
+// the masks' bits itself, one lane per row i stepping through its set bits:
+// 44% of that kernel's instructions.)  A tile is a chain over the tested atoms:
+// four wavefronts shorten it where there are few tiles (81 atoms: 18 us with
+// one, 9 with four), and repeat the setup and the scan where there are many
+// (98,304 atoms: 200 us with one, 349 with four; 12,288 atoms are even).
+constexpr int kOneWaveRows = 16384;  // row entries (twice the tiles)
+template <int W>
+__global__ __launch_bounds__(W * kTile) void k_nl_masks(int n, const int* __restrict__ rstart, const int* __restrict__ rows,
                                                  const int* __restrict__ owner, const float4* __restrict__ bmin,
                                                  const float4* __restrict__ bmax, const double4* __restrict__ pos,
                                                  const int* __restrict__ partners, const int* __restrict__ npart,
                                                  int pstride, Box<double> box, double rc2,
-                                                 const int* __restrict__ chg,
+                                                 const unsigned long long* __restrict__ bmask,
                                                  unsigned long long* __restrict__ nmask,
-                                                 unsigned long long* __restrict__ tmask,
-                                                 unsigned long long* __restrict__ tmaskcc,
                                                  int* __restrict__ flag, int cap, int4* __restrict__ act,
+                                                 unsigned short* __restrict__ plist, int tcap,
+                                                 int2* __restrict__ groups, int group,
                                                  const int* __restrict__ ustart) {
     __shared__ double4 sp[kTile];
-    const int r = blockIdx.x, lane = threadIdx.x;
+    __shared__ unsigned long long shits[kTile];             // [atom of J]: the atoms of I within the cutoff
+    __shared__ unsigned long long sm[W][kTile];             // [][atom of I]: a wavefront's part of its mask
+    const int r = blockIdx.x, lane = threadIdx.x & (kTile - 1), wave = threadIdx.x / kTile;
     const int nbk = (n + kTile - 1) / kTile;
     if (r >= min(rstart[nbk], cap)) return;  // uniform: the grid may cover the capacity, not the count
     const int I = owner[r], J = rows[r];
@@ -272,9 +283,11 @@ __global__ __launch_bounds__(64) void k_nl_masks(int n, const int* __restrict__ 
     const bool iv = i < n, jv = j < n;
     const int ic = iv ? i : n - 1, jc = jv ? j : n - 1;
     const double4 pi = pos[ic], pj = pos[jc];
-    const bool ibare = iv && chg[ic] != 0;
-    const unsigned long long jbare = __ballot(jv && chg[jc] != 0);
-    sp[lane] = pj;
+    const unsigned long long ibare = bmask[I], jbare = bmask[J];
+    if (wave == 0) {
+        sp[lane] = pj;
+        shits[lane] = 0ull;
+    }
     // candidates: atoms of J whose distance to block I's box is within the
     // cutoff (minimum image; never rejects a pair within the cutoff)
     bool cand;
@@ -294,7 +307,7 @@ __global__ __launch_bounds__(64) void k_nl_masks(int n, const int* __restrict__ 
         cand = jv && gap_within((float)pj.x - cI[0], (float)pj.y - cI[1], (float)pj.z - cI[2], hI[0], hI[1], hI[2],
                                 fb, rcf);
     }
-    unsigned long long cmask = __ballot(cand);
+    const unsigned long long cmask = __ballot(cand);
     unsigned long long skip = J == I ? 1ull << lane : 0ull;
     const int np = iv ? npart[ic] : 0;
     const int* parts = partners + (size_t)ic * pstride;
@@ -302,36 +315,91 @@ __global__ __launch_bounds__(64) void k_nl_masks(int n, const int* __restrict__ 
         const int p = parts[k] >> 2;
         if ((p >> 6) == J) skip |= 1ull << (p & 63);
     }
-    if (!iv) cmask = 0;  // lanes past the last atom list nothing
     __syncthreads();
-    unsigned long long m = 0;
-    while (cmask) {
-        const int jj = __ffsll((long long)cmask) - 1;
-        cmask &= cmask - 1ull;
-        const double4 q = sp[jj];
-        const V3<double> dr = min_image(mk(q.x - pi.x, q.y - pi.y, q.z - pi.z), box);
-        if (dot(dr, dr) <= rc2) m |= 1ull << jj;
-    }
-    m &= ~skip;
-    nmask[(size_t)r * kTile + lane] = m;
-    // tile-mask bits: j > i, i.e. all of J when J > I, those above the lane when J == I;
-    // pairs of two bare charges go to their own list (their interaction is q q erfc(a r) / r)
-    const unsigned long long upper = J > I ? ~0ull : ~((2ull << lane) - 1ull);
-    const unsigned long long cc = ibare ? (m & jbare) : 0ull;
-    tmask[(size_t)r * kTile + lane] = (m & ~cc) & upper;
-    tmaskcc[(size_t)r * kTile + lane] = cc & upper;
     // the tile's entry in the electrostatics kernels' work list: the row
     // entries J >= I of row I are its last upper[I] entries, placed at
-    // ustart[I] (the exclusive scan of upper) in the same order; a tile
-    // without pairs is marked r = -1
-    const bool has_pairs = __ballot((m & upper) != 0ull) != 0ull;
-    if (lane == 0) act[ustart[I + 1] - (rstart[I + 1] - r)] = make_int4(has_pairs ? r : -1, I, J, 0);
-    if (J > I) {
-        unsigned long long t = 0;
-        for (int k = 0; k < kTile; k++) {
-            const unsigned long long col = __ballot((m >> k) & 1ull);
-            if (lane == k) t = col;
+    // ustart[I] (the exclusive scan of upper) in the same order
+    const int u = ustart[I + 1] - (rstart[I + 1] - r);
+    if (u >= tcap) return;  // uniform: only when the rows exceeded their capacity (the host then builds again)
+    unsigned short* list = plist + (size_t)u * kTilePairs;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const bool mine = ((ibare >> lane) & 1ull) != 0;  // this lane's atom of I is a bare charge
+    const unsigned long long part = W == 4 ? cmask & (0x1111111111111111ull << wave) : cmask;
+    unsigned long long m = 0;
+    for (unsigned long long cm = part; cm;) {
+        constexpr int kAhead = 4;  // distances formed at once
+        unsigned long long bit[kAhead];
+        int jj[kAhead];
+        bool hit[kAhead];
+#pragma unroll
+        for (int k = 0; k < kAhead; k++) {
+            bit[k] = cm & (0ull - cm);  // the lowest one left, or none
+            jj[k] = __ffsll((long long)cm) - 1;
+            cm &= cm - 1ull;
+            const double4 q = sp[max(jj[k], 0)];
+            const V3<double> dr = min_image(mk(q.x - pi.x, q.y - pi.y, q.z - pi.z), box);
+            hit[k] = iv && dot(dr, dr) <= rc2 && (bit[k] & ~skip) != 0ull;
         }
+#pragma unroll
+        for (int k = 0; k < kAhead; k++) {
+            const unsigned long long hits = __ballot(hit[k]);
+            if (hit[k]) m |= bit[k];
+            if (lane == 0 && bit[k]) shits[jj[k]] = hits;
+        }
+    }
+    sm[wave][lane] = m;
+    __syncthreads();
+    // lane jj: the pairs of J's atom jj.  Those whose two sites are alike (both
+    // bare, or neither) go to the front, two bare charges first; those with
+    // one bare site to the back.
+    const unsigned long long hits = shits[lane];
+    const bool jb = ((jbare >> lane) & 1ull) != 0;
+    const unsigned long long pairs = J > I ? hits : hits & below;  // j > i
+    const unsigned long long alike = jb ? pairs & ibare : pairs & ~ibare, mixed = pairs & ~alike;
+    const int na = __popcll(alike), nm = __popcll(mixed);
+    int front = jb ? na : na << 16, back = nm;  // scans: two bare | general << 16, one bare
+#pragma unroll
+    for (int off = 1; off < kTile; off <<= 1) {
+        const int f = __shfl_up(front, off), k = __shfl_up(back, off);
+        if (lane >= off) {
+            front += f;
+            back += k;
+        }
+    }
+    const int totals = __builtin_amdgcn_readlane(front, kTile - 1);
+    const int ncc = totals & 0xffff, nup = ncc + (int)((unsigned)totals >> 16);
+    const int none = __builtin_amdgcn_readlane(back, kTile - 1);
+    front = jb ? (front & 0xffff) - na : ncc + (int)((unsigned)front >> 16) - na;
+    back = kTilePairs - 1 - (back - nm);
+    const unsigned long long own = (mine ? ibare : ~ibare) & below;  // this lane's class, the atoms before it
+    // the entry without its atom of J, for a bare one and for another one there
+    const int ent = lane << 8, ent_bare = ent, ent_other = mine ? ent | 0x8000 : ent;
+    for (unsigned long long cm = part; cm; cm &= cm - 1ull) {
+        const int jj = __ffsll((long long)cm) - 1;  // uniform
+        const unsigned lo = __builtin_amdgcn_readlane((unsigned)pairs, jj);
+        const unsigned hi = __builtin_amdgcn_readlane((unsigned)(pairs >> 32), jj);
+        const unsigned long long all = ((unsigned long long)hi << 32) | lo;
+        const bool jbb = ((jbare >> jj) & 1ull) != 0, same = mine == jbb;
+        const int f = __builtin_amdgcn_readlane(front, jj), k = __builtin_amdgcn_readlane(back, jj);
+        const int rank = __popcll(all & own);
+        if ((all >> lane) & 1ull)
+            list[same ? f + rank : k - rank] = (unsigned short)((jbb ? ent_bare : ent_other) | jj);
+    }
+    if (wave != 0) return;
+    m = 0;
+#pragma unroll
+    for (int w = 0; w < W; w++) m |= sm[w][lane];
+    nmask[(size_t)r * kTile + lane] = m;
+    if (lane == 0) {
+        act[u] = make_int4(ncc | ((nup - ncc) << 16), I, J, none);
+        if (group > 1) {
+            const int u0 = ustart[I], u1 = ustart[I + 1], slot = u0 / group + I, k = u - u0;
+            if (k % group == 0) groups[slot + k / group] = make_int2(u, min(group, u1 - u));
+            if (u + 1 == u1)  // the row's slot that it does not need, if there is one
+                for (int s = slot + (u1 - u0 + group - 1) / group; s <= u1 / group + I; s++) groups[s] = make_int2(0, 0);
+        }
+    }
+    if (J > I) {
         // the mirrored entry: I in the ascending row of J
         int lo = min(rstart[J], cap), hi = min(rstart[J + 1], cap) - 1;
         while (lo < hi) {
@@ -339,7 +407,7 @@ __global__ __launch_bounds__(64) void k_nl_masks(int n, const int* __restrict__ 
             if (rows[mid] < I) lo = mid + 1;
             else hi = mid;
         }
-        if (lo <= hi && rows[lo] == I) nmask[(size_t)lo * kTile + lane] = t;
+        if (lo <= hi && rows[lo] == I) nmask[(size_t)lo * kTile + lane] = hits;
         else if (lane == 0) atomicOr(flag, 1);
     }
 }
@@ -621,14 +689,16 @@ void launch_nl_build(hipStream_t s, int n, int nrows, int rcap, bool all, const 
                      const int* owner, const float4* bmin, const float4* bmax, const double4* pos,
                      const int* partners, const int* npart, int pstride, Box<double> box, double rc2, int cap,
                      unsigned long long* nmask, const unsigned long long* polmask, const int* polstart, int* nbr,
-                     int* count, int* scalars, unsigned long long* tmask, int* pnbr, int* pcount, const int* chg,
-                     unsigned long long* tmaskcc, int4* act, const int* ustart, int* pol_idx, int ntiles,
+                     int* count, int* scalars, int* pnbr, int* pcount, const unsigned long long* bmask, int4* act,
+                     unsigned short* plist, int tcap, int2* groups, int group, const int* ustart, int* pol_idx, int ntiles,
                      const int* tstart, int* tpstart) {
     const int nb = (n + kTile - 1) / kTile;
-    if (nrows > 0)
-        hipLaunchKernelGGL(k_nl_masks, dim3(nrows), dim3(kTile), 0, s, n, rstart, rows, owner, bmin, bmax, pos,
-                           partners, npart, pstride, box, rc2, chg, nmask, tmask, tmaskcc, scalars + 1, rcap, act,
-                           ustart);
+    if (nrows > 0) {
+        const bool one = nrows > kOneWaveRows;
+        hipLaunchKernelGGL((one ? &k_nl_masks<1> : &k_nl_masks<4>), dim3(nrows), dim3(one ? kTile : 4 * kTile), 0, s, n,
+                           rstart, rows, owner, bmin, bmax, pos, partners, npart, pstride, box, rc2, bmask, nmask,
+                           scalars + 1, rcap, act, plist, tcap, groups, group, ustart);
+    }
     hipLaunchKernelGGL(k_nl_fill, dim3(nb), dim3(kFillWaves * kTile), 0, s, n, all ? 1 : 0, rstart, rows, polmask,
                        polstart, nmask, cap, nbr, count, scalars, pnbr, pcount, rcap, pol_idx, ntiles, tstart, tpstart);
 }

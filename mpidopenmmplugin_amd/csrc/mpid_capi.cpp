@@ -278,12 +278,15 @@ struct mpid_context {
     // of capacity nl_cap, and the tile masks of the row entries with J >= I
     DBuf<float4> bmin, bmax;
     DBuf<int> brow_work, brow_start, brows, brow_owner, nbr, ncount, nl_scalars;
-    DBuf<int4> tile_act;  // the electrostatics kernels' tiles {r, I, J} (row entries with J >= I)
+    DBuf<int4> tile_act;  // the electrostatics kernels' tiles (TileList; row entries with J >= I)
     DBuf<int> brow_ustart;  // exclusive scan of the block rows' entries with J >= I
     // polarisable neighbours only (pnbr/pcount), and the sorted indices of the polarisable atoms
     DBuf<int> pnbr, pcount, polcnt, polstart, pol_idx;
     int npol = 0;
-    DBuf<unsigned long long> tmask, tmaskcc, nmask, polmask;
+    DBuf<unsigned long long> nmask, polmask, baremask;
+    DBuf<unsigned short> tile_pairs;  // the tiles' pair lists (TileList)
+    DBuf<int2> tile_groups_buf;       // and their groups of tile_group tiles
+    int tile_group = 1;
     int rows_total = 0;
     bool rows_pending = false;  // the block-row count of this build is still on its way to hnl[2]
     int rows_grow_to = 0;       // a row count that overflowed the capacity (grown before the retry)
@@ -680,6 +683,7 @@ struct mpid_context {
         pcount.resize(n);
         polcnt.resize(nb);
         polmask.resize(nb);
+        baremask.resize(nb);
         polstart.resize(nb + 1);
         pol_idx.resize(n);
         nl_scalars.resize(4);
@@ -883,7 +887,7 @@ struct mpid_context {
             const AtomState out{spos.p, smol.p, saxes.p, sthole.p, spol.p, spart.p, snpart.p, lab.p, labpol.p,
                                 sqrtpol.p, damp.p, aniso.p, chg.p, pd.pos.p, pd.td.p, mixed ? pf.pos.p : nullptr,
                                 mixed ? pf.lab.p : nullptr, mixed ? pf.td.p : nullptr, bmin.p, bmax.p, polmask.p,
-                                polcnt.p, nl_scalars.p, tiled_spread ? tstart.p : nullptr, 3 * (10 - tgeom.m),
+                                polcnt.p, baremask.p, nl_scalars.p, tiled_spread ? tstart.p : nullptr, 3 * (10 - tgeom.m),
                                 tgeom.ntiles, all ? nullptr : E0.p, mud.p, pd.mu.p, mixed ? pf.mu.p : nullptr};
             launch_sorted_atoms(stream, n, dbox, d_pos, in, out);
         });
@@ -925,14 +929,17 @@ struct mpid_context {
         const int nb = (n + kTile - 1) / kTile;
         return ((rows_pending ? (int)brows.n : rows_total) + nb) / 2 + 1;
     }
+    TileList tiles() const { return TileList{tile_act.p, nl_scalars.p + 2, tile_pairs.p, tile_groups_buf.p}; }
     void grow_rows(int count) {
         if ((size_t)count <= brows.n) return;
         const size_t cap = count + count / 4 + 64;
         brows.resize(cap);
         brow_owner.resize(cap);
         tile_act.resize(cap);
-        tmask.resize(cap * kTile);
-        tmaskcc.resize(cap * kTile);
+        // tiles J >= I: half of the row entries and of the diagonal
+        const size_t nb = (n + kTile - 1) / kTile, tcap = (cap + nb) / 2 + 1;
+        tile_pairs.resize(tcap * kTilePairs);
+        tile_groups_buf.resize(tcap / 2 + nb + 1);
         nmask.resize(cap * kTile);
     }
 
@@ -950,6 +957,7 @@ struct mpid_context {
                 nl_cap = std::min<int>((int)(1.3 * mean) + 64, n);
             }
         }
+        tile_group = tiles_per_group(tile_bound(), opt.precision != MPID_PRECISION_MIXED);
         for (int attempt = 0; attempt < 2; attempt++) {
             nl_cap = (nl_cap + kNlSplit - 1) / kNlSplit * kNlSplit;
             nbr.resize((size_t)n * nl_cap);
@@ -959,8 +967,9 @@ struct mpid_context {
                 launch_nl_build(stream, n, rows_pending ? (int)brows.n : rows_total, (int)brows.n, all_lists,
                                 brow_start.p, brows.p, brow_owner.p, bmin.p, bmax.p,
                                 pd.pos.p, spart.p, snpart.p, pstride, dbox, opt.cutoff * opt.cutoff, nl_cap, nmask.p,
-                                polmask.p, polstart.p, nbr.p, ncount.p, nl_scalars.p, tmask.p, pnbr.p,
-                                pcount.p, chg.p, tmaskcc.p, tile_act.p, brow_ustart.p, pol_idx.p, tgeom.ntiles,
+                                polmask.p, polstart.p, nbr.p, ncount.p, nl_scalars.p, pnbr.p,
+                                pcount.p, baremask.p, tile_act.p, tile_pairs.p,
+                                (int)(tile_pairs.n / kTilePairs), tile_groups_buf.p, tile_group, brow_ustart.p, pol_idx.p, tgeom.ntiles,
                                 tstart.p, tiled_spread ? tpstart.p : nullptr);
             });
             check_launch();
@@ -1624,11 +1633,9 @@ struct mpid_context {
         recip_cycle_induced(P);  // phidp
         // this category's events bracket the one kernel (its live time in the benchmark)
         timed(P_ELEC, [&] {
-            launch_electrostatics_pairs<R>(stream, tile_bound(), tile_act.p, nl_scalars.p + 2,
-                                           brows.p, brow_owner.p,
-                                           tmask.p, tmaskcc.p, chg.p,
-                                           pair_atoms(P), P.mu.p, pair_params<R>(), pd.pos.p, lab.p,
-                                           pair_params<double>(), force_acc(), torque_acc(), energy_acc());
+            launch_electrostatics_pairs<R>(stream, n, tile_bound(), tile_group, tiles(), brow_ustart.p, baremask.p, pair_atoms(P),
+                                           P.mu.p, pair_params<R>(), pd.pos.p, lab.p, pair_params<double>(),
+                                           force_acc(), torque_acc(), energy_acc());
         });
         timed_on(rstream, P_RECIP, [&] {
             launch_final_atoms<R>(rstream, n, opt.polarization == MPID_POLARIZATION_MUTUAL ? 1 : 0, pd.phi.p,
@@ -1797,12 +1804,9 @@ struct mpid_context {
         });
         recip_cycle_induced(P);  // phidp at every atom
         timed(P_ELEC, [&] {
-            launch_electrostatics_pot<R>(stream, tile_bound(), tile_act.p, nl_scalars.p + 2,
-                                           brows.p, brow_owner.p,
-                                         tmask.p, tmaskcc.p, chg.p,
-                                         pair_atoms(P), P.mu.p, pair_params<R>(), pd.pos.p, lab.p,
-                                         pair_params<double>(), force_acc(), torque_acc(), energy_acc(), pot_acc.p,
-                                         all_sites ? 1 : 0);
+            launch_electrostatics_pot<R>(stream, tile_bound(), tiles(), baremask.p, pair_atoms(P), P.mu.p,
+                                         pair_params<R>(), pd.pos.p, lab.p, pair_params<double>(), force_acc(),
+                                         torque_acc(), energy_acc(), pot_acc.p, all_sites ? 1 : 0);
         });
         timed_on(rstream, P_RECIP, [&] {
             launch_final_atoms<R>(rstream, n, mutual ? 1 : 0, pd.phi.p, P.phidp.p, mud.p, frac_transform<double>(),

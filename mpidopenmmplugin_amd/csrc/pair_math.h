@@ -449,13 +449,13 @@ template <class R> struct ElecOut {
 // about r (see PairParams::fix_torque).
 template <class R> MPID_HD void qi_frame(V3<R> dr, R rinv, V3<R>& ex, V3<R>& ey, V3<R>& ez) {
     ez = dr * rinv;
+    // Selects, not a branch: in the FP64 covalent-pair kernel of the gradients
+    // the compiler (ROCm 7.2) spilled ez.z^2 ahead of the join's exec restore,
+    // so that a pair along x read an older pair's.
+    const bool on_x = dr.y == R(0) && dr.z == R(0);
     const R syz2 = ez.y * ez.y + ez.z * ez.z;
-    if (dr.y != R(0) || dr.z != R(0)) {
-        const R is = rsqrt_r(syz2);
-        ex = mk(syz2 * is, -ez.x * ez.y * is, -ez.x * ez.z * is);
-    } else {
-        ex = mk(R(0), R(1), R(0));
-    }
+    const R is = rsqrt_r(on_x ? R(1) : syz2);
+    ex = mk(syz2 * is, on_x ? R(1) : -ez.x * ez.y * is, -ez.x * ez.z * is);
     ey = cross(ez, ex);
 }
 
