@@ -319,7 +319,9 @@ struct FftStage {
 };
 struct FftAxis {
     int n, nst;
+    int a, b;  // n = a b in two register steps (a <= b <= 16), 0 if n has no such split
     FastDiv nd;
+    float rn, ra, rb;  // 1 / n, 1 / a, 1 / b
     FftStage st[kFftMaxStages];
 };
 bool make_fft_axis(int n, FftAxis& ax);  // false unless n = 2^a 3^b 5^c with at most 8 stages
@@ -328,7 +330,7 @@ template <class R> struct FftPlan {
     const R2<R>* tw[3];  // per-axis twiddles exp(-2 pi i k / n), k < n
 };
 template <class R> struct ConvParams {
-    const R* infl;       // the influence function on the half spectrum, [kz][ky][kx] (launch_influence_table)
+    const R* infl;       // the influence function on the half spectrum, [kz][kx][ky] (launch_influence_table)
     const double* skip;  // the solver's stop flag in the FFT passes of a solver iteration, else null
 };
 // Inputs of the influence-function table, FP64
@@ -338,7 +340,7 @@ struct InflParams {
     double sc;                            // 1 / (pi V)
     double r00, r10, r11, r20, r21, r22;  // box^-1 (lower triangular): m = box^-1 k
 };
-// out[(kz * n1 + ky) * n0 + kx], kz < n2 / 2 + 1; moduli64: |b(k)|^2, [n0 | n1 | n2]
+// out[(kz * n0 + kx) * n1 + ky], kz < n2 / 2 + 1; moduli64: |b(k)|^2, [n0 | n1 | n2]
 template <class R> void launch_influence_table(hipStream_t s, InflParams ip, const double* moduli64, R* out);
 // Fold for tilings with W = T + 8 <= 2T in every dimension: one workgroup per
 // Morton cell sums, for each point of its T^3 core, its own window and those

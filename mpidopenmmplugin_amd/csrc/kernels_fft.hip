@@ -18,9 +18,11 @@
 // Like the reference's fftpack transforms, neither direction is normalised;
 // the convolution constants carry the scale.
 //
-// Every pass loads a batch of T lines into LDS, runs Stockham stages of radix
-// 4, 2, 3 and 5 (twiddles staged in LDS) and writes the lines back.  Index
-// arithmetic uses precomputed multiply-shift division by the stage constants.
+// An axis of n = a b points, a and b at most 16, is transformed in two register
+// steps, and planes that fit in LDS take passes 2 to 4 in one kernel.  Other
+// axes (75, 125, 135 and most above 144) load a batch of T lines into LDS and
+// run Stockham stages of radix 4, 2, 3 and 5 (twiddles staged in LDS, index
+// arithmetic by precomputed multiply-shift division).
 #include <algorithm>
 
 #include "engine.h"
@@ -305,12 +307,12 @@ __global__ __launch_bounds__(fft_threads<R>()) void k_fft_x_convolve(R2<R>* __re
     }
     __syncthreads();
     Cx<R>* res = fft_in_lds<R>(A, B, ax, T, W, R(-1));
-    // the influence function, from its table ([kz][ky][kx])
+    // the influence function, from its table ([kz][kx][ky])
     const R* gz = cp.infl + (size_t)kz * n1 * n;
     for (int idx = threadIdx.x; idx < T * n; idx += blockDim.x) {
         const int kx = idx >> Tshift, t = idx & (T - 1);
         const int y = y0 + t;
-        const R et = t < count ? gz[(size_t)y * n + kx] : R(0);
+        const R et = t < count ? gz[(size_t)kx * n1 + y] : R(0);
         Cx<R>& v = res[t * n + kx];
         v.x *= et;
         v.y *= et;
@@ -328,105 +330,8 @@ __global__ __launch_bounds__(fft_threads<R>()) void k_fft_x_convolve(R2<R>* __re
 }
 
 // ---------------------------------------------------------------------------
-// Small planes (two n0 x n1 buffers and both twiddle tables within 64 KB of
-// LDS): passes 2-4 fused, one workgroup per kz plane.  The plane is loaded as
-// n0 lines along y, transformed, transposed to n1 lines along x, transformed,
-// multiplied by the influence function (as k_fft_x_convolve), transformed
-// back along x, transposed back, transformed back along y and stored: one
-// dispatch instead of three for the grids of small systems.
-template <class R> __host__ __device__ constexpr size_t plane_small_lds(int n0, int n1) {
-    return (2 * (size_t)n0 * n1 + n0 + n1) * sizeof(Cx<R>);
-}
-constexpr size_t kPlaneSmallLds = 65536;
-
-template <class R>
-__global__ __launch_bounds__(fft_threads<R>()) void k_fft_plane_small(R2<R>* __restrict__ S, FftAxis ax0, FftAxis ax1,
-                                                                 const R2<R>* __restrict__ tw0,
-                                                                 const R2<R>* __restrict__ tw1, int n2,
-                                                                 ConvParams<R> cp) {
-    if (skipped(cp.skip)) return;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    const int n0 = ax0.n, n1 = ax1.n, np = n0 * n1;
-    Cx<R>* A = reinterpret_cast<Cx<R>*>(smem_raw);
-    Cx<R>* B = A + np;
-    Cx<R>* W0 = B + np;
-    Cx<R>* W1 = W0 + n0;
-    const int kz = blockIdx.x;
-    R2<R>* base = S + (size_t)kz * np;
-    for (int idx = threadIdx.x; idx < np; idx += blockDim.x) {
-        const R2<R> v = base[idx];
-        A[idx] = Cx<R>{v.x, v.y};
-    }
-    stage_twiddles(W0, tw0, n0);
-    stage_twiddles(W1, tw1, n1);
-    __syncthreads();
-    // y forward: n0 lines [x][y]
-    Cx<R>* res = fft_in_lds<R>(A, B, ax1, n0, W1, R(-1));
-    Cx<R>* other = (res == A) ? B : A;
-    // transpose [x][y] -> [y][x]
-    for (int idx = threadIdx.x; idx < np; idx += blockDim.x) {
-        const int x = idx / n1, y = idx - x * n1;
-        other[y * n0 + x] = res[idx];
-    }
-    __syncthreads();
-    // x forward: n1 lines [y][kx]
-    res = fft_in_lds<R>(other, res, ax0, n1, W0, R(-1));
-    // the influence function, from its table ([kz][ky][kx])
-    const R* gz = cp.infl + (size_t)kz * np;
-    for (int idx = threadIdx.x; idx < np; idx += blockDim.x) {
-        const R et = gz[idx];
-        res[idx].x *= et;
-        res[idx].y *= et;
-    }
-    __syncthreads();
-    other = (res == A) ? B : A;
-    // x backward
-    res = fft_in_lds<R>(res, other, ax0, n1, W0, R(1));
-    other = (res == A) ? B : A;
-    // transpose [y][x] -> [x][y]
-    for (int idx = threadIdx.x; idx < np; idx += blockDim.x) {
-        const int y = idx / n0, x = idx - y * n0;
-        other[x * n1 + y] = res[idx];
-    }
-    __syncthreads();
-    // y backward
-    res = fft_in_lds<R>(other, res, ax1, n0, W1, R(1));
-    for (int idx = threadIdx.x; idx < np; idx += blockDim.x) base[idx] = R2<R>{res[idx].x, res[idx].y};
-}
-
-template <class R> static bool plane_small_pass(hipStream_t s, const FftPlan<R>& p, R2<R>* S, int n2h, int n2,
-                                                ConvParams<R> cp) {
-    const int n0 = p.ax[0].n, n1 = p.ax[1].n;
-    const size_t lds = plane_small_lds<R>(n0, n1);
-    if (lds > kPlaneSmallLds) return false;
-    hipLaunchKernelGGL(k_fft_plane_small<R>, dim3(n2h), dim3(fft_threads<R>()), lds, s, S, p.ax[0], p.ax[1], p.tw[0],
-                       p.tw[1], n2, cp);
-    return true;
-}
-
+// Register transforms
 // ---------------------------------------------------------------------------
-// FP32, n0 = n1 = 128: passes 2-4 fused, one workgroup per kz plane.
-// The 128 x 128 complex plane S[kz][.][.] (128 KB) is held in LDS, and the
-// y transform, the x transform, the influence function and both inverse
-// transforms run on it without leaving the chip.  A line of 128 = 16 x 8 is
-// transformed in two register steps (four-step algorithm): 16-point DFTs at
-// stride 8 with the twiddles w^(b k1), then 8-point DFTs over contiguous
-// groups of 8, which leaves X[k1 + 16 k2] in slot 8 k1 + k2 (digit-reversed
-// order).  The influence function is applied in that order and the inverse
-// runs the steps backwards, so no permutation pass is needed.
-// LDS layout: element (x, y) at x * 152 + 9 (y / 8) + y % 8 (a pad word after
-// every group of 8 and a row pitch of 8 mod 16 complex words keep the
-// accesses of both steps, along rows and along columns, free of bank
-// conflicts).
-// ---------------------------------------------------------------------------
-namespace plane {
-constexpr int N = 128, A = 16, B = 8;
-constexpr int kThreads = 1024;
-constexpr int kPitch = (N / B) * (B + 1) + 8;  // 152
-__device__ __forceinline__ int slot(int y) { return (y >> 3) * (B + 1) + (y & 7); }
-
-typedef Cx<float> C;
-// the register steps below serve both precisions (the z passes also run in FP64)
 template <class R> __device__ __forceinline__ Cx<R> tw_s(const Cx<R>* tw, int j, R s) {
     return Cx<R>{tw[j].x, -s * tw[j].y};
 }
@@ -473,7 +378,443 @@ template <class R> __device__ __forceinline__ void dft16(Cx<R>* v, R s) {
         for (int l = 0; l < 4; l++) v[k + 4 * l] = y[l];
     }
 }
+// cos and sin of 2 pi j / N
+template <int N> struct Roots;
+template <> struct Roots<6> {
+    static constexpr double c[6] = {1.0, 0.5, -0.5, -1.0, -0.5, 0.5};
+    static constexpr double s[6] = {0.0, 0.8660254037844386, 0.8660254037844387, 0.0, -0.8660254037844384,
+                                    -0.8660254037844386};
+};
+template <> struct Roots<9> {
+    static constexpr double c[9] = {1.0, 0.766044443118978, 0.17364817766693041, -0.5, -0.9396926207859083,
+                                    -0.9396926207859084, -0.5, 0.17364817766692997, 0.7660444431189778};
+    static constexpr double s[9] = {0.0, 0.6427876096865393, 0.984807753012208, 0.8660254037844387, 0.3420201433256689,
+                                    -0.34202014332566866, -0.8660254037844384, -0.9848077530122081, -0.6427876096865396};
+};
+template <> struct Roots<10> {
+    static constexpr double c[10] = {1.0, 0.8090169943749475, 0.30901699437494745, -0.30901699437494734,
+                                    -0.8090169943749473, -1.0, -0.8090169943749476, -0.30901699437494756,
+                                    0.30901699437494723, 0.8090169943749473};
+    static constexpr double s[10] = {0.0, 0.5877852522924731, 0.9510565162951535, 0.9510565162951536, 0.5877852522924732,
+                                    0.0, -0.587785252292473, -0.9510565162951535, -0.9510565162951536, -0.5877852522924734};
+};
+template <> struct Roots<12> {
+    static constexpr double c[12] = {1.0, 0.8660254037844387, 0.5, 0.0, -0.5, -0.8660254037844387, -1.0,
+                                    -0.8660254037844388, -0.5, 0.0, 0.5, 0.8660254037844384};
+    static constexpr double s[12] = {0.0, 0.5, 0.8660254037844386, 1.0, 0.8660254037844387, 0.5, 0.0, -0.5,
+                                    -0.8660254037844384, -1.0, -0.8660254037844386, -0.5};
+};
+// P Q points from transforms of P and of Q: element Q p + q, result k + P l
+template <class R, int P, int Q> __device__ __forceinline__ void dft_composite(Cx<R>* v, R s) {
+    typedef Roots<P * Q> W;
+    Cx<R> d[Q][P];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+#pragma unroll
+        for (int p = 0; p < P; p++) d[q][p] = v[Q * p + q];
+        dft_small<R, P>(d[q], s);
+    }
+#pragma unroll
+    for (int k = 0; k < P; k++) {
+        Cx<R> y[Q];
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            y[q] = q * k == 0 ? d[q][k] : cmul(d[q][k], Cx<R>{R(W::c[q * k]), s * R(W::s[q * k])});
+        dft_small<R, Q>(y, s);
+#pragma unroll
+        for (int l = 0; l < Q; l++) v[k + P * l] = y[l];
+    }
+}
+template <class R, int N> __device__ __forceinline__ void dft_reg(Cx<R>* v, R s) {
+    if constexpr (N <= 5) dft_small<R, N>(v, s);
+    else if constexpr (N == 6) dft_composite<R, 2, 3>(v, s);
+    else if constexpr (N == 8) dft8<R>(v, s);
+    else if constexpr (N == 9) dft_composite<R, 3, 3>(v, s);
+    else if constexpr (N == 10) dft_composite<R, 2, 5>(v, s);
+    else if constexpr (N == 12) dft_composite<R, 3, 4>(v, s);
+    else dft16<R>(v, s);
+}
+template <int N> struct Radix {
+    static constexpr int n = N;
+};
+// f(Radix<n>) for the radix n of a two-step axis (uniform)
+template <class F> __device__ __forceinline__ void with_radix(int n, F f) {
+    switch (n) {
+        case 2: f(Radix<2>()); break;
+        case 3: f(Radix<3>()); break;
+        case 4: f(Radix<4>()); break;
+        case 5: f(Radix<5>()); break;
+        case 6: f(Radix<6>()); break;
+        case 8: f(Radix<8>()); break;
+        case 9: f(Radix<9>()); break;
+        case 10: f(Radix<10>()); break;
+        case 12: f(Radix<12>()); break;
+        default: f(Radix<16>()); break;
+    }
+}
 
+// ---------------------------------------------------------------------------
+// Axes of n = a b points, a and b at most 16, in two register steps (four-step
+// algorithm): a-point DFTs over elements j, j + b, ... with the twiddles
+// w^(j k1), then b-point DFTs over groups of b neighbours, which leaves
+// X[k1 + a k2] in place b k1 + k2.  The inverse runs the steps backwards, so
+// the spectrum is used in that order and never permuted.  A step reads and
+// writes LDS once where radix-4 passes need three for 64 points, with a
+// barrier each.  A place's slot in LDS leaves a word free after every group of
+// an even b, so that lanes at consecutive groups reach different banks.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int pad_group(const FftAxis& ax) { return ax.b + 1 - (ax.b & 1); }
+__host__ __device__ constexpr int line_slots(int a, int b) { return a * (b + 1 - (b & 1)); }
+
+// t / d for t below 2^20, r = 1 / d in FP32: (t + 1/2) / d lies 1 / (2 d) or more
+// from a whole number, the rounding moves it by less
+__device__ __forceinline__ int small_div(int t, float r) { return (int)(((float)t + 0.5f) * r); }
+
+// Planes that fit in LDS: passes 2-4 fused, one workgroup per kz plane, as
+// seven steps: y in two, x in two, the second of which multiplies by the
+// influence function and takes the first step of the inverse in the same
+// registers, and three back.  The first step loads the plane from global
+// memory and the last stores it there, in runs of b words.
+// What bounds it: one workgroup's latency (n2 / 2 + 1 planes leave most CUs
+// idle), that is its six barriers, LDS traffic and dependent arithmetic.
+// One plane pass and, in brackets, the passes with radix-4 stages it replaced
+// (without the gaps between them): 64 x 64 FP32 12.4 us (20), FP64 14.1 (25);
+// 24 x 24 FP32 7.5 (11), FP64 8.3 (15).
+constexpr int kPlaneThreads = 512;
+constexpr size_t kPlaneLds = 163840;
+template <class R> static size_t plane_lds(const FftAxis& x, const FftAxis& y) {
+    return ((size_t)x.n * line_slots(y.a, y.b) + x.n + y.n) * sizeof(Cx<R>);
+}
+
+template <class R>
+__global__ __launch_bounds__(kPlaneThreads) void k_fft_plane(R2<R>* __restrict__ S, FftAxis x, FftAxis y,
+                                                             const R2<R>* __restrict__ twx,
+                                                             const R2<R>* __restrict__ twy, ConvParams<R> cp) {
+    if (skipped(cp.skip)) return;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int gy = pad_group(y), pitch = y.a * gy;  // slots: a row per x place, y in padded groups
+    const int y_pad = gy - y.b, xb_pitch = x.b * pitch, infl_step = x.a * y.n;
+    Cx<R>* L = reinterpret_cast<Cx<R>*>(smem_raw);
+    Cx<R>* Wx = L + (size_t)x.n * pitch;
+    Cx<R>* Wy = Wx + x.n;
+    R2<R>* base = S + (size_t)blockIdx.x * x.n * y.n;
+    const R* infl = cp.infl + (size_t)blockIdx.x * x.n * y.n;
+    stage_twiddles(Wx, twx, x.n);
+    stage_twiddles(Wy, twy, y.n);
+    __syncthreads();
+    // step k: y a, y b, x a, x b (and back), x a, y b, y a
+    for (int k = 0; k < 7; k++) {
+        const bool col = k >= 2 && k <= 4, over_a = k == 0 || k == 2 || k == 4 || k == 6;
+        const FftAxis& ax = col ? x : y;
+        const int rad = over_a ? ax.a : ax.b, m = over_a ? ax.b : ax.a;
+        const R s = k < 4 ? R(-1) : R(1);
+        const Cx<R>* W = col ? Wx : Wy;
+        const bool twiddle = k == 0 || k == 2 || k == 3 || k == 5;
+        const int div = col ? y.n : over_a ? y.b : y.a, tasks = (col ? y.n : x.n) * m;
+        const float rdiv = col ? y.rn : over_a ? y.rb : y.ra;
+        const int step = col ? (over_a ? xb_pitch : pitch) : over_a ? gy : 1;      // between a butterfly's elements
+        const int qstep = col ? (over_a ? pitch : xb_pitch) : over_a ? 1 : gy;     // between butterflies of a line
+        with_radix(rad, [&](auto radix) {
+            constexpr int N = decltype(radix)::n;
+            for (int t = threadIdx.x; t < tasks; t += blockDim.x) {
+                // line and the butterfly's index q in it; lanes run along y.
+                // (Sums and FP32 quotients where a multiply would do: the
+                // integer one takes four times the issue slots, and the
+                // addresses are a third of a step's instructions.)
+                const int hi = small_div(t, rdiv), lo = t - __umul24(hi, div);
+                const int line = col ? lo : hi, q = col ? hi : lo;
+                const int ly = small_div(line, y.rb);  // (columns: the line's group)
+                const int at = (col ? line + __umul24(ly, y_pad) : __umul24(line, pitch)) + __umul24(q, qstep);
+                unsigned g = __umul24(line, y.n) + q;  // steps 0 and 6
+                Cx<R> v[N];
+                if (k == 0) {
+#pragma unroll
+                    for (int r = 0; r < N; r++, g += y.b) {
+                        const R2<R> e = base[g];
+                        v[r] = Cx<R>{e.x, e.y};
+                    }
+                } else {
+                    int e = at;
+#pragma unroll
+                    for (int r = 0; r < N; r++, e += step) v[r] = L[e];
+                }
+                R w = s;
+                if (k == 3) {
+                    unsigned f = __umul24(q, y.n) + ly + __umul24(y.a, line - __umul24(ly, y.b));
+                    R fv[N];
+#pragma unroll
+                    for (int r = 0; r < N; r++, f += infl_step) fv[r] = infl[f];
+                    dft_reg<R, N>(v, s);
+#pragma unroll
+                    for (int r = 0; r < N; r++) {
+                        v[r].x *= fv[r];
+                        v[r].y *= fv[r];
+                    }
+                    w = R(1);
+                }
+                dft_reg<R, N>(v, w);
+                if (k == 6) {
+#pragma unroll
+                    for (int r = 0; r < N; r++, g += y.b) base[g] = R2<R>{v[r].x, v[r].y};
+                } else {
+                    if (twiddle) {
+                        int c = q;
+#pragma unroll
+                        for (int r = 1; r < N; r++, c += q) v[r] = cmul(v[r], Cx<R>{W[c].x, -w * W[c].y});
+                    }
+                    int e = at;
+#pragma unroll
+                    for (int r = 0; r < N; r++, e += step) L[e] = v[r];
+                }
+            }
+        });
+        if (k < 6) __syncthreads();
+    }
+}
+
+template <class R>
+static bool plane_two_step(hipStream_t s, const FftPlan<R>& p, R2<R>* S, int n2h, ConvParams<R> cp) {
+    const FftAxis &x = p.ax[0], &y = p.ax[1];
+    if (!x.a || !y.a || plane_lds<R>(x, y) > kPlaneLds) return false;
+    // a thread per butterfly of the step that has most, up to kPlaneThreads (b >= a)
+    const int threads = std::min(kPlaneThreads, (std::max(x.n * y.b, y.n * x.b) + 63) / 64 * 64);
+    hipLaunchKernelGGL(k_fft_plane<R>, dim3(n2h), dim3(threads), plane_lds<R>(x, y), s, S, x, y, p.tw[0], p.tw[1], cp);
+    return true;
+}
+
+// Larger planes: the passes along y and x by the same two steps, batches of T
+// lines per workgroup through LDS.  Global memory keeps the natural order: the
+// second forward step holds X[k1 + a k2] for one k1, so lanes at consecutive k1
+// store runs of a words, and the inverse loads them so.  Bound by the grid's
+// bytes (34 MB read and written per pass at 128^3 in FP64) and by a
+// workgroup's few steps.  At 128^3 in FP64:
+// y 15.9 us (radix-4 stages 19.7), x with the convolution 17.9 (31.0).
+constexpr int kLineThreads = 256;
+constexpr int kLineBatch = 16;
+template <class R>
+__global__ __launch_bounds__(kLineThreads) void k_fft_y2(R2<R>* __restrict__ S, FftAxis ax,
+                                                         const R2<R>* __restrict__ tw, int n0, int nxb, int dir,
+                                                         const double* skip) {
+    if (skipped(skip)) return;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int n = ax.n, a = ax.a, b = ax.b, gb = pad_group(ax), pitch = a * gb;
+    Cx<R>* L = reinterpret_cast<Cx<R>*>(smem_raw);
+    Cx<R>* W = L + kLineBatch * pitch;
+    const int kz = blockIdx.x / nxb, x0 = (blockIdx.x - kz * nxb) * kLineBatch;
+    const int count = min(kLineBatch, n0 - x0);
+    R2<R>* base = S + ((size_t)kz * n0 + x0) * n;
+    stage_twiddles(W, tw, n);
+    __syncthreads();
+    const R s = (R)dir;
+    for (int k = 0; k < 2; k++) {
+        // over a (butterflies of elements j, j + b, ...: b of them), or over b
+        const bool over_a = (dir < 0) == (k == 0);
+        const int m = over_a ? b : a, step = over_a ? gb : 1, qstep = over_a ? 1 : gb;
+        const float rm = over_a ? ax.rb : ax.ra;
+        with_radix(over_a ? a : b, [&](auto radix) {
+            constexpr int N = decltype(radix)::n;
+            for (int t = threadIdx.x; t < count * m; t += kLineThreads) {
+                const int line = small_div(t, rm), q = t - __umul24(line, m);
+                const int at = __umul24(line, pitch) + __umul24(q, qstep);
+                unsigned g = __umul24(line, n) + q;
+                Cx<R> v[N];
+                if (k == 0) {
+#pragma unroll
+                    for (int r = 0; r < N; r++, g += m) {
+                        const R2<R> e = base[g];
+                        v[r] = Cx<R>{e.x, e.y};
+                    }
+                } else {
+                    int e = at;
+#pragma unroll
+                    for (int r = 0; r < N; r++, e += step) v[r] = L[e];
+                }
+                dft_reg<R, N>(v, s);
+                if (k == 0) {
+                    int c = q, e = at + step;
+                    L[at] = v[0];
+#pragma unroll
+                    for (int r = 1; r < N; r++, c += q, e += step) L[e] = cmul(v[r], Cx<R>{W[c].x, -s * W[c].y});
+                } else {
+#pragma unroll
+                    for (int r = 0; r < N; r++, g += m) base[g] = R2<R>{v[r].x, v[r].y};
+                }
+            }
+        });
+        if (k == 0) __syncthreads();
+    }
+}
+
+// The z passes by two steps: lines l, T per workgroup.  The step over a runs
+// its lanes along z in the real lines, the step over b along the lines, T
+// consecutive words of a half-spectrum plane.  dir < 0: Q -> S (with `clear` Q
+// is left zero, as by k_fft_z), else S -> Q.
+// 64^3: FP32 4.1 us (radix-4 stages 5.7), FP64 4.4 (6.6); 24^3 3.7 and 3.9 (4.9,
+// 5.2).
+template <class R>
+__global__ __launch_bounds__(kLineThreads) void k_fft_z2(R* __restrict__ Q, R2<R>* __restrict__ S, FftAxis ax,
+                                                         const R2<R>* __restrict__ tw, int nlines, int dir, int clear,
+                                                         const double* skip) {
+    if (skipped(skip)) return;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    constexpr int T = kLineBatch;
+    const int n = ax.n, a = ax.a, b = ax.b, gb = pad_group(ax), pitch = (a * gb) | 1;
+    Cx<R>* L = reinterpret_cast<Cx<R>*>(smem_raw);
+    Cx<R>* W = L + T * pitch;
+    const int l0 = blockIdx.x * T, count = min(T, nlines - l0);
+    R* real = Q + (size_t)l0 * n;
+    R2<R>* half = S + l0;
+    stage_twiddles(W, tw, n);
+    __syncthreads();
+    const R s = (R)dir;
+    for (int k = 0; k < 2; k++) {
+        const bool over_a = (dir < 0) == (k == 0);
+        const int tasks = over_a ? count * b : T * a;
+        with_radix(over_a ? a : b, [&](auto radix) {
+            constexpr int N = decltype(radix)::n;
+            for (int t = threadIdx.x; t < tasks; t += blockDim.x) {
+                const int hi = over_a ? small_div(t, ax.rb) : t / T, lo = over_a ? t - __umul24(hi, b) : t & (T - 1);
+                const int line = over_a ? hi : lo, q = over_a ? lo : hi;
+                if (line >= count) continue;
+                const int at = __umul24(line, pitch) + (over_a ? q : __umul24(q, gb)), step = over_a ? gb : 1;
+                Cx<R> v[N];
+                if (k == 1) {
+                    int e = at;
+#pragma unroll
+                    for (int r = 0; r < N; r++, e += step) v[r] = L[e];
+                } else if (over_a) {
+                    unsigned g = __umul24(line, n) + q;
+#pragma unroll
+                    for (int r = 0; r < N; r++, g += b) v[r] = Cx<R>{real[g], R(0)};
+                    if (clear) {
+                        g = __umul24(line, n) + q;
+#pragma unroll
+                        for (int r = 0; r < N; r++, g += b) real[g] = R(0);
+                    }
+                } else {
+                    int kz = q;
+#pragma unroll
+                    for (int r = 0; r < N; r++, kz += a) {
+                        const bool cj = kz > n / 2;  // the other half by Hermitian symmetry
+                        const R2<R> e = half[(size_t)(cj ? n - kz : kz) * nlines + line];
+                        v[r] = Cx<R>{e.x, cj ? -e.y : e.y};
+                    }
+                }
+                dft_reg<R, N>(v, s);
+                if (k == 0) {
+                    int c = q, e = at + step;
+                    L[at] = v[0];
+#pragma unroll
+                    for (int r = 1; r < N; r++, c += q, e += step) L[e] = cmul(v[r], Cx<R>{W[c].x, -s * W[c].y});
+                } else if (over_a) {
+                    unsigned g = __umul24(line, n) + q;
+#pragma unroll
+                    for (int r = 0; r < N; r++, g += b) real[g] = v[r].x;
+                } else {
+                    int kz = q;
+#pragma unroll
+                    for (int r = 0; r < N; r++, kz += a)
+                        if (kz <= n / 2) half[(size_t)kz * nlines + line] = R2<R>{v[r].x, v[r].y};
+                }
+            }
+        });
+        if (k == 0) __syncthreads();
+    }
+}
+
+// x forward, the influence function, x backward: three steps, the middle one
+// with both transforms over b and the multiplication in registers.  Lanes run
+// along y, T consecutive words of one kz plane.
+template <class R>
+__global__ __launch_bounds__(kLineThreads) void k_fft_x2(R2<R>* __restrict__ S, FftAxis ax,
+                                                         const R2<R>* __restrict__ tw, int n1, int nyb,
+                                                         ConvParams<R> cp) {
+    if (skipped(cp.skip)) return;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    constexpr int T = kLineBatch;
+    const int n = ax.n, a = ax.a, b = ax.b;
+    Cx<R>* L = reinterpret_cast<Cx<R>*>(smem_raw);
+    Cx<R>* W = L + T * n;
+    const int kz = blockIdx.x / nyb, y0 = (blockIdx.x - kz * nyb) * T;
+    const int count = min(T, n1 - y0);
+    R2<R>* base = S + (size_t)kz * n * n1 + y0;
+    const R* infl = cp.infl + (size_t)kz * n * n1 + y0;
+    stage_twiddles(W, tw, n);
+    __syncthreads();
+    for (int k = 0; k < 3; k++) {
+        const bool over_a = k != 1;
+        const int tasks = (over_a ? b : a) * T, step = over_a ? b * T : T, qstep = over_a ? T : b * T;
+        with_radix(over_a ? a : b, [&](auto radix) {
+            constexpr int N = decltype(radix)::n;
+            for (int t = threadIdx.x; t < tasks; t += kLineThreads) {
+                const int y = t & (T - 1), q = t / T;
+                if (y >= count) continue;
+                const int at = y + q * qstep;
+                unsigned g = __umul24(q, n1) + y;  // steps 0 and 2: elements q + b r
+                Cx<R> v[N];
+                if (k == 0) {
+#pragma unroll
+                    for (int r = 0; r < N; r++, g += b * n1) {
+                        const R2<R> e = base[g];
+                        v[r] = Cx<R>{e.x, e.y};
+                    }
+                } else {
+                    int e = at;
+#pragma unroll
+                    for (int r = 0; r < N; r++, e += step) v[r] = L[e];
+                }
+                R w = k == 2 ? R(1) : R(-1);
+                if (k == 1) {
+                    R f[N];
+                    unsigned at_f = g;  // kx = q + a r
+#pragma unroll
+                    for (int r = 0; r < N; r++, at_f += a * n1) f[r] = infl[at_f];
+                    dft_reg<R, N>(v, w);
+#pragma unroll
+                    for (int r = 0; r < N; r++) {
+                        v[r].x *= f[r];
+                        v[r].y *= f[r];
+                    }
+                    w = R(1);
+                }
+                dft_reg<R, N>(v, w);
+                if (k < 2) {
+                    int c = q, e = at + step;
+                    L[at] = v[0];
+#pragma unroll
+                    for (int r = 1; r < N; r++, c += q, e += step) L[e] = cmul(v[r], Cx<R>{W[c].x, -w * W[c].y});
+                } else {
+#pragma unroll
+                    for (int r = 0; r < N; r++, g += b * n1) base[g] = R2<R>{v[r].x, v[r].y};
+                }
+            }
+        });
+        if (k < 2) __syncthreads();
+    }
+}
+
+// ---------------------------------------------------------------------------
+// FP32, n0 = n1 = 128: passes 2-4 fused, one workgroup per kz plane.
+// The 128 x 128 complex plane S[kz][.][.] (128 KB) is held in LDS, and the
+// y transform, the x transform, the influence function and both inverse
+// transforms run on it without leaving the chip.  A line of 128 = 16 x 8 is
+// transformed in two register steps (four-step algorithm): 16-point DFTs at
+// stride 8 with the twiddles w^(b k1), then 8-point DFTs over contiguous
+// groups of 8, which leaves X[k1 + 16 k2] in slot 8 k1 + k2 (digit-reversed
+// order).  The influence function is applied in that order and the inverse
+// runs the steps backwards, so no permutation pass is needed.
+// LDS layout: element (x, y) at x * 152 + 9 (y / 8) + y % 8 (a pad word after
+// every group of 8 and a row pitch of 8 mod 16 complex words keep the
+// accesses of both steps, along rows and along columns, free of bank
+// conflicts).
+// ---------------------------------------------------------------------------
+namespace plane {
+constexpr int N = 128, A = 16, B = 8;
+constexpr int kThreads = 1024;
+constexpr int kPitch = (N / B) * (B + 1) + 8;  // 152
+__device__ __forceinline__ int slot(int y) { return (y >> 3) * (B + 1) + (y & 7); }
+
+typedef Cx<float> C;
 // address of element k of line `line`: ROW lines run along y in row x = line,
 // column lines along x in column y = line
 template <bool ROW> __device__ __forceinline__ int addr(int line, int k) {
@@ -548,14 +889,14 @@ __global__ __launch_bounds__(plane::kThreads) void k_fft_plane128_convolve(R2<fl
     __syncthreads();
     step8<false, true>(P, W, -1.f);
     __syncthreads();
-    // the influence function at (kx, ky, kz) from its table ([kz][ky][kx]),
+    // the influence function at (kx, ky, kz) from its table ([kz][kx][ky]),
     // slots in digit-reversed order
     {
         const float* gz = cp.infl + (size_t)kz * N * N;
         for (int idx = threadIdx.x; idx < N * N; idx += kThreads) {
             const int sx = idx >> 7, sy = idx & 127;
             const int kx = (sx >> 3) + A * (sx & 7), ky = (sy >> 3) + A * (sy & 7);
-            const float et = gz[ky * N + kx];
+            const float et = gz[kx * N + ky];
             C& v = P[sx * kPitch + slot(sy)];
             v.x *= et;
             v.y *= et;
@@ -636,11 +977,11 @@ __global__ __launch_bounds__(zline::threads<R>()) void k_fft_z128_r2c(R* __restr
         C v[A];
 #pragma unroll
         for (int a = 0; a < A; a++) v[a] = L[at(t, a * B + b)];
-        plane::dft16<R>(v, R(-1));
+        dft16<R>(v, R(-1));
 #pragma unroll
         for (int k1 = 0; k1 < A; k1++) {
             C r = v[k1];
-            if (b * k1 != 0) r = cmul(r, plane::tw_s<R>(W, b * k1, R(-1)));
+            if (b * k1 != 0) r = cmul(r, tw_s<R>(W, b * k1, R(-1)));
             L[at(t, k1 * B + b)] = r;
         }
     }
@@ -652,7 +993,7 @@ __global__ __launch_bounds__(zline::threads<R>()) void k_fft_z128_r2c(R* __restr
         C v[B];
 #pragma unroll
         for (int j = 0; j < B; j++) v[j] = L[at(t, k1 * B + j)];
-        plane::dft8<R>(v, R(-1));
+        dft8<R>(v, R(-1));
 #pragma unroll
         for (int k2 = 0; k2 < B; k2++) {
             const int kz = k1 + A * k2;
@@ -688,11 +1029,11 @@ __global__ __launch_bounds__(zline::threads<R>()) void k_fft_z128_c2r(R* __restr
             const R2<R> sv = S[(size_t)(cj ? N - kz : kz) * nlines + l0 + t];
             v[k2] = C{sv.x, cj ? -sv.y : sv.y};
         }
-        plane::dft8<R>(v, R(1));
+        dft8<R>(v, R(1));
 #pragma unroll
         for (int j = 0; j < B; j++) {
             C r = v[j];
-            if (j * k1 != 0) r = cmul(r, plane::tw_s<R>(W, j * k1, R(1)));
+            if (j * k1 != 0) r = cmul(r, tw_s<R>(W, j * k1, R(1)));
             L[at(t, k1 * B + j)] = r;
         }
     }
@@ -702,7 +1043,7 @@ __global__ __launch_bounds__(zline::threads<R>()) void k_fft_z128_c2r(R* __restr
         C v[A];
 #pragma unroll
         for (int k1 = 0; k1 < A; k1++) v[k1] = L[at(t, k1 * B + b)];
-        plane::dft16<R>(v, R(1));
+        dft16<R>(v, R(1));
 #pragma unroll
         for (int a = 0; a < A; a++) L[at(t, a * B + b)] = v[a];
     }
@@ -749,6 +1090,18 @@ bool make_fft_axis(int n, FftAxis& ax) {
         ax.st[k].twstep = n / (Ns * rad[k]);
         Ns *= rad[k];
     }
+    // two register steps, the most even split (b the larger: runs of b words)
+    ax.a = ax.b = 0;
+    static const int steps[] = {2, 3, 4, 5, 6, 8, 9, 10, 12, 16};
+    for (int a : steps)
+        for (int b : steps)
+            if (a * b == n && a <= b) {
+                ax.a = a;
+                ax.b = b;
+            }
+    ax.rn = 1.0f / (float)n;
+    ax.ra = 1.0f / (float)std::max(ax.a, 1);
+    ax.rb = 1.0f / (float)std::max(ax.b, 1);
     return true;
 }
 
@@ -767,19 +1120,27 @@ static int log2i(int v) {
 }
 template <class R> static size_t fft_lds(int T, int n) { return (2 * (size_t)T * n + n) * sizeof(R2<R>); }
 
-// the z passes with the register-step kernels where they apply (n2 = 128,
-// whole batches of 64 lines in FP32, 32 in FP64)
+// the z passes with the register-step kernels where they apply: the ones for
+// n2 = 128 and whole batches of 64 lines in FP32, 32 in FP64, or the general one
 template <class R>
 static bool zline_pass(hipStream_t s, const FftPlan<R>& p, R* Q, R2<R>* S, int dir, int clear, const double* skip) {
     constexpr int T = zline::lines<R>();
     const int nlines = p.ax[0].n * p.ax[1].n;
-    if (p.ax[2].n != zline::N || nlines % T != 0) return false;
-    if (dir < 0)
-        hipLaunchKernelGGL(k_fft_z128_r2c<R>, dim3(nlines / T), dim3(zline::threads<R>()), 0, s, Q, S, p.tw[2], nlines,
-                           clear, skip);
-    else
-        hipLaunchKernelGGL(k_fft_z128_c2r<R>, dim3(nlines / T), dim3(zline::threads<R>()), 0, s, Q, S, p.tw[2], nlines,
-                           skip);
+    const FftAxis& z = p.ax[2];
+    if (z.n == zline::N && nlines % T == 0) {
+        if (dir < 0)
+            hipLaunchKernelGGL(k_fft_z128_r2c<R>, dim3(nlines / T), dim3(zline::threads<R>()), 0, s, Q, S, p.tw[2],
+                               nlines, clear, skip);
+        else
+            hipLaunchKernelGGL(k_fft_z128_c2r<R>, dim3(nlines / T), dim3(zline::threads<R>()), 0, s, Q, S, p.tw[2],
+                               nlines, skip);
+        return true;
+    }
+    if (!z.a) return false;
+    const int threads = std::min(kLineThreads, (kLineBatch * z.b + 63) / 64 * 64);
+    hipLaunchKernelGGL(k_fft_z2<R>, dim3((nlines + kLineBatch - 1) / kLineBatch), dim3(threads),
+                       (kLineBatch * (line_slots(z.a, z.b) | 1) + z.n) * sizeof(Cx<R>), s, Q, S, z, p.tw[2], nlines, dir,
+                       clear, skip);
     return true;
 }
 
@@ -822,7 +1183,7 @@ __global__ void k_influence_table(InflParams ip, const double* __restrict__ mod,
     const size_t total = (size_t)n2h * n1 * n0;
     for (size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
          idx += (size_t)gridDim.x * blockDim.x) {
-        const int kx = (int)(idx % n0), ky = (int)((idx / n0) % n1), kz = (int)(idx / ((size_t)n0 * n1));
+        const int ky = (int)(idx % n1), kx = (int)((idx / n1) % n0), kz = (int)(idx / ((size_t)n0 * n1));
         const double g = influence_at(kx, ky, kz, ip, mod);
         const double gm = influence_at((n0 - kx) % n0, (n1 - ky) % n1, (n2 - kz) % n2, ip, mod);
         out[idx] = (R)(0.5 * (g + gm));
@@ -850,16 +1211,32 @@ void launch_recip_convolution(hipStream_t s, const FftPlan<R>& p, R* Q, R2<R>* S
     if (!zline_pass<R>(s, p, Q, S, -1, clear, cp.skip))
         hipLaunchKernelGGL(k_fft_z<R>, dim3((nlines + Tz - 1) / Tz), dim3(fft_threads<R>()), fft_lds<R>(Tz, n2), s, Q,
                            S, p.ax[2], Tz, log2i(Tz), p.tw[2], nlines, -1, clear, cp.skip);
-    if (!plane_pass<R>(s, p, S, n2h, n2, cp) && !plane_small_pass<R>(s, p, S, n2h, n2, cp)) {
+    if (!plane_pass<R>(s, p, S, n2h, n2, cp) && !plane_two_step<R>(s, p, S, n2h, cp)) {
         // 2. y forward
-        hipLaunchKernelGGL(k_fft_y<R>, dim3(n2h * nxb), dim3(fft_threads<R>()), fft_lds<R>(Ty, n1), s, S, p.ax[1], Ty,
-                           p.tw[1], n0, nxb, -1, cp.skip);
+        auto along_y = [&](int dir) {
+            const FftAxis& y = p.ax[1];
+            if (y.a) {
+                const int nb = (n0 + kLineBatch - 1) / kLineBatch;
+                hipLaunchKernelGGL(k_fft_y2<R>, dim3(n2h * nb), dim3(kLineThreads),
+                                   (kLineBatch * line_slots(y.a, y.b) + n1) * sizeof(Cx<R>), s, S, y, p.tw[1], n0, nb,
+                                   dir, cp.skip);
+            } else {
+                hipLaunchKernelGGL(k_fft_y<R>, dim3(n2h * nxb), dim3(fft_threads<R>()), fft_lds<R>(Ty, n1), s, S, y, Ty,
+                                   p.tw[1], n0, nxb, dir, cp.skip);
+            }
+        };
+        along_y(-1);
         // 3. x forward, convolution, x backward
-        hipLaunchKernelGGL(k_fft_x_convolve<R>, dim3(n2h * nyb), dim3(fft_threads<R>()), fft_lds<R>(Tx, n0), s, S,
-                           p.ax[0], Tx, log2i(Tx), p.tw[0], n1, n2, nyb, cp);
+        if (p.ax[0].a) {
+            const int nb = (n1 + kLineBatch - 1) / kLineBatch;
+            hipLaunchKernelGGL(k_fft_x2<R>, dim3(n2h * nb), dim3(kLineThreads),
+                               (kLineBatch + 1) * n0 * sizeof(Cx<R>), s, S, p.ax[0], p.tw[0], n1, nb, cp);
+        } else {
+            hipLaunchKernelGGL(k_fft_x_convolve<R>, dim3(n2h * nyb), dim3(fft_threads<R>()), fft_lds<R>(Tx, n0), s, S,
+                               p.ax[0], Tx, log2i(Tx), p.tw[0], n1, n2, nyb, cp);
+        }
         // 4. y backward
-        hipLaunchKernelGGL(k_fft_y<R>, dim3(n2h * nxb), dim3(fft_threads<R>()), fft_lds<R>(Ty, n1), s, S, p.ax[1], Ty,
-                           p.tw[1], n0, nxb, 1, cp.skip);
+        along_y(1);
     }
     // 5. z backward
     if (!zline_pass<R>(s, p, V, S, 1, 0, cp.skip))
