@@ -194,6 +194,7 @@ void launch_torque_to_force(hipStream_t s, int n, Box<double> box, const double4
                             const acc_t* torque, acc_t* force, int exact_threefold);
 void launch_output_forces(hipStream_t s, int n, const int* perm, const acc_t* force, double* out, int accumulate,
                           const acc_t* energy, acc_t* esum, const double* gate);
+void launch_copy(hipStream_t s, int count, const double* in, double* out);  // count >= 1 words
 void launch_unpermute3(hipStream_t s, int n, const int* perm, const double* in, double* out);
 void launch_zero_acc(hipStream_t s, acc_t* p, size_t count);
 size_t sort_temp_bytes(int n);

@@ -1182,6 +1182,11 @@ __global__ __launch_bounds__(256) void k_output_forces(int n, const int* __restr
     }
 }
 
+__global__ void k_copy(int count, const double* __restrict__ in, double* __restrict__ out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < count) out[i] = in[i];
+}
+
 __global__ void k_unpermute3(int n, const int* __restrict__ perm, const double* __restrict__ in, double* out) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
@@ -1269,6 +1274,9 @@ void launch_output_forces(hipStream_t s, int n, const int* perm, const acc_t* fo
                           const acc_t* energy, acc_t* esum, const double* gate) {
     hipLaunchKernelGGL(k_output_forces, out ? blocks_for(n, 256) : dim3(1), dim3(256), 0, s, n, perm, force, out,
                        accumulate, energy, esum, gate);
+}
+void launch_copy(hipStream_t s, int count, const double* in, double* out) {
+    hipLaunchKernelGGL(k_copy, blocks_for(count, 256), dim3(256), 0, s, count, in, out);
 }
 void launch_unpermute3(hipStream_t s, int n, const int* perm, const double* in, double* out) {
     hipLaunchKernelGGL(k_unpermute3, blocks_for(n, 256), dim3(256), 0, s, n, perm, in, out);
