@@ -261,31 +261,39 @@ __global__ __launch_bounds__(256) void k_spread_tiled(const R4<R>* __restrict__ 
 // copy of the core and writes the core to the grid once.  No scratch, no
 // fold and no clearing of the grid: every point is written by its owner.
 // ---------------------------------------------------------------------------
-// candidate atoms examined per pass (the slots of their spline weights in LDS)
-template <class R, int MODE> constexpr int owner_cand() { return MODE == 0 ? 64 : 128; }
+//
+// Every thread tests one candidate per pass; the atoms that meet the core then
+// take their spline weights in chunks of kOwnerChunk, one wavefront per axis and
+// the fourth for the source and the count of stencil rows, so that a chunk's
+// chain is one spline and not three.  A core is a chain of dependent loads and
+// short steps, and what bounds the kernel is how many cores a CU holds (LDS and
+// registers) and the length of that chain.  Induced dipoles, 98,304 atoms on
+// 128^3: FP64 73 us with one wavefront taking all three splines of 128
+// candidates, 56 so; FP32 37 and 33; 12,288 atoms on 64^3 FP32 12 and 9.
+constexpr int kOwnerChunk = 64;
 // stencil rows (of 6) along an axis inside a core of T points, for a stencil
 // starting at r relative to the core (r in [-5, T - 1] for a stencil that meets it)
 __device__ __forceinline__ int owner_rows(int r, int T) { return min(kOrder, T - r) - max(0, -r); }
 
 template <class R, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_spread_owner(const R4<R>* __restrict__ pos, const R* __restrict__ src,
-                                                      PmeGeom<R> g, TileGeom tg, const int* __restrict__ atoms,
-                                                      const int* __restrict__ tstart, const int* __restrict__ tend,
-                                                      R* __restrict__ grid) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ? 3 : 4))) void k_spread_owner(
+    const R4<R>* __restrict__ pos, const R* __restrict__ src, PmeGeom<R> g, TileGeom tg, const int* __restrict__ atoms,
+    const int* __restrict__ tstart, const int* __restrict__ tend, R* __restrict__ grid) {
     if (skipped(g.skip)) return;
     constexpr int ND = MODE == 0 ? 3 : 1;   // spline derivatives needed
     constexpr int NC = MODE == 0 ? 20 : 3;  // fractional components
-    constexpr int kOwnerCand = owner_cand<R, MODE>();
+    constexpr int kCand = 256;              // candidates per pass, one per thread
+    static_assert(kOwnerChunk == kTile && kCand == 4 * kTile, "a wavefront per axis, and one for the source");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int T0 = tg.T[0], T1 = tg.T[1], T2 = tg.T[2];
     const int TV = T0 * T1 * T2;
     double* core = reinterpret_cast<double*>(smem_raw);
-    R* sth = reinterpret_cast<R*>(core + TV);                       // [kOwnerCand][3][6][ND+1]
-    R* smf = sth + kOwnerCand * 3 * kOrder * (ND + 1);              // [kOwnerCand][NC]
-    int* srel = reinterpret_cast<int*>(smf + kOwnerCand * NC);      // [kOwnerCand][3] stencil start - core origin
-    __shared__ int sbeg[8], send_[8], soff[9], snv, snrows;
-    __shared__ int sfirst[kOwnerCand];
-    static_assert(kOwnerCand % kTile == 0 && kOwnerCand <= 256, "slots: whole wavefronts, at most the block");
+    R* sth = reinterpret_cast<R*>(core + TV);            // [kOwnerChunk][3][6][ND+1]
+    R* smf = sth + kOwnerChunk * 3 * kOrder * (ND + 1);  // [kOwnerChunk][NC]
+    __shared__ int sbeg[8], soff[9], snv;
+    // the atoms that meet the core: stencil start - core origin (+ 8 per byte), atom, first stencil row
+    __shared__ int srel[kCand], satom[kCand], sfirst[kCand + 1];
+    const int tid = threadIdx.x, lane = tid & (kTile - 1), wave = tid / kTile;
     const int t = blockIdx.x;
     const int nt = tg.tiles_per_axis;
     const int c[3] = {(int)compact_bits((unsigned)t >> 2), (int)compact_bits((unsigned)t >> 1),
@@ -293,151 +301,149 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     int w0[3];
 #pragma unroll
     for (int k = 0; k < 3; k++) w0[k] = ((c[k] * tg.T[k] + (g.n[k] >> 1) - 6) % g.n[k] + g.n[k]) % g.n[k];
-    for (int i = threadIdx.x; i < TV; i += blockDim.x) core[i] = 0.0;
-    if (threadIdx.x < 8) {
-        const int d = threadIdx.x;
-        const unsigned tx = (unsigned)((c[0] - ((d >> 2) & 1) + nt) % nt),
-                       ty = (unsigned)((c[1] - ((d >> 1) & 1) + nt) % nt), tz = (unsigned)((c[2] - (d & 1) + nt) % nt);
+    if (tid < 8) {
+        const unsigned tx = (unsigned)((c[0] - ((tid >> 2) & 1) + nt) % nt),
+                       ty = (unsigned)((c[1] - ((tid >> 1) & 1) + nt) % nt), tz = (unsigned)((c[2] - (tid & 1) + nt) % nt);
         const unsigned tile = (spread_bits_pme(tx) << 2) | (spread_bits_pme(ty) << 1) | spread_bits_pme(tz);
-        sbeg[d] = tstart[tile];
-        send_[d] = tend[tile];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        // cells c - 1 and c coincide only with one cell per axis: count each cell once
-        int o = 0;
-        for (int d = 0; d < 8; d++) {
-            bool dup = false;
-            for (int e = 0; e < d; e++) dup = dup || (sbeg[e] == sbeg[d] && send_[e] == send_[d] && send_[d] > sbeg[d]);
-            soff[d] = o;
-            if (!dup) o += max(0, send_[d] - sbeg[d]);
-            else send_[d] = sbeg[d];
+        const int beg = tstart[tile];
+        // cells c - 1 and c coincide with one cell per axis only: count it once
+        int o = nt == 1 && tid > 0 ? 0 : max(0, tend[tile] - beg);
+#pragma unroll
+        for (int off = 1; off < 8; off <<= 1) {
+            const int v = __shfl_up(o, off);
+            if (tid >= off) o += v;
         }
-        soff[8] = o;
+        sbeg[tid] = beg;
+        soff[tid + 1] = o;
+        if (tid == 0) soff[0] = snv = 0;
     }
+    for (int i = tid; i < TV; i += blockDim.x) core[i] = 0.0;
     __syncthreads();
     const int ncand = soff[8];
-    for (int c0 = 0; c0 < ncand; c0 += kOwnerCand) {
-        if (threadIdx.x == 0) snv = 0;
-        __syncthreads();
-        if ((int)threadIdx.x < kOwnerCand && c0 + (int)threadIdx.x < ncand) {
-            const int q = c0 + threadIdx.x;
+    for (int c0 = 0; c0 < ncand; c0 += kCand) {
+        if (c0 + tid < ncand) {
+            const int q = c0 + tid;
             int d = 0;
-            while (soff[d + 1] <= q) d++;
+#pragma unroll
+            for (int k = 1; k < 8; k++) d += soff[k] <= q ? 1 : 0;
             const int s = sbeg[d] + (q - soff[d]);
             const int a = atoms ? atoms[s] : s;
             const R4<R> p = pos[a];
             const V3<R> fp = to_frac(mk(p.x, p.y, p.z), g.box);
             const R px[3] = {fp.x, fp.y, fp.z};
-            int ig[3], rel[3];
-            R w[3];
+            int rel = 0;
             bool meets = true;
 #pragma unroll
             for (int k = 0; k < 3; k++) {
-                grid_coord(px[k], g.n[k], ig[k], w[k]);
-                int r = ig[k] - w0[k];
+                int ig;
+                R w;
+                grid_coord(px[k], g.n[k], ig, w);
+                int r = ig - w0[k];
                 if (r < -(g.n[k] >> 1)) r += g.n[k];
                 if (r >= g.n[k] - (g.n[k] >> 1)) r -= g.n[k];
-                rel[k] = r;
+                rel |= (r + 8) << (8 * k);
                 meets = meets && r + kOrder - 1 >= 0 && r < tg.T[k];
             }
             if (meets) {
                 const int slot = atomicAdd(&snv, 1);
-#pragma unroll
-                for (int k = 0; k < 3; k++) {
-                    R th[kOrder][ND + 1];
-                    bspline6<R, ND>(w[k], th);
-                    for (int m = 0; m < kOrder; m++)
-                        for (int r = 0; r <= ND; r++) sth[((slot * 3 + k) * kOrder + m) * (ND + 1) + r] = th[m][r];
-                    srel[slot * 3 + k] = rel[k];
-                }
-                R* mf = smf + slot * NC;
-                    if (MODE == 0) {
-                    frac_moments(src + (size_t)a * kMP, g.A, mf);
-                } else {
-                    const V3<R> uf =
-                        frac_vector(mk(src[3 * (size_t)a], src[3 * (size_t)a + 1], src[3 * (size_t)a + 2]), g.A);
-                    mf[0] = uf.x;
-                    mf[1] = uf.y;
-                    mf[2] = uf.z;
-                }
+                srel[slot] = rel;
+                satom[slot] = a;
             }
         }
         __syncthreads();
         const int nv = snv;
-        // The listed atoms' stencil rows (iy, iz) inside the core, numbered
-        // atom by atom (sfirst[la]: the first row of atom la), so that every
-        // thread's item below is a row with points to add: about 14 of an
-        // atom's 36 rows meet the core (T = 8).  One wavefront counts them.
-        if (threadIdx.x < kTile) {
-            int cnt[kOwnerCand / kTile], inc[kOwnerCand / kTile];
+        for (int s0 = 0; s0 < nv; s0 += kOwnerChunk) {
+            const int la = s0 + lane;
+            if (wave < 3) {
+                if (la < nv) {
+                    const R4<R> p = pos[satom[la]];
+                    const V3<R> fp = to_frac(mk(p.x, p.y, p.z), g.box);
+                    int ig;
+                    R w, th[kOrder][ND + 1];
+                    grid_coord(wave == 0 ? fp.x : wave == 1 ? fp.y : fp.z, g.n[wave], ig, w);
+                    bspline6<R, ND>(w, th);
+                    R* o = sth + (lane * 3 + wave) * kOrder * (ND + 1);
 #pragma unroll
-            for (int h = 0; h < kOwnerCand / kTile; h++) {
-                const int la = h * kTile + (int)threadIdx.x;
-                cnt[h] = la < nv ? owner_rows(srel[la * 3 + 1], T1) * owner_rows(srel[la * 3 + 2], T2) : 0;
-                inc[h] = cnt[h];
-            }
+                    for (int m = 0; m < kOrder; m++)
 #pragma unroll
-            for (int off = 1; off < kTile; off <<= 1) {
+                        for (int r = 0; r <= ND; r++) o[m * (ND + 1) + r] = th[m][r];
+                }
+            } else {
+                // The atoms' stencil rows (iy, iz) inside the core, numbered atom
+                // by atom, so that every thread's item below is a row with points
+                // to add: about 14 of an atom's 36 rows meet the core (T = 8).
+                int cnt = 0;
+                if (la < nv) {
+                    const int rel = srel[la];
+                    cnt = owner_rows(((rel >> 8) & 0xff) - 8, T1) * owner_rows((rel >> 16) - 8, T2);
+                }
+                int inc = cnt;
 #pragma unroll
-                for (int h = 0; h < kOwnerCand / kTile; h++) {
-                    const int v = __shfl_up(inc[h], off);
-                    if ((int)threadIdx.x >= off) inc[h] += v;
+                for (int off = 1; off < kTile; off <<= 1) {
+                    const int v = __shfl_up(inc, off);
+                    if (lane >= off) inc += v;
+                }
+                sfirst[lane + 1] = inc;
+                if (lane == 0) sfirst[0] = 0;
+                if (la < nv) {
+                    R* mf = smf + lane * NC;
+                    const size_t a = satom[la];
+                    if (MODE == 0) {
+                        frac_moments(src + a * kMP, g.A, mf);
+                    } else {
+                        const V3<R> uf = frac_vector(mk(src[3 * a], src[3 * a + 1], src[3 * a + 2]), g.A);
+                        mf[0] = uf.x;
+                        mf[1] = uf.y;
+                        mf[2] = uf.z;
+                    }
                 }
             }
-            int base = 0;
+            __syncthreads();
+            const int nrows = sfirst[kOwnerChunk];
+            // one item = (atom, iy, iz): the points of the stencil row along x inside the core
+            for (int it = tid; it < nrows; it += blockDim.x) {
+                int la = 0;  // the last slot with sfirst[la] <= it (every atom has a row)
 #pragma unroll
-            for (int h = 0; h < kOwnerCand / kTile; h++) {
-                const int la = h * kTile + (int)threadIdx.x;
-                if (la < nv) sfirst[la] = base + inc[h] - cnt[h];
-                base += __shfl(inc[h], kTile - 1);
+                for (int step = kOwnerChunk / 2; step >= 1; step >>= 1)
+                    if (sfirst[la + step] <= it) la += step;
+                const int rel = srel[s0 + la];
+                const int rx = (rel & 0xff) - 8, ry = ((rel >> 8) & 0xff) - 8, rz = (rel >> 16) - 8;
+                const int y0 = max(0, -ry), z0 = max(0, -rz);
+                const int nz = min(kOrder, T2 - rz) - z0;
+                const int loc = it - sfirst[la], dy = (int)(((float)loc + 0.5f) / (float)nz);
+                const int iy = y0 + dy, iz = z0 + (loc - dy * nz);
+                const int ly = ry + iy, lz = rz + iz;
+                const R* tx = sth + ((la * 3 + 0) * kOrder) * (ND + 1);
+                const R* ty = sth + ((la * 3 + 1) * kOrder + iy) * (ND + 1);
+                const R* tz = sth + ((la * 3 + 2) * kOrder + iz) * (ND + 1);
+                const R* mf = smf + la * NC;
+                R t0, t1, t2 = R(0), t3 = R(0);
+                if (MODE == 0) {
+                    const R u0 = ty[0], u1 = ty[1], u2 = ty[2], u3 = ty[ND >= 3 ? 3 : 0];
+                    const R v0 = tz[0], v1 = tz[1], v2 = tz[2], v3 = tz[ND >= 3 ? 3 : 0];
+                    t0 = mf[0] * u0 * v0 + mf[2] * u1 * v0 + mf[3] * u0 * v1 + mf[7] * u2 * v0 + mf[9] * u0 * v2 +
+                         mf[8] * u1 * v1 + mf[16] * u3 * v0 + mf[17] * u2 * v1 + mf[18] * u1 * v2 + mf[19] * u0 * v3;
+                    t1 = mf[1] * u0 * v0 + mf[5] * u1 * v0 + mf[6] * u0 * v1 + mf[13] * u2 * v0 + mf[14] * u1 * v1 +
+                         mf[15] * u0 * v2;
+                    t2 = mf[4] * u0 * v0 + mf[11] * u1 * v0 + mf[12] * u0 * v1;
+                    t3 = mf[10] * u0 * v0;
+                } else {
+                    t0 = mf[1] * ty[1] * tz[0] + mf[2] * ty[0] * tz[1];
+                    t1 = mf[0] * ty[0] * tz[0];
+                }
+#pragma unroll
+                for (int ix = 0; ix < kOrder; ix++) {
+                    const int lx = rx + ix;
+                    if (lx < 0 || lx >= T0) continue;
+                    R v = t0 * tx[ix * (ND + 1)] + t1 * tx[ix * (ND + 1) + 1];
+                    if (MODE == 0) v += t2 * tx[ix * (ND + 1) + 2] + t3 * tx[ix * (ND + 1) + ND];
+                    atomicAdd(&core[(lx * T1 + ly) * T2 + lz], (double)v);
+                }
             }
-            if (threadIdx.x == 0) snrows = base;
+            __syncthreads();
         }
-        __syncthreads();
-        const int nrows = snrows;
-        // one item = (atom, iy, iz): the points of the stencil row along x inside the core
-        for (int it = threadIdx.x; it < nrows; it += blockDim.x) {
-            // the atom: the last la with sfirst[la] <= it (every atom has a row)
-            int la = 0;
-#pragma unroll
-            for (int step = kOwnerCand / 2; step >= 1; step >>= 1)
-                if (la + step < nv && sfirst[la + step] <= it) la += step;
-            const int ry = srel[la * 3 + 1], rz = srel[la * 3 + 2];
-            const int y0 = max(0, -ry), z0 = max(0, -rz);
-            const int nz = min(kOrder, T2 - rz) - z0;
-            const int loc = it - sfirst[la], dy = loc / nz;
-            const int iy = y0 + dy, iz = z0 + (loc - dy * nz);
-            const int ly = ry + iy, lz = rz + iz;
-            const R* tx = sth + ((la * 3 + 0) * kOrder) * (ND + 1);
-            const R* ty = sth + ((la * 3 + 1) * kOrder + iy) * (ND + 1);
-            const R* tz = sth + ((la * 3 + 2) * kOrder + iz) * (ND + 1);
-            const R* mf = smf + la * NC;
-            R t0, t1, t2 = R(0), t3 = R(0);
-            if (MODE == 0) {
-                const R u0 = ty[0], u1 = ty[1], u2 = ty[2], u3 = ty[ND >= 3 ? 3 : 0];
-                const R v0 = tz[0], v1 = tz[1], v2 = tz[2], v3 = tz[ND >= 3 ? 3 : 0];
-                t0 = mf[0] * u0 * v0 + mf[2] * u1 * v0 + mf[3] * u0 * v1 + mf[7] * u2 * v0 + mf[9] * u0 * v2 +
-                     mf[8] * u1 * v1 + mf[16] * u3 * v0 + mf[17] * u2 * v1 + mf[18] * u1 * v2 + mf[19] * u0 * v3;
-                t1 = mf[1] * u0 * v0 + mf[5] * u1 * v0 + mf[6] * u0 * v1 + mf[13] * u2 * v0 + mf[14] * u1 * v1 +
-                     mf[15] * u0 * v2;
-                t2 = mf[4] * u0 * v0 + mf[11] * u1 * v0 + mf[12] * u0 * v1;
-                t3 = mf[10] * u0 * v0;
-            } else {
-                t0 = mf[1] * ty[1] * tz[0] + mf[2] * ty[0] * tz[1];
-                t1 = mf[0] * ty[0] * tz[0];
-            }
-            const int lx0 = srel[la * 3 + 0];
-#pragma unroll
-            for (int ix = 0; ix < kOrder; ix++) {
-                const int lx = lx0 + ix;
-                if (lx < 0 || lx >= T0) continue;
-                R v = t0 * tx[ix * (ND + 1)] + t1 * tx[ix * (ND + 1) + 1];
-                if (MODE == 0) v += t2 * tx[ix * (ND + 1) + 2] + t3 * tx[ix * (ND + 1) + ND];
-                atomicAdd(&core[(lx * T1 + ly) * T2 + lz], (double)v);
-            }
-        }
-        __syncthreads();
+        if (tid == 0) snv = 0;
+        if (c0 + kCand < ncand) __syncthreads();
     }
     for (int i = threadIdx.x; i < TV; i += blockDim.x) {
         const int lx = i / (T1 * T2), rem = i - lx * T1 * T2;
@@ -763,14 +769,13 @@ void launch_spread_induced_tiled(hipStream_t s, const R4<R>* pos, const R* mu, P
 template <class R, int MODE> static size_t owner_lds(const TileGeom& tg) {
     constexpr int ND = MODE == 0 ? 3 : 1;
     constexpr int NC = MODE == 0 ? 20 : 3;
-    constexpr int K = owner_cand<R, MODE>();
-    return (size_t)tg.T[0] * tg.T[1] * tg.T[2] * sizeof(double) + K * (3 * kOrder * (ND + 1) + NC) * sizeof(R) +
-           K * 3 * sizeof(int);
+    return (size_t)tg.T[0] * tg.T[1] * tg.T[2] * sizeof(double) +
+           kOwnerChunk * (3 * kOrder * (ND + 1) + NC) * sizeof(R);
 }
 bool spread_by_owner(const TileGeom& tg) {
     for (int k = 0; k < 3; k++)
         if (tg.T[k] < 8) return false;
-    return owner_lds<double, 0>(tg) <= 65536;
+    return owner_lds<double, 0>(tg) + kOwnerChunk * 3 * sizeof(int) <= 65536;  // (T <= 13: three bytes hold a start)
 }
 template <class R>
 void launch_spread_fixed_owner(hipStream_t s, const R4<R>* pos, const R* lab, PmeGeom<R> g, TileGeom tg,
