@@ -271,6 +271,10 @@ __global__ __launch_bounds__(256) void k_spread_tiled(const R4<R>* __restrict__ 
 // 128^3: FP64 73 us with one wavefront taking all three splines of 128
 // candidates, 56 so; FP32 37 and 33; 12,288 atoms on 64^3 FP32 12 and 9.
 constexpr int kOwnerChunk = 64;
+// words of a slot's spline weights and source components: odd, so that lanes at
+// different slots read different LDS banks
+template <int MODE> constexpr int owner_weights() { return 3 * kOrder * (MODE == 0 ? 4 : 2) + 1; }
+template <int MODE> constexpr int owner_source() { return MODE == 0 ? 21 : 3; }
 // stencil rows (of 6) along an axis inside a core of T points, for a stencil
 // starting at r relative to the core (r in [-5, T - 1] for a stencil that meets it)
 __device__ __forceinline__ int owner_rows(int r, int T) { return min(kOrder, T - r) - max(0, -r); }
@@ -281,15 +285,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ?
     const int* __restrict__ tstart, const int* __restrict__ tend, R* __restrict__ grid) {
     if (skipped(g.skip)) return;
     constexpr int ND = MODE == 0 ? 3 : 1;   // spline derivatives needed
-    constexpr int NC = MODE == 0 ? 20 : 3;  // fractional components
+    constexpr int NW = owner_weights<MODE>(), NC = owner_source<MODE>();
     constexpr int kCand = 256;              // candidates per pass, one per thread
     static_assert(kOwnerChunk == kTile && kCand == 4 * kTile, "a wavefront per axis, and one for the source");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int T0 = tg.T[0], T1 = tg.T[1], T2 = tg.T[2];
     const int TV = T0 * T1 * T2;
     double* core = reinterpret_cast<double*>(smem_raw);
-    R* sth = reinterpret_cast<R*>(core + TV);            // [kOwnerChunk][3][6][ND+1]
-    R* smf = sth + kOwnerChunk * 3 * kOrder * (ND + 1);  // [kOwnerChunk][NC]
+    R* sth = reinterpret_cast<R*>(core + TV);            // [kOwnerChunk][NW]: [3][6][ND+1]
+    R* smf = sth + kOwnerChunk * NW;  // [kOwnerChunk][NC]
     __shared__ int sbeg[8], soff[9], snv;
     // the atoms that meet the core: stencil start - core origin (+ 8 per byte), atom, first stencil row
     __shared__ int srel[kCand], satom[kCand], sfirst[kCand + 1];
@@ -362,7 +366,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ?
                     R w, th[kOrder][ND + 1];
                     grid_coord(wave == 0 ? fp.x : wave == 1 ? fp.y : fp.z, g.n[wave], ig, w);
                     bspline6<R, ND>(w, th);
-                    R* o = sth + (lane * 3 + wave) * kOrder * (ND + 1);
+                    R* o = sth + lane * NW + wave * kOrder * (ND + 1);
 #pragma unroll
                     for (int m = 0; m < kOrder; m++)
 #pragma unroll
@@ -413,9 +417,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ?
                 const int loc = it - sfirst[la], dy = (int)(((float)loc + 0.5f) / (float)nz);
                 const int iy = y0 + dy, iz = z0 + (loc - dy * nz);
                 const int ly = ry + iy, lz = rz + iz;
-                const R* tx = sth + ((la * 3 + 0) * kOrder) * (ND + 1);
-                const R* ty = sth + ((la * 3 + 1) * kOrder + iy) * (ND + 1);
-                const R* tz = sth + ((la * 3 + 2) * kOrder + iz) * (ND + 1);
+                const R* tx = sth + la * NW;
+                const R* ty = tx + (kOrder + iy) * (ND + 1);
+                const R* tz = tx + (2 * kOrder + iz) * (ND + 1);
                 const R* mf = smf + la * NC;
                 R t0, t1, t2 = R(0), t3 = R(0);
                 if (MODE == 0) {
@@ -767,15 +771,13 @@ void launch_spread_induced_tiled(hipStream_t s, const R4<R>* pos, const R* mu, P
     k_spread_tiled<R, 1><<<dim3(tg.ntiles), dim3(256), shm, s>>>(pos, mu, g, tg, atoms, tstart, tend, scratch, grid);
 }
 template <class R, int MODE> static size_t owner_lds(const TileGeom& tg) {
-    constexpr int ND = MODE == 0 ? 3 : 1;
-    constexpr int NC = MODE == 0 ? 20 : 3;
     return (size_t)tg.T[0] * tg.T[1] * tg.T[2] * sizeof(double) +
-           kOwnerChunk * (3 * kOrder * (ND + 1) + NC) * sizeof(R);
+           kOwnerChunk * (owner_weights<MODE>() + owner_source<MODE>()) * sizeof(R);
 }
 bool spread_by_owner(const TileGeom& tg) {
     for (int k = 0; k < 3; k++)
         if (tg.T[k] < 8) return false;
-    return owner_lds<double, 0>(tg) + kOwnerChunk * 3 * sizeof(int) <= 65536;  // (T <= 13: three bytes hold a start)
+    return (size_t)tg.T[0] * tg.T[1] * tg.T[2] <= 2208;  // 64 KB with the weights (and T <= 34: a byte holds a start)
 }
 template <class R>
 void launch_spread_fixed_owner(hipStream_t s, const R4<R>* pos, const R* lab, PmeGeom<R> g, TileGeom tg,
