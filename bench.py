@@ -202,7 +202,7 @@ def run(args):
 
     km = make(args.precision)
     # live HIP events on the dominant kernel (the real-space electrostatics,
-    # outside the solver's graph replays) over the timed evaluations
+    # with the general pairs' kernel in FP64) over the timed evaluations
     km.setProfileFamilies(["electrostatic_pairs"])
     ms_step, energy = timed_rate(km, args.steps, args.warmup)
     live_ms, live_n = km.profile(reset=True)["electrostatic_pairs"]
@@ -310,7 +310,7 @@ def run(args):
     e_ach = e_flops / (e_avg * 1e-3) / 1e12
     roof = {"bound": "valu", "achieved": e_ach, "peak": e_peak, "unit": "TFLOP/s", "frac": e_ach / e_peak,
             "traffic": traffic.get("electrostatic_pairs"), "kernel": "k_electrostatics_" +
-            ("f32" if mixed else "f64"), "avg_launch_ms": e_avg, "launches_timed": live_n,
+            ("f32" if mixed else "f64, k_general_pairs"), "avg_launch_ms": e_avg, "launches_timed": live_n,
             "flops_per_launch": e_flops,
             "note": "vector ALU arithmetic, no matrix instructions; peak is MI355X's published dense FP32/FP64 "
                     "rate; traffic in bytes per launch" +
@@ -421,7 +421,7 @@ def batch_leg(args):
     del systems
     print(f"[bench] batch: {len(ev)} systems, {atoms} atoms, generated in {gen_s:.1f} s, contexts in {init_s:.1f} s",
           file=sys.stderr, flush=True)
-    ev.execute()  # first evaluation builds lists and solver graphs
+    ev.execute()  # first evaluation builds the lists
     reps = max(1, args.batch_reps)
     t = time.perf_counter()
     for _ in range(reps):

@@ -840,7 +840,7 @@ __global__ __launch_bounds__(kTile) void k_final_atoms(int n, int nb, int mutual
 // with the moments eps sum mf.phidp (phidp: the potential of the induced
 // dipoles), so dE/dm_k = eps c_k (phi + phidp) at the index of component k.
 // Self terms: the derivatives of calculatePmeSelfEnergy's expression
-// (MPIDReferenceForce.cpp:4283-4318, as in k_recip_atoms) with the dipole-
+// (MPIDReferenceForce.cpp:4283-4318, as in recip_atom) with the dipole-
 // induced dipole product counted twice, as -mu.E_self carries it at fixed
 // induced dipoles.
 template <class R>

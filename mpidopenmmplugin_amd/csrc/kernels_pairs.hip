@@ -6,8 +6,8 @@
 // come within the cutoff; the neighbour-list build leaves, for every tile, the
 // list of its pairs within the cutoff that are not covalent partners, sorted
 // into three classes (two bare charges, general, one bare charge; TileList).
-// One workgroup (four wavefronts) owns one tile and walks each class in chunks
-// of 64 entries, one chunk per wavefront.  Every thread thus works on a pair
+// One workgroup (four wavefronts) owns a tile, or two of one block row, and its
+// wavefronts take chunks of 64 entries of a class.  Every thread works on a pair
 // inside the cutoff, whatever the tile's fill, and each class runs its own
 // formula without divergence.  Both sides accumulate in LDS (atomic adds) and
 // are flushed to the fixed-point global accumulators once per tile.
@@ -627,15 +627,15 @@ void k_electrostatics_pot(TileList T, const unsigned long long* __restrict__ bma
                           int all_general) {
     electrostatics_tiles<R, true, true>(1, T, bmask, A, mu, P, pos64, lab64, P64, force, torque, energy, pot, all_general);
 }
-// the kernel, and whether it leaves the general pairs to k_general_pairs
+// the kernel, and whether one of them leaves the general pairs to k_general_pairs
 template <class R> struct ElecKernel;
 template <> struct ElecKernel<float> {
+    static constexpr bool kSplit = false;
     static constexpr auto fn(int) { return k_electrostatics_f32; }
-    static bool split(int) { return false; }
 };
 template <> struct ElecKernel<double> {
+    static constexpr bool kSplit = true;  // above kSmallTiles
     static constexpr auto fn(int tiles) { return tiles > kSmallTiles ? k_electrostatics_f64 : k_electrostatics_f64_small; }
-    static bool split(int tiles) { return tiles > kSmallTiles; }
 };
 
 // ---------------------------------------------------------------------------
@@ -747,7 +747,8 @@ void launch_electrostatics_pairs(hipStream_t s, int n, int maxtiles, int group, 
     hipLaunchKernelGGL(ElecKernel<R>::fn(maxtiles), dim3(group == 1 ? maxtiles : tile_groups(maxtiles, n, group)),
                        dim3(TileShape<R, false>::kThreads), 0, s, group, t, bmask, a, mu, p, pos64, lab64, p64, force,
                        torque, energy);
-    if (ElecKernel<R>::split(maxtiles)) {
+    if constexpr (ElecKernel<R>::kSplit) {
+        if (maxtiles <= kSmallTiles) return;
         // about 512 workgroups (two per CU), at most 32 per block row: at 192 blocks
         // 2 per row take 49 us, 4 59 us and 8 90 us (shorter queues, emptier last
         // chunks)

@@ -275,7 +275,7 @@ struct mpid_context {
     DBuf<int> tpstart;  // the same over the polarisable atoms (indices into pol_idx)
     // 64-atom blocks: bounding boxes, block rows (CSR: for each block I the
     // blocks J within the cutoff, with their owner I), per-atom neighbour lists
-    // of capacity nl_cap, and the tile masks of the row entries with J >= I
+    // of capacity nl_cap, and the pair lists of the row entries with J >= I
     DBuf<float4> bmin, bmax;
     DBuf<int> brow_work, brow_start, brows, brow_owner, nbr, ncount, nl_scalars;
     DBuf<int4> tile_act;  // the electrostatics kernels' tiles (TileList; row entries with J >= I)
@@ -893,7 +893,7 @@ struct mpid_context {
             launch_sorted_atoms(stream, n, dbox, d_pos, in, out);
         });
         check_launch();
-        // Block rows, neighbour lists and tile masks.  The FP64 reciprocal
+        // Block rows, neighbour and pair lists.  The FP64 reciprocal
         // cycle of the permanent multipoles is issued first (to rstream).
         // After a verified build for the current parameters the row count is
         // not waited for: the row kernels run over the capacity and stop at
