@@ -334,10 +334,14 @@ __global__ __launch_bounds__(W * kTile) void k_nl_masks(int n, const int* __rest
     __syncthreads();
     // the tile's entry in the electrostatics kernels' work list: the row
     // entries J >= I of row I are its last upper[I] entries, placed at
-    // ustart[I] (the exclusive scan of upper) in the same order
+    // ustart[I] (the exclusive scan of upper) in the same order.  When the rows
+    // exceed their capacity, the stored ones can hold more such entries than
+    // the tile list: those have no tile, but their masks and the mirrored ones
+    // are written all the same, since k_nl_fill reads the mask of every stored
+    // row entry (the host then builds again).
     const int u = ustart[I + 1] - (rstart[I + 1] - r);
-    if (u >= tcap) return;  // uniform: only when the rows exceeded their capacity (the host then builds again)
-    unsigned short* list = plist + (size_t)u * kTilePairs;
+    const bool tile = u < tcap;  // uniform
+    unsigned short* list = plist + (size_t)(tile ? u : 0) * kTilePairs;
     const unsigned long long below = (1ull << lane) - 1ull;
     const bool mine = ((ibare >> lane) & 1ull) != 0;  // this lane's atom of I is a bare charge
     const unsigned long long part = W == 4 ? cmask & (0x1111111111111111ull << wave) : cmask;
@@ -391,7 +395,7 @@ __global__ __launch_bounds__(W * kTile) void k_nl_masks(int n, const int* __rest
     const unsigned long long own = (mine ? ibare : ~ibare) & below;  // this lane's class, the atoms before it
     // the entry without its atom of J, for a bare one and for another one there
     const int ent = lane << 8, ent_bare = ent, ent_other = mine ? ent | 0x8000 : ent;
-    for (unsigned long long cm = part; cm; cm &= cm - 1ull) {
+    for (unsigned long long cm = tile ? part : 0ull; cm; cm &= cm - 1ull) {
         const int jj = __ffsll((long long)cm) - 1;  // uniform
         const unsigned lo = __builtin_amdgcn_readlane((unsigned)pairs, jj);
         const unsigned hi = __builtin_amdgcn_readlane((unsigned)(pairs >> 32), jj);
@@ -407,7 +411,7 @@ __global__ __launch_bounds__(W * kTile) void k_nl_masks(int n, const int* __rest
 #pragma unroll
     for (int w = 0; w < W; w++) m |= sm[w][lane];
     nmask[(size_t)r * kTile + lane] = m;
-    if (lane == 0) {
+    if (tile && lane == 0) {
         act[u] = make_int4(ncc | ((nup - ncc) << 16), I, J, none);
         if (group > 1) {
             const int u0 = ustart[I], u1 = ustart[I + 1], slot = u0 / group + I, k = u - u0;
