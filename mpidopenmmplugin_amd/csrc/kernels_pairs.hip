@@ -414,16 +414,26 @@ __device__ __forceinline__ void electrostatics_tiles(int tiles, const TileList& 
 // the lanes of this class, the one with by far the longest formula, were 40%
 // full, and in FP64 its registers (308) held the tile kernel to one wavefront
 // per SIMD; here the chunks are full to the last one of a row, and the tile
-// kernel needs 132.  Block I's side accumulates in LDS over the row; the other
-// side goes to the fixed-point accumulators, through LDS so that three lanes
-// hold a site's three consecutive words: the adds are taken by the memory side
-// in 64-byte pieces, and one component per instruction, 64 pieces each, made
-// this kernel 2-3 times slower (540 against 365 us in FP64 at 98,304 atoms).
+// kernel needs 132.
+//
+// Both sides accumulate in LDS in FP64: block I's over the row, and those of the
+// tiles' blocks J over a pass, in one slot per site that is not a bare charge
+// (kGenSlots hold the 21 of 64 of 72 water tiles, or 24 tiles of general
+// sites).  One workgroup per CU is what the registers leave, so its LDS is
+// free.  A slot goes to the fixed-point accumulators once per tile.  (Adding
+// every pair's J side there truncated each of them to 2^-32, and six adds a
+// pair bound the kernel wherever tiles are dense.)  Three lanes hold a site's
+// three consecutive words: the memory side takes adds in 64-byte pieces, and
+// one component per instruction was 2-3 times slower.
 // splits: workgroups per block row, so that small systems fill the chip.
-// At 98,304 atoms in FP64: 260 us here and 440 in the tile kernel, where one
-// kernel for all pairs took 1,870.  The adds of the other side bound it.
+// FP64, with every pair's J side added to the fixed-point accumulators in
+// brackets: 98,304 atoms of water 258 us (303) beside 500 in the tile kernel,
+// where one kernel for all pairs took 1,870; 64,000 general sites 565 us of
+// electrostatics (747), 3,000 without a cutoff 715 (1,615).
 constexpr int kGenTiles = 64;             // tiles ranked per pass
 constexpr int kGenQueue = kTilePairs;     // queue entries: at least one tile's most
+constexpr int kGenSlots = 1536;           // sites of the pass's blocks J, a multiple of 32
+constexpr int kGenPitch = kGenSlots + 21;  // a flush reads components of 21 slots: 63 different places
 template <class R>
 __global__ __launch_bounds__(kElecThreads) void k_general_pairs(int splits, TileList T, const int* __restrict__ ustart,
                                                                 const unsigned long long* __restrict__ bmask,
@@ -434,17 +444,19 @@ __global__ __launch_bounds__(kElecThreads) void k_general_pairs(int splits, Tile
     constexpr int kV = 16 / (int)sizeof(R);  // reals per 16-byte vector
     constexpr int kWaves = kElecThreads / kTile;
     typedef R vec __attribute__((ext_vector_type(kV)));
-    __shared__ unsigned queue[kGenQueue];  // atom of I << 12 | tile of the pass << 6 | atom of J
-    __shared__ int sfirst[kGenTiles], soff[kGenTiles + 1], sfit, sJ[kGenTiles];
+    __shared__ unsigned queue[kGenQueue];  // slot of J's site << 6 | atom of I
+    __shared__ int sfirst[kGenTiles], soff[kGenTiles + 1], sslot[kGenTiles + 1], sfit, sJ[kGenTiles];
+    __shared__ unsigned long long sgen[kGenTiles];  // the sites of J that are not bare charges
     static_assert(kGenTiles == kTile, "a pass's tiles are ranked by one wavefront");
+    static_assert(kGenSlots >= kTile && kGenQueue >= kTilePairs, "a pass takes at least one tile");
+    __shared__ double accj[6][kGenPitch];
+    __shared__ int satom[kGenSlots];
     __shared__ double acc[6][kTile];
     __shared__ R4<R> spos[kTile];
     __shared__ __align__(16) R smp[kTile * kMP];
     __shared__ R smu[kTile * 3];
     __shared__ int san[kTile];
     __shared__ double sen[kWaves];
-    __shared__ double sother[kWaves][3 * kTile];
-    __shared__ int sj[kWaves][kTile];
     if (*T.nact == 0) return;
     const int n = P.n;
     const int tid = threadIdx.x, lane = tid & (kTile - 1), wave = tid / kTile;
@@ -468,6 +480,7 @@ __global__ __launch_bounds__(kElecThreads) void k_general_pairs(int splits, Tile
 #pragma unroll
         for (int k = 0; k < 6; k++) acc[k][lane] = 0.0;
     }
+    for (int k = tid; k < 6 * kGenPitch; k += kElecThreads) (&accj[0][0])[k] = 0.0;
     double en = 0.0;
     // as in the tile kernel: neighbours in the queue share a site, and spreading
     // them over the lanes keeps one instruction's atomic adds off a common address
@@ -477,29 +490,41 @@ __global__ __launch_bounds__(kElecThreads) void k_general_pairs(int splits, Tile
         if (wave == 0) {
             const int4 t = T.act[u0 + (b0 + min(lane, nt - 1)) * splits];
             int c = lane < nt ? t.x >> 16 : 0;
+            const unsigned long long gen = c > 0 ? ~bmask[t.z] : 0ull;  // (atoms past the last have slots, no pairs)
+            int sl = __popcll(gen);
             sfirst[lane] = t.x & 0xffff;
             sJ[lane] = t.z;
+            sgen[lane] = gen;
 #pragma unroll
             for (int off = 1; off < kTile; off <<= 1) {
-                const int v = __shfl_up(c, off);
-                if (lane >= off) c += v;
+                const int v = __shfl_up(c, off), w = __shfl_up(sl, off);
+                if (lane >= off) {
+                    c += v;
+                    sl += w;
+                }
             }
             soff[lane + 1] = c;
-            const int fit = __popcll(__ballot(lane < nt && c <= kGenQueue));  // tiles of this pass (at least one)
+            sslot[lane + 1] = sl;
+            // tiles of this pass (at least one)
+            const int fit = __popcll(__ballot(lane < nt && c <= kGenQueue && sl <= kGenSlots));
             if (lane == 0) {
-                soff[0] = 0;
+                soff[0] = sslot[0] = 0;
                 sfit = fit;
             }
         }
         __syncthreads();
-        const int fit = sfit, total = soff[fit];
-        // the tiles' general entries, 16 lanes per tile
+        const int fit = sfit, total = soff[fit], nslots = sslot[fit];
+        // the tiles' general entries and sites, 16 lanes per tile
         for (int k = tid >> 4; k < fit; k += kElecThreads >> 4) {
             const unsigned short* list = T.list + (size_t)(u0 + (b0 + k) * splits) * kTilePairs + sfirst[k];
-            const int o = soff[k], c = soff[k + 1] - o;
+            const int o = soff[k], c = soff[k + 1] - o, so = sslot[k], a0 = sJ[k] * kTile;
+            const unsigned long long gen = sgen[k];
+            for (int a = tid & 15; a < kTile; a += 16)
+                if ((gen >> a) & 1ull) satom[so + __popcll(gen & ((1ull << a) - 1ull))] = a0 + a;
             for (int e = tid & 15; e < c; e += 16) {
                 const unsigned ent = list[e];
-                queue[o + e] = ((ent >> 8) << 12) | (unsigned)(k << 6) | (ent & 63u);
+                const int slot = so + __popcll(gen & ((1ull << (ent & 63u)) - 1ull));
+                queue[o + e] = ((unsigned)slot << 6) | (ent >> 8);
             }
         }
         __syncthreads();
@@ -507,8 +532,8 @@ __global__ __launch_bounds__(kElecThreads) void k_general_pairs(int splits, Tile
             const int q = q0 + perm;
             const bool qv = q < total;
             const unsigned ent = queue[qv ? q : total - 1];
-            const int il = (int)(ent >> 12);
-            const size_t j = (size_t)sJ[(ent >> 6) & 63u] * kTile + (ent & 63u);
+            const int il = (int)(ent & 63u), slot = (int)(ent >> 6);
+            const size_t j = satom[slot];
             const R4<R> pi = spos[il], pj = A.pos[j];
             const V3<R> dr = min_image(mk(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z), P.box);
             R mi[kMP], mj[kMP];
@@ -536,33 +561,27 @@ __global__ __launch_bounds__(kElecThreads) void k_general_pairs(int splits, Tile
                 atomicAdd(&acc[3][il], (double)o.ti.x);
                 atomicAdd(&acc[4][il], (double)o.ti.y);
                 atomicAdd(&acc[5][il], (double)o.ti.z);
-            }
-            // the other side (the wavefront's own LDS: no barrier between its lanes)
-            double* so = sother[wave];
-            int* jw = sj[wave];
-            jw[lane] = qv ? (int)j : -1;
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const V3<R> v = h == 0 ? o.f : o.tj;
-                so[3 * lane] = (double)v.x;
-                so[3 * lane + 1] = (double)v.y;
-                so[3 * lane + 2] = (double)v.z;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                acc_t* dst = h == 0 ? force : torque;
-#pragma unroll
-                for (int w = 0; w < 3; w++) {
-                    const int e = w * kTile + lane, pl = e / 3, jj = jw[pl];
-                    if (jj >= 0) acc_add(&dst[3 * (size_t)jj + (e - 3 * pl)], so[e]);
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                atomicAdd(&accj[0][slot], (double)o.f.x);
+                atomicAdd(&accj[1][slot], (double)o.f.y);
+                atomicAdd(&accj[2][slot], (double)o.f.z);
+                atomicAdd(&accj[3][slot], (double)o.tj.x);
+                atomicAdd(&accj[4][slot], (double)o.tj.y);
+                atomicAdd(&accj[5][slot], (double)o.tj.z);
             }
         }
         b0 += fit;
-        __syncthreads();  // the queue is read before the next pass rewrites it
+        __syncthreads();
+        // the slots, left zero for the next pass
+        for (int e = tid; e < 3 * nslots; e += kElecThreads) {
+            const int slot = e / 3, k = e - 3 * slot;
+            const double f = accj[k][slot], t = accj[3 + k][slot];
+            accj[k][slot] = 0.0;
+            accj[3 + k][slot] = 0.0;
+            const size_t at = 3 * (size_t)satom[slot] + k;
+            if (f != 0.0) acc_add(&force[at], f);
+            if (t != 0.0) acc_add(&torque[at], t);
+        }
+        __syncthreads();  // the queue and the slots are read before the next pass rewrites them
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) en += __shfl_xor(en, off);
