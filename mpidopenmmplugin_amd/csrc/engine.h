@@ -460,13 +460,13 @@ constexpr int kOneSites = 2048;     // sites whose update fits one workgroup
 // real-space field of mu at the polarisable sites (lists and covalent partners)
 template <class R>
 void launch_list_field(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p, const R* mu,
-                       R* field);
+                       double* field);
 // Av = v - S (E_rec + E_real + selfc mu), mu = S v in place; pot: the potential
 // grid (null: none).  field: launch_list_field's, or null to add the
 // real-space field in the same kernel.  Returns the number of partial sums of
 // v.Av left in partial (if given).
 template <class R>
-int launch_operator(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const R* field, NbrList l,
+int launch_operator(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const double* field, NbrList l,
                     PairAtoms<R> a, PairParams<R> p, const R* mu, double selfc, const double* v, double* Av,
                     double* partial);
 // Check 0 of a solve: r = rhs - Ax (Ax null: x = 0), p = r, mu = S p; the
@@ -510,11 +510,11 @@ struct ExtrapOrder {
 // real-space field and gradient of mu (9 per site)
 template <class R>
 void launch_extrap_list(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p, const R* mu,
-                        R* field);
+                        double* field);
 // field null: the real-space part in the same kernel.  mu_next (by atom) must
 // not be mu.
 template <class R>
-void launch_extrap_order(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const R* field, NbrList l,
+void launch_extrap_order(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const double* field, NbrList l,
                          PairAtoms<R> a, PairParams<R> p, const R* mu, R* mu_next, FracT<double> A, double selfc,
                          const double* labpol, const ExtrapOrder& o, const double* mud);
 // S v: by atom in mu and mud, by site in at (each may be null)

@@ -92,6 +92,10 @@ __device__ __forceinline__ double operator_row(const SolverSites& st, int t, int
     return dot(pv, a);
 }
 
+// The parts of a site's field (reciprocal, listed neighbours, covalent partners)
+// are formed in R and meet in FP64: a partner's field can be far smaller than
+// the list's sum.
+//
 // Everything after the inverse transform in one kernel, 32 lanes per site:
 // the site's splines (lanes 0-2, one axis each, through LDS), the stencil's
 // points over the lanes, the neighbours over the lanes, the covalent partners.
@@ -184,21 +188,15 @@ __global__ __launch_bounds__(256) void k_operator_fused(SolverSites st, PmeGeom<
             rz += fi.z;
         }
         const V3<R> c = partner_field<R>(i, lane, kOpLanes, A, mu, P);
-        rx += c.x;
-        ry += c.y;
-        rz += c.z;
+        D3 e = mk((double)ex + (double)rx + (double)c.x, (double)ey + (double)ry + (double)c.y,
+                  (double)ez + (double)rz + (double)c.z);
 #pragma unroll
         for (int off = 1; off < kOpLanes; off <<= 1) {
-            ex += __shfl_xor(ex, off);
-            ey += __shfl_xor(ey, off);
-            ez += __shfl_xor(ez, off);
-            rx += __shfl_xor(rx, off);
-            ry += __shfl_xor(ry, off);
-            rz += __shfl_xor(rz, off);
+            e.x += __shfl_xor(e.x, off);
+            e.y += __shfl_xor(e.y, off);
+            e.z += __shfl_xor(e.z, off);
         }
-        if (tv && lane == 0)
-            acc += operator_row<R>(st, t, i, mk((double)ex + (double)rx, (double)ey + (double)ry, (double)ez + (double)rz),
-                                   mu, selfc, v, Av);
+        if (tv && lane == 0) acc += operator_row<R>(st, t, i, e, mu, selfc, v, Av);
     }
     if (partial) {
         if (lane == 0) sdot[grp] = acc;
@@ -218,7 +216,7 @@ __global__ __launch_bounds__(256) void k_operator_fused(SolverSites st, PmeGeom<
 // plane, all loads in flight).
 template <class R>
 __global__ __launch_bounds__(256) void k_list_field(SolverSites st, NbrList L, PairAtoms<R> A, PairParams<R> P,
-                                                    const R* __restrict__ mu, R* __restrict__ field) {
+                                                    const R* __restrict__ mu, double* __restrict__ field) {
     if (skipped(P.skip)) return;
     const unsigned gth = (unsigned)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     const int t = (int)(gth / kNlSplit), sub = (int)(gth % kNlSplit);
@@ -245,27 +243,22 @@ __global__ __launch_bounds__(256) void k_list_field(SolverSites st, NbrList L, P
         ez += fi.z;
     }
     const V3<R> c = partner_field<R>(i, sub, kNlSplit, A, mu, P);
-    ex += c.x;
-    ey += c.y;
-    ez += c.z;
+    D3 e = mk((double)ex + (double)c.x, (double)ey + (double)c.y, (double)ez + (double)c.z);
 #pragma unroll
     for (int off = 1; off < kNlSplit; off <<= 1) {
-        ex += __shfl_xor(ex, off);
-        ey += __shfl_xor(ey, off);
-        ez += __shfl_xor(ez, off);
+        e.x += __shfl_xor(e.x, off);
+        e.y += __shfl_xor(e.y, off);
+        e.z += __shfl_xor(e.z, off);
     }
-    if (tv && sub == 0) {
-        field[3 * (size_t)t] = ex;
-        field[3 * (size_t)t + 1] = ey;
-        field[3 * (size_t)t + 2] = ez;
-    }
+    if (tv && sub == 0) store3(field, t, e);
 }
 
 constexpr int kGatherSites = 32;  // sites per workgroup
 template <class R>
 __global__ __launch_bounds__(256) void k_operator_gather(SolverSites st, PmeGeom<R> g, const R* __restrict__ pot,
-                                                         const R* __restrict__ field, const R4<R>* __restrict__ pos,
-                                                         const R* __restrict__ mu, double selfc,
+                                                         const double* __restrict__ field,
+                                                         const R4<R>* __restrict__ pos, const R* __restrict__ mu,
+                                                         double selfc,
                                                          const double* __restrict__ v, double* __restrict__ Av,
                                                          double* __restrict__ partial) {
     if (skipped(g.skip)) return;
@@ -336,10 +329,8 @@ __global__ __launch_bounds__(256) void k_operator_gather(SolverSites st, PmeGeom
         }
         if (tv && iz == 0) {
             const V3<R> e = cart_vector(mk(s100, s010, s001), g.A);
-            const R* f = field + 3 * (size_t)t;
-            acc += operator_row<R>(st, t, i, mk((double)f[0] - (double)e.x, (double)f[1] - (double)e.y,
-                                                (double)f[2] - (double)e.z),
-                                   mu, selfc, v, Av);
+            acc += operator_row<R>(st, t, i, load3(field, t) - mk((double)e.x, (double)e.y, (double)e.z), mu, selfc, v,
+                                   Av);
         }
     }
     if (partial) {
@@ -367,7 +358,7 @@ __global__ __launch_bounds__(256) void k_operator_gather(SolverSites st, PmeGeom
 // s: field and gradient (xx yy zz xy xz yz) of the lists; q: the potential's
 // grid derivatives 100 010 001 200 020 002 110 101 011.
 template <class R>
-__device__ __forceinline__ void extrap_finish(const SolverSites& st, int t, int i, const R (&s)[9], const R (&q)[9],
+__device__ __forceinline__ void extrap_finish(const SolverSites& st, int t, int i, const double (&s)[9], const R (&q)[9],
                                               const FracT<double>& F, double selfc, const double* __restrict__ labpol,
                                               const ExtrapOrder& o, const double* __restrict__ mud, R* __restrict__ mu) {
     const D3 c1 = cart_vector(mk((double)q[0], (double)q[1], (double)q[2]), F);
@@ -399,14 +390,27 @@ __device__ __forceinline__ void extrap_finish(const SolverSites& st, int t, int 
     }
     const D3 m = o.mus_in ? load3(o.mus_in, t) : load3(mud, i);
     if (!o.mus_in) store3(o.mu0, t, m);  // mu_(0) = alpha E0, so far by atom
-    const D3 e = mk((double)s[0] - c1.x + selfc * m.x, (double)s[1] - c1.y + selfc * m.y,
-                    (double)s[2] - c1.z + selfc * m.z);
+    const D3 e = mk(s[0] - c1.x + selfc * m.x, s[1] - c1.y + selfc * m.y, s[2] - c1.z + selfc * m.z);
     store3(o.E, t, e);
 #pragma unroll
-    for (int c = 0; c < 6; c++) o.G[6 * (size_t)t + c] = (double)s[3 + c] - c2[c];
+    for (int c = 0; c < 6; c++) o.G[6 * (size_t)t + c] = s[3 + c] - c2[c];
     const D3 nx = sym_mul6(labpol + 6 * (size_t)i, e);
     store3(o.mus_out, t, nx);
     store_mu<R>(mu, i, nx);
+}
+
+// f = s, a lane's part of the listed neighbours' field and gradient, and in
+// FP64 the lane's covalent partners'
+template <class R>
+__device__ __forceinline__ void add_partners(int i, int lane, int lanes, const PairAtoms<R>& A, const R* mu,
+                                             const PairParams<R>& P, const R (&s)[9], double (&f)[9]) {
+    R g[6] = {};
+    const V3<R> c = partner_field_grad<R>(i, lane, lanes, A, mu, P, g);
+    f[0] = (double)s[0] + (double)c.x;
+    f[1] = (double)s[1] + (double)c.y;
+    f[2] = (double)s[2] + (double)c.z;
+#pragma unroll
+    for (int k = 0; k < 6; k++) f[3 + k] = (double)s[3 + k] + (double)g[k];
 }
 
 // As k_operator_fused: 32 lanes per site for everything after the inverse
@@ -491,24 +495,22 @@ __global__ __launch_bounds__(256) void k_extrap_fused(SolverSites st, PmeGeom<R>
         s[2] += e.z;
         induced_grad_add<R>(uj, dr, f.f2, f.f3, s + 3);
     }
-    const V3<R> c = partner_field_grad<R>(i, lane, kOpLanes, A, mu, P, s + 3);
-    s[0] += c.x;
-    s[1] += c.y;
-    s[2] += c.z;
+    double f[9];
+    add_partners<R>(i, lane, kOpLanes, A, mu, P, s, f);
 #pragma unroll
     for (int off = 1; off < kOpLanes; off <<= 1)
 #pragma unroll
         for (int k = 0; k < 9; k++) {
             q[k] += __shfl_xor(q[k], off);
-            s[k] += __shfl_xor(s[k], off);
+            f[k] += __shfl_xor(f[k], off);
         }
-    if (tv && lane == 0) extrap_finish<R>(st, t, i, s, q, F, selfc, labpol, o, mud, mu_next);
+    if (tv && lane == 0) extrap_finish<R>(st, t, i, f, q, F, selfc, labpol, o, mud, mu_next);
 }
 
 // The same in two kernels (see k_list_field and k_operator_gather)
 template <class R>
 __global__ __launch_bounds__(256) void k_extrap_list(SolverSites st, NbrList L, PairAtoms<R> A, PairParams<R> P,
-                                                     const R* __restrict__ mu, R* __restrict__ field) {
+                                                     const R* __restrict__ mu, double* __restrict__ field) {
     const unsigned gth = (unsigned)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     const int t0 = (int)(gth / kNlSplit), sub = (int)(gth % kNlSplit);
     const bool tv = t0 < st.npol;
@@ -534,22 +536,20 @@ __global__ __launch_bounds__(256) void k_extrap_list(SolverSites st, NbrList L, 
         s[2] += e.z;
         induced_grad_add<R>(uj, dr, f.f2, f.f3, s + 3);
     }
-    const V3<R> c = partner_field_grad<R>(i, sub, kNlSplit, A, mu, P, s + 3);
-    s[0] += c.x;
-    s[1] += c.y;
-    s[2] += c.z;
+    double f[9];
+    add_partners<R>(i, sub, kNlSplit, A, mu, P, s, f);
 #pragma unroll
     for (int off = 1; off < kNlSplit; off <<= 1)
 #pragma unroll
-        for (int k = 0; k < 9; k++) s[k] += __shfl_xor(s[k], off);
+        for (int k = 0; k < 9; k++) f[k] += __shfl_xor(f[k], off);
     if (tv && sub == 0)
 #pragma unroll
-        for (int k = 0; k < 9; k++) field[9 * (size_t)t + k] = s[k];
+        for (int k = 0; k < 9; k++) field[9 * (size_t)t + k] = f[k];
 }
 template <class R>
 __global__ __launch_bounds__(256) void k_extrap_gather(SolverSites st, PmeGeom<R> g, const R* __restrict__ pot,
-                                                       const R* __restrict__ field, const R4<R>* __restrict__ pos,
-                                                       FracT<double> F, double selfc,
+                                                       const double* __restrict__ field,
+                                                       const R4<R>* __restrict__ pos, FracT<double> F, double selfc,
                                                        const double* __restrict__ labpol, ExtrapOrder o,
                                                        const double* __restrict__ mud, R* __restrict__ mu_next) {
     const int gt = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
@@ -620,7 +620,7 @@ __global__ __launch_bounds__(256) void k_extrap_gather(SolverSites st, PmeGeom<R
             for (int k = 0; k < 9; k++) q[k] += __shfl_xor(q[k], off);
     }
     if (tv && iz == 0) {
-        R s[9];
+        double s[9];
 #pragma unroll
         for (int k = 0; k < 9; k++) s[k] = field[9 * (size_t)t + k];
         extrap_finish<R>(st, t, i, s, q, F, selfc, labpol, o, mud, mu_next);
@@ -963,13 +963,13 @@ static int site_blocks(int npol) { return std::max(1, std::min((npol + 255) / 25
 
 template <class R>
 void launch_list_field(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p, const R* mu,
-                       R* field) {
+                       double* field) {
     if (st.npol <= 0) return;
     const unsigned blocks = ((unsigned)st.npol * kNlSplit + 255) / 256;
     hipLaunchKernelGGL(k_list_field<R>, dim3(blocks), dim3(256), 0, s, st, l, a, p, mu, field);
 }
 template <class R>
-int launch_operator(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const R* field, NbrList l,
+int launch_operator(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const double* field, NbrList l,
                     PairAtoms<R> a, PairParams<R> p, const R* mu, double selfc, const double* v, double* Av,
                     double* partial) {
     if (st.npol <= 0) return 0;
@@ -1046,13 +1046,13 @@ void launch_final_start(hipStream_t s, SolverSites st, const double* v, const Ex
 }
 template <class R>
 void launch_extrap_list(hipStream_t s, SolverSites st, NbrList l, PairAtoms<R> a, PairParams<R> p, const R* mu,
-                        R* field) {
+                        double* field) {
     if (st.npol <= 0) return;
     const unsigned blocks = ((unsigned)st.npol * kNlSplit + 255) / 256;
     hipLaunchKernelGGL(k_extrap_list<R>, dim3(blocks), dim3(256), 0, s, st, l, a, p, mu, field);
 }
 template <class R>
-void launch_extrap_order(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const R* field, NbrList l,
+void launch_extrap_order(hipStream_t s, SolverSites st, PmeGeom<R> g, const R* pot, const double* field, NbrList l,
                          PairAtoms<R> a, PairParams<R> p, const R* mu, R* mu_next, FracT<double> A, double selfc,
                          const double* labpol, const ExtrapOrder& o, const double* mud) {
     if (st.npol <= 0) return;
@@ -1073,8 +1073,8 @@ void launch_residual(hipStream_t s, SolverSites st, const double* b, const doubl
 
 #define MPID_INSTANTIATE(R)                                                                                         \
     template void launch_list_field<R>(hipStream_t, SolverSites, NbrList, PairAtoms<R>, PairParams<R>, const R*,    \
-                                       R*);                                                                        \
-    template int launch_operator<R>(hipStream_t, SolverSites, PmeGeom<R>, const R*, const R*, NbrList,              \
+                                       double*);                                                                   \
+    template int launch_operator<R>(hipStream_t, SolverSites, PmeGeom<R>, const R*, const double*, NbrList,         \
                                     PairAtoms<R>, PairParams<R>, const R*, double, const double*, double*,          \
                                     double*);                                                                      \
     template void launch_cg_start<R>(hipStream_t, SolverSites, const double*, const double*, double*, double*,      \
@@ -1090,8 +1090,8 @@ void launch_residual(hipStream_t s, SolverSites st, const double* b, const doubl
     template void launch_final_start<R>(hipStream_t, SolverSites, const double*, const ExtrapCoefficients&,         \
                                         const double*, R*, double*, acc_t*, size_t);                               \
     template void launch_extrap_list<R>(hipStream_t, SolverSites, NbrList, PairAtoms<R>, PairParams<R>, const R*,   \
-                                        R*);                                                                       \
-    template void launch_extrap_order<R>(hipStream_t, SolverSites, PmeGeom<R>, const R*, const R*, NbrList,         \
+                                        double*);                                                                  \
+    template void launch_extrap_order<R>(hipStream_t, SolverSites, PmeGeom<R>, const R*, const double*, NbrList,    \
                                          PairAtoms<R>, PairParams<R>, const R*, R*, FracT<double>, double,          \
                                          const double*, const ExtrapOrder&, const double*);                        \
     template void launch_apply_S<R>(hipStream_t, SolverSites, const double*, R*, double*, double*);

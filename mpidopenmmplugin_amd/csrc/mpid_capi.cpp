@@ -161,7 +161,7 @@ template <class R> struct Prec {
     DBuf<R> mu;       // induced dipoles in this precision (matvec input)
     DBuf<R> mu_next;  // Extrapolated polarization: the next order's
     DBuf<R> erec;     // reciprocal induced field (inspection entry point)
-    DBuf<R> elist;    // real-space induced field at the polarisable sites
+    DBuf<double> elist;  // real-space induced field (and gradient) at the polarisable sites
     DBuf<R> phi, phidp;
     DBuf<R> grid;       // real charge grid [n0][n1][n2]; left zero between cycles unless owned cores write it whole
     DBuf<R> pot;        // potential grid (the charge grid itself when owned cores write that whole)
