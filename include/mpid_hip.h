@@ -132,12 +132,17 @@ typedef struct {
  * families' times can overlap).  MPID_PROF_FFT covers the whole reciprocal
  * convolution (the influence function is applied inside the FFT passes), so
  * MPID_PROF_CONVOLVE stays zero.  MPID_PROF_ELECTROSTATIC_PAIRS times the
- * one real-space electrostatics kernel alone. */
+ * real-space electrostatics alone: one kernel, and in FP64 beyond 256 block
+ * pairs the general pairs' kernel after it.  The scaled covalent pairs' share
+ * of the permanent and induced fields is part of the kernels that form these
+ * (FIXED_PAIRS, INDUCED_PAIRS).  Up to 8,192 polarisable sites one kernel
+ * gathers the reciprocal field and adds the real-space one: INDUCED_PAIRS. */
 enum {
     MPID_PROF_SORT = 0, MPID_PROF_ROTATE, MPID_PROF_TILES, MPID_PROF_SPREAD, MPID_PROF_FFT, MPID_PROF_CONVOLVE,
     MPID_PROF_GATHER, MPID_PROF_FIXED_PAIRS, MPID_PROF_INDUCED_PAIRS, MPID_PROF_ELECTROSTATIC_PAIRS,
     MPID_PROF_RECIP_ATOMS, MPID_PROF_SOLVER, MPID_PROF_OTHER,
-    MPID_PROF_COVALENT_PAIRS, /* the scaled covalent pairs (FP64 permanent field and electrostatics) */
+    MPID_PROF_COVALENT_PAIRS, /* the scaled covalent pairs' FP64 electrostatics: a dispatch of their own while this
+                                 family is timed, part of RECIP_ATOMS' otherwise */
     MPID_PROF_REFINEMENT,     /* mixed precision: the FP64 operator applications of the refinement */
     MPID_PROF_COUNT
 };

@@ -249,12 +249,13 @@ struct ExtrapResponse {
     const double* E;
     const double* G;
 };
-// reciprocal-space energy, forces and torques, self terms (per atom), and
-// (cov) the covalent pairs' electrostatics and the response forces; energy:
-// 2 kEnergySlots words
+// The per-atom terms of the final pass; energy: 2 kEnergySlots words.  parts:
+// reciprocal-space energy, forces and torques, self terms and the response
+// forces, the covalent pairs' electrostatics, or both
+constexpr int kFinalRecip = 1, kFinalCov = 2;
 template <class R>
 void launch_final_atoms(hipStream_t s, int n, int mutual, const double* phi, const R* phidp, const double* mu,
-                        FracT<double> A, double alpha, PairAtoms<double> c, PairParams<double> p, bool cov,
+                        FracT<double> A, double alpha, PairAtoms<double> c, PairParams<double> p, int parts,
                         const ExtrapResponse& x, acc_t* force, acc_t* torque, acc_t* energy);
 
 // ---- PME (kernels_pme.hip) ----------------------------------------------------

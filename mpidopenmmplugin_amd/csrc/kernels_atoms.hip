@@ -802,23 +802,26 @@ __device__ __forceinline__ void extrap_response(const ExtrapResponse& x, int t, 
     }
 }
 
-// The per-atom terms of the final pass, one dispatch: workgroups [0, nb) take
-// the reciprocal and self terms of 64 atoms each (their energy to the second
-// kEnergySlots words), workgroups [nb, 2 nb) the covalent pairs (to the first),
-// workgroups beyond the response terms of Extrapolated polarization.
+// The per-atom terms of the final pass, one dispatch: nb workgroups take the
+// reciprocal and self terms of 64 atoms each (their energy to the second
+// kEnergySlots words), the next xb the response terms of Extrapolated
+// polarization, and nb the covalent pairs (to the first kEnergySlots words).
+// first: the dispatch's first workgroup in that order.
 template <class R, bool COV>
-__global__ __launch_bounds__(kTile) void k_final_atoms(int n, int nb, int mutual, const double* __restrict__ phi,
+__global__ __launch_bounds__(kTile) void k_final_atoms(int n, int nb, int xb, int first, int mutual,
+                                                       const double* __restrict__ phi,
                                                        const R* __restrict__ phidp, const double* __restrict__ mu,
                                                        FracT<double> A, double alpha, PairAtoms<double> C,
                                                        PairParams<double> P, ExtrapResponse X, acc_t* force,
                                                        acc_t* torque, acc_t* energy) {
-    if (COV && (int)blockIdx.x >= 2 * nb) {
-        const int t = (blockIdx.x - 2 * nb) * kTile + threadIdx.x;
+    const int b = blockIdx.x + first;
+    if (COV && b >= nb && b < nb + xb) {
+        const int t = (b - nb) * kTile + threadIdx.x;
         if (t < X.npol) extrap_response(X, t, C.aniso, force, torque);
         return;
     }
-    const bool cov = COV && (int)blockIdx.x >= nb;
-    const int block = cov ? blockIdx.x - nb : blockIdx.x;
+    const bool cov = COV && b >= nb;
+    const int block = cov ? b - nb - xb : b;
     const int s = block * kTile + threadIdx.x;
     double en = 0.0;
     if (s < n)
@@ -1351,15 +1354,17 @@ void launch_sub(hipStream_t s, int m, const double* a, const double* b_, double*
 }
 template <class R>
 void launch_final_atoms(hipStream_t s, int n, int mutual, const double* phi, const R* phidp, const double* mu,
-                        FracT<double> A, double alpha, PairAtoms<double> c, PairParams<double> p, bool cov,
+                        FracT<double> A, double alpha, PairAtoms<double> c, PairParams<double> p, int parts,
                         const ExtrapResponse& x, acc_t* force, acc_t* torque, acc_t* energy) {
-    const int nb = (n + kTile - 1) / kTile;
-    if (cov)
-        hipLaunchKernelGGL((k_final_atoms<R, true>), dim3(2 * nb + (x.npol + kTile - 1) / kTile), dim3(kTile), 0, s, n,
-                           nb, mutual, phi, phidp, mu, A, alpha, c, p, x, force, torque, energy);
-    else
-        hipLaunchKernelGGL((k_final_atoms<R, false>), dim3(nb), dim3(kTile), 0, s, n, nb, mutual, phi, phidp, mu, A,
-                           alpha, c, p, x, force, torque, energy);
+    const int nb = (n + kTile - 1) / kTile, xb = (x.npol + kTile - 1) / kTile;
+    if ((parts & kFinalCov) || xb > 0) {
+        const int first = (parts & kFinalRecip) ? 0 : nb + xb, last = (parts & kFinalCov) ? 2 * nb + xb : nb + xb;
+        hipLaunchKernelGGL((k_final_atoms<R, true>), dim3(last - first), dim3(kTile), 0, s, n, nb, xb, first, mutual,
+                           phi, phidp, mu, A, alpha, c, p, x, force, torque, energy);
+    } else {
+        hipLaunchKernelGGL((k_final_atoms<R, false>), dim3(nb), dim3(kTile), 0, s, n, nb, xb, 0, mutual, phi, phidp,
+                           mu, A, alpha, c, p, x, force, torque, energy);
+    }
 }
 
 #define MPID_INSTANTIATE(R)                                                                                         \
@@ -1367,7 +1372,7 @@ void launch_final_atoms(hipStream_t s, int n, int mutual, const double* phi, con
     template void launch_fixed_field_finish<R>(hipStream_t, int, const R*, const double*, const acc_t*, FracT<double>, \
                                                double, double*);                                                    \
     template void launch_final_atoms<R>(hipStream_t, int, int, const double*, const R*, const double*,              \
-                                        FracT<double>, double, PairAtoms<double>, PairParams<double>, bool,         \
+                                        FracT<double>, double, PairAtoms<double>, PairParams<double>, int,          \
                                         const ExtrapResponse&, acc_t*, acc_t*, acc_t*);                             \
     template void launch_field_sum<R>(hipStream_t, int, const acc_t*, const R*, const R*, double, double*);                    \
     template void launch_recip_potential<R>(hipStream_t, int, int, const double*, const R*, const double*,            \

@@ -1638,12 +1638,16 @@ struct mpid_context {
                                            P.mu.p, pair_params<R>(), pd.pos.p, lab.p, pair_params<double>(),
                                            force_acc(), torque_acc(), energy_acc());
         });
-        timed_on(rstream, P_RECIP, [&] {
+        auto final_atoms = [&](int parts) {
             launch_final_atoms<R>(rstream, n, opt.polarization == MPID_POLARIZATION_MUTUAL ? 1 : 0, pd.phi.p,
                                   P.phidp.p, mud.p, frac_transform<double>(), opt.ewald_alpha, pair_atoms(pd),
-                                  pair_params<double>(), true, extrap_response(), force_acc(), torque_acc(),
+                                  pair_params<double>(), parts, extrap_response(), force_acc(), torque_acc(),
                                   energy_acc());
-        });
+        };
+        // one dispatch; the covalent pairs have their own while their family is timed
+        const bool apart = (prof_mask >> P_COV) & 1u;
+        timed_on(rstream, P_RECIP, [&] { final_atoms(apart ? kFinalRecip : kFinalRecip | kFinalCov); });
+        if (apart) timed_on(rstream, P_COV, [&] { final_atoms(kFinalCov); });
         check_launch();
         final_issued = true;
     }
@@ -1814,7 +1818,7 @@ struct mpid_context {
         });
         timed_on(rstream, P_RECIP, [&] {
             launch_final_atoms<R>(rstream, n, mutual ? 1 : 0, pd.phi.p, P.phidp.p, mud.p, frac_transform<double>(),
-                                  opt.ewald_alpha, pair_atoms(pd), pair_params<double>(), false, ExtrapResponse{}, force_acc(),
+                                  opt.ewald_alpha, pair_atoms(pd), pair_params<double>(), kFinalRecip, ExtrapResponse{}, force_acc(),
                                   torque_acc(), energy_acc());
             launch_recip_potential<R>(rstream, n, pme() ? 1 : 0, pd.phi.p, P.phidp.p, lab.p, mud.p, frac_transform<double>(),
                                       opt.ewald_alpha, pot_acc.p);
