@@ -45,9 +45,11 @@ struct MpidError : std::runtime_error {
 #define HIP_CHECK(call)                                                                                         \
     do {                                                                                                        \
         hipError_t e_ = (call);                                                                                 \
-        if (e_ != hipSuccess)                                                                                   \
+        if (e_ != hipSuccess) {                                                                                 \
+            (void)hipGetLastError(); /* reported here: not to be found by the next check_launch() */            \
             throw HipError(std::string("HIP error ") + hipGetErrorString(e_) + " at " + __FILE__ + ":" +        \
                            std::to_string(__LINE__));                                                           \
+        }                                                                                                       \
     } while (0)
 
 // Owning device buffer.
@@ -872,6 +874,7 @@ struct mpid_context {
     // beside the neighbour-list build); fixed_field() joins it.
     void prepare(const double* d_pos, bool all = false, bool fixed_recip = true) {
         all_lists = all;
+        fixed_recip_rest = false;  // (an evaluation that failed may have left it)
         update_influence(pd);
         if (opt.precision == MPID_PRECISION_MIXED) update_influence(pf);
         timed(P_SORT, [&] {
@@ -933,15 +936,19 @@ struct mpid_context {
     TileList tiles() const { return TileList{tile_act.p, nl_scalars.p + 2, tile_pairs.p, tile_groups_buf.p}; }
     void grow_rows(int count) {
         if ((size_t)count <= brows.n) return;
-        const size_t cap = count + count / 4 + 64;
-        brows.resize(cap);
-        brow_owner.resize(cap);
-        tile_act.resize(cap);
+        const size_t cap = (size_t)count + count / 4 + 64;
+        // The size of brows is what the kernels and the next growth go by: it
+        // is released first and allocated last, so that an allocation that
+        // fails leaves a context without rows, not rows without masks.
+        brows.release();
         // tiles J >= I: half of the row entries and of the diagonal
         const size_t nb = (n + kTile - 1) / kTile, tcap = (cap + nb) / 2 + 1;
         tile_pairs.resize(tcap * kTilePairs);
         tile_groups_buf.resize(tcap / 2 + nb + 1);
+        tile_act.resize(cap);
         nmask.resize(cap * kTile);
+        brow_owner.resize(cap);
+        brows.resize(cap);
     }
 
     // Per-atom lists: of the polarisable atoms (by position in pol_idx) for an
