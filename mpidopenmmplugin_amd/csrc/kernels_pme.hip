@@ -774,10 +774,19 @@ template <class R, int MODE> static size_t owner_lds(const TileGeom& tg) {
     return (size_t)tg.T[0] * tg.T[1] * tg.T[2] * sizeof(double) +
            kOwnerChunk * (owner_weights<MODE>() + owner_source<MODE>()) * sizeof(R);
 }
+// LDS of an owned core at most, with the weights and sources of its chunk in
+// FP64: 2,208 points at order 6, 2,976 at order 5.  With the static arrays
+// (candidates, cells) two cores fit the 160 KB of a CU, and T is at most 46, so
+// that a byte holds a stencil's start.
+constexpr size_t kOwnerLds = 65792;
+constexpr size_t kOwnerStatic = (256 + 256 + 257 + 8 + 9 + 1) * sizeof(int);
+static_assert(2 * (kOwnerLds + kOwnerStatic) <= 163840, "two cores per CU");
+static_assert((kOwnerLds - kOwnerChunk * (owner_weights<0>() + owner_source<0>()) * sizeof(double)) / sizeof(double) / 64 +
+                      16 < 256, "a stencil's start in a byte");
 bool spread_by_owner(const TileGeom& tg) {
     for (int k = 0; k < 3; k++)
         if (tg.T[k] < 8) return false;
-    return (size_t)tg.T[0] * tg.T[1] * tg.T[2] <= 2208;  // 64 KB with the weights (and T <= 34: a byte holds a start)
+    return owner_lds<double, 0>(tg) <= kOwnerLds;
 }
 template <class R>
 void launch_spread_fixed_owner(hipStream_t s, const R4<R>* pos, const R* lab, PmeGeom<R> g, TileGeom tg,

@@ -184,7 +184,7 @@ template <class R> struct Prec {
 // ---- tilings of the PME spreading ---------------------------------------------
 // (level, mode) as mpid_options takes them: level -1 without tiles; level m
 // >= 1 cuts each axis of the grid into 2^m tiles of T_k = n_k / 2^m >= 6
-// points, spread by owned cores (T_k >= 8 and the core's LDS within 64 KiB)
+// points, spread by owned cores (T_k >= 8 and the core's LDS within kOwnerLds)
 // or by windows of T_k + 8 points folded into the grid (at most 3 windows
 // per point and axis, and the window's LDS within 64 KiB).
 enum { kSpreadUntiled = 0, kSpreadOwner = 1, kSpreadWindows = 2 };
