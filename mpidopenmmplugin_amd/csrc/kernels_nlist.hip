@@ -258,6 +258,9 @@ __global__ __launch_bounds__(1024) void k_block_rows_one(int nb, const float4* _
 // four wavefronts shorten it where there are few tiles (81 atoms: 18 us with
 // one, 9 with four), and repeat the setup and the scan where there are many
 // (98,304 atoms: 160 us with one, 349 with four; 12,288 atoms are even).
+// Evaluations with direct polarization, four and one: 1,111 tiles 215 and 221 us,
+// 3,292 268 and 274, 9,892 335 both, 17,000 442 and 419.  (The line is taken on the
+// row entries launched: the capacity while the count of the build is pending.)
 constexpr int kOneWaveRows = 16384;  // row entries (twice the tiles)
 template <int W>
 __global__ __launch_bounds__(W * kTile) void k_nl_masks(int n, const int* __restrict__ rstart, const int* __restrict__ rows,

@@ -19,7 +19,7 @@
 
 namespace mpid {
 
-constexpr int kElecThreads = 256;  // four wavefronts share one tile
+constexpr int kElecThreads = 256;  // four wavefronts share one workgroup's tiles
 
 // kPot (the energy gradients): also the potential vectors dE/dm of every
 // pair (20 stored lab components per atom, induced dipoles fixed) into pot;
@@ -45,7 +45,6 @@ constexpr int kElecThreads = 256;  // four wavefronts share one tile
 typedef int per_tile __attribute__((ext_vector_type(4)));  // (in registers, where the compiler kept arrays in memory)
 template <class R, bool kPot> struct TileShape {
     static constexpr int kM = kPot ? 1 : sizeof(R) == 4 ? 2 : 1;  // tiles per workgroup
-    static constexpr int kThreads = 256;
 };
 template <class R, bool kPot, bool kGen>
 __device__ __forceinline__ void electrostatics_tiles(int tiles, const TileList& T,
@@ -56,7 +55,7 @@ __device__ __forceinline__ void electrostatics_tiles(int tiles, const TileList& 
                                                      acc_t* __restrict__ force, acc_t* __restrict__ torque,
                                                      acc_t* __restrict__ energy, acc_t* __restrict__ pot,
                                                      int all_general) {
-    constexpr int kM = TileShape<R, kPot>::kM, kT = TileShape<R, kPot>::kThreads;
+    constexpr int kM = TileShape<R, kPot>::kM, kT = kElecThreads;
     constexpr int kWaves = kT / kTile, kSides = 1 + kM;
     // Multipole rows of 20 reals, read as 16-byte vectors: with a 20-word
     // stride, 16 lanes reading 16 different rows cover each bank once.
@@ -604,14 +603,16 @@ __global__ __launch_bounds__(kElecThreads) void k_general_pairs(int splits, Tile
 }
 
 // Where the general pairs run.  FP32: in the tile kernel, whose registers they
-// do not raise above 128 (98,304 atoms: the evaluation takes 2,280 us with the
+// do not raise above 128 (98,304 atoms: the evaluation took 2,280 us with the
 // kernel of their own, 2,195 without).  FP64: in their own kernel, except for
 // systems of at most kSmallTiles tiles, which leave CUs idle whatever the
-// registers: they are spared the dependent dispatch.
+// registers: they are spared the dependent dispatch.  Evaluations with direct
+// polarization, in the tile kernel and apart: 66 tiles 188 and 198 us, 190 193
+// and 195, 560 to 1,111 even, 3,292 317 and 286.
 constexpr int kSmallTiles = 256;
 
 // FP32: at most 128 VGPRs, so that four wavefronts fit per SIMD
-__global__ __launch_bounds__((TileShape<float, false>::kThreads)) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(kElecThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void k_electrostatics_f32(int tiles, TileList T, const unsigned long long* __restrict__ bmask, PairAtoms<float> A,
                           const float* __restrict__ mu, PairParams<float> P, const double4* __restrict__ pos64,
                           const double* __restrict__ lab64, PairParams<double> P64, acc_t* __restrict__ force,
@@ -619,7 +620,7 @@ void k_electrostatics_f32(int tiles, TileList T, const unsigned long long* __res
     electrostatics_tiles<float, false, true>(tiles, T, bmask, A, mu, P, pos64, lab64, P64, force, torque,
                                                                 energy, nullptr, 0);
 }
-__global__ __launch_bounds__((TileShape<double, false>::kThreads)) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(kElecThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void k_electrostatics_f64(int tiles, TileList T, const unsigned long long* __restrict__ bmask, PairAtoms<double> A,
                           const double* __restrict__ mu, PairParams<double> P, const double4* __restrict__ pos64,
                           const double* __restrict__ lab64, PairParams<double> P64, acc_t* __restrict__ force,
@@ -627,7 +628,7 @@ void k_electrostatics_f64(int tiles, TileList T, const unsigned long long* __res
     electrostatics_tiles<double, false, false>(tiles, T, bmask, A, mu, P, pos64, lab64, P64, force, torque,
                                                                   energy, nullptr, 0);
 }
-__global__ __launch_bounds__((TileShape<double, false>::kThreads))
+__global__ __launch_bounds__(kElecThreads)
 void k_electrostatics_f64_small(int tiles, TileList T, const unsigned long long* __restrict__ bmask,
                                 PairAtoms<double> A, const double* __restrict__ mu, PairParams<double> P,
                                 const double4* __restrict__ pos64, const double* __restrict__ lab64,
@@ -764,13 +765,17 @@ void launch_electrostatics_pairs(hipStream_t s, int n, int maxtiles, int group, 
                                  acc_t* torque, acc_t* energy) {
     if (maxtiles <= 0) return;
     hipLaunchKernelGGL(ElecKernel<R>::fn(maxtiles), dim3(group == 1 ? maxtiles : tile_groups(maxtiles, n, group)),
-                       dim3(TileShape<R, false>::kThreads), 0, s, group, t, bmask, a, mu, p, pos64, lab64, p64, force,
+                       dim3(kElecThreads), 0, s, group, t, bmask, a, mu, p, pos64, lab64, p64, force,
                        torque, energy);
     if constexpr (ElecKernel<R>::kSplit) {
         if (maxtiles <= kSmallTiles) return;
-        // about 512 workgroups (two per CU), at most 32 per block row: at 192 blocks
-        // 2 per row take 49 us, 4 59 us and 8 90 us (shorter queues, emptier last
-        // chunks)
+        // About 512 workgroups, two for each that the chip holds (the first rows
+        // have most tiles J >= I), at most 32 per block row.  Where tiles are
+        // sparse longer queues would do: evaluations of 192 blocks of water with
+        // direct polarization take 350 us with one workgroup per row, 359 with two,
+        // 372 with four and 409 with eight.  Where they are dense a row has to be
+        // cut: 3,000 general sites without a cutoff (47 blocks) take 1,230 us of
+        // electrostatics with five per row and 713 with ten.
         const int nb = (n + kTile - 1) / kTile;
         const int splits = std::max(1, std::min(32, 512 / nb));
         hipLaunchKernelGGL(k_general_pairs<R>, dim3(nb * splits), dim3(kElecThreads), 0, s, splits, t, ustart, bmask, a,

@@ -653,7 +653,8 @@ __device__ __forceinline__ void cg_publish(double* scal, double* hcheck, int c, 
 // r = rhs - Ax (Ax null: x = 0, r = rhs), p = r, mu = S p.  Else one iteration
 // from Ap and the partials of p.Ap: a = rr / p.Ap, x += a p, r -= a Ap, the
 // check, p = r + beta p and mu = S p.  More sites: the same in two kernels
-// (k_cg_step, k_cg_direction) over many workgroups.
+// (k_cg_step, k_cg_direction) over many workgroups.  Evaluations one way and the
+// other: 216 sites 0.46 and 0.50 ms, 1,000 0.52 and 0.54, 2,048 0.63 both.
 constexpr int kOneThreads = 1024, kOnePer = kOneSites / kOneThreads;
 template <class R, bool START>
 __global__ __launch_bounds__(kOneThreads) void k_cg_one(SolverSites st, const double* __restrict__ rhs,

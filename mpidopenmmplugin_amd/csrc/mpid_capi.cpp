@@ -1221,10 +1221,11 @@ struct mpid_context {
     SolverSites sites() const { return SolverSites{npol, pol_idx.p, sqrtpol.p}; }
     // Up to kFusedSites polarisable sites the operator's kernel adds the
     // real-space field itself; beyond, the list kernel runs on rstream beside
-    // the reciprocal chain.  At 4,096 sites an evaluation takes 0.91 ms this
-    // way against 1.03 ms with the two kernels and their cross-stream waits
-    // (FP64: 1.04 against 1.14 ms); at 32,768 sites the list walk (20 us in
-    // FP32) would sit on the critical path, where it now overlaps the chain.
+    // the reciprocal chain.  Evaluations one way and the other: 2,000 sites 0.64
+    // and 0.70 ms, 4,096 0.68 and 0.75 (FP64 0.73 and 0.78), 8,192 0.91 and 0.93
+    // (FP64 1.04 both; Extrapolated 0.63 and 0.61), 16,384 1.65 and 1.64 (FP64
+    // 1.92 and 1.84; Extrapolated 1.16 and 1.13): there the list walk sits on the
+    // critical path, where it overlaps the chain in a kernel of its own.
     static constexpr int kFusedSites = 8192;
 
     // Av = v - S T S v with P.mu = S v in place; returns the number of partial
