@@ -265,7 +265,10 @@ __global__ __launch_bounds__(256) void k_spread_tiled(const R4<R>* __restrict__ 
 // Every thread tests one candidate per pass; the atoms that meet the core then
 // take their spline weights in chunks of kOwnerChunk, one wavefront per axis and
 // the fourth for the source and the count of stencil rows, so that a chunk's
-// chain is one spline and not three.  A core is a chain of dependent loads and
+// chain is one spline and not three.  An atom's stencil start and its offset
+// from it are evaluated once, together: evaluated again, the compiler contracts
+// the products differently, and an atom within a rounding of a grid plane would
+// get the weights of one start at the points of the next.  A core is a chain of dependent loads and
 // short steps, and what bounds the kernel is how many cores a CU holds (LDS and
 // registers) and the length of that chain.  Induced dipoles, 98,304 atoms on
 // 128^3: FP64 73 us with one wavefront taking all three splines of 128
@@ -297,6 +300,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ?
     __shared__ int sbeg[8], soff[9], snv;
     // the atoms that meet the core: stencil start - core origin (+ 8 per byte), atom, first stencil row
     __shared__ int srel[kCand], satom[kCand], sfirst[kCand + 1];
+    __shared__ R sw[3][kCand];  // their offsets from the stencil start
     const int tid = threadIdx.x, lane = tid & (kTile - 1), wave = tid / kTile;
     const int t = blockIdx.x;
     const int nt = tg.tiles_per_axis;
@@ -337,11 +341,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ?
             const R px[3] = {fp.x, fp.y, fp.z};
             int rel = 0;
             bool meets = true;
+            R w[3];
 #pragma unroll
             for (int k = 0; k < 3; k++) {
                 int ig;
-                R w;
-                grid_coord(px[k], g.n[k], ig, w);
+                grid_coord(px[k], g.n[k], ig, w[k]);
                 int r = ig - w0[k];
                 if (r < -(g.n[k] >> 1)) r += g.n[k];
                 if (r >= g.n[k] - (g.n[k] >> 1)) r -= g.n[k];
@@ -352,6 +356,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ?
                 const int slot = atomicAdd(&snv, 1);
                 srel[slot] = rel;
                 satom[slot] = a;
+#pragma unroll
+                for (int k = 0; k < 3; k++) sw[k][slot] = w[k];
             }
         }
         __syncthreads();
@@ -360,12 +366,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ?
             const int la = s0 + lane;
             if (wave < 3) {
                 if (la < nv) {
-                    const R4<R> p = pos[satom[la]];
-                    const V3<R> fp = to_frac(mk(p.x, p.y, p.z), g.box);
-                    int ig;
-                    R w, th[kOrder][ND + 1];
-                    grid_coord(wave == 0 ? fp.x : wave == 1 ? fp.y : fp.z, g.n[wave], ig, w);
-                    bspline6<R, ND>(w, th);
+                    R th[kOrder][ND + 1];
+                    bspline6<R, ND>(sw[wave][la], th);
                     R* o = sth + lane * NW + wave * kOrder * (ND + 1);
 #pragma unroll
                     for (int m = 0; m < kOrder; m++)
@@ -779,7 +781,7 @@ template <class R, int MODE> static size_t owner_lds(const TileGeom& tg) {
 // (candidates, cells) two cores fit the 160 KB of a CU, and T is at most 46, so
 // that a byte holds a stencil's start.
 constexpr size_t kOwnerLds = 65792;
-constexpr size_t kOwnerStatic = (256 + 256 + 257 + 8 + 9 + 1) * sizeof(int);
+constexpr size_t kOwnerStatic = (256 + 256 + 257 + 8 + 9 + 1) * sizeof(int) + 3 * 256 * sizeof(double);
 static_assert(2 * (kOwnerLds + kOwnerStatic) <= 163840, "two cores per CU");
 static_assert((kOwnerLds - kOwnerChunk * (owner_weights<0>() + owner_source<0>()) * sizeof(double)) / sizeof(double) / 64 +
                       16 < 256, "a stencil's start in a byte");
