@@ -968,8 +968,14 @@ struct mpid_context {
         tile_group = tiles_per_group(tile_bound(), opt.precision != MPID_PRECISION_MIXED);
         for (int attempt = 0; attempt < 2; attempt++) {
             nl_cap = (nl_cap + kNlSplit - 1) / kNlSplit * kNlSplit;
-            nbr.resize((size_t)n * nl_cap);
-            pnbr.resize((size_t)n * nl_cap);
+            try {
+                nbr.resize((size_t)n * nl_cap);
+                pnbr.resize((size_t)n * nl_cap);
+            } catch (...) {
+                nl_cap = 0;  // the next build takes it from its own density
+                npol_cached = -1;
+                throw;
+            }
             timed(P_TILES, [&] {
                 if (attempt > 0) launch_fill<int>(stream, nl_scalars.p, 2, 0);
                 launch_nl_build(stream, n, rows_pending ? (int)brows.n : rows_total, (int)brows.n, all_lists,

@@ -1,11 +1,13 @@
-"""A context whose row buffers could not be allocated can be used again.
+"""A context whose list buffers could not be allocated can be used again.
 
 720,000 charges squeezed into 1.9 nm: most of the 11,250 blocks are within the
 0.9 nm cutoff of each other, and the pair lists of their tiles would take 470 GB
-(8 KB each), more than the 288 of the card, so that the evaluation ends in an
-error before it builds a list.  The same context at an ordinary density then
-gives what a fresh one gives: the same kernels on the same inputs, 1e-9 relative
-in the energy and 1e-6 in the forces for the order of the sums on the grid.
+(8 KB each), more than the 288 of the card.  300,000 in 1.84 nm: the pair lists fit
+(80 GB), the neighbour lists of 190,000 entries an atom (230 GB) do not.  Both
+evaluations end in an error before a list is built.  The same context at an
+ordinary density then gives what a fresh one gives: the same kernels on the same
+inputs, 1e-9 relative in the energy and 1e-6 in the forces for the order of the
+sums on the grid.
 """
 import numpy as np
 import pytest
@@ -39,11 +41,12 @@ class ManyCharges(MPIDForce):
         return flat
 
 
-def test_context_after_a_failed_allocation():
-    n = 720000
-    cells = np.indices((90, 90, 90)).reshape(3, -1).T[:n]
-    pos = (cells + 0.5) * (19.0 / 90) + np.random.default_rng(7).uniform(-0.05, 0.05, size=(n, 3))
-    box = np.full(3, 19.0)
+@pytest.mark.parametrize("n,cells,squeeze", [(720000, 90, 0.1), (300000, 67, 0.13)], ids=["rows", "lists"])
+def test_context_after_a_failed_allocation(n, cells, squeeze):
+    edge = cells * (19.0 / 90)
+    sites = np.indices((cells,) * 3).reshape(3, -1).T[:n]
+    pos = (sites + 0.5) * (19.0 / 90) + np.random.default_rng(7).uniform(-0.05, 0.05, size=(n, 3))
+    box = np.full(3, edge)
     force = ManyCharges(n)
     force.setNonbondedMethod(MPIDForce.PME)
     force.setPolarizationType(MPIDForce.Direct)
@@ -53,7 +56,7 @@ def test_context_after_a_failed_allocation():
     k.initialize(n, force)
     print("[gpu] an allocation beyond the card's memory", flush=True)
     with pytest.raises(RuntimeError, match="memory"):
-        k.execute(0.1 * pos, 0.1 * box)
+        k.execute(squeeze * pos, squeeze * box)
     print("[gpu] the same context at an ordinary density", flush=True)
     e1, f1 = k.execute(pos, box)
     fresh = HipCalcMPIDForceKernel("mixed")
