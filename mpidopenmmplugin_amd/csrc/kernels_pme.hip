@@ -272,7 +272,7 @@ __global__ __launch_bounds__(256) void k_spread_tiled(const R4<R>* __restrict__ 
 // short steps, and what bounds the kernel is how many cores a CU holds (LDS and
 // registers) and the length of that chain.  Induced dipoles, 98,304 atoms on
 // 128^3: FP64 73 us with one wavefront taking all three splines of 128
-// candidates, 56 so; FP32 37 and 33; 12,288 atoms on 64^3 FP32 12 and 9.
+// candidates, 56 so; FP32 37 and 31; 12,288 atoms on 64^3 FP32 12 and 9.
 constexpr int kOwnerChunk = 64;
 // words of a slot's spline weights and source components: odd, so that lanes at
 // different slots read different LDS banks
